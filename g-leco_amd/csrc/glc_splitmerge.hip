@@ -8,28 +8,38 @@
 // parallel reductions here give the same costs -- hence the same boundaries --
 // as a sequential evaluation of the same definition.
 //
+//   blocks  the column is cut into blocks of B values (B divides m, at most
+//           128).  Per block: exact sums (prefix sums over the column, so any
+//           candidate's sums are two differences) and the vertices of the convex
+//           hull of its points (k_sm_blocks), about 11 for 128 noisy values;
 //   split   every start s = j*m (m = minimum size) is evaluated at once: the
 //           candidate sizes m*{1,2,3,4,5,7,...,17,21,25,29} (step m, then 2m
 //           above 4m, then 4m above 16m, at most 32m); the smallest cost per
-//           value wins (first on ties).  For m <= 128 a workgroup takes four
-//           starts, their values staged in LDS, their sums from exact block
-//           prefix sums of the column (k_sm_block_pfx); otherwise one start
-//           per workgroup with one pass for the sums (nested prefixes) and
-//           one for the maximum error;
+//           value wins (first on ties);
 //   chain   the greedy walk 0 -> end(0) -> end(end(0)) ... keeps the starts it
-//           reaches: pointer doubling marks them in log2(N/m) rounds;
-//   merge   up to 10 left-to-right passes.  Pass: the merged cost of every
-//           adjacent pair in parallel, then the list is walked in segments
-//           at once with a one-workgroup fix-up where the true walk enters a
-//           segment elsewhere than the segment's own walk (k_sm_seg,
-//           k_sm_fix).  While a group is a single partition its decision is
-//           the precomputed pair test, otherwise the workgroup fits the grown
-//           group on the spot (the reference's sequential semantics).
+//           reaches: pointer doubling inside chunks, one walk over the chunks;
+//   merge   up to 10 left-to-right passes.  The group that starts at a
+//           partition does not depend on how the walk got there, so every
+//           partition's group is grown at once, one wave each (k_sm_grow), and
+//           the chain keeps the groups the walk from partition 0 reaches.
+//
+// The maximum residual of a line over a range.  A cost needs only the bit
+// width of max |v_i - round(pr_i)|, pr_i = t0 + t1 * i in FP64.  Over a block the
+// real-valued residual of any line is largest at a hull vertex, so with D the
+// largest |v - pr| and H the largest |v - round(pr)| over the vertices,
+//     H <= max <= D + 0.5 + 3 eps,  eps = 2^-52 (|t0| + |t1| n)
+// (eps bounds one prediction's FP64 error; values and predictions within 2^52,
+// where every difference of two integers is exact).  Both ends have the same bit
+// width except when a power of two lies between them; then, and for blocks or
+// candidates outside the exact range, the values themselves are read.  That makes
+// one evaluation about 10 times cheaper than a pass over the values: 2^26 uint64
+// piecewise-linear values, m = 128: split 8.1 -> 1.33 ms, and growing every
+// partition's group takes 0.32 ms a pass where the sequential walk (one
+// workgroup regrowing groups across segments) took 23.4 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <cfloat>
-#include <cstdlib>
 #include <map>
 #include <mutex>
 #include <vector>
@@ -41,9 +51,11 @@ namespace glc {
 namespace {
 
 constexpr int kSmThreads = 256;
-constexpr int kPfxChunk = kSmThreads;  // block-prefix positions per chunk (k_sm_block_pfx)
+constexpr int kPfxChunk = 64;  // block-prefix positions per chunk (k_sm_blocks, k_sm_chunk_pfx)
 constexpr int kMaxCand = 14;  // m * {1,2,3,4,5,7,9,11,13,15,17,21,25,29}
 __constant__ int kCandUnits[kMaxCand] = {1, 2, 3, 4, 5, 7, 9, 11, 13, 15, 17, 21, 25, 29};
+// units of the candidates before candidate k (of one start)
+__constant__ int kCandCum[kMaxCand + 1] = {0, 1, 3, 6, 10, 15, 22, 31, 42, 55, 70, 87, 108, 133, 162};
 
 typedef __int128 i128;
 typedef unsigned __int128 u128;
@@ -129,21 +141,22 @@ template <class T> __device__ __forceinline__ int64_t abs_err(T v, double t0, do
 }
 
 // Residual magnitude in FP64 when it is exact.  For values v and rounded
-// predictions p of magnitude <= 2^50 (inside T for 32-bit types), x86_cast is
+// predictions p of magnitude <= 2^52 (inside T for 32-bit types), x86_cast is
 // the identity on p, calc_delta is v - p without wrap or saturation, and the
 // FP64 difference of two such integers is exact; so fabs(v - round(pr)) is
 // abs_err's result.  The prediction t0 + t1 * i is monotonic in i, so its two
 // end values bound a candidate's whole range.
+constexpr double kExact = 4503599627370496.0;  // 2^52
 template <class T> __device__ __forceinline__ bool small_value(T x) {
     if constexpr (sizeof(T) == 4) return true;
-    else if constexpr (std::is_signed<T>::value) return x >= -(int64_t(1) << 50) && x <= (int64_t(1) << 50);
-    else return x <= (uint64_t(1) << 50);
+    else if constexpr (std::is_signed<T>::value) return x >= -(int64_t(1) << 52) && x <= (int64_t(1) << 52);
+    else return x <= (uint64_t(1) << 52);
 }
 template <class T> __device__ __forceinline__ bool small_pred(double pr) {  // false for NaN
     if constexpr (std::is_same<T, int32_t>::value) return pr >= -2147483647.0 && pr <= 2147483646.0;
     else if constexpr (std::is_same<T, uint32_t>::value) return pr >= 0.0 && pr <= 4294967294.0;
-    else if constexpr (std::is_signed<T>::value) return pr >= -1125899906842624.0 && pr <= 1125899906842624.0;
-    else return pr >= 0.0 && pr <= 1125899906842624.0;
+    else if constexpr (std::is_signed<T>::value) return pr >= -kExact && pr <= kExact;
+    else return pr >= 0.0 && pr <= kExact;
 }
 
 __device__ __forceinline__ int32_t bits_of(int64_t mx) {
@@ -165,75 +178,66 @@ template <int NT> struct FitLdsT {
 };
 typedef FitLdsT<kSmThreads> FitLds;
 
-// Block prefix sums of the column (k_sm_block_pfx) when they exist (p1 null
-// otherwise): G1(p), G2(p) over the first min(p m, n) values.
+// Prefix sums of the column at block granularity: G1(p) = sum of y_q and
+// G2(p) = sum of q * y_q over q < min(p * B, n), for p in [0, JB].
+// G(p) = p(p) + c(p / kPfxChunk).
 struct SmPrefix {
     const i128 *p1, *p2, *c1, *c2;
-    int64_t m, n, J;
+    int64_t n, JB;
+    int32_t B;
 };
 __device__ __forceinline__ i128 pfx_at(const i128* p, const i128* c, int64_t i) {
     return p[i] + c[i / kPfxChunk];
 }
 
-// Cost of [s, e) computed by the whole workgroup (all threads call it).  The
-// sums come from the block prefixes when s is a block start and e a block
-// start or the column's end (every split/merge boundary is), otherwise from a
-// pass over the values.  The maximum residual takes the exact FP64 form for
-// values within small_value's range when both end predictions are in range.
-template <class T, int NT = kSmThreads>
-__device__ double wg_cost(const T* __restrict__ v, int64_t s, int64_t e, FitLdsT<NT>& L,
-                          const SmPrefix& pf) {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int64_t n = e - s;
-    const bool use_pfx = pf.p1 != nullptr && s % pf.m == 0 && (e == pf.n || e % pf.m == 0);
-    if (use_pfx) {
-        if (tid == 0) {
-            const int64_t ib = s / pf.m, ie = (e == pf.n) ? pf.J : e / pf.m;
-            const i128 sy = pfx_at(pf.p1, pf.c1, ie) - pfx_at(pf.p1, pf.c1, ib);
-            const i128 sxy = pfx_at(pf.p2, pf.c2, ie) - pfx_at(pf.p2, pf.c2, ib) - static_cast<i128>(s) * sy;
-            sm_theta(sy, sxy, n, L.t0, L.t1);
-            L.fast = small_pred<T>(L.t0 + L.t1 * 0.0) && small_pred<T>(L.t0 + L.t1 * static_cast<double>(n - 1));
-        }
-    } else {
-        i128 sy = 0, sxy = 0;
-        for (int64_t i = tid; i < n; i += NT) {
-            const i128 y = wide<T>(v[s + i]);
-            sy += y;
-            sxy += y * static_cast<i128>(i);
-        }
-        sy = wave_sum(sy);
-        sxy = wave_sum(sxy);
-        if (lane == 0) {
-            L.sy[w] = sy;
-            L.sxy[w] = sxy;
-        }
-        __syncthreads();
-        if (tid == 0) {
-            i128 a = 0, b = 0;
-#pragma unroll 1
-            for (int k = 0; k < NT / 64; ++k) {
-                a += L.sy[k];
-                b += L.sxy[k];
-            }
-            sm_theta(a, b, n, L.t0, L.t1);
-            L.fast = small_pred<T>(L.t0 + L.t1 * 0.0) && small_pred<T>(L.t0 + L.t1 * static_cast<double>(n - 1));
-        }
-    }
-    __syncthreads();
-    const double t0 = L.t0, t1 = L.t1;
-    const bool fast = L.fast != 0;
+// Hull vertices of the blocks: vertex k of block b at
+// ((b / 64) * slots + k) * 64 + b % 64, so that lanes on consecutive blocks read
+// consecutive memory; y its value, x its index in the block.  nv[b]: the number of
+// vertices, or kHullScan for a block that has to be read value by value (more
+// than `slots` vertices, or a value outside small_value's range).  slots = 0: no
+// hulls, every range is read.
+constexpr int kHullSlots = 24;
+constexpr int kHullScan = 255;
+constexpr int kHullMaxB = 128;
+struct SmHull {
+    double* y;
+    uint8_t* x;
+    uint8_t* nv;
+    int32_t slots;
+};
+__device__ __forceinline__ int64_t hull_at(int32_t slots, int64_t b, int k) {
+    return ((b >> 6) * slots + k) * 64 + (b & 63);
+}
+
+// A candidate's line over [s, e) (s a block start, e one or n) from the
+// prefix sums, and whether its two end predictions are within small_pred.
+template <class T>
+__device__ __forceinline__ void range_line(const SmPrefix& pf, int64_t s, int64_t e, double& t0, double& t1,
+                                           bool& fast) {
+    const int64_t ib = s / pf.B, ie = (e == pf.n) ? pf.JB : e / pf.B;
+    const i128 sy = pfx_at(pf.p1, pf.c1, ie) - pfx_at(pf.p1, pf.c1, ib);
+    const i128 sxy = pfx_at(pf.p2, pf.c2, ie) - pfx_at(pf.p2, pf.c2, ib) - static_cast<i128>(s) * sy;
+    sm_theta(sy, sxy, e - s, t0, t1);
+    fast = small_pred<T>(t0 + t1 * 0.0) && small_pred<T>(t0 + t1 * static_cast<double>(e - s - 1));
+}
+
+// Largest residual magnitude of values x0, x0 + step, ... < n of a range at v
+// (four loads in flight; one lane's share).
+template <class T>
+__device__ __forceinline__ int64_t scan_err(const T* __restrict__ v, int64_t x0, int64_t n, int step, double t0,
+                                            double t1, bool fast) {
     int64_t mx = 0;
     double md = 0.0;
-    for (int64_t i0 = tid; i0 < n; i0 += 4 * NT) {
+    for (int64_t i0 = x0; i0 < n; i0 += 4 * step) {
         T x[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {  // four loads in flight (index clamped; the extra ones are skipped)
-            const int64_t i = i0 + k * NT;
-            x[k] = v[s + (i < n ? i : n - 1)];
+        for (int k = 0; k < 4; ++k) {  // index clamped; the extra ones are skipped
+            const int64_t i = i0 + k * step;
+            x[k] = v[i < n ? i : n - 1];
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int64_t i = i0 + k * NT;
+            const int64_t i = i0 + k * step;
             if (i >= n) break;
             if (fast && small_value<T>(x[k])) {
                 const double pr = t0 + t1 * static_cast<double>(i);  // no contraction (-ffp-contract=off)
@@ -245,8 +249,63 @@ __device__ double wg_cost(const T* __restrict__ v, int64_t s, int64_t e, FitLdsT
         }
     }
     const int64_t mdi = static_cast<int64_t>(md);
-    mx = mdi > mx ? mdi : mx;
-    mx = wave_max(mx);
+    return mdi > mx ? mdi : mx;
+}
+
+// D and H (see the top of the file) over the vertices of one block whose
+// first value has index x0 in the range.  y, x: the block's vertices, `stride`
+// apart.
+__device__ __forceinline__ void hull_err(const double* __restrict__ y, const uint8_t* __restrict__ x, int stride,
+                                         int nv, int64_t x0, double t0, double t1, double& D, double& H) {
+#pragma unroll 4
+    for (int k = 0; k < nv; ++k) {
+        const double yv = y[k * stride];
+        const double pr = t0 + t1 * static_cast<double>(x0 + x[k * stride]);  // no contraction (-ffp-contract=off)
+        D = __builtin_fmax(D, __builtin_fabs(yv - pr));
+        H = __builtin_fmax(H, __builtin_fabs(yv - round_away(pr)));
+    }
+}
+
+// The bit width that D and H (both <= 2^53 + 1) settle for a range of n
+// values, -1 if a power of two lies between the two bounds.
+__device__ __forceinline__ int32_t hull_bits(double D, double H, double t0, double t1, int64_t n) {
+    const double eps = (__builtin_fabs(t0) + __builtin_fabs(t1) * static_cast<double>(n)) * 2.220446049250313e-16;
+    const int32_t lo = bits_of(static_cast<int64_t>(H));
+    const int32_t hi = bits_of(static_cast<int64_t>(D * (1.0 + 4.44e-16) + 0.5 + 3.0 * eps));  // D is rounded itself
+    return lo == hi ? lo : -1;
+}
+
+// Cost of [s, e) by a pass for the sums and one for the maximum residual,
+// computed by the whole workgroup (all threads call it).
+template <class T, int NT = kSmThreads>
+__device__ double wg_cost(const T* __restrict__ v, int64_t s, int64_t e, FitLdsT<NT>& L) {
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int64_t n = e - s;
+    i128 sy = 0, sxy = 0;
+    for (int64_t i = tid; i < n; i += NT) {
+        const i128 y = wide<T>(v[s + i]);
+        sy += y;
+        sxy += y * static_cast<i128>(i);
+    }
+    sy = wave_sum(sy);
+    sxy = wave_sum(sxy);
+    if (lane == 0) {
+        L.sy[w] = sy;
+        L.sxy[w] = sxy;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        i128 a = 0, b = 0;
+#pragma unroll 1
+        for (int k = 0; k < NT / 64; ++k) {
+            a += L.sy[k];
+            b += L.sxy[k];
+        }
+        sm_theta(a, b, n, L.t0, L.t1);
+        L.fast = small_pred<T>(L.t0 + L.t1 * 0.0) && small_pred<T>(L.t0 + L.t1 * static_cast<double>(n - 1));
+    }
+    __syncthreads();
+    const int64_t mx = wave_max(scan_err<T>(v + s, tid, n, NT, L.t0, L.t1, L.fast != 0));
     if (lane == 0) L.mx[w] = mx;
     __syncthreads();
     if (tid == 0) {
@@ -279,7 +338,7 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split(const T* __restrict__ v
     while (K < kMaxCand && static_cast<int64_t>(kCandUnits[K]) * m <= max_size) ++K;
     if (K == 0) {  // fewer than m values left: one partition [cur, n)
         __shared__ FitLds L;
-        const double c = wg_cost<T>(v, cur, n, L, SmPrefix{nullptr, nullptr, nullptr, nullptr, m, n, J});
+        const double c = wg_cost<T>(v, cur, n, L);
         if (tid == 0) {
             best_end[j] = static_cast<int32_t>(n);
             best_cost[j] = c;
@@ -383,36 +442,252 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split(const T* __restrict__ v
     }
 }
 
-// Exact prefix sums at block granularity: for p in [0, J], G1(p) = sum of
-// y_q and G2(p) = sum of q * y_q over q < min(p * m, n) (q the column index).
-// |G2| < 2^126 for n < 2^31, so i128 holds them.  k_sm_block_pfx: one
-// workgroup per chunk of kPfxChunk positions, one thread per block sum, then
-// an exclusive scan inside the chunk (p1, p2) and the chunk totals (c1, c2);
-// k_sm_chunk_scan turns the totals into chunk offsets (exclusive).
-// G(p) = p(p) + c(p / kPfxChunk).
+// Block sums, prefixes and hulls.  One workgroup per chunk of kPfxChunk = 64
+// blocks, staged in LDS (rows of B | 1 values: 64 lanes reading the same index
+// of 64 blocks hit different banks).
+//   filter  a value is no vertex of the upper (lower) hull if the mean of its
+//           neighbours at some equal distance is not below (above) it; the
+//           survivors of distances 1, 2, 4, ..., 32 are one ballot per 64 values;
+//   hull    wave 0 walks the survivors of the upper hulls, wave 1 those of the
+//           lower ones, a block per lane: Andrew's monotone chain with the kept
+//           vertices as a 128-bit mask, cross products exact in int64
+//           (differences <= 2^53, index distances < 2^7);
+//   sums    wave 2, a block per lane, and the scan over the 64 blocks.
+// p1, p2 receive the exclusive prefix inside the chunk, c1, c2 the chunk's
+// totals (k_sm_chunk_scan turns those into chunk offsets).  A block per lane
+// with values straight from memory (one cache line per lane and step) read the
+// column at 0.55 TB/s.
+struct HullMask {
+    uint64_t lo, hi;
+    __device__ __forceinline__ int top() const {  // highest set bit, -1 if none
+        return hi ? 127 - __builtin_clzll(hi) : lo ? 63 - __builtin_clzll(lo) : -1;
+    }
+    __device__ __forceinline__ int next() const {  // lowest set bit (there is one)
+        return lo ? __builtin_ctzll(lo) : 64 + __builtin_ctzll(hi);
+    }
+    __device__ __forceinline__ void flip(int i) {
+        if (i < 64) lo ^= 1ULL << i;
+        else hi ^= 1ULL << (i - 64);
+    }
+};
+
+// One block's upper (UP) or lower hull among the points of `in`.
+template <bool UP>
+__device__ __forceinline__ HullMask hull_chain(const int64_t* __restrict__ row, HullMask in) {
+    HullMask out{0, 0};
+    int n = 0, xa = 0, xb = 0, xi = -1;
+    int64_t ya = 0, yb = 0, yi = 0;
+    for (;;) {
+        if (xi < 0) {  // the next point
+            if ((in.lo | in.hi) == 0) break;
+            xi = in.next();
+            in.flip(xi);
+            yi = row[xi];
+        }
+        const int64_t l = (ya - yb) * (xi - xa), r = (yi - ya) * (xa - xb);
+        if (n >= 2 && (UP ? l <= r : l >= r)) {  // the last vertex is not outside the chord past it
+            out.flip(xa);
+            --n;
+            xa = xb;
+            ya = yb;
+            if (n >= 2) {
+                HullMask m = out;
+                m.flip(xa);
+                xb = m.top();
+                yb = row[xb];
+            }
+        } else {
+            out.flip(xi);
+            xb = xa;
+            yb = ya;
+            xa = xi;
+            ya = yi;
+            ++n;
+            xi = -1;
+        }
+    }
+    return out;
+}
+
+__device__ __forceinline__ i128 shfl_up_i128(i128 v, int o) {
+    const uint64_t lo = static_cast<uint64_t>(static_cast<u128>(v));
+    const uint64_t hi = static_cast<uint64_t>(static_cast<u128>(v) >> 64);
+    const uint64_t l2 = __shfl_up(lo, o, 64), h2 = __shfl_up(hi, o, 64);
+    return static_cast<i128>((static_cast<u128>(h2) << 64) | l2);
+}
+
+inline __host__ __device__ int hull_stride(int32_t B) { return B | 1; }
+inline size_t hull_lds(int32_t B) { return static_cast<size_t>(64) * hull_stride(B) * 8; }
+
 template <class T>
-__global__ __launch_bounds__(kSmThreads) void k_sm_block_pfx(const T* __restrict__ v, int64_t n, int32_t m,
-                                                             int64_t J, i128* __restrict__ p1,
-                                                             i128* __restrict__ p2, i128* __restrict__ c1,
-                                                             i128* __restrict__ c2) {
-    __shared__ i128 s1[kPfxChunk], s2[kPfxChunk];
-    const int tid = threadIdx.x;
-    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kPfxChunk;
-    {  // thread tid: block p0 + tid, values [(p0+tid) m, (p0+tid+1) m) in order
-        const int64_t j = p0 + tid;
-        i128 a1 = 0, a2 = 0;
-        if (j < J) {
-            const int64_t lo = j * m;
-            const int64_t hi = (lo + m < n) ? lo + m : n;
-            for (int64_t q = lo; q < hi; ++q) {
-                const i128 y = wide<T>(v[q]);
+__global__ __launch_bounds__(kSmThreads) void k_sm_blocks(const T* __restrict__ v, int64_t n, int32_t B, int64_t JB,
+                                                          i128* __restrict__ p1, i128* __restrict__ p2,
+                                                          i128* __restrict__ c1, i128* __restrict__ c2, SmHull h) {
+    extern __shared__ int64_t s_v[];  // 64 rows
+    __shared__ HullMask s_mask[2][64];
+    __shared__ int32_t s_big[64];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int stride = hull_stride(B);
+    const uint32_t rcp = 0xFFFFFFFFu / static_cast<uint32_t>(B) + 1u;  // i / B, exact for i * B < 2^32
+    const int64_t b0 = static_cast<int64_t>(blockIdx.x) * kPfxChunk;
+    const int64_t q0 = b0 * B;
+    int32_t cnt = 64 * B;  // values of these 64 blocks
+    if (q0 + cnt > n) cnt = n > q0 ? static_cast<int32_t>(n - q0) : 0;
+    if (tid < 64) s_big[tid] = 0;
+    __syncthreads();
+    for (int32_t i0 = tid; i0 < cnt; i0 += 8 * kSmThreads) {
+        T y[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {  // eight loads in flight (index clamped)
+            const int32_t i = i0 + k * kSmThreads;
+            y[k] = v[q0 + (i < cnt ? i : cnt - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int32_t i = i0 + k * kSmThreads;
+            if (i >= cnt) break;
+            const int32_t blk = B == 1 ? i : static_cast<int32_t>(__umulhi(static_cast<uint32_t>(i), rcp));
+            s_v[blk * stride + (i - blk * B)] = static_cast<int64_t>(y[k]);
+            if (!small_value<T>(y[k])) s_big[blk] = 1;
+        }
+    }
+    __syncthreads();
+    for (int b = w; b < 64; b += kSmThreads / 64) {  // filter: a block per wave
+        const int len = cnt - b * B < B ? cnt - b * B : B;
+        const int64_t* row = s_v + b * stride;
+        HullMask up{0, 0}, dn{0, 0};
+        for (int half = 0; half < 2; ++half) {
+            const int i = half * 64 + lane;
+            bool u = i < len, d = u;
+            if (u) {
+                const int64_t y2 = 2 * row[i];
+#pragma unroll
+                for (int o = 1; o <= 32; o *= 2) {
+                    if (i >= o && i + o < len) {
+                        const int64_t s = row[i - o] + row[i + o];
+                        u = u && y2 > s;
+                        d = d && y2 < s;
+                    }
+                }
+            }
+            const uint64_t bu = __ballot(u), bd = __ballot(d);
+            if (half) up.hi = bu, dn.hi = bd;
+            else up.lo = bu, dn.lo = bd;
+            if (len <= 64) break;
+        }
+        if (lane == 0) s_mask[0][b] = up, s_mask[1][b] = dn;
+    }
+    __syncthreads();
+    const int64_t* row = s_v + lane * stride;
+    if (w == 0) {
+        s_mask[0][lane] = hull_chain<true>(row, s_mask[0][lane]);
+    } else if (w == 1) {
+        s_mask[1][lane] = hull_chain<false>(row, s_mask[1][lane]);
+    } else if (w == 2) {
+        const int len = cnt - lane * B < B ? cnt - lane * B : B;
+        i128 a1 = 0, a2 = 0;  // sum of y, of i * y
+        if (s_big[lane]) {
+            for (int i = 0; i < len; ++i) {
+                const i128 y = wide<T>(static_cast<T>(row[i]));
                 a1 += y;
-                a2 += y * static_cast<i128>(q);
+                a2 += y * static_cast<i128>(i);
+            }
+        } else {  // |y| <= 2^52: a block's sum fits 64 bits, eight products too
+            int64_t s1 = 0;
+            for (int i = 0; i < len; i += 8) {
+                int64_t s2 = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    const int64_t y = row[i + k < len ? i + k : i];
+                    if (i + k < len) {
+                        s1 += y;
+                        s2 += y * (i + k);
+                    }
+                }
+                a2 += s2;
+            }
+            a1 = s1;
+        }
+        a2 += a1 * static_cast<i128>(q0 + static_cast<int64_t>(lane) * B);  // q = first + i
+        i128 s1 = a1, s2 = a2;  // inclusive scan over the 64 blocks
+        for (int o = 1; o < 64; o <<= 1) {
+            const i128 x1 = shfl_up_i128(s1, o), x2 = shfl_up_i128(s2, o);
+            if (lane >= o) {
+                s1 += x1;
+                s2 += x2;
             }
         }
-        s1[tid] = a1;
-        s2[tid] = a2;
+        if (b0 + lane <= JB) {
+            p1[b0 + lane] = s1 - a1;
+            p2[b0 + lane] = s2 - a2;
+        }
+        if (lane == 63) {
+            c1[blockIdx.x] = s1;
+            c2[blockIdx.x] = s2;
+        }
     }
+    __syncthreads();
+    // vertices: lane = block, wave w the mask bits [32 w, 32 w + 32)
+    const int64_t b = b0 + lane;
+    const uint64_t lo = s_mask[0][lane].lo | s_mask[1][lane].lo, hi = s_mask[0][lane].hi | s_mask[1][lane].hi;
+    const int total = __popcll(lo) + __popcll(hi);
+    if (b >= JB) return;
+    if (total > h.slots || s_big[lane]) {
+        if (w == 0) h.nv[b] = kHullScan;
+        return;
+    }
+    if (w == 0) h.nv[b] = static_cast<uint8_t>(total);
+    uint32_t bits = static_cast<uint32_t>((w < 2 ? lo : hi) >> ((w & 1) * 32));
+    int k = (w >= 2 ? __popcll(lo) : 0) + ((w & 1) ? __popc(static_cast<uint32_t>(w < 2 ? lo : hi)) : 0);
+    while (bits) {
+        const int i = w * 32 + __builtin_ctz(bits);
+        bits &= bits - 1;
+        h.y[hull_at(h.slots, b, k)] = static_cast<double>(row[i]);
+        h.x[hull_at(h.slots, b, k)] = static_cast<uint8_t>(i);
+        ++k;
+    }
+}
+
+// Sums without hulls, for block sizes above kHullMaxB: a workgroup per block,
+// then the exclusive scan inside each chunk.
+template <class T>
+__global__ __launch_bounds__(kSmThreads) void k_sm_sums(const T* __restrict__ v, int64_t n, int32_t B,
+                                                        i128* __restrict__ p1, i128* __restrict__ p2) {
+    __shared__ i128 s1[kSmThreads / 64], s2[kSmThreads / 64];
+    const int tid = threadIdx.x;
+    const int64_t q0 = static_cast<int64_t>(blockIdx.x) * B;
+    const int64_t q1 = (q0 + B < n) ? q0 + B : n;
+    i128 a1 = 0, a2 = 0;
+    for (int64_t q = q0 + tid; q < q1; q += kSmThreads) {
+        const i128 y = wide<T>(v[q]);
+        a1 += y;
+        a2 += y * static_cast<i128>(q);
+    }
+    a1 = wave_sum(a1);
+    a2 = wave_sum(a2);
+    if ((tid & 63) == 0) {
+        s1[tid >> 6] = a1;
+        s2[tid >> 6] = a2;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        for (int k = 1; k < kSmThreads / 64; ++k) {
+            a1 += s1[k];
+            a2 += s2[k];
+        }
+        p1[blockIdx.x] = a1;
+        p2[blockIdx.x] = a2;
+    }
+}
+__global__ __launch_bounds__(kPfxChunk) void k_sm_chunk_pfx(int64_t JB, i128* __restrict__ p1, i128* __restrict__ p2,
+                                                             i128* __restrict__ c1, i128* __restrict__ c2) {
+    __shared__ i128 s1[kPfxChunk], s2[kPfxChunk];
+    const int tid = threadIdx.x;
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * kPfxChunk + tid;
+    const i128 a1 = p < JB ? p1[p] : static_cast<i128>(0), a2 = p < JB ? p2[p] : static_cast<i128>(0);
+    s1[tid] = a1;
+    s2[tid] = a2;
     __syncthreads();
     for (int o = 1; o < kPfxChunk; o <<= 1) {  // inclusive scan
         const i128 x1 = (tid >= o) ? s1[tid - o] : static_cast<i128>(0);
@@ -422,10 +697,9 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_block_pfx(const T* __restrict
         s2[tid] += x2;
         __syncthreads();
     }
-    const int64_t p = p0 + tid;
-    if (p <= J) {
-        p1[p] = tid ? s1[tid - 1] : static_cast<i128>(0);
-        p2[p] = tid ? s2[tid - 1] : static_cast<i128>(0);
+    if (p <= JB) {
+        p1[p] = s1[tid] - a1;
+        p2[p] = s2[tid] - a2;
     }
     if (tid == kPfxChunk - 1) {
         c1[blockIdx.x] = s1[tid];
@@ -433,11 +707,12 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_block_pfx(const T* __restrict
     }
 }
 // exclusive scan of C chunk totals in place (one workgroup, serial chunks)
-__global__ __launch_bounds__(kSmThreads) void k_sm_chunk_scan(i128* __restrict__ c1, i128* __restrict__ c2,
+constexpr int kChunkScanThreads = 1024;
+__global__ __launch_bounds__(kChunkScanThreads) void k_sm_chunk_scan(i128* __restrict__ c1, i128* __restrict__ c2,
                                                               int64_t C) {
-    __shared__ i128 s1[kSmThreads], s2[kSmThreads];
+    __shared__ i128 s1[kChunkScanThreads], s2[kChunkScanThreads];
     const int tid = threadIdx.x;
-    const int64_t per = (C + kSmThreads - 1) / kSmThreads;
+    const int64_t per = (C + kChunkScanThreads - 1) / kChunkScanThreads;
     const int64_t b0 = tid * per;
     const int64_t b1 = (b0 + per < C) ? b0 + per : C;
     i128 a1 = 0, a2 = 0;
@@ -448,7 +723,7 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_chunk_scan(i128* __restrict__
     s1[tid] = a1;
     s2[tid] = a2;
     __syncthreads();
-    for (int o = 1; o < kSmThreads; o <<= 1) {
+    for (int o = 1; o < kChunkScanThreads; o <<= 1) {
         const i128 x1 = (tid >= o) ? s1[tid - o] : static_cast<i128>(0);
         const i128 x2 = (tid >= o) ? s2[tid - o] : static_cast<i128>(0);
         __syncthreads();
@@ -466,183 +741,235 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_chunk_scan(i128* __restrict__
     }
 }
 
-// The same evaluation for m <= kStageMin, kSplitStarts consecutive starts per
-// workgroup: their candidates lie in one window of (kSplitStarts - 1 + 29) m
-// values, loaded into LDS once with all loads of a thread in flight.  The sums
-// come from the block prefixes.  The maximum-error pass runs candidate by
-// candidate with theta in registers (one accumulator, reduced as soon as the
-// candidate is done).
-constexpr int kStageMin = 128;
-constexpr int kSplitStarts = 4;
-constexpr int kStage = (kSplitStarts - 1 + 29) * kStageMin;  // the window, values
+// The same evaluation from prefix sums and hulls, S consecutive starts per
+// workgroup (m = U * B, S = 8 / U): their candidates lie in a window of
+// (S - 1 + 29) U blocks, whose vertices are staged in LDS.  Each thread takes
+// (start, candidate, block) triples and raises the candidate's D and H; a
+// candidate that the bounds do not settle is read value by value.
+constexpr int kSplitMaxU = 8;
+inline __host__ __device__ int split_starts(int U) { return U >= kSplitMaxU ? 1 : 8 / U; }
+inline __host__ __device__ int split_window(int U) { return (split_starts(U) - 1 + 29) * U; }
+inline size_t split_lds(int U, int32_t slots) { return static_cast<size_t>(split_window(U)) * (slots * 9 + 1); }
+
 template <class T>
-__global__ __launch_bounds__(kSmThreads) void k_sm_split_lds(const T* __restrict__ v, int64_t n, int32_t m,
-                                                             int64_t J, const i128* __restrict__ p1,
-                                                             const i128* __restrict__ p2,
-                                                             const i128* __restrict__ c1,
-                                                             const i128* __restrict__ c2,
-                                                             int32_t* __restrict__ best_end,
-                                                             double* __restrict__ best_cost) {
-    typedef typename std::make_unsigned<T>::type U;
-    __shared__ uint64_t s_v[kStage];  // T's bits; FP64 values in the exact pass
-    __shared__ double s_t[kSplitStarts][kMaxCand][2];
-    __shared__ int64_t s_mx[kSmThreads / 64][kSplitStarts][kMaxCand];
-    __shared__ bool s_fast[kSplitStarts][kMaxCand];
+__global__ __launch_bounds__(kSmThreads) void k_sm_split_hull(const T* __restrict__ v, int64_t n, int32_t m, int64_t J,
+                                                              int U, SmPrefix pf, SmHull h,
+                                                              int32_t* __restrict__ best_end,
+                                                              double* __restrict__ best_cost) {
+    constexpr int kS = 8, kTasks = kS * kMaxCand;
+    extern __shared__ double s_y[];  // [slots][W], then x [slots][W], nv [W]
+    __shared__ double s_t[kTasks][2];
+    __shared__ unsigned long long s_D[kTasks], s_H[kTasks];  // bits of non-negative doubles: ordered as integers
+    __shared__ int32_t s_bits[kTasks], s_scan[kTasks], s_fast[kTasks];
+    __shared__ int s_list[kTasks], s_cnt;
+    __shared__ int64_t s_mx[kSmThreads / 64];
     __shared__ FitLds L;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int64_t j0 = static_cast<int64_t>(blockIdx.x) * kSplitStarts;
-    if (j0 >= J) return;
-    const int64_t cur0 = j0 * m;
-    // candidates of start s: K[s] (0: fewer than m values left, only the column's last start)
-    int K[kSplitStarts];
-    int ns = 0, Kmax = 0;
-    bool tail = false;
-#pragma unroll
-    for (int q = 0; q < kSplitStarts; ++q) {
-        K[q] = 0;
-        const int64_t cur = cur0 + static_cast<int64_t>(q) * m;
-        if (j0 + q >= J) continue;
-        ns = q + 1;
-        const int64_t max_size = (n - cur < static_cast<int64_t>(m) * 32) ? n - cur : static_cast<int64_t>(m) * 32;
-        int k = 0;
-        while (k < kMaxCand && static_cast<int64_t>(kCandUnits[k]) * m <= max_size) ++k;
-        K[q] = k;
-        Kmax = k > Kmax ? k : Kmax;
-        tail = tail || k == 0;
+    const int S = split_starts(U), W = split_window(U);
+    uint8_t* s_x = reinterpret_cast<uint8_t*>(s_y + h.slots * W);
+    uint8_t* s_nv = s_x + h.slots * W;
+    const int64_t j0 = static_cast<int64_t>(blockIdx.x) * S;
+    const int64_t bw = j0 * U;  // first block of the window
+    int most = 0;
+    for (int i = tid; i < W; i += kSmThreads) {
+        const int c = bw + i < pf.JB ? h.nv[bw + i] : 0;
+        s_nv[i] = static_cast<uint8_t>(c);
+        most = c != kHullScan && c > most ? c : most;
     }
-    // window [cur0, cur0 + W): every candidate of every start, W <= kStage, cur0 + W <= n
-    int64_t W = 0;
-#pragma unroll
-    for (int q = 0; q < kSplitStarts; ++q)
-        if (K[q] > 0) {
-            const int64_t end = static_cast<int64_t>(q) * m + static_cast<int64_t>(kCandUnits[K[q] - 1]) * m;
-            W = end > W ? end : W;
-        }
-    constexpr int kPer = (kStage + kSmThreads - 1) / kSmThreads;
-    int big = 0;  // a value outside small_value's range
-    if (W > 0) {
-        T y[kPer];
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const int64_t i = tid + q * kSmThreads;
-            y[q] = v[cur0 + (i < W ? i : W - 1)];
-        }
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const int64_t i = tid + q * kSmThreads;
-            if (i < W) {
-                big |= small_value<T>(y[q]) ? 0 : 1;
-                s_v[i] = static_cast<uint64_t>(static_cast<U>(y[q]));
-            }
+    if (tid == 0) s_cnt = 0;
+    // task q * 14 + k: candidate k of start j0 + q
+    const int tq = tid / kMaxCand, tk = tid % kMaxCand;
+    const int64_t cur = (j0 + tq) * m, size = static_cast<int64_t>(kCandUnits[tk]) * m;
+    const bool live = tid < S * kMaxCand && cur + size <= n;
+    if (tid < kTasks) {
+        s_D[tid] = s_H[tid] = 0;
+        s_bits[tid] = live ? 0 : -1;
+        s_scan[tid] = 0;
+        if (live) {
+            bool fast;
+            range_line<T>(pf, cur, cur + size, s_t[tid][0], s_t[tid][1], fast);
+            s_fast[tid] = fast;
+            s_scan[tid] = !fast;
         }
     }
-    const int any_big = __syncthreads_or(big);
-    if (tid < kSplitStarts * kMaxCand) {  // candidate k of start q: sums from the prefixes
-        const int q = tid / kMaxCand, k = tid % kMaxCand;
-        if (k < K[q]) {
-            const int64_t j = j0 + q, cur = cur0 + static_cast<int64_t>(q) * m;
-            const int64_t e = j + kCandUnits[k];  // e * m <= n, so e <= J
-            const i128 sy = (p1[e] + c1[e / kPfxChunk]) - (p1[j] + c1[j / kPfxChunk]);
-            const i128 sxy =
-                (p2[e] + c2[e / kPfxChunk]) - (p2[j] + c2[j / kPfxChunk]) - static_cast<i128>(cur) * sy;
-            double t0, t1;
-            const int64_t size = static_cast<int64_t>(kCandUnits[k]) * m;
-            sm_theta(sy, sxy, size, t0, t1);
-            s_t[q][k][0] = t0;
-            s_t[q][k][1] = t1;
-            const double pr0 = t0 + t1 * 0.0, pr1 = t0 + t1 * static_cast<double>(size - 1);
-            s_fast[q][k] = small_pred<T>(pr0) && small_pred<T>(pr1);
+    const int rows = __syncthreads_or(most > 16) ? h.slots : h.slots < 16 ? h.slots : 16;
+    for (int i = tid; i < rows * W; i += kSmThreads) {
+        const int k = i / W, b = i - k * W;
+        if (bw + b < pf.JB) {  // slots past a block's vertices hold whatever was there and are not read below
+            s_y[i] = h.y[hull_at(h.slots, bw + b, k)];
+            s_x[i] = h.x[hull_at(h.slots, bw + b, k)];
         }
     }
     __syncthreads();
-    bool fast = !any_big;
-    for (int q = 0; q < ns; ++q)
-        for (int k = 0; k < K[q]; ++k) fast = fast && s_fast[q][k];
-    if (fast) {  // workgroup-uniform: every residual is exact in FP64
-        for (int64_t i = tid; i < W; i += kSmThreads)
-            s_v[i] = static_cast<uint64_t>(
-                __double_as_longlong(static_cast<double>(static_cast<T>(static_cast<U>(s_v[i])))));
+    const int per = kCandCum[kMaxCand] * U;  // blocks of one start's candidates
+    for (int t = tid; t < S * per; t += kSmThreads) {
+        const int q = t / per, r = t - q * per;
+        int k = 0;
+#pragma unroll
+        for (int step = 8; step; step >>= 1)
+            if (k + step < kMaxCand && r >= kCandCum[k + step] * U) k += step;
+        const int task = q * kMaxCand + k;
+        if (s_bits[task] < 0 || s_scan[task]) continue;
+        const int u = r - kCandCum[k] * U, b = q * U + u;
+        const int nv = s_nv[b];
+        if (nv == kHullScan) {
+            s_scan[task] = 1;
+            continue;
+        }
+        double D = 0.0, H = 0.0;
+        hull_err(s_y + b, s_x + b, W, nv, static_cast<int64_t>(u) * pf.B, s_t[task][0], s_t[task][1], D, H);
+        atomicMax(&s_D[task], static_cast<unsigned long long>(__double_as_longlong(D)));
+        atomicMax(&s_H[task], static_cast<unsigned long long>(__double_as_longlong(H)));
+    }
+    __syncthreads();
+    if (live) {
+        int32_t b = -1;
+        if (!s_scan[tid])
+            b = hull_bits(__longlong_as_double(static_cast<long long>(s_D[tid])),
+                          __longlong_as_double(static_cast<long long>(s_H[tid])), s_t[tid][0], s_t[tid][1], size);
+        if (b < 0) s_list[atomicAdd(&s_cnt, 1)] = tid;
+        else s_bits[tid] = b;
+    }
+    __syncthreads();
+    for (int i = 0; i < s_cnt; ++i) {  // read by the whole workgroup
+        const int task = s_list[i];
+        const int64_t c = (j0 + task / kMaxCand) * m, z = static_cast<int64_t>(kCandUnits[task % kMaxCand]) * m;
+        const int64_t mx = wave_max(
+            scan_err<T>(v + c, tid, z, kSmThreads, s_t[task][0], s_t[task][1], s_fast[task] != 0));
+        if (lane == 0) s_mx[w] = mx;
+        __syncthreads();
+        if (tid == 0) {
+            int64_t r = s_mx[0];
+            for (int x = 1; x < kSmThreads / 64; ++x) r = s_mx[x] > r ? s_mx[x] : r;
+            s_bits[task] = bits_of(r);
+        }
         __syncthreads();
     }
-    for (int q = 0; q < ns; ++q) {
-        const uint64_t* sv = s_v + q * m;  // start q's values
-        for (int k = 0; k < K[q]; ++k) {
-            const int size = kCandUnits[k] * m;
-            const double t0 = s_t[q][k][0], t1 = s_t[q][k][1];
-            int64_t mx = 0;
-            if (fast) {
-                double md = 0.0;
-                for (int i = tid; i < size; i += kSmThreads) {
-                    const double pr = t0 + t1 * static_cast<double>(i);  // no contraction (-ffp-contract=off)
-                    md = __builtin_fmax(md, __builtin_fabs(__longlong_as_double(static_cast<long long>(sv[i])) -
-                                                           round_away(pr)));
-                }
-                mx = static_cast<int64_t>(md);
-            } else {
-                for (int i = tid; i < size; i += kSmThreads) {
-                    const int64_t a = abs_err<T>(static_cast<T>(static_cast<U>(sv[i])), t0, t1, i);
-                    mx = a > mx ? a : mx;
-                }
-            }
-            mx = wave_max(mx);
-            if (lane == 0) s_mx[w][q][k] = mx;
-        }
-    }
-    __syncthreads();
-    if (tid < ns && K[tid] > 0) {  // start tid: the smallest cost per value, the first on ties
-        const int q = tid;
-        const int64_t cur = cur0 + static_cast<int64_t>(q) * m;
+    if (tid < S && j0 + tid < J && s_bits[tid * kMaxCand] >= 0) {  // smallest cost per value, the first on ties
+        const int64_t c0 = (j0 + tid) * m;
         double best = DBL_MAX, bc = 0.0;
-        int64_t be = (cur + m < n) ? cur + m : n;
-        for (int k = 0; k < K[q]; ++k) {
-            int64_t r = s_mx[0][q][k];
-            for (int x = 1; x < kSmThreads / 64; ++x) r = s_mx[x][q][k] > r ? s_mx[x][q][k] : r;
-            const int64_t size = static_cast<int64_t>(kCandUnits[k]) * m;
-            const double c = cost_of(size, bits_of(r));
-            const double cpe = c / static_cast<double>(size);
+        int64_t be = (c0 + m < n) ? c0 + m : n;
+        for (int k = 0; k < kMaxCand && s_bits[tid * kMaxCand + k] >= 0; ++k) {
+            const int64_t z = static_cast<int64_t>(kCandUnits[k]) * m;
+            const double c = cost_of(z, s_bits[tid * kMaxCand + k]);
+            const double cpe = c / static_cast<double>(z);
             if (cpe < best) {
                 best = cpe;
-                be = cur + size;
+                be = c0 + z;
                 bc = c;
             }
         }
-        best_end[j0 + q] = static_cast<int32_t>(be);
-        best_cost[j0 + q] = bc;
+        best_end[j0 + tid] = static_cast<int32_t>(be);
+        best_cost[j0 + tid] = bc;
     }
-    if (tail) {  // workgroup-uniform: the column's last start has fewer than m values, one partition [cur, n)
-        for (int q = 0; q < ns; ++q) {
-            if (K[q] != 0) continue;
-            const int64_t cur = cur0 + static_cast<int64_t>(q) * m;
-            const double c = wg_cost<T>(v, cur, n, L, SmPrefix{p1, p2, c1, c2, m, n, J});
-            if (tid == 0) {
-                best_end[j0 + q] = static_cast<int32_t>(n);
-                best_cost[j0 + q] = c;
-            }
+    // the column's last start may have fewer than m values: one partition [cur, n)
+    const int64_t last = (J - 1) * m;
+    if (J - 1 >= j0 && J - 1 < j0 + S && n - last < m) {
+        const double c = wg_cost<T>(v, last, n, L);
+        if (tid == 0) {
+            best_end[J - 1] = static_cast<int32_t>(n);
+            best_cost[J - 1] = c;
         }
     }
 }
 
-// ---- chain: mark the starts the greedy walk from 0 reaches -----------------
-__global__ void k_sm_chain_init(const int32_t* __restrict__ best_end, int64_t J, int32_t m,
-                                int32_t* __restrict__ jump, int32_t* __restrict__ mark) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= J) return;
-    const int64_t e = best_end[j];
-    jump[j] = static_cast<int32_t>((e % m == 0 && e / m < J) ? e / m : J);  // J = past the end
-    mark[j] = (j == 0);
+// ---- chain: mark the entries that a walk from entry 0 reaches ----------------
+// next[i] > i is the entry after i (J or more: the end).  k_sm_chain_exit: a
+// workgroup per chunk of kChain entries replaces next by the first entry past
+// the chunk, by pointer doubling in LDS; k_sm_chain_walk hops from chunk to
+// chunk (one dependent load each) and notes where the walk enters each;
+// k_sm_chain_mark marks a chunk's entries from there, again by doubling.  Three
+// launches where doubling over the whole list took 2 log2(J).
+constexpr int kChainThreads = 1024;
+constexpr int kChainPer = 8;
+constexpr int kChain = kChainThreads * kChainPer;
+
+// one doubling step over the chunk's LDS copy; true while some entry is inside
+__device__ __forceinline__ bool chain_double(int32_t* s_j, int32_t cnt) {
+    int32_t t[kChainPer];
+    bool inside = false;
+#pragma unroll
+    for (int q = 0; q < kChainPer; ++q) {
+        const int32_t i = threadIdx.x + q * kChainThreads;
+        t[q] = i < cnt ? s_j[i] : cnt;
+        if (t[q] < cnt) t[q] = s_j[t[q]];
+        inside = inside || t[q] < cnt;
+    }
+    const bool any = __syncthreads_or(inside);
+#pragma unroll
+    for (int q = 0; q < kChainPer; ++q) {
+        const int32_t i = threadIdx.x + q * kChainThreads;
+        if (i < cnt) s_j[i] = t[q];
+    }
+    __syncthreads();
+    return any;
 }
-// marked nodes mark their jump target; then jump <- jump o jump
-__global__ void k_sm_chain_mark(const int32_t* __restrict__ jump, int64_t J, int32_t* __restrict__ mark) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= J || !mark[j]) return;
-    const int32_t t = jump[j];
-    if (t < J) mark[t] = 1;
+
+// next[] of entry i: its target entry, J past the end
+struct ChainSplit {  // split: best_end[i] / m where that is an entry
+    const int32_t* best_end;
+    int64_t J;
+    int32_t m;
+    __device__ int64_t operator()(int64_t i) const {
+        const uint32_t e = static_cast<uint32_t>(best_end[i]), j = e / static_cast<uint32_t>(m);
+        return (j * static_cast<uint32_t>(m) == e && j < J) ? j : J;
+    }
+};
+struct ChainMerge {  // merge: the group that starts at partition i ends before partition gend[i]
+    const int32_t* gend;
+    __device__ int64_t operator()(int64_t i) const { return gend[i]; }
+};
+
+template <class F>
+__global__ __launch_bounds__(kChainThreads) void k_sm_chain_exit(F next, int64_t J, int32_t* __restrict__ out) {
+    __shared__ int32_t s_j[kChain];
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kChain;
+    const int32_t cnt = static_cast<int32_t>(J - base < kChain ? J - base : kChain);
+    // targets relative to the chunk; one past it is kept as it is (>= cnt) and
+    // never followed inside
+    bool inside = false;
+    for (int32_t i = threadIdx.x; i < cnt; i += kChainThreads) {
+        s_j[i] = static_cast<int32_t>(next(base + i) - base);
+        inside = inside || s_j[i] < cnt;
+    }
+    bool any = __syncthreads_or(inside);
+    while (any) any = chain_double(s_j, cnt);
+    for (int32_t i = threadIdx.x; i < cnt; i += kChainThreads) out[base + i] = static_cast<int32_t>(base + s_j[i]);
 }
-__global__ void k_sm_chain_double(const int32_t* __restrict__ jin, int64_t J, int32_t* __restrict__ jout) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= J) return;
-    const int32_t t = jin[j];
-    jout[j] = (t < J) ? jin[t] : static_cast<int32_t>(J);
+__global__ void k_sm_chain_walk(const int32_t* __restrict__ exits, int64_t J, int64_t chunks,
+                                int32_t* __restrict__ entry) {
+    for (int64_t c = threadIdx.x; c < chunks; c += blockDim.x) entry[c] = -1;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t e = 0;
+        while (e < J) {
+            entry[e / kChain] = static_cast<int32_t>(e);
+            e = exits[e];
+        }
+    }
+}
+template <class F>
+__global__ __launch_bounds__(kChainThreads) void k_sm_chain_mark(F next, int64_t J, const int32_t* __restrict__ entry,
+                                                                 int32_t* __restrict__ mark) {
+    __shared__ int32_t s_j[kChain];
+    __shared__ uint8_t s_m[kChain];
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * kChain;
+    const int32_t cnt = static_cast<int32_t>(J - base < kChain ? J - base : kChain);
+    const int32_t e = entry[blockIdx.x];
+    bool inside = false;
+    for (int32_t i = threadIdx.x; i < cnt; i += kChainThreads) {
+        s_j[i] = static_cast<int32_t>(next(base + i) - base);
+        s_m[i] = e >= 0 && base + i == e;
+        inside = inside || s_j[i] < cnt;
+    }
+    bool any = __syncthreads_or(inside) && e >= 0;
+    while (any) {  // entries on the walk mark their targets, then every target doubles
+        for (int32_t i = threadIdx.x; i < cnt; i += kChainThreads)
+            if (s_m[i] && s_j[i] < cnt) s_m[s_j[i]] = 1;
+        __syncthreads();
+        any = chain_double(s_j, cnt);
+    }
+    for (int32_t i = threadIdx.x; i < cnt; i += kChainThreads) mark[base + i] = s_m[i];
 }
 
 // exclusive scan of mark[] into pos[]; *count = total (one workgroup)
@@ -723,206 +1050,98 @@ __global__ void k_sm_emit(const int32_t* __restrict__ mark, const int32_t* __res
 }
 
 // ---- merge -------------------------------------------------------------------
-// pair test of partitions i, i+1 as a fresh group: merged cost and decision
+// The group that starts at partition e (CpuPartitioner.cuh:207-236): it takes
+// in partition j while the refitted whole costs less than the group so far and
+// j apart.  Whether the walk starts a group at e or not, what the group would
+// be depends on e alone, so all are grown at once, a wave each; gend[e] is the
+// first partition after the group, gcost[e] its cost.  A group holds at most
+// about 46341 values (past that the cost model's int32 n * (n - 1) wraps and
+// the fit is useless), which bounds the work per start.  The lines of the next
+// kGrowLook candidates are computed by as many lanes at once; one candidate's
+// residuals take the hulls of its blocks, a block per lane.
+constexpr int kGrowLook = 16;
+
+// Bit width of the residuals of line t0, t1 over [gs, ge), computed by a
+// wave (gs a block start, ge one or n).
 template <class T>
-__global__ __launch_bounds__(kSmThreads) void k_sm_pair(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                        const int32_t* __restrict__ en,
-                                                        const double* __restrict__ cost, int64_t P,
-                                                        double* __restrict__ mc, int32_t* __restrict__ flag,
-                                                        SmPrefix pf) {
-    __shared__ FitLds L;
-    for (int64_t i = blockIdx.x; i + 1 < P; i += gridDim.x) {
-        const double c = wg_cost<T>(v, st[i], en[i + 1], L, pf);
-        if (threadIdx.x == 0) {
-            mc[i] = c;
-            flag[i] = c < cost[i] + cost[i + 1];
-        }
-    }
-}
-
-// A pass's walk (CpuPartitioner.cuh:207-236) keeps one state: the current
-// group [gs, ge) with its cost.  At a group start that state is fixed by the
-// start's index alone, so the walk from any group start is the same whoever
-// reaches it.  The pass therefore runs as
-//   k_sm_seg  every segment of `seg` consecutive partitions is walked at once,
-//             one workgroup each, as if a group started at its first entry;
-//             the walk records its group starts inside the segment (spec = 1,
-//             group end index, group cost) and its exit, the first group start
-//             at or past the segment's end;
-//   k_sm_fix  one workgroup follows the true walk from partition 0 across the
-//             segments: where it reaches a start that the segment's walk also
-//             made, the segment's result from there on is the true one and the
-//             walk jumps to the segment's exit; elsewhere it grows the group
-//             itself and rewrites spec / end / cost for the entries it covers.
-// Either way every entry of every segment ends up with the true walk's
-// decision, so the pass result equals the sequential walk's.
-constexpr int kWin = 256;
-
-template <class T>
-__global__ __launch_bounds__(kSmThreads) void k_sm_seg(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                       const int32_t* __restrict__ en,
-                                                       const double* __restrict__ cost,
-                                                       const double* __restrict__ mc,
-                                                       const int32_t* __restrict__ flag, int64_t P, int64_t seg,
-                                                       int32_t* __restrict__ spec, int32_t* __restrict__ gend,
-                                                       double* __restrict__ gcost, int32_t* __restrict__ exitk,
-                                                       SmPrefix pf) {
-    __shared__ FitLds L;
-    __shared__ int32_t w_st[kWin + 1], w_en[kWin + 1], w_flag[kWin + 1];
-    __shared__ double w_c[kWin + 1], w_mc[kWin + 1];
-    const int tid = threadIdx.x;
-    const int64_t a0 = static_cast<int64_t>(blockIdx.x) * seg;
-    if (a0 >= P) return;
-    const int64_t a1 = (a0 + seg < P) ? a0 + seg : P;
-    int64_t base = a0;  // the window holds entries [base, base + kWin]
-    auto load = [&](int64_t b) {
-        __syncthreads();
-        for (int k = tid; k <= kWin; k += kSmThreads) {
-            const int64_t i = b + k;
-            if (i < P) {
-                w_st[k] = st[i];
-                w_en[k] = en[i];
-                w_c[k] = cost[i];
-                w_mc[k] = (i + 1 < P) ? mc[i] : 0.0;
-                w_flag[k] = (i + 1 < P) ? flag[i] : 0;
-            }
-        }
-        __syncthreads();
-    };
-    load(a0);
-    int64_t g = a0;  // index of the current group's first partition
-    int64_t gs = w_st[0];
-    double gc = w_c[0];
-    bool single = true;
-    int64_t i = a0 + 1;
-    for (; i < P; ++i) {
-        if (i - base >= kWin) {  // entries i-1 and i must be in the window
-            base = i - 1;
-            load(base);
-        }
-        const int k = static_cast<int>(i - base);
-        const double ci = w_c[k];
-        bool merge;
-        double merged;
-        if (single) {
-            merge = w_flag[k - 1] != 0;
-            merged = w_mc[k - 1];
-        } else {
-            merged = wg_cost<T>(v, gs, w_en[k], L, pf);
-            merge = merged < gc + ci;
-        }
-        if (merge) {
-            gc = merged;
-            single = false;
-            if (tid == 0 && i < a1) spec[i] = 0;
-        } else {
-            if (tid == 0) {
-                spec[g] = 1;
-                gend[g] = static_cast<int32_t>(i);
-                gcost[g] = gc;
-            }
-            if (i >= a1) break;
-            g = i;
-            gs = w_st[k];
-            gc = ci;
-            single = true;
-        }
-    }
-    if (tid == 0) {
-        if (i == P) {  // the last group reaches the end of the list
-            spec[g] = 1;
-            gend[g] = static_cast<int32_t>(P);
-            gcost[g] = gc;
-        }
-        exitk[blockIdx.x] = static_cast<int32_t>(i);
-    }
-}
-
-// The group that starts at partition e: returns the index of the first
-// partition after it and its cost (all threads call it).
-template <class T, int NT>
-__device__ int64_t sm_grow(const T* __restrict__ v, const int32_t* __restrict__ st, const int32_t* __restrict__ en,
-                           const double* __restrict__ cost, const double* __restrict__ mc,
-                           const int32_t* __restrict__ flag, int64_t P, int64_t e, double& gc_out, FitLdsT<NT>& L,
-                           const SmPrefix& pf) {
-    const int64_t gs = st[e];
-    double gc = cost[e];
-    bool single = true;
-    int64_t j = e + 1;
-    for (; j < P; ++j) {
-        const double cj = cost[j];
-        bool merge;
-        double merged;
-        if (single) {
-            merge = flag[j - 1] != 0;
-            merged = mc[j - 1];
-        } else {
-            merged = wg_cost<T, NT>(v, gs, en[j], L, pf);
-            merge = merged < gc + cj;
-        }
-        if (!merge) break;
-        gc = merged;
-        single = false;
-    }
-    gc_out = gc;
-    return j;
-}
-
-constexpr int kFixWin = 2048;
-// One workgroup of 16 waves (4 per SIMD): its regrowth scans are the only
-// work on the GPU while it runs, and 4 waves per SIMD hide their load latency
-// where 1 did not.
-constexpr int kFixThreads = 1024;
-template <class T>
-__global__ __launch_bounds__(kFixThreads) void k_sm_fix(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                       const int32_t* __restrict__ en,
-                                                       const double* __restrict__ cost,
-                                                       const double* __restrict__ mc,
-                                                       const int32_t* __restrict__ flag, int64_t P, int64_t seg,
-                                                       int64_t K, int32_t* __restrict__ spec,
-                                                       int32_t* __restrict__ gend, double* __restrict__ gcost,
-                                                       const int32_t* __restrict__ exitk, SmPrefix pf) {
-    __shared__ FitLdsT<kFixThreads> L;
-    __shared__ int32_t s_spec[kFixWin], s_exit[kFixWin];
-    const int tid = threadIdx.x;
-    // Every write below is to an entry before the walk's position e, every
-    // read of spec at or after it, so the windows never hold a stale entry
-    // that is read.
-    int64_t wb = -1, xb = -1;  // windows: spec [wb, wb + kFixWin), exits [xb, xb + kFixWin)
-    int64_t e = 0;             // the true walk's next group start
-    for (int64_t k = 0; k < K; ++k) {
-        const int64_t a0 = k * seg;
-        const int64_t a1 = (a0 + seg < P) ? a0 + seg : P;
-        const int64_t c = e < a1 ? e : a1;
-        for (int64_t a = a0 + tid; a < c; a += kFixThreads) spec[a] = 0;  // inside the group before e
-        while (e < a1) {
-            if (wb < 0 || e >= wb + kFixWin) {
-                __syncthreads();
-                wb = e;
-                for (int q = tid; q < kFixWin; q += kFixThreads) s_spec[q] = (wb + q < P) ? spec[wb + q] : 0;
-                __syncthreads();
-            }
-            if (s_spec[e - wb]) {  // the segment's own walk from e is the true one
-                if (xb < 0 || k >= xb + kFixWin) {
-                    __syncthreads();
-                    xb = k;
-                    for (int q = tid; q < kFixWin; q += kFixThreads) s_exit[q] = (xb + q < K) ? exitk[xb + q] : 0;
-                    __syncthreads();
-                }
-                e = s_exit[k - xb];
+__device__ __forceinline__ int32_t range_bits(const T* __restrict__ v, int64_t gs, int64_t ge, double t0, double t1,
+                                              bool fast, const SmPrefix& pf, const SmHull& h, int lane) {
+    const int64_t len = ge - gs;
+    int32_t bits = -1;
+    if (fast && h.slots > 0) {
+        const int64_t ib = gs / pf.B, ie = (ge == pf.n) ? pf.JB : ge / pf.B;
+        double D = 0.0, H = 0.0;
+        int64_t mx = 0;  // of blocks read value by value
+        bool settled = true;
+        for (int64_t b0 = ib; b0 < ie; b0 += 64) {
+            const int64_t b = b0 + lane;
+            int nv = b < ie ? h.nv[b] : 0;
+            uint64_t odd = __ballot(nv == kHullScan);
+            if (__popcll(odd) > 8) {  // mostly such blocks: one pass over the range is faster
+                settled = false;
                 break;
             }
-            double gc;
-            const int64_t j = sm_grow<T, kFixThreads>(v, st, en, cost, mc, flag, P, e, gc, L, pf);
-            if (tid == 0) {
-                spec[e] = 1;
-                gend[e] = static_cast<int32_t>(j);
-                gcost[e] = gc;
+            if (nv == kHullScan) nv = 0;
+            const int64_t at = hull_at(h.slots, b < ie ? b : ib, 0);
+            hull_err(h.y + at, h.x + at, 64, nv, (b - ib) * pf.B, t0, t1, D, H);
+            while (odd) {  // wave-uniform
+                const int64_t q = (b0 + __builtin_ctzll(odd)) * pf.B;
+                odd &= odd - 1;
+                const int64_t hi = q + pf.B < ge ? q + pf.B : ge;
+                const int64_t a = scan_err<T>(v + gs, q - gs + lane, hi - gs, 64, t0, t1, true);
+                mx = a > mx ? a : mx;
             }
-            const int64_t hi = j < a1 ? j : a1;
-            for (int64_t a = e + 1 + tid; a < hi; a += kFixThreads) spec[a] = 0;
-            e = j;
         }
+        for (int o = 32; o > 0; o >>= 1) {
+            D = __builtin_fmax(D, __shfl_xor(D, o, 64));
+            H = __builtin_fmax(H, __shfl_xor(H, o, 64));
+        }
+        mx = wave_max(mx);
+        bits = settled ? hull_bits(D, H, t0, t1, len) : -1;
+        if (bits >= 0) bits = bits_of(mx) > bits ? bits_of(mx) : bits;
+    }
+    return bits >= 0 ? bits : bits_of(wave_max(scan_err<T>(v + gs, lane, len, 64, t0, t1, fast)));
+}
+
+template <class T>
+__global__ __launch_bounds__(kSmThreads) void k_sm_grow(const T* __restrict__ v, const int32_t* __restrict__ st,
+                                                        const int32_t* __restrict__ en,
+                                                        const double* __restrict__ cost, int64_t P, SmPrefix pf,
+                                                        SmHull h, int32_t* __restrict__ gend,
+                                                        double* __restrict__ gcost) {
+    const int lane = threadIdx.x & 63;
+    const int64_t e = static_cast<int64_t>(blockIdx.x) * (kSmThreads / 64) +
+                      __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (e >= P) return;
+    const int64_t gs = st[e];
+    double gc = cost[e];
+    int64_t j = e + 1;
+    bool open = true;
+    while (open && j < P) {
+        double lt0 = 0.0, lt1 = 0.0, lc = 0.0;
+        int32_t le = 0;
+        bool lf = false;
+        if (lane < kGrowLook && j + lane < P) {
+            le = en[j + lane];
+            lc = cost[j + lane];
+            range_line<T>(pf, gs, le, lt0, lt1, lf);
+        }
+        const int look = P - j < kGrowLook ? static_cast<int>(P - j) : kGrowLook;
+        for (int c = 0; c < look && open; ++c) {
+            const int64_t ge = __shfl(le, c, 64);
+            const double merged =
+                cost_of(ge - gs, range_bits<T>(v, gs, ge, __shfl(lt0, c, 64), __shfl(lt1, c, 64),
+                                               __shfl(static_cast<int>(lf), c, 64) != 0, pf, h, lane));
+            open = merged < gc + __shfl(lc, c, 64);
+            if (open) {
+                gc = merged;
+                ++j;
+            }
+        }
+    }
+    if (lane == 0) {
+        gend[e] = static_cast<int32_t>(j);
+        gcost[e] = gc;
     }
 }
 
@@ -951,14 +1170,14 @@ template <class F> int dispatch_dtype(int dtype, F&& f) {
 
 unsigned blocks(int64_t n, int b) { return static_cast<unsigned>((n + b - 1) / b); }
 
-// Partitions per speculative merge segment: GLC_SPLITMERGE_SEGMENT (1..2^30),
-// default 32.  Any value gives the same boundaries; it only moves work
-// between the parallel segment walks and the one-workgroup fix-up.
 // Scratch of one split/merge call, kept per device between calls and grown
 // when a larger column needs more (a per-call hipMalloc/hipFree pair costs
 // hundreds of microseconds and the free synchronises the device).  Held
-// until the process ends; the lock covers a whole call, which ends with its
-// stream synchronised.
+// until the process ends while it is at most kSmKeep bytes (a column of about
+// 2^28 values at minimum size 128; larger ones give it back, their call is 100
+// times longer than the allocation); the lock covers a whole call, which ends
+// with its stream synchronised.
+constexpr int64_t kSmKeep = int64_t(1) << 30;
 struct SmScratch {
     std::mutex mu;
     void* p = nullptr;
@@ -973,13 +1192,6 @@ SmScratch& sm_scratch(int device) {
     return *e;
 }
 
-int64_t merge_segment_length() {
-    const char* e = std::getenv("GLC_SPLITMERGE_SEGMENT");
-    if (!e || !*e) return 32;
-    const long long x = std::atoll(e);
-    return (x >= 1 && x <= (1LL << 30)) ? x : 32;
-}
-
 }  // namespace
 
 // Partition d_values[0, n) on the device; the boundaries end up in host
@@ -991,16 +1203,33 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
     if (n <= 0) return GLC_OK;
     if (m <= 0 || m > (1 << 20)) return fail(GLC_ERR_INVALID_ARG, "split/merge minimum size must be in [1, 2^20]");
     const int64_t J = (n + m - 1) / m;
-    // scratch: best_end, jump x2, mark, pos, st x2, en x2, flag (int32 x J each);
-    // best_cost, cost x2, mc (double x J each); result (2 x int64)
-    // with m <= kStageMin also block prefixes p1, p2 (i128 x (J + 1)) and chunk offsets c1, c2 (i128 x C)
+    // blocks: B = m up to kHullMaxB; above, the largest divisor of m from 32
+    // to kHullMaxB with m / B <= kSplitMaxU (wide enough to make hulls pay, few
+    // enough for the split window).  No such divisor: B = m, sums only.
+    int32_t B = m;
+    if (m > kHullMaxB)
+        for (int32_t d = kHullMaxB; d >= 32; --d)
+            if (m % d == 0 && m / d <= kSplitMaxU) {
+                B = d;
+                break;
+            }
+    const bool hulls = B <= kHullMaxB;
+    const int32_t slots = hulls ? std::min<int32_t>(kHullSlots, B) : 0;
+    const int U = m / B;
+    const int64_t JB = (n + B - 1) / B;
+    // scratch: best_end, exits, mark, pos, st x2, en x2, gend (int32 x J each);
+    // best_cost, cost x2, gcost (double x J each); result (2 x int64); block
+    // prefixes p1, p2 (i128 x (JB + 1)) and chunk offsets c1, c2 (i128 x C); scan
+    // tile totals and offsets (int32 x T), chain entries (int32); hull vertices
+    // y (double), x (byte) x slots and counts (byte) per block, 64 blocks at a time
     const int64_t i4 = align_up(J * 4, 256), d8 = align_up(J * 8, 256);
-    const bool staged = m <= kStageMin;
-    const int64_t C = (J + 1 + kPfxChunk - 1) / kPfxChunk;
-    const int64_t q16 = staged ? align_up((J + 1) * 16, 256) : 0, c16 = staged ? align_up(C * 16, 256) : 0;
-    const int64_t T = (J + kScanTile - 1) / kScanTile;  // scan tiles; tile totals and offsets: int32 x T each
+    const int64_t C = (JB + 1 + kPfxChunk - 1) / kPfxChunk;
+    const int64_t q16 = align_up((JB + 1) * 16, 256), c16 = align_up(C * 16, 256);
+    const int64_t T = (J + kScanTile - 1) / kScanTile;
     const int64_t t4 = align_up(T * 4, 256);
-    const int64_t bytes = 10 * i4 + 4 * d8 + 256 + 2 * q16 + 2 * c16 + 2 * t4;
+    const int64_t jb64 = align_up(JB, 64);
+    const int64_t hy = align_up(jb64 * slots * 8, 256), hx = align_up(jb64 * slots, 256), hn = align_up(jb64, 256);
+    const int64_t bytes = 9 * i4 + 4 * d8 + 256 + 2 * q16 + 2 * c16 + 3 * t4 + (hulls ? hy + hx + hn : 0);
     int dev = 0;
     GLC_HIP(hipGetDevice(&dev));
     SmScratch& sc = sm_scratch(dev);
@@ -1019,52 +1248,63 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
     }
     char* p = static_cast<char*>(sc.p);
     auto I = [&](int k) { return reinterpret_cast<int32_t*>(p + k * i4); };
-    auto D = [&](int k) { return reinterpret_cast<double*>(p + 10 * i4 + k * d8); };
-    int32_t *best_end = I(0), *jump0 = I(1), *jump1 = I(2), *mark = I(3), *pos = I(4);
-    int32_t *st0 = I(5), *st1 = I(6), *en0 = I(7), *en1 = I(8), *flag = I(9);
-    double *best_cost = D(0), *cost0 = D(1), *cost1 = D(2), *mc = D(3);
-    int64_t* result = reinterpret_cast<int64_t*>(p + 10 * i4 + 4 * d8);
-    char* pq = p + 10 * i4 + 4 * d8 + 256;
+    auto D = [&](int k) { return reinterpret_cast<double*>(p + 9 * i4 + k * d8); };
+    int32_t *best_end = I(0), *exits = I(1), *mark = I(2), *pos = I(3);
+    int32_t *st0 = I(4), *st1 = I(5), *en0 = I(6), *en1 = I(7), *gend = I(8);
+    double *best_cost = D(0), *cost0 = D(1), *cost1 = D(2), *gcost = D(3);
+    int64_t* result = reinterpret_cast<int64_t*>(p + 9 * i4 + 4 * d8);
+    char* pq = p + 9 * i4 + 4 * d8 + 256;
     i128 *pf1 = reinterpret_cast<i128*>(pq), *pf2 = reinterpret_cast<i128*>(pq + q16);
     i128 *cf1 = reinterpret_cast<i128*>(pq + 2 * q16), *cf2 = reinterpret_cast<i128*>(pq + 2 * q16 + c16);
-    int32_t* tile_tot = reinterpret_cast<int32_t*>(pq + 2 * q16 + 2 * c16);
-    int32_t* tile_off = reinterpret_cast<int32_t*>(pq + 2 * q16 + 2 * c16 + t4);
-    // exclusive scan of flags[0, N) into pos, the total into result[0]
-    auto scan_flags = [&](const int32_t* flags, int64_t N) {
+    char* pt = pq + 2 * q16 + 2 * c16;
+    int32_t* tile_tot = reinterpret_cast<int32_t*>(pt);
+    int32_t* tile_off = reinterpret_cast<int32_t*>(pt + t4);
+    int32_t* entry = reinterpret_cast<int32_t*>(pt + 2 * t4);  // ceil(J / kChain) <= T entries
+    static_assert(kChain >= kScanTile, "chain entries fit the scan tiles' array");
+    char* ph = pt + 3 * t4;
+    const SmHull h{reinterpret_cast<double*>(ph), reinterpret_cast<uint8_t*>(ph + hy),
+                   reinterpret_cast<uint8_t*>(ph + hy + hx), slots};
+    const SmPrefix pf{pf1, pf2, cf1, cf2, n, JB, B};
+    // exclusive scan of mark[0, N) into pos, the total into result[0]
+    auto scan_marks = [&](int64_t N) {
         const int64_t nt = (N + kScanTile - 1) / kScanTile;
-        hipLaunchKernelGGL(k_sm_scan_local, dim3(static_cast<unsigned>(nt)), dim3(kSmThreads), 0, s, flags, N, pos,
+        hipLaunchKernelGGL(k_sm_scan_local, dim3(static_cast<unsigned>(nt)), dim3(kSmThreads), 0, s, mark, N, pos,
                            tile_tot);
         hipLaunchKernelGGL(k_sm_scan, dim3(1), dim3(kScan), 0, s, tile_tot, nt, tile_off, result);
         hipLaunchKernelGGL(k_sm_scan_add, dim3(blocks(N, 256)), dim3(256), 0, s, pos, N, tile_off);
     };
-    // merge passes reuse the split phase's arrays: group start flags in mark,
-    // group end indices in jump0, segment exits in jump1, group costs in best_cost
-    int32_t *spec = mark, *gend = jump0, *exitk = jump1;
-    double* gcost = best_cost;
-    const int64_t seg = merge_segment_length();
+    // mark[i] = the walk from entry 0 over next() reaches entry i
+    auto chain = [&](auto next, int64_t N) {
+        using F = decltype(next);
+        const unsigned nc = blocks(N, kChain);
+        hipLaunchKernelGGL(k_sm_chain_exit<F>, dim3(nc), dim3(kChainThreads), 0, s, next, N, exits);
+        hipLaunchKernelGGL(k_sm_chain_walk, dim3(1), dim3(64), 0, s, exits, N, static_cast<int64_t>(nc), entry);
+        hipLaunchKernelGGL(k_sm_chain_mark<F>, dim3(nc), dim3(kChainThreads), 0, s, next, N, entry, mark);
+    };
     int rc = dispatch_dtype(dtype, [&](auto t) -> int {
         using T = decltype(t);
         const T* v = static_cast<const T*>(d_values);
-        if (staged) {
-            hipLaunchKernelGGL(k_sm_block_pfx<T>, dim3(static_cast<unsigned>(C)), dim3(kSmThreads), 0, s, v, n, m, J,
-                               pf1, pf2, cf1, cf2);
-            hipLaunchKernelGGL(k_sm_chunk_scan, dim3(1), dim3(kSmThreads), 0, s, cf1, cf2, C);
-            hipLaunchKernelGGL(k_sm_split_lds<T>, dim3(static_cast<unsigned>((J + kSplitStarts - 1) / kSplitStarts)),
-                               dim3(kSmThreads), 0, s, v, n, m, J, pf1, pf2, cf1, cf2, best_end, best_cost);
-        } else
+        if (hulls) {
+            hipLaunchKernelGGL(k_sm_blocks<T>, dim3(static_cast<unsigned>(C)), dim3(kSmThreads), hull_lds(B), s, v, n,
+                               B, JB, pf1, pf2, cf1, cf2, h);
+        } else {
+            hipLaunchKernelGGL(k_sm_sums<T>, dim3(static_cast<unsigned>(JB)), dim3(kSmThreads), 0, s, v, n, B, pf1,
+                               pf2);
+            hipLaunchKernelGGL(k_sm_chunk_pfx, dim3(static_cast<unsigned>(C)), dim3(kPfxChunk), 0, s, JB, pf1, pf2,
+                               cf1, cf2);
+        }
+        GLC_HIP(hipGetLastError());
+        hipLaunchKernelGGL(k_sm_chunk_scan, dim3(1), dim3(kChunkScanThreads), 0, s, cf1, cf2, C);
+        if (hulls) {
+            hipLaunchKernelGGL(k_sm_split_hull<T>, dim3(blocks(J, split_starts(U))), dim3(kSmThreads),
+                               split_lds(U, slots), s, v, n, m, J, U, pf, h, best_end, best_cost);
+        } else {
             hipLaunchKernelGGL(k_sm_split<T>, dim3(static_cast<unsigned>(J)), dim3(kSmThreads), 0, s, v, n, m, J,
                                best_end, best_cost);
-        GLC_HIP(hipGetLastError());
-        hipLaunchKernelGGL(k_sm_chain_init, dim3(blocks(J, 256)), dim3(256), 0, s, best_end, J, m, jump0, mark);
-        GLC_HIP(hipGetLastError());
-        int32_t *ja = jump0, *jb = jump1;
-        for (int64_t reach = 1; reach < J + 1; reach <<= 1) {
-            hipLaunchKernelGGL(k_sm_chain_mark, dim3(blocks(J, 256)), dim3(256), 0, s, ja, J, mark);
-            hipLaunchKernelGGL(k_sm_chain_double, dim3(blocks(J, 256)), dim3(256), 0, s, ja, J, jb);
-            GLC_HIP(hipGetLastError());
-            std::swap(ja, jb);
         }
-        scan_flags(mark, J);
+        GLC_HIP(hipGetLastError());
+        chain(ChainSplit{best_end, J, m}, J);
+        scan_marks(J);
         hipLaunchKernelGGL(k_sm_emit, dim3(blocks(J, 256)), dim3(256), 0, s, mark, pos, best_end, best_cost, J, m,
                            st0, en0, cost0);
         GLC_HIP(hipGetLastError());
@@ -1072,21 +1312,14 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
         GLC_HIP(hipMemcpyAsync(&P, result, 8, hipMemcpyDeviceToHost, s));
         GLC_HIP(hipStreamSynchronize(s));
         if (P < 1 || P > J) return fail(GLC_ERR_STATE, "split phase produced an invalid partition count");
-        const SmPrefix pf{staged ? pf1 : nullptr, pf2, cf1, cf2, m, n, J};  // merge refits: sums from the prefixes
         int32_t *sa = st0, *sb = st1, *ea = en0, *eb = en1;
         double *ca = cost0, *cb = cost1;
         for (int iter = 0; iter < 10 && P > 1; ++iter) {  // CpuPartitioner.cuh:198-242
-            const unsigned g = static_cast<unsigned>(std::min<int64_t>(P - 1, 1 << 20));
-            hipLaunchKernelGGL(k_sm_pair<T>, dim3(g), dim3(kSmThreads), 0, s, v, sa, ea, ca, P, mc, flag, pf);
-            // at most 2^20 segments (one workgroup each)
-            const int64_t sg = std::max<int64_t>(seg, (P + (1 << 20) - 1) >> 20);
-            const int64_t K = (P + sg - 1) / sg;
-            hipLaunchKernelGGL(k_sm_seg<T>, dim3(static_cast<unsigned>(K)), dim3(kSmThreads), 0, s, v, sa, ea, ca, mc,
-                               flag, P, sg, spec, gend, gcost, exitk, pf);
-            hipLaunchKernelGGL(k_sm_fix<T>, dim3(1), dim3(kFixThreads), 0, s, v, sa, ea, ca, mc, flag, P, sg, K, spec,
-                               gend, gcost, exitk, pf);
-            scan_flags(spec, P);
-            hipLaunchKernelGGL(k_sm_emit_groups, dim3(blocks(P, 256)), dim3(256), 0, s, spec, pos, gend, gcost, sa, ea,
+            hipLaunchKernelGGL(k_sm_grow<T>, dim3(blocks(P, kSmThreads / 64)), dim3(kSmThreads), 0, s, v, sa, ea, ca,
+                               P, pf, h, gend, gcost);
+            chain(ChainMerge{gend}, P);
+            scan_marks(P);
+            hipLaunchKernelGGL(k_sm_emit_groups, dim3(blocks(P, 256)), dim3(256), 0, s, mark, pos, gend, gcost, sa, ea,
                                P, sb, eb, cb);
             GLC_HIP(hipGetLastError());
             int64_t Pn = 0;
@@ -1108,6 +1341,11 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
         return GLC_OK;
     });
     if (rc) (void)hipStreamSynchronize(s);  // no kernel of this call may outlive the lock on the scratch
+    if (sc.bytes > kSmKeep) {
+        (void)hipFree(sc.p);
+        sc.p = nullptr;
+        sc.bytes = 0;
+    }
     return rc;
 }
 
