@@ -587,11 +587,309 @@ __device__ __forceinline__ void wave_slow(const DecArgs& a, int64_t e0, int64_t 
     }
 }
 
+// V adjacent values of a lane at p: those with index in [lo, hi) of them, one
+// 16- or 8-byte store when that is all (p is aligned to it).
+template <class O, int V>
+__device__ __forceinline__ void put_values(O* p, const O (&v)[V], int32_t lo, int32_t hi) {
+    if (lo <= 0 && hi >= V) {
+        if constexpr (V * sizeof(O) == 16) {
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            u32x4 q;
+            if constexpr (sizeof(O) == 8) {
+                q.x = static_cast<uint32_t>(static_cast<uint64_t>(v[0]));
+                q.y = static_cast<uint32_t>(static_cast<uint64_t>(v[0]) >> 32);
+                q.z = static_cast<uint32_t>(static_cast<uint64_t>(v[1]));
+                q.w = static_cast<uint32_t>(static_cast<uint64_t>(v[1]) >> 32);
+            } else {
+                q.x = static_cast<uint32_t>(v[0]);
+                q.y = static_cast<uint32_t>(v[1]);
+                q.z = static_cast<uint32_t>(v[2]);
+                q.w = static_cast<uint32_t>(v[3]);
+            }
+            put(reinterpret_cast<u32x4*>(p), q);
+        } else if constexpr (V == 2) {
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            u32x2 q;
+            q.x = static_cast<uint32_t>(v[0]);
+            q.y = static_cast<uint32_t>(v[1]);
+            put(reinterpret_cast<u32x2*>(p), q);
+        } else {
+            put(p, v[0]);
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < V; ++k)
+            if (k >= lo && k < hi) put(p + k, v[k]);
+    }
+}
+
+// Tiles that hold several partitions (or a gap, or a decode-only polynomial
+// model), kSegParts at most: partition by partition, the whole wave on one at a
+// time, so that the model and the bit width are wave-uniform and neighbouring
+// lanes read neighbouring words.  Lanes take V adjacent values aligned to V in
+// the tile (one 16-byte store where all of them are the partition's), V fields
+// of V * bits <= 64 from three words loaded together.  The next partition's
+// descriptor is loaded before the current one is decoded.  5e7 uint32 values in
+// partitions of 1000: 67 us, where a search per value (wave_slow) took 225 us and
+// wave_many takes 95; from about 300 values a partition down wave_many is the
+// faster one (300: 95 against 134 us).
+constexpr int kSegParts = 3;
+
+// Values [s, t) of partition p (descriptor d; s, t in elements) of the tile at
+// e0.  FAST as in narrow_v_rows; 0 also takes DIRECT_COPY and POLY2.
+template <class T, int OP, int V, int FAST>
+__device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t s, int64_t t,
+                                         int lane) {
+    typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
+    constexpr int kSegRows = V == 4 ? 2 : 4;  // in flight; more only cost registers (V = 1: 128 against 117 us)
+    O* __restrict__ out = static_cast<O*>(a.out);
+    const int b = desc_bits(d.packed);
+    const int32_t type = desc_type(d.packed);
+    const int64_t off = desc_off(d.packed);
+    const double t2 = (FAST == 0 && OP != OP_UNPACK && type == MODEL_POLY2) ? a.params[4 * p + 2] : 0.0;
+    const int32_t lo = static_cast<int32_t>(s - e0), hi = static_cast<int32_t>(t - e0);  // in the tile
+    const int32_t kb = static_cast<int32_t>(e0 - d.start);  // tile position x is value kb + x of the partition
+    for (int32_t x0 = lo / V * V + lane * V; x0 - lane * V < hi; x0 += kSegRows * 64 * V) {
+        uint32_t w[kSegRows][3];
+        int64_t pl[kSegRows][V];
+#pragma unroll
+        for (int r = 0; r < kSegRows; ++r) {
+            const int32_t x = x0 + r * 64 * V;
+            if constexpr (OP == OP_PLAIN) {
+#pragma unroll
+                for (int j = 0; j < V; ++j) pl[r][j] = a.plain[e0 + (x + j < lo ? lo : x + j < hi ? x + j : hi - 1)];
+            } else {  // the three words from the lane's first field of the partition on
+                const int32_t xf = x < lo ? lo : x < hi ? x : hi - 1;
+                const int64_t wi = (off + static_cast<int64_t>(kb + xf) * b) >> 5;
+                w[r][0] = a.words[wi];
+                w[r][1] = a.words[wi + 1];
+                w[r][2] = a.words[wi + 2];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kSegRows; ++r) {
+            const int32_t x = x0 + r * 64 * V;
+            const int32_t xf = x < lo ? lo : x < hi ? x : hi - 1;
+            const uint32_t sh = static_cast<uint32_t>(off + static_cast<int64_t>(kb + xf) * b) & 31;
+            O v[V];
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                uint64_t raw;
+                int64_t delta;
+                if constexpr (OP == OP_PLAIN) {
+                    delta = pl[r][j];
+                    raw = static_cast<uint64_t>(delta);
+                } else if constexpr (V == 1) {
+                    raw = static_cast<uint64_t>(__builtin_amdgcn_alignbit(w[r][2], w[r][1], sh)) << 32 |
+                          __builtin_amdgcn_alignbit(w[r][1], w[r][0], sh);
+                    delta = sign_extend(raw, b);
+                    raw = b >= 64 ? raw : raw & ((1ULL << b) - 1ULL);
+                } else {
+                    const int32_t jj = x + j - xf;  // fields after the first loaded one
+                    const uint32_t sk = sh + static_cast<uint32_t>(jj < 0 ? 0 : jj) * b;
+                    const uint32_t idx = sk >> 5;
+                    const uint32_t l = idx == 0 ? w[r][0] : idx == 1 ? w[r][1] : w[r][2];
+                    const uint32_t h = idx == 0 ? w[r][1] : w[r][2];
+                    const uint32_t f = __builtin_amdgcn_alignbit(h, l, sk & 31);
+                    raw = b == 32 ? f : f & ((1u << b) - 1u);
+                    // the builtin returns an unsigned: sign-extend through int32
+                    delta = b == 32 ? static_cast<int64_t>(static_cast<int32_t>(f))
+                                    : static_cast<int64_t>(static_cast<int32_t>(__builtin_amdgcn_sbfe(
+                                          static_cast<int>(f), 0u, static_cast<unsigned>(b))));
+                }
+                const int32_t i = kb + x + j;
+                if constexpr (FAST != 0) v[j] = apply_delta<T>(dec_pred_fast<T, FAST>(d.theta0, d.theta1, i), delta);
+                else if constexpr (OP == OP_UNPACK)
+                    v[j] = type == MODEL_DIRECT_COPY ? static_cast<int64_t>(static_cast<T>(raw)) : delta;
+                else
+                    v[j] = type == MODEL_DIRECT_COPY
+                               ? static_cast<T>(raw)
+                               : apply_delta<T>(dec_pred_poly<T>(type, d.theta0, d.theta1, t2, i), delta);
+            }
+            put_values<O, V>(out + e0 + x, v, lo - x, hi - x);
+        }
+    }
+}
+
+// Values [s, t) of one partition of the tile at e0 (wave-uniform arguments).
+template <class T, int OP>
+__device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t s,
+                                           int64_t t, int lane) {
+    constexpr int kWide = (OP == OP_UNPACK || sizeof(T) == 8) ? 2 : 4;  // values of a 16-byte store
+    const int b = desc_bits(d.packed);
+    const int32_t type = desc_type(d.packed);
+    if constexpr (OP == OP_PACKED) {
+        const double p0 = __builtin_fma(d.theta1, static_cast<double>(s - d.start), d.theta0);
+        const double p1 = __builtin_fma(d.theta1, static_cast<double>(t - 1 - d.start), d.theta0);
+        const bool line = type != MODEL_DIRECT_COPY && type != MODEL_POLY2;
+        const int tier = !line ? 0 : dec_fast_range<T, 1>(p0, p1) ? 1 : (sizeof(T) == 8 && dec_fast_range<T, 2>(p0, p1)) ? 2 : 0;
+        const int u = __builtin_amdgcn_readfirstlane(tier);
+        if (b <= 64 / kWide && b <= 32) {
+            if (u == 1) seg_rows<T, OP, kWide, 1>(a, d, p, e0, s, t, lane);
+            else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, kWide, 2>(a, d, p, e0, s, t, lane);
+            else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+        } else if (sizeof(T) == 4 && b <= 32 && u == 1) {
+            seg_rows<T, OP, 2, 1>(a, d, p, e0, s, t, lane);
+        } else {
+            seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+        }
+    } else if constexpr (OP == OP_UNPACK) {
+        if (b <= 32) seg_rows<T, OP, 2, 0>(a, d, p, e0, s, t, lane);
+        else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+    } else {
+        seg_rows<T, OP, 2, 0>(a, d, p, e0, s, t, lane);
+    }
+}
+
+// Tiles of more than kSegParts partitions, a value per lane.  The tile's
+// descriptors are staged in LDS; the starts set bits of a 1024-bit map, and a
+// value's partition is the number of bits up to it (a popcount of the rows
+// before and a masked count in its own), so no value searches and the payload
+// loads of four rows are in flight together.  5e7 values in partitions of 64:
+// 97-138 us by type and width where the search took 300-350.  Returns false
+// (nothing written) where two partitions share a start (empty ones): the caller
+// searches, as it does for more than kManyParts partitions (3 KB of LDS a wave
+// keeps 8 waves per SIMD).
+constexpr int kManyParts = 96;
+struct ManyLds {
+    Desc d[kManyParts];
+    uint32_t bits[kWaveTile / 32];
+};
+
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <class T, int OP>
+__device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int np, int lane,
+                                          ManyLds& L) {
+    typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
+    O* __restrict__ out = static_cast<O*>(a.out);
+    if (lane < kWaveTile / 32) L.bits[lane] = 0;
+    wave_lds_fence();
+    int wide = 0, starts = 0;
+    for (int i = lane; i < np; i += 64) {
+        const Desc d = a.desc[plo + i];
+        L.d[i] = d;
+        wide |= desc_bits(d.packed) > 32 ? 1 : 0;
+        const int64_t x = d.start - e0;
+        if (i > 0 && x < kWaveTile) {  // x > 0: plo is the last partition that starts at or before e0
+            atomicOr(&L.bits[x >> 5], 1u << (x & 31));
+            ++starts;
+        }
+    }
+    const bool any_wide = __any(wide) != 0;
+    wave_lds_fence();
+    int set = lane < kWaveTile / 32 ? __popc(L.bits[lane]) : 0;
+    for (int o = 32; o > 0; o >>= 1) {
+        set += __shfl_xor(set, o, 64);
+        starts += __shfl_xor(starts, o, 64);
+    }
+    if (set != starts) return false;
+    int base = 0;  // partitions that start in the rows before
+    for (int r0 = 0; r0 < kWaveRows; r0 += 4) {
+        int idx[4];
+        uint32_t w0[4], w1[4], w2[4];
+        int64_t pl[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t lo = __builtin_amdgcn_readfirstlane(L.bits[2 * (r0 + k)]);
+            const uint32_t hi = __builtin_amdgcn_readfirstlane(L.bits[2 * (r0 + k) + 1]);
+            const uint32_t own = lane < 32 ? (lo >> lane) & 1 : (hi >> (lane - 32)) & 1;
+            idx[k] = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, own)));
+            base += __popc(lo) + __popc(hi);
+            const int64_t e = e0 + (r0 + k) * 64 + lane;
+            const Desc& d = L.d[idx[k]];
+            const int64_t i = e - d.start;
+            const bool in = e < e1 && i >= 0 && i < d.len;
+            if constexpr (OP == OP_PLAIN) {
+                pl[k] = a.plain[in ? e : e0];
+            } else {
+                const int64_t wi = in ? (desc_off(d.packed) + i * desc_bits(d.packed)) >> 5 : 0;
+                w0[k] = a.words[wi];
+                w1[k] = a.words[wi + 1];
+                w2[k] = any_wide ? a.words[wi + 2] : 0u;
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int64_t e = e0 + (r0 + k) * 64 + lane;
+            const Desc& d = L.d[idx[k]];
+            const int64_t i = e - d.start;
+            const int32_t type = desc_type(d.packed);
+            O v = O(0);
+            if (i >= 0 && i < d.len) {
+                uint64_t raw;
+                int64_t delta;
+                if constexpr (OP == OP_PLAIN) {
+                    delta = pl[k];
+                    raw = static_cast<uint64_t>(delta);
+                } else {
+                    const int b = desc_bits(d.packed);
+                    const uint32_t sh = static_cast<uint32_t>(desc_off(d.packed) + i * b) & 31;
+                    raw = static_cast<uint64_t>(__builtin_amdgcn_alignbit(w2[k], w1[k], sh)) << 32 |
+                          __builtin_amdgcn_alignbit(w1[k], w0[k], sh);
+                    delta = sign_extend(raw, b);
+                    raw = b >= 64 ? raw : raw & ((1ULL << b) - 1ULL);
+                }
+                if constexpr (OP == OP_UNPACK) {
+                    v = type == MODEL_DIRECT_COPY ? static_cast<int64_t>(static_cast<T>(raw)) : delta;
+                } else if (type == MODEL_DIRECT_COPY) {
+                    v = static_cast<T>(raw);
+                } else {
+                    const int32_t ii = static_cast<int32_t>(i);
+                    v = type == MODEL_POLY2
+                            ? apply_delta<T>(dec_pred_poly<T>(type, d.theta0, d.theta1, a.params[4 * (plo + idx[k]) + 2], ii),
+                                             delta)
+                            : apply_delta<T>(dec_pred<T>(d.theta0, d.theta1, ii), delta);
+                }
+            }
+            if (e < e1) put(out + e, v);
+        }
+    }
+    return true;
+}
+
+// A tile of the partition-spanning path.  out must be 16-byte aligned (VEC).
+template <class T, int OP>
+__device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int lane,
+                                          ManyLds* L) {
+    typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
+    const int64_t phi = a.tile_part[(e1 + kIndexTile - 1) >> kIndexShift];
+    if (phi - plo >= kSegParts) {
+        const int64_t np = phi - plo + 1;
+        if (np > kManyParts || !wave_many<T, OP>(a, e0, e1, plo, static_cast<int>(np), lane, *L))
+            wave_slow<T, OP>(a, e0, e1, plo, lane);
+        return;
+    }
+    O* __restrict__ out = static_cast<O*>(a.out);
+    int64_t done = e0;  // everything before is written
+    Desc next = a.desc[plo];
+    for (int64_t p = plo; p <= phi; ++p) {
+        const Desc d = next;
+        next = a.desc[p < phi ? p + 1 : p];
+        const int64_t ds = d.start, de = ds + d.len;
+        const int64_t s = ds > e0 ? ds : e0, t = de < e1 ? de : e1;
+        if (s >= t) continue;
+        for (int64_t e = done + lane; e < s; e += 64) out[e] = O(0);  // a gap
+        seg_decode<T, OP>(a, d, p, e0, s, t, lane);
+        done = t;
+    }
+    for (int64_t e = done + lane; e < e1; e += 64) out[e] = O(0);
+}
+
 // VEC: narrow tiles take the wide-store path (wave_narrow_v), which needs a
 // 16-byte aligned output; the host picks the instantiation by the output's
 // alignment, so each kernel carries one narrow path only.
-template <class T, int OP, bool VEC = true>
-__device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane) {
+// SEGS: partition-spanning tiles take wave_segs.  Left out where no tile of the
+// launch can span partitions (batches) and of the half-tile kernel: its
+// extra registers (46 -> 72 VGPRs for 64-bit types) leave the whole-tile
+// kernels as fast on columns without such tiles (uint64 2^28 430 against 437
+// us) but cost the half tiles 4 % (420 against 404 us).
+template <class T, int OP, bool VEC = true, bool SEGS = false>
+__device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane, ManyLds* L = nullptr) {
     const int64_t e0 = t * kWaveTile;
     const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
     const TileInfo x = a.tinfo[t];
@@ -601,6 +899,7 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane)
             if constexpr (VEC) wave_plain_v<T>(a, x, e0, e1, lane);
             else wave_plain<T>(a, x, e0, e1, lane);
         }
+        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, a.tile_part[t], lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     } else {
         if (path == TILE_NARROW) {
@@ -610,6 +909,7 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane)
             else wave_narrow_v<T, OP, 2>(a, x, e0, e1, lane);
         }
         else if (path == TILE_WIDE) wave_wide<T, OP>(a, x, e0, e1, lane);
+        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, a.tile_part[t], lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     }
 }
@@ -627,7 +927,12 @@ __global__ __launch_bounds__(64 * WPG) void k_decode_wave(DecArgs a) {
     const int wave = (WPG == 1) ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t t = static_cast<int64_t>(blockIdx.x) * WPG + wave;
     if (t * kWaveTile >= a.n) return;
-    wave_tile<T, OP, VEC>(a, t, lane);
+    if constexpr (VEC) {
+        __shared__ ManyLds L[WPG];
+        wave_tile<T, OP, true, true>(a, t, lane, &L[wave]);
+    } else {
+        wave_tile<T, OP, false>(a, t, lane);
+    }
 }
 
 // Half tiles (packed decode): one-wave workgroup g decodes half g & 1 of
@@ -705,12 +1010,17 @@ __device__ __forceinline__ void batch_tile_unaligned(const DecArgs& a, int64_t t
     wave_slow<T, OP_PACKED>(a, e0, e1, a.tile_part[t], lane);
 }
 
-template <int WPG, int TPW>
+template <int WPG, int TPW, bool SEGS>
 __global__ __launch_bounds__(64 * WPG) void k_batch_decode(const BatchCol* __restrict__ cols,
                                                            const int32_t* __restrict__ tile_col,
                                                            void* const* __restrict__ outs, int64_t Ttot) {
     const int lane = threadIdx.x & 63;
     const int wave = (WPG == 1) ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    ManyLds* L = nullptr;
+    if constexpr (SEGS) {
+        __shared__ ManyLds s_many[WPG];
+        L = &s_many[wave];
+    }
     for (int k = 0; k < TPW; ++k) {
         const int64_t g = (static_cast<int64_t>(blockIdx.x) * WPG + wave) * TPW + k;
         if (g >= Ttot) return;
@@ -735,10 +1045,10 @@ __global__ __launch_bounds__(64 * WPG) void k_batch_decode(const BatchCol* __res
         const int64_t t = g - c.tile_base;
         if (a.vec16) {
             switch (c.dtype) {
-                case GLC_I32: wave_tile<int32_t, OP_PACKED, true>(a, t, lane); break;
-                case GLC_U32: wave_tile<uint32_t, OP_PACKED, true>(a, t, lane); break;
-                case GLC_I64: wave_tile<int64_t, OP_PACKED, true>(a, t, lane); break;
-                default: wave_tile<uint64_t, OP_PACKED, true>(a, t, lane); break;
+                case GLC_I32: wave_tile<int32_t, OP_PACKED, true, SEGS>(a, t, lane, L); break;
+                case GLC_U32: wave_tile<uint32_t, OP_PACKED, true, SEGS>(a, t, lane, L); break;
+                case GLC_I64: wave_tile<int64_t, OP_PACKED, true, SEGS>(a, t, lane, L); break;
+                default: wave_tile<uint64_t, OP_PACKED, true, SEGS>(a, t, lane, L); break;
             }
         } else {
             switch (c.dtype) {
@@ -847,7 +1157,8 @@ DecArgs make_args(const glc_column* c, void* out) {
     return a;
 }
 
-template <class T, int OP, bool VEC> void launch_static(const DecArgs& a, int dsched, int64_t nwt, hipStream_t s) {
+template <class T, int OP, bool VEC>
+void launch_static(const DecArgs& a, int dsched, int64_t nwt, hipStream_t s) {
     if (dsched == GLC_DECODE_HALF_TILE_W1 && OP == OP_PACKED)
         hipLaunchKernelGGL((k_decode_half<T, VEC>), dim3(static_cast<unsigned>(2 * nwt)), dim3(64), 0, s, a, nwt);
     else if (dsched != GLC_DECODE_TILE_W4)
@@ -1006,10 +1317,21 @@ int launch_batch_decode(const BatchPlan& b, int wpg, int tpw, hipStream_t s) {
     auto grid = [&](int w, int t) {
         return dim3(static_cast<unsigned>((b.Ttot + static_cast<int64_t>(w) * t - 1) / (static_cast<int64_t>(w) * t)));
     };
+    // partitions that are no multiple of a tile leave partition-spanning tiles
+    // all over: the instantiation with the segment rows, one or four waves per
+    // workgroup (the other schedules group whole-partition tiles)
+    if (b.S % kIndexTile != 0) {
+        if (wpg == 1) hipLaunchKernelGGL((k_batch_decode<1, 1, true>), grid(1, 1), dim3(64), 0, s, b.cols, b.tile_col,
+                                         b.outs, b.Ttot);
+        else hipLaunchKernelGGL((k_batch_decode<4, 1, true>), grid(4, 1), dim3(256), 0, s, b.cols, b.tile_col, b.outs,
+                                b.Ttot);
+        GLC_HIP(hipGetLastError());
+        return GLC_OK;
+    }
 #define GLC_BATCH_CASE(W, TP)                                                                                     \
     if (wpg == W && tpw == TP) {                                                                                  \
-        hipLaunchKernelGGL((k_batch_decode<W, TP>), grid(W, TP), dim3(64 * W), 0, s, b.cols, b.tile_col, b.outs,   \
-                           b.Ttot);                                                                       \
+        hipLaunchKernelGGL((k_batch_decode<W, TP, false>), grid(W, TP), dim3(64 * W), 0, s, b.cols, b.tile_col,    \
+                           b.outs, b.Ttot);                                                               \
         GLC_HIP(hipGetLastError());                                                                               \
         return GLC_OK;                                                                                            \
     }
