@@ -242,6 +242,7 @@ int finish_index(glc_column* c, hipStream_t s, IndexSummary* out) {
     }
     c->max_bits = out->max_bits;
     c->has_poly = out->has_poly;
+    c->spans = out->unaligned != 0;
     return launch_build_tinfo(c, s);
 }
 

@@ -5,9 +5,8 @@
 //   k_scan        exclusive scan of len*bits -> bit offsets
 //                 (replaces the O(P^2) setBitOffsetsKernel, :222-238)
 //   k_build_index 32-byte decode descriptors + 1024-element tile index
-//   k_pack        bit packer: one workgroup per 2048-element tile, deltas ORed
-//                 into an LDS window, interior words stored once, only the two
-//                 edge words of a tile use a global atomicOr
+//   k_pack_*      bit packer: one wave per 1024-element tile, every word of the
+//                 payload stored once, partial words merged inside a workgroup
 //                 (replaces the per-element atomicOr packer, :243-372)
 //   k_v6_*        GPUVariableLengthPartitionerV6 (compression/GpuPartitioner.cuh:34-214,
 //                 compression/PartitioningKernels.cuh:648-744) without atomics
@@ -739,7 +738,7 @@ __global__ __launch_bounds__(kIndexThreads) void k_build_index(const int32_t* __
                               IndexSummary* __restrict__ sum) {
     const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     const bool live = p < P;  // every lane stays for the wave reductions
-    int bad = 0, bad_bits = 0, poly = 0, not_fixed = 0;
+    int bad = 0, bad_bits = 0, poly = 0, not_fixed = 0, unaligned = 0;
     int32_t b = 0;
     int64_t endbit = 0;
     int32_t s = 0, s_next = 0x7FFFFFFF;
@@ -762,6 +761,7 @@ __global__ __launch_bounds__(kIndexThreads) void k_build_index(const int32_t* __
         if (p + 1 < P && s_next < s) bad = 1;
         bad_bits = (b < 0 || b > 64) ? 1 : 0;
         poly = ty == MODEL_POLY2 ? 1 : 0;
+        unaligned = (len > 0 && (s % kIndexTile != 0 || (e % kIndexTile != 0 && e != n))) ? 1 : 0;
         endbit = off[p] + static_cast<int64_t>(len) * b;
         // fixed-size detection against S = len of partition 0
         const int64_t S = static_cast<int64_t>(en[0]) - st[0];
@@ -772,7 +772,7 @@ __global__ __launch_bounds__(kIndexThreads) void k_build_index(const int32_t* __
     __shared__ int32_t s_flags[kIndexThreads / 64], s_bits[kIndexThreads / 64];
     __shared__ uint64_t s_end[kIndexThreads / 64];
     const int flags = (__any(bad) ? 1 : 0) | (__any(bad_bits) ? 2 : 0) | (__any(poly) ? 4 : 0) |
-                      (__any(not_fixed) ? 8 : 0) | (__any(live) ? 16 : 0);
+                      (__any(not_fixed) ? 8 : 0) | (__any(live) ? 16 : 0) | (__any(unaligned) ? 32 : 0);
     const int32_t wmax_bits = wave_max_all(live ? b : INT32_MIN);
     const uint64_t wend = wave_max_all(live ? static_cast<uint64_t>(endbit) : 0ULL);  // unsigned, as the atomic
     if ((threadIdx.x & 63) == 0) {
@@ -795,6 +795,7 @@ __global__ __launch_bounds__(kIndexThreads) void k_build_index(const int32_t* __
             if (f & 2) atomicOr(&sum->bad_bits, 1);
             if (f & 4) atomicOr(&sum->has_poly, 1);
             if (f & 8) atomicOr(&sum->not_fixed, 1);
+            if (f & 32) atomicOr(&sum->unaligned, 1);
             atomicMax(&sum->max_bits, mb);
             atomicMax(reinterpret_cast<unsigned long long*>(&sum->total_bits), static_cast<unsigned long long>(me));
         }
@@ -865,14 +866,10 @@ __global__ void k_build_tinfo_batch(const BatchCol* __restrict__ cols, const int
 }
 
 // ---------------------------------------------------------------------------
-// Pack.  Tiles inside one partition: one wave per 1024-value tile, word-major
-// (pack_wave).  Other tiles: one workgroup assembles the tile's words in LDS
-// (pack_tile).
+// Pack, one wave per 1024-value tile.  Tiles inside one partition: word-major
+// (pack_wave).  Other tiles: the codes are ORed into the tile's words in LDS
+// (pack_span).
 // ---------------------------------------------------------------------------
-constexpr int kPackThreads = 256;
-constexpr int kPackTile = 1024;                 // values per LDS-assembled tile (one index tile)
-constexpr int kPackWords = kPackTile * 2 + 8;   // 64-bit fields + the 3 words past the last one
-
 // bit position of element e's first bit, or of the next stored bit when e is
 // in a gap / past the end of the last partition with start <= e.
 __device__ __forceinline__ int64_t bitpos_lb(const Desc* __restrict__ desc, int64_t plo, int64_t phi, int64_t e) {
@@ -889,61 +886,6 @@ __device__ __forceinline__ int64_t bitpos_lb(const Desc* __restrict__ desc, int6
     return desc_off(d.packed) + k * desc_bits(d.packed);
 }
 
-// Pack elements [e0, e1) of one column into its payload (zeroed beforehand).
-template <class T>
-__device__ __forceinline__ void pack_tile(const T* __restrict__ v, const Desc* __restrict__ desc,
-                                          const int32_t* __restrict__ tile_part, int64_t e0, int64_t e1,
-                                          uint32_t* __restrict__ words, uint32_t* s_w, int64_t* s_ww) {
-    const int tid = threadIdx.x;
-    const int64_t plo = tile_part[e0 >> kIndexShift];
-    const int64_t phi = tile_part[(e1 + kIndexTile - 1) >> kIndexShift];
-    if (tid == 0) {
-        s_ww[0] = bitpos_lb(desc, plo, phi, e0);
-        s_ww[1] = bitpos_lb(desc, plo, phi, e1 - 1);
-    }
-    for (int i = tid; i < kPackWords; i += kPackThreads) s_w[i] = 0u;
-    __syncthreads();
-    const int64_t wbase = s_ww[0] >> 5;  // first word touched by this tile
-    for (int64_t e = e0 + tid; e < e1; e += kPackThreads) {
-        int64_t lo = plo, hi = phi;
-        while (lo < hi) {
-            int64_t m = (lo + hi + 1) >> 1;
-            if (desc[m].start <= e) lo = m; else hi = m - 1;
-        }
-        const Desc d = desc[lo];
-        if (e < d.start || e >= static_cast<int64_t>(d.start) + d.len) continue;
-        const int b = desc_bits(d.packed);
-        if (b == 0) continue;
-        const int32_t i = static_cast<int32_t>(e - d.start);
-        uint64_t code;
-        if (desc_type(d.packed) == MODEL_DIRECT_COPY) {
-            code = static_cast<uint64_t>(v[e]);
-        } else {
-            code = static_cast<uint64_t>(calc_delta<T>(v[e], enc_pred<T>(d.theta0, d.theta1, i)));
-        }
-        if (b < 64) code &= (1ULL << b) - 1ULL;
-        const int64_t pos = desc_off(d.packed) + static_cast<int64_t>(i) * b;
-        const uint32_t rel = static_cast<uint32_t>(pos - (wbase << 5));
-        const uint32_t wi = rel >> 5, sh = rel & 31;
-        atomicOr(&s_w[wi], static_cast<uint32_t>(code << sh));
-        if (sh + b > 32) atomicOr(&s_w[wi + 1], static_cast<uint32_t>(code >> (32 - sh)));
-        if (sh + b > 64) atomicOr(&s_w[wi + 2], static_cast<uint32_t>(code >> (64 - sh)));
-    }
-    __syncthreads();
-    // words [wbase, wlast]; the first and last may be shared with neighbours
-    const int64_t wlast = (s_ww[1] >= 0) ? (s_ww[1] + 64) >> 5 : wbase;  // covers the last element
-    const int64_t nw = wlast - wbase + 1;
-    for (int64_t k = tid; k < nw && k < kPackWords; k += kPackThreads) {
-        const uint32_t val = s_w[k];
-        if (k == 0 || k >= nw - 3) {
-            if (val) atomicOr(&words[wbase + k], val);
-        } else {
-            words[wbase + k] = val;
-        }
-    }
-    __syncthreads();  // LDS reused by the next tile
-}
-
 // Wave pack of one 1024-value tile that lies inside one partition (the
 // tile's TileInfo path is not TILE_SLOW).  Phase 1: coalesced loads, one
 // residual code per value (lane l: values l, l+64, ...), parked in the
@@ -953,6 +895,10 @@ __device__ __forceinline__ void pack_tile(const T* __restrict__ v, const Desc* _
 // tile.  Every word the tile covers completely is stored whole.  A word the
 // tile starts or ends inside is shared with the neighbouring tile; its
 // partial value is returned as an edge (wave-uniform) for merge_edges.
+// EDGES = false: a column without partition-spanning tiles.  Its partitions
+// start on tiles and its tiles hold 1024 * bits bits, so every tile starts on a
+// word and only the column's last word can be partial, with nothing after it:
+// every word is stored whole, nothing has to be zeroed or merged.
 constexpr int kPackWaves = 4;
 
 struct PackEdge {
@@ -960,7 +906,7 @@ struct PackEdge {
     uint32_t v;
 };
 
-template <class T>
+template <class T, bool EDGES>
 __device__ __forceinline__ void pack_wave(const T* __restrict__ v, const Desc* __restrict__ desc, const TileInfo& x,
                                           int64_t e0, int64_t e1, uint32_t* __restrict__ words, int lane,
                                           uint64_t* __restrict__ s_code, PackEdge& ef, PackEdge& el) {
@@ -1025,10 +971,11 @@ __device__ __forceinline__ void pack_wave(const T* __restrict__ v, const Desc* _
             const int32_t pos = k * b - lo_bit;  // in (-b, 32)
             wv |= (pos >= 0) ? static_cast<uint32_t>(code << pos) : static_cast<uint32_t>(code >> (-pos));
         }
-        if (j == 0 && start_partial) vf = wv;
-        else if (j == Wt - 1 && end_partial) vl = wv;
+        if (EDGES && j == 0 && start_partial) vf = wv;
+        else if (EDGES && j == Wt - 1 && end_partial) vl = wv;
         else words[w0 + j] = wv;
     }
+    if constexpr (!EDGES) return;
     // word 0 is lane 0's first word; word Wt - 1 is lane (Wt - 1) % 64's last
     if (start_partial) ef = PackEdge{words + w0, static_cast<uint32_t>(__builtin_amdgcn_readlane(vf, 0))};
     if (end_partial && !(start_partial && Wt == 1))
@@ -1075,7 +1022,7 @@ __device__ __forceinline__ void merge_edges(const PackEdge* __restrict__ e, int 
     }
 }
 
-template <class T>
+template <class T, bool EDGES>
 __global__ __launch_bounds__(64 * kPackWaves) void k_pack_wave(const T* __restrict__ v, const Desc* __restrict__ desc,
                                                                const TileInfo* __restrict__ tinfo, int64_t n,
                                                                uint32_t* __restrict__ words) {
@@ -1090,9 +1037,10 @@ __global__ __launch_bounds__(64 * kPackWaves) void k_pack_wave(const T* __restri
         const TileInfo x = tinfo[t];
         if (tile_path(x.info) != TILE_SLOW) {
             const int64_t e1 = (e0 + kIndexTile < n) ? e0 + kIndexTile : n;
-            pack_wave<T>(v, desc, x, e0, e1, words, lane, s_code[wave], ef, el);
+            pack_wave<T, EDGES>(v, desc, x, e0, e1, words, lane, s_code[wave], ef, el);
         }
     }
+    if constexpr (!EDGES) return;
     if (lane == 0) {
         s_edge[2 * wave] = ef;
         s_edge[2 * wave + 1] = el;
@@ -1101,43 +1049,210 @@ __global__ __launch_bounds__(64 * kPackWaves) void k_pack_wave(const T* __restri
     if (threadIdx.x == 0) merge_edges(s_edge, 2 * kPackWaves);
 }
 
-// The tiles the wave pack leaves (several partitions, gaps, POLY models):
-// LDS assembly per 1024-value tile.  A workgroup scans kSlowChunk tiles at a
-// time (one path read per thread), lists the slow ones in LDS and packs them
-// one after another; small chunks spread columns with many slow tiles (a
-// partition boundary inside every few tiles) over many workgroups.
-constexpr int kSlowChunk = 8;
+// Pack of one tile of the partition-spanning path by a wave: a value per lane
+// and row, its partition from the staged map (a search over the tile's candidates
+// where that does not apply), its code ORed into the tile's words in LDS (a
+// tile's bits are contiguous: gaps and empty partitions store none), then the
+// words stored in order.  A first or last word that the tile does not fill is
+// returned as an edge (wave-uniform); a tile inside one word that continues on
+// both sides returns that word twice, the second time empty.  2e7 int64 values in
+// partitions of 1000: 63.5 us where a workgroup per tile with a search per
+// value took 130 us; instructions bound it (uint32, half the bytes: 51 us).
+// Values are loaded at once and packed kSpanRows rows at a time, the last
+// partial word carried over, so that a wave needs 5 KB of LDS (the whole tile's
+// words would take 11 and leave 3 waves per SIMD: 97 us).
+constexpr int kSpanRows = 4;
+constexpr int kSpanWords = 2 * 64 * kSpanRows + 4;  // 64-bit fields from any bit of the first word on
+
+// A partition as pack_span takes it, relative to the tile: value x of the tile
+// is the partition's value x - sx and its first bit is bit off + x * bits from the
+// tile's first word on (mod 2^32; a tile has at most 2^16 bits).  32-bit index and
+// bit arithmetic and the branch-free residual where the whole partition allows
+// it: 63.5 us where the same loop on Desc took 75.
+struct alignas(16) SpanDesc {
+    double t0, t1;
+    int32_t sx;
+    uint32_t len;
+    uint32_t off;
+    int32_t info;  // bits | DIRECT_COPY << 8 | enc_fast_range << 9
+};
+struct SpanMap {
+    SpanDesc d[kManyParts];
+    uint32_t bits[kIndexTile / 32];
+};
+
+template <class T> __device__ __forceinline__ SpanDesc span_desc(const Desc& d, int64_t e0, int64_t W0) {
+    const int b = desc_bits(d.packed);
+    const int32_t sx = static_cast<int32_t>(d.start - e0);  // > -2^31: starts are int32 >= 0
+    const bool direct = desc_type(d.packed) == MODEL_DIRECT_COPY;
+    const bool fast =
+        !direct && d.len > 0 &&
+        enc_fast_range<T>(__builtin_fma(d.theta1, 0.0, d.theta0),
+                          __builtin_fma(d.theta1, static_cast<double>(d.len - 1), d.theta0));
+    return SpanDesc{d.theta0, d.theta1, sx, static_cast<uint32_t>(d.len),
+                    static_cast<uint32_t>(desc_off(d.packed) - (W0 & ~31LL)) -
+                        static_cast<uint32_t>(sx) * static_cast<uint32_t>(b),
+                    b | (direct ? 256 : 0) | (fast ? 512 : 0)};
+}
+
 template <class T>
-__global__ __launch_bounds__(kPackThreads) void k_pack_slow(const T* __restrict__ v, const Desc* __restrict__ desc,
-                                                            const int32_t* __restrict__ tile_part,
-                                                            const TileInfo* __restrict__ tinfo, int64_t n,
-                                                            int64_t ntiles, uint32_t* __restrict__ words) {
-    __shared__ uint32_t s_w[kPackWords];
-    __shared__ int64_t s_ww[2];
-    __shared__ int64_t s_list[kSlowChunk];
-    __shared__ int s_cnt;
-    for (int64_t c0 = static_cast<int64_t>(blockIdx.x) * kSlowChunk; c0 < ntiles;
-         c0 += static_cast<int64_t>(gridDim.x) * kSlowChunk) {
-        if (threadIdx.x == 0) s_cnt = 0;
-        __syncthreads();
-        const int64_t t = c0 + threadIdx.x;
-        if (threadIdx.x < kSlowChunk && t < ntiles && tile_path(tinfo[t].info) == TILE_SLOW)
-            s_list[atomicAdd(&s_cnt, 1)] = t;
-        __syncthreads();
-        const int cnt = s_cnt;
-        for (int k = 0; k < cnt; ++k) {
-            const int64_t e0 = s_list[k] * kIndexTile;
-            const int64_t e1 = (e0 + kIndexTile < n) ? e0 + kIndexTile : n;
-            pack_tile<T>(v, desc, tile_part, e0, e1, words, s_w, s_ww);
+__device__ __forceinline__ void pack_span(const T* __restrict__ v, const Desc* __restrict__ desc,
+                                          const int32_t* __restrict__ tile_part, int64_t e0, int64_t e1,
+                                          uint32_t* __restrict__ words, int lane, SpanMap& L, uint32_t* s_w,
+                                          PackEdge& ef, PackEdge& el) {
+    ef = PackEdge{nullptr, 0};
+    el = PackEdge{nullptr, 0};
+    const int32_t cnt = static_cast<int32_t>(e1 - e0);
+    const T* __restrict__ vt = v + e0;
+    T val[kIndexTile / 64];
+#pragma unroll
+    for (int r = 0; r < kIndexTile / 64; ++r) {
+        const int32_t x = r * 64 + lane;
+        val[r] = vt[x < cnt ? x : cnt - 1];
+    }
+    const int64_t plo = tile_part[e0 >> kIndexShift];
+    const int64_t phi = tile_part[(e1 + kIndexTile - 1) >> kIndexShift];
+    const int64_t W0 = bitpos_lb(desc, plo, plo, e0);
+    const bool mapped = phi - plo < kManyParts &&
+                        many_stage(plo, static_cast<int>(phi - plo + 1), lane, L.bits, [&](int64_t p, int i) {
+                            const SpanDesc d = span_desc<T>(desc[p], e0, W0);
+                            L.d[i] = d;
+                            return d.sx;
+                        });
+    int base = 0;
+    uint32_t* __restrict__ out = words + (W0 >> 5);  // word of s_w[0]
+    uint32_t done = 0;                               // bits of the tile's words stored so far
+    int32_t used = static_cast<int32_t>(W0 & 31);    // bits of s_w[0] before this step's
+    uint32_t carry = 0;                              // and their value, of this tile's own bits
+    bool first = used != 0;                          // s_w[0] is the tile's partial first word
+#pragma unroll
+    for (int r0 = 0; r0 < kIndexTile / 64; r0 += kSpanRows) {
+        for (int i = lane; i < kSpanWords; i += 64) s_w[i] = i == 0 ? carry : 0;
+        wave_lds_fence();
+        int32_t end = used;  // bits used, from s_w[0]'s bit 0
+#pragma unroll
+        for (int k = 0; k < kSpanRows; ++k) {
+            const int32_t x = (r0 + k) * 64 + lane;
+            SpanDesc d;
+            if (mapped) {
+                d = L.d[many_index(L.bits, r0 + k, lane, base)];
+            } else {
+                int64_t lo = plo, hi = phi;
+                while (lo < hi) {
+                    const int64_t m = (lo + hi + 1) >> 1;
+                    if (desc[m].start <= e0 + x) lo = m; else hi = m - 1;
+                }
+                d = span_desc<T>(desc[lo], e0, W0);
+            }
+            const int b = d.info & 255;
+            const int32_t i = x - d.sx;
+            if (x >= cnt || static_cast<uint32_t>(i) >= d.len || b == 0) continue;
+            uint64_t code;
+            if (d.info & 512) code = static_cast<uint64_t>(enc_delta_fast<T>(val[r0 + k], d.t0, d.t1, i));
+            else if (d.info & 256) code = static_cast<uint64_t>(val[r0 + k]);
+            else code = static_cast<uint64_t>(calc_delta<T>(val[r0 + k], enc_pred<T>(d.t0, d.t1, i)));
+            const uint32_t rel = d.off + static_cast<uint32_t>(x) * static_cast<uint32_t>(b) - done;
+            const uint32_t wi = rel >> 5, sh = rel & 31;
+            if (b <= 32) {
+                const uint32_t c = static_cast<uint32_t>(code) & (0xFFFFFFFFu >> (32 - b));
+                atomicOr(&s_w[wi], c << sh);
+                if (sh + b > 32) atomicOr(&s_w[wi + 1], c >> (32 - sh));
+            } else {
+                if (b < 64) code &= (1ULL << b) - 1ULL;
+                atomicOr(&s_w[wi], static_cast<uint32_t>(code << sh));
+                if (sh + b > 32) atomicOr(&s_w[wi + 1], static_cast<uint32_t>(code >> (32 - sh)));
+                if (sh + b > 64) atomicOr(&s_w[wi + 2], static_cast<uint32_t>(code >> (64 - sh)));
+            }
+            end = static_cast<int32_t>(rel) + b;  // increases along a lane's values
         }
-        __syncthreads();  // s_cnt / s_list reused by the next chunk
+        for (int o = 32; o > 0; o >>= 1) {
+            const int32_t y = __shfl_xor(end, o, 64);
+            end = y > end ? y : end;
+        }
+        wave_lds_fence();
+        const int32_t full = end >> 5;  // words complete after this step
+        for (int32_t j = lane; j < full; j += 64)
+            if (j > 0 || !first) out[j] = s_w[j];
+        if (full > 0 && first) {
+            ef = PackEdge{out, s_w[0]};
+            first = false;
+        }
+        carry = s_w[full];
+        used = end & 31;
+        out += full;
+        done += static_cast<uint32_t>(full) << 5;
+        wave_lds_fence();  // s_w is the next rows'
+    }
+    // the word the tile ends inside (a tile may also begin inside it)
+    if (used == 0) return;
+    if (first) {
+        if (used == (W0 & 31)) return;  // nothing stored
+        ef = PackEdge{out, carry};
+        carry = 0;
+    }
+    el = PackEdge{out, carry};
+}
+
+// The edges of a workgroup's spanning tiles (first and last of each tile, in
+// bit order; null where there is none).  A run of equal words is the word's
+// whole content when it begins with a tile's last word and ends with a tile's
+// first one, and is stored; every other word has more bits in another tile (of
+// another workgroup, or packed by k_pack_wave before) and is ORed.  One thread.
+__device__ __forceinline__ void merge_span_edges(const PackEdge* __restrict__ e, int m) {
+    int k = 0;
+    while (k < m) {
+        if (!e[k].p) {
+            ++k;
+            continue;
+        }
+        uint32_t v = e[k].v;
+        const bool from_last = (k & 1) != 0;
+        int last = k, q = k + 1;
+        for (; q < m; ++q) {
+            if (!e[q].p) continue;
+            if (e[q].p != e[k].p) break;
+            v |= e[q].v;
+            last = q;
+        }
+        if (from_last && !(last & 1)) *e[k].p = v;
+        else if (v) atomicOr(e[k].p, v);
+        k = q;
     }
 }
 
+struct SpanLds {
+    SpanMap many[kPackWaves];
+    uint32_t w[kPackWaves][kSpanWords];
+    PackEdge edge[2 * kPackWaves];
+};
+
+template <class T>
+__global__ __launch_bounds__(64 * kPackWaves) void k_pack_span(const T* __restrict__ v, const Desc* __restrict__ desc,
+                                                               const int32_t* __restrict__ tile_part,
+                                                               const TileInfo* __restrict__ tinfo, int64_t n,
+                                                               uint32_t* __restrict__ words) {
+    __shared__ SpanLds S;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t t = static_cast<int64_t>(blockIdx.x) * kPackWaves + wave;
+    const int64_t e0 = t * kIndexTile;
+    PackEdge ef{nullptr, 0}, el{nullptr, 0};
+    if (e0 < n && tile_path(tinfo[t].info) == TILE_SLOW) {
+        const int64_t e1 = (e0 + kIndexTile < n) ? e0 + kIndexTile : n;
+        pack_span<T>(v, desc, tile_part, e0, e1, words, lane, S.many[wave], S.w[wave], ef, el);
+    }
+    if (lane == 0) {
+        S.edge[2 * wave] = ef;
+        S.edge[2 * wave + 1] = el;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) merge_span_edges(S.edge, 2 * kPackWaves);
+}
 
 // Batched wave pack over the 1024-value tiles of every column, every element
 // type in one launch (the type comes from the column); tiles that span
-// partitions are left to k_pack_batch.
+// partitions are left to k_pack_span_batch.
+template <bool EDGES>
 __global__ __launch_bounds__(64 * kPackWaves) void k_pack_wave_batch(const BatchCol* __restrict__ cols,
                                                                      const int32_t* __restrict__ tile_col, int64_t Ttot) {
     __shared__ uint64_t s_code[kPackWaves][kIndexTile];
@@ -1156,25 +1271,26 @@ __global__ __launch_bounds__(64 * kPackWaves) void k_pack_wave_batch(const Batch
                 const int64_t e1 = (e0 + kIndexTile < c.n) ? e0 + kIndexTile : c.n;
                 switch (c.dtype) {
                     case GLC_I32:
-                        pack_wave<int32_t>(static_cast<const int32_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
+                        pack_wave<int32_t, EDGES>(static_cast<const int32_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
                                            s_code[wave], ef, el);
                         break;
                     case GLC_U32:
-                        pack_wave<uint32_t>(static_cast<const uint32_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
+                        pack_wave<uint32_t, EDGES>(static_cast<const uint32_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
                                             s_code[wave], ef, el);
                         break;
                     case GLC_I64:
-                        pack_wave<int64_t>(static_cast<const int64_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
+                        pack_wave<int64_t, EDGES>(static_cast<const int64_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
                                            s_code[wave], ef, el);
                         break;
                     default:
-                        pack_wave<uint64_t>(static_cast<const uint64_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
+                        pack_wave<uint64_t, EDGES>(static_cast<const uint64_t*>(c.values), c.desc, x, e0, e1, c.words, lane,
                                             s_code[wave], ef, el);
                         break;
                 }
             }
         }
     }
+    if constexpr (!EDGES) return;
     // tiles of different columns never share a word (separate payloads), so
     // their edges never pair
     if (lane == 0) {
@@ -1185,36 +1301,47 @@ __global__ __launch_bounds__(64 * kPackWaves) void k_pack_wave_batch(const Batch
     if (threadIdx.x == 0) merge_edges(s_edge, 2 * kPackWaves);
 }
 
-template <class T>
-__global__ __launch_bounds__(kPackThreads) void k_pack_batch(const BatchCol* __restrict__ cols,
-                                                             const int32_t* __restrict__ tile_col, int64_t Ttot,
-                                                             int dtype) {
-    __shared__ uint32_t s_w[kPackWords];
-    __shared__ int64_t s_ww[2];
-    __shared__ int64_t s_list[kSlowChunk];
-    __shared__ int s_cnt;
-    for (int64_t c0 = static_cast<int64_t>(blockIdx.x) * kSlowChunk; c0 < Ttot;
-         c0 += static_cast<int64_t>(gridDim.x) * kSlowChunk) {
-        if (threadIdx.x == 0) s_cnt = 0;
-        __syncthreads();
-        const int64_t g = c0 + threadIdx.x;
-        if (threadIdx.x < kSlowChunk && g < Ttot) {
-            const BatchCol& c = cols[tile_col[g]];
-            if (c.dtype == dtype && c.payload_words <= c.words_reserved &&
-                tile_path(c.tinfo[g - c.tile_base].info) == TILE_SLOW)
-                s_list[atomicAdd(&s_cnt, 1)] = g;
-        }
-        __syncthreads();
-        const int cnt = s_cnt;
-        for (int k = 0; k < cnt; ++k) {
-            const int64_t gk = s_list[k];
-            const BatchCol& c = cols[tile_col[gk]];
-            const int64_t e0 = (gk - c.tile_base) * kIndexTile;
+// The spanning tiles of every column of a batch.
+__global__ __launch_bounds__(64 * kPackWaves) void k_pack_span_batch(const BatchCol* __restrict__ cols,
+                                                                     const int32_t* __restrict__ tile_col, int64_t Ttot) {
+    __shared__ SpanLds S;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t g = static_cast<int64_t>(blockIdx.x) * kPackWaves + wave;
+    PackEdge ef{nullptr, 0}, el{nullptr, 0};
+    if (g < Ttot) {
+        const BatchCol& c = cols[tile_col[g]];
+        const int64_t t = g - c.tile_base;
+        if (c.payload_words <= c.words_reserved && tile_path(c.tinfo[t].info) == TILE_SLOW) {
+            const int64_t e0 = t * kIndexTile;
             const int64_t e1 = (e0 + kIndexTile < c.n) ? e0 + kIndexTile : c.n;
-            pack_tile<T>(static_cast<const T*>(c.values), c.desc, c.tile_part, e0, e1, c.words, s_w, s_ww);
+            switch (c.dtype) {
+                case GLC_I32:
+                    pack_span<int32_t>(static_cast<const int32_t*>(c.values), c.desc, c.tile_part, e0, e1, c.words, lane,
+                                       S.many[wave], S.w[wave], ef, el);
+                    break;
+                case GLC_U32:
+                    pack_span<uint32_t>(static_cast<const uint32_t*>(c.values), c.desc, c.tile_part, e0, e1, c.words,
+                                        lane, S.many[wave], S.w[wave], ef, el);
+                    break;
+                case GLC_I64:
+                    pack_span<int64_t>(static_cast<const int64_t*>(c.values), c.desc, c.tile_part, e0, e1, c.words, lane,
+                                       S.many[wave], S.w[wave], ef, el);
+                    break;
+                default:
+                    pack_span<uint64_t>(static_cast<const uint64_t*>(c.values), c.desc, c.tile_part, e0, e1, c.words,
+                                        lane, S.many[wave], S.w[wave], ef, el);
+                    break;
+            }
         }
-        __syncthreads();
     }
+    // tiles of different columns never share a word (separate payloads)
+    if (lane == 0) {
+        S.edge[2 * wave] = ef;
+        S.edge[2 * wave + 1] = el;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) merge_span_edges(S.edge, 2 * kPackWaves);
 }
 
 // ---------------------------------------------------------------------------
@@ -1498,11 +1625,11 @@ int launch_build_tinfo(glc_column* c, hipStream_t s) {
     return GLC_OK;
 }
 
-// Single-column form of k_zero_edges_batch: tile t's first payload word and
-// the three words ending at the one past its last element's first bit are
-// the only words the pack kernels write with atomicOr (merge_edges' outer
-// edges, pack_tile's k == 0 / k >= nw - 3); every other word of the payload
-// is stored whole, so these are all a compress must clear.
+// Columns with partition-spanning tiles: tile t's first payload word and the
+// three words ending at the one past its last element's first bit hold every
+// word that the pack kernels write with atomicOr (the edges of merge_edges and
+// merge_span_edges); every other word of the payload is stored whole, so these
+// are all a compress must clear.  (2^28 uint64 V6: 19 us, now not run.)
 __global__ void k_zero_edges(const Desc* __restrict__ desc, const int32_t* __restrict__ tile_part, int64_t n,
                              int64_t ntiles, uint32_t* __restrict__ words) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1520,7 +1647,7 @@ __global__ void k_zero_edges(const Desc* __restrict__ desc, const int32_t* __res
 
 int launch_zero_edges(glc_column* c, hipStream_t s) {
     const int64_t ntiles = c->n_index - 1;
-    if (c->P == 0 || c->n == 0 || c->total_bits == 0 || ntiles <= 0) return GLC_OK;
+    if (c->P == 0 || c->n == 0 || c->total_bits == 0 || ntiles <= 0 || !c->spans) return GLC_OK;
     hipLaunchKernelGGL(k_zero_edges, dim3(grid_for(ntiles, 256)), dim3(256), 0, s, c->d_desc, c->d_tile_part, c->n,
                        ntiles, c->d_words);
     GLC_HIP(hipGetLastError());
@@ -1532,15 +1659,20 @@ int launch_pack(int dtype, const void* d_values, glc_column* c, hipStream_t s) {
     return dispatch_dtype(dtype, [&](auto t) {
         using T = decltype(t);
         const int64_t ntiles = c->n_index - 1;
-        hipLaunchKernelGGL(k_pack_wave<T>, dim3(grid_for(ntiles, kPackWaves)), dim3(64 * kPackWaves), 0, s,
-                           static_cast<const T*>(d_values),
-                           c->d_desc, c->d_tinfo, c->n, c->d_words);
-        GLC_HIP(hipGetLastError());
-        const int64_t chunks = (ntiles + kSlowChunk - 1) / kSlowChunk;
-        const unsigned gs = static_cast<unsigned>(chunks < 8192 ? (chunks > 0 ? chunks : 1) : 8192);
-        hipLaunchKernelGGL(k_pack_slow<T>, dim3(gs), dim3(kPackThreads), 0, s, static_cast<const T*>(d_values),
-                           c->d_desc, c->d_tile_part, c->d_tinfo, c->n, ntiles, c->d_words);
-        GLC_HIP(hipGetLastError());
+        if (!c->spans) {
+            hipLaunchKernelGGL((k_pack_wave<T, false>), dim3(grid_for(ntiles, kPackWaves)), dim3(64 * kPackWaves), 0, s,
+                               static_cast<const T*>(d_values), c->d_desc, c->d_tinfo, c->n, c->d_words);
+            GLC_HIP(hipGetLastError());
+        } else {
+            hipLaunchKernelGGL((k_pack_wave<T, true>), dim3(grid_for(ntiles, kPackWaves)), dim3(64 * kPackWaves), 0, s,
+                               static_cast<const T*>(d_values), c->d_desc, c->d_tinfo, c->n, c->d_words);
+            GLC_HIP(hipGetLastError());
+            // the other tiles, after every wave-packed word
+            hipLaunchKernelGGL(k_pack_span<T>, dim3(grid_for(ntiles, kPackWaves)), dim3(64 * kPackWaves), 0, s,
+                               static_cast<const T*>(d_values), c->d_desc, c->d_tile_part, c->d_tinfo, c->n,
+                               c->d_words);
+            GLC_HIP(hipGetLastError());
+        }
         return GLC_OK;
     });
 }
@@ -1597,9 +1729,9 @@ __global__ void k_batch_prologue(const BatchCol* __restrict__ cols, int C) {
     if (i < C) *cols[i].sum = IndexSummary{};
 }
 
-// Zero the payload words a 1024-element tile shares with its neighbours (its
-// first word and last three, the ones k_pack_batch ORs into); every other
-// payload word is written whole by exactly one tile.
+// Zero the payload words a 1024-element tile can share with its neighbours
+// (its first word and last three, which hold every word the pack kernels OR
+// into); every other payload word is written whole by exactly one tile.
 __global__ void k_zero_edges_batch(const BatchCol* __restrict__ cols, const int32_t* __restrict__ tile_col,
                                    int64_t Ttot) {
     const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -1657,23 +1789,19 @@ int launch_batch_compress(const BatchPlan& b, hipStream_t s) {
     GLC_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_set_payload_words, dim3(grid_for(b.C, 256)), dim3(256), 0, s, b.cols, b.col_bits, b.C);
     GLC_HIP(hipGetLastError());
+    const unsigned gp = grid_for(b.Ttot, kPackWaves);
+    if (b.S % kIndexTile == 0) {  // no tile spans partitions
+        hipLaunchKernelGGL(k_pack_wave_batch<false>, dim3(gp), dim3(64 * kPackWaves), 0, s, b.cols, b.tile_col, b.Ttot);
+        GLC_HIP(hipGetLastError());
+        return GLC_OK;
+    }
     hipLaunchKernelGGL(k_zero_edges_batch, dim3(grid_for(b.Ttot, 256)), dim3(256), 0, s, b.cols, b.tile_col, b.Ttot);
     GLC_HIP(hipGetLastError());
-    const int64_t pchunks = (b.Ttot + kSlowChunk - 1) / kSlowChunk;
-    const unsigned gp = static_cast<unsigned>(pchunks < 8192 ? (pchunks > 0 ? pchunks : 1) : 8192);
-    hipLaunchKernelGGL(k_pack_wave_batch, dim3(grid_for(b.Ttot, kPackWaves)), dim3(64 * kPackWaves), 0, s, b.cols,
-                       b.tile_col, b.Ttot);
+    hipLaunchKernelGGL(k_pack_wave_batch<true>, dim3(gp), dim3(64 * kPackWaves), 0, s, b.cols, b.tile_col, b.Ttot);
     GLC_HIP(hipGetLastError());
-    for (int dt = GLC_I32; dt <= GLC_U64; ++dt) {  // the partition-spanning tiles, after every wave-packed word
-        if (!b.has_dtype[dt]) continue;
-        int rc = dispatch_dtype(dt, [&](auto t) {
-            using T = decltype(t);
-            hipLaunchKernelGGL(k_pack_batch<T>, dim3(gp), dim3(kPackThreads), 0, s, b.cols, b.tile_col, b.Ttot, dt);
-            GLC_HIP(hipGetLastError());
-            return GLC_OK;
-        });
-        if (rc) return rc;
-    }
+    // the partition-spanning tiles, after every wave-packed word
+    hipLaunchKernelGGL(k_pack_span_batch, dim3(gp), dim3(64 * kPackWaves), 0, s, b.cols, b.tile_col, b.Ttot);
+    GLC_HIP(hipGetLastError());
     return GLC_OK;
 }
 

@@ -631,8 +631,8 @@ __device__ __forceinline__ void put_values(O* p, const O (&v)[V], int32_t lo, in
 // of V * bits <= 64 from three words loaded together.  The next partition's
 // descriptor is loaded before the current one is decoded.  5e7 uint32 values in
 // partitions of 1000: 67 us, where a search per value (wave_slow) took 225 us and
-// wave_many takes 95; from about 300 values a partition down wave_many is the
-// faster one (300: 95 against 134 us).
+// wave_many takes 90; from about 300 values a partition down wave_many is the
+// faster one (300: 81 against 134 us).
 constexpr int kSegParts = 3;
 
 // Values [s, t) of partition p (descriptor d; s, t in elements) of the tile at
@@ -741,53 +741,51 @@ __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int6
     }
 }
 
-// Tiles of more than kSegParts partitions, a value per lane.  The tile's
-// descriptors are staged in LDS; the starts set bits of a 1024-bit map, and a
-// value's partition is the number of bits up to it (a popcount of the rows
-// before and a masked count in its own), so no value searches and the payload
-// loads of four rows are in flight together.  5e7 values in partitions of 64:
-// 97-138 us by type and width where the search took 300-350.  Returns false
-// (nothing written) where two partitions share a start (empty ones): the caller
-// searches, as it does for more than kManyParts partitions (3 KB of LDS a wave
-// keeps 8 waves per SIMD).
-constexpr int kManyParts = 96;
+// Tiles of more than kSegParts partitions, a value per lane: the staged
+// partition map (ManyLds) instead of a search, the payload loads of four rows in
+// flight together.  5e7 values in partitions of 64: 83-121 us by type and width
+// where the search took 300-350.  Returns false (nothing written) where the map
+// does not apply: the caller searches.
+//
+// The staged form: value x of the tile is the partition's value x - sx and its
+// first bit is bit off + x * bits of the payload.
+struct alignas(8) ManyDesc {
+    double t0, t1;
+    int64_t off;
+    int32_t sx;
+    uint32_t len;
+    int32_t info;  // bits | type << 8 | tier << 12 (dec_fast_range over the whole partition, 0 = none)
+    int32_t pad;
+};
 struct ManyLds {
-    Desc d[kManyParts];
+    ManyDesc d[kManyParts];
     uint32_t bits[kWaveTile / 32];
 };
-
-__device__ __forceinline__ void wave_lds_fence() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 template <class T, int OP>
 __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int np, int lane,
                                           ManyLds& L) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
-    O* __restrict__ out = static_cast<O*>(a.out);
-    if (lane < kWaveTile / 32) L.bits[lane] = 0;
-    wave_lds_fence();
-    int wide = 0, starts = 0;
-    for (int i = lane; i < np; i += 64) {
-        const Desc d = a.desc[plo + i];
-        L.d[i] = d;
-        wide |= desc_bits(d.packed) > 32 ? 1 : 0;
-        const int64_t x = d.start - e0;
-        if (i > 0 && x < kWaveTile) {  // x > 0: plo is the last partition that starts at or before e0
-            atomicOr(&L.bits[x >> 5], 1u << (x & 31));
-            ++starts;
+    O* __restrict__ out = static_cast<O*>(a.out) + e0;
+    int wide = 0;
+    const bool ok = many_stage(plo, np, lane, L.bits, [&](int64_t p, int i) {
+        const Desc d = a.desc[p];
+        const int b = desc_bits(d.packed), type = desc_type(d.packed);
+        const int32_t sx = static_cast<int32_t>(d.start - e0);
+        int tier = 0;
+        if (OP != OP_UNPACK && type != MODEL_DIRECT_COPY && type != MODEL_POLY2 && d.len > 0) {
+            const double p0 = __builtin_fma(d.theta1, 0.0, d.theta0);
+            const double p1 = __builtin_fma(d.theta1, static_cast<double>(d.len - 1), d.theta0);
+            tier = dec_fast_range<T, 1>(p0, p1) ? 1 : (sizeof(T) == 8 && dec_fast_range<T, 2>(p0, p1)) ? 2 : 0;
         }
-    }
+        L.d[i] = ManyDesc{d.theta0, d.theta1, desc_off(d.packed) - static_cast<int64_t>(sx) * b, sx,
+                          static_cast<uint32_t>(d.len), b | (type << 8) | (tier << 12), 0};
+        wide |= b > 32 ? 1 : 0;
+        return sx;
+    });
+    if (!ok) return false;
     const bool any_wide = __any(wide) != 0;
-    wave_lds_fence();
-    int set = lane < kWaveTile / 32 ? __popc(L.bits[lane]) : 0;
-    for (int o = 32; o > 0; o >>= 1) {
-        set += __shfl_xor(set, o, 64);
-        starts += __shfl_xor(starts, o, 64);
-    }
-    if (set != starts) return false;
+    const int32_t cnt = static_cast<int32_t>(e1 - e0);
     int base = 0;  // partitions that start in the rows before
     for (int r0 = 0; r0 < kWaveRows; r0 += 4) {
         int idx[4];
@@ -795,19 +793,14 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
         int64_t pl[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const uint32_t lo = __builtin_amdgcn_readfirstlane(L.bits[2 * (r0 + k)]);
-            const uint32_t hi = __builtin_amdgcn_readfirstlane(L.bits[2 * (r0 + k) + 1]);
-            const uint32_t own = lane < 32 ? (lo >> lane) & 1 : (hi >> (lane - 32)) & 1;
-            idx[k] = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, own)));
-            base += __popc(lo) + __popc(hi);
-            const int64_t e = e0 + (r0 + k) * 64 + lane;
-            const Desc& d = L.d[idx[k]];
-            const int64_t i = e - d.start;
-            const bool in = e < e1 && i >= 0 && i < d.len;
+            idx[k] = many_index(L.bits, r0 + k, lane, base);
+            const int32_t x = (r0 + k) * 64 + lane;
+            const ManyDesc& d = L.d[idx[k]];
+            const bool in = x < cnt && static_cast<uint32_t>(x - d.sx) < d.len;
             if constexpr (OP == OP_PLAIN) {
-                pl[k] = a.plain[in ? e : e0];
+                pl[k] = a.plain[e0 + (in ? x : 0)];
             } else {
-                const int64_t wi = in ? (desc_off(d.packed) + i * desc_bits(d.packed)) >> 5 : 0;
+                const int64_t wi = in ? (d.off + static_cast<int64_t>(x) * (d.info & 255)) >> 5 : 0;
                 w0[k] = a.words[wi];
                 w1[k] = a.words[wi + 1];
                 w2[k] = any_wide ? a.words[wi + 2] : 0u;
@@ -815,38 +808,47 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int64_t e = e0 + (r0 + k) * 64 + lane;
-            const Desc& d = L.d[idx[k]];
-            const int64_t i = e - d.start;
-            const int32_t type = desc_type(d.packed);
+            const int32_t x = (r0 + k) * 64 + lane;
+            const ManyDesc& d = L.d[idx[k]];
+            const int32_t i = x - d.sx;
+            const int32_t type = (d.info >> 8) & 15;
             O v = O(0);
-            if (i >= 0 && i < d.len) {
+            if (static_cast<uint32_t>(i) < d.len) {
                 uint64_t raw;
                 int64_t delta;
                 if constexpr (OP == OP_PLAIN) {
                     delta = pl[k];
                     raw = static_cast<uint64_t>(delta);
                 } else {
-                    const int b = desc_bits(d.packed);
-                    const uint32_t sh = static_cast<uint32_t>(desc_off(d.packed) + i * b) & 31;
-                    raw = static_cast<uint64_t>(__builtin_amdgcn_alignbit(w2[k], w1[k], sh)) << 32 |
-                          __builtin_amdgcn_alignbit(w1[k], w0[k], sh);
-                    delta = sign_extend(raw, b);
-                    raw = b >= 64 ? raw : raw & ((1ULL << b) - 1ULL);
+                    const int b = d.info & 255;
+                    const uint32_t sh = (static_cast<uint32_t>(d.off) + static_cast<uint32_t>(x) * static_cast<uint32_t>(b)) & 31;
+                    const uint32_t f = __builtin_amdgcn_alignbit(w1[k], w0[k], sh);
+                    if (any_wide) {  // wave-uniform
+                        raw = static_cast<uint64_t>(__builtin_amdgcn_alignbit(w2[k], w1[k], sh)) << 32 | f;
+                        delta = sign_extend(raw, b);
+                        raw = b >= 64 ? raw : raw & ((1ULL << b) - 1ULL);
+                    } else {
+                        raw = b == 32 ? f : f & ((1u << b) - 1u);
+                        // the builtin returns an unsigned: sign-extend through int32
+                        delta = b == 32 ? static_cast<int64_t>(static_cast<int32_t>(f))
+                                        : static_cast<int64_t>(static_cast<int32_t>(__builtin_amdgcn_sbfe(
+                                              static_cast<int>(f), 0u, static_cast<unsigned>(b))));
+                    }
                 }
                 if constexpr (OP == OP_UNPACK) {
                     v = type == MODEL_DIRECT_COPY ? static_cast<int64_t>(static_cast<T>(raw)) : delta;
-                } else if (type == MODEL_DIRECT_COPY) {
-                    v = static_cast<T>(raw);
                 } else {
-                    const int32_t ii = static_cast<int32_t>(i);
-                    v = type == MODEL_POLY2
-                            ? apply_delta<T>(dec_pred_poly<T>(type, d.theta0, d.theta1, a.params[4 * (plo + idx[k]) + 2], ii),
-                                             delta)
-                            : apply_delta<T>(dec_pred<T>(d.theta0, d.theta1, ii), delta);
+                    const int tier = d.info >> 12;
+                    if (tier == 1) v = apply_delta<T>(dec_pred_fast<T, 1>(d.t0, d.t1, i), delta);
+                    else if (sizeof(T) == 8 && tier == 2) v = apply_delta<T>(dec_pred_fast<T, 2>(d.t0, d.t1, i), delta);
+                    else if (type == MODEL_DIRECT_COPY) v = static_cast<T>(raw);
+                    else
+                        v = apply_delta<T>(dec_pred_poly<T>(type, d.t0, d.t1,
+                                                            type == MODEL_POLY2 ? a.params[4 * (plo + idx[k]) + 2] : 0.0, i),
+                                           delta);
                 }
             }
-            if (e < e1) put(out + e, v);
+            if (x < cnt) put(out + x, v);
         }
     }
     return true;

@@ -224,6 +224,56 @@ __device__ __forceinline__ T decode_value(int32_t type, double t0, double t1, in
     return apply_delta<T>(dec_pred<T>(t0, t1, local), sign_extend(raw, bits));
 }
 
+// The partitions of one 1024-value tile, staged by a wave: their descriptors
+// (the caller's form) and a bit map of the values at which one starts.  A value's
+// partition is then the number of starts up to it: a popcount of the rows of 64
+// before and a masked count in its own, no search.  At most kManyParts partitions
+// (3-4 KB of LDS a wave).
+constexpr int kManyParts = 96;
+
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Stage partitions plo .. plo + np - 1 (np <= kManyParts; plo the last one
+// that starts at or before the tile's first value, or the column's first):
+// stage(p, i) stores partition p as entry i and returns its start relative to
+// the tile.  False where two of them share a start (empty partitions): the map
+// cannot tell them apart.
+template <class F>
+__device__ __forceinline__ bool many_stage(int64_t plo, int np, int lane, uint32_t* bits, F stage) {
+    if (lane < kIndexTile / 32) bits[lane] = 0;
+    wave_lds_fence();
+    int starts = 0;
+    for (int i = lane; i < np; i += 64) {
+        const int32_t x = stage(plo + i, i);
+        if (i > 0 && x < kIndexTile) {  // x > 0
+            atomicOr(&bits[x >> 5], 1u << (x & 31));
+            ++starts;
+        }
+    }
+    wave_lds_fence();
+    int set = lane < kIndexTile / 32 ? __popc(bits[lane]) : 0;
+    for (int o = 32; o > 0; o >>= 1) {
+        set += __shfl_xor(set, o, 64);
+        starts += __shfl_xor(starts, o, 64);
+    }
+    return set == starts;
+}
+
+// Index among the staged partitions of the lane's value in row r; base: starts
+// in the rows before, advanced (call it for r = 0, 1, ... in order).
+__device__ __forceinline__ int many_index(const uint32_t* bits, int r, int lane, int& base) {
+    const uint32_t lo = __builtin_amdgcn_readfirstlane(bits[2 * r]);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane(bits[2 * r + 1]);
+    const uint32_t own = lane < 32 ? (lo >> lane) & 1 : (hi >> (lane - 32)) & 1;
+    const int idx = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, own)));
+    base += __popc(lo) + __popc(hi);
+    return idx;
+}
+
 template <class T> __device__ __forceinline__ void store_out(T* p, T v) { __builtin_nontemporal_store(v, p); }
 
 }  // namespace glc

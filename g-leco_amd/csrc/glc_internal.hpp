@@ -88,7 +88,7 @@ __host__ __device__ inline TileInfo make_tile_info(const Desc& d, int64_t e0, in
 constexpr int kSchedBytes = 1024;  // per-XCD work-stealing queues (16 ints apart) + a done counter
 
 // Summary computed on the device when the index is built (one D2H copy).
-struct IndexSummary {
+struct alignas(64) IndexSummary {  // one 64-byte fill clears it (a fill of 40 bytes is two launches)
     int32_t max_bits;
     int32_t malformed;      // unsorted / overlapping / out-of-range partitions
     int32_t fixed_size;     // S if every partition is [pS, min((p+1)S, N)), else 0
@@ -96,7 +96,9 @@ struct IndexSummary {
     int32_t not_fixed;      // scratch flag for fixed-size detection
     int32_t bad_bits;       // delta_bits outside [0, 64]
     int64_t total_bits;     // max end bit over partitions
+    int32_t unaligned;      // a partition starts, or ends before N, inside a 1024-value tile
 };
+static_assert(sizeof(IndexSummary) == 64, "the scratch slot after the summary is at byte 64");
 
 // Column table entry of a batch (device resident).  Every array pointer
 // points into the batch's shared allocations.
@@ -176,6 +178,7 @@ struct glc_column {
     int32_t fit_block = 0;
     int32_t fit_form = 0;           // contraction form of the fit (glc_opts.fit_form)
     int32_t has_poly = 0;
+    bool spans = false;             // some tile holds several partitions or a gap (IndexSummary::unaligned)
     int32_t dec_sched = GLC_DECODE_TILE_W4;  // packed full-decode schedule (glc_column_set_decode_schedule)
     int32_t dec_pace = 0;                    // pause per decoded row (glc_column_set_decode_pace)
     // arena
