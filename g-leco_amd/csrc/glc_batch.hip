@@ -188,8 +188,6 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
     std::vector<BatchCol> cols(num_columns);
     std::vector<int32_t> part_col, tile_col;
     int64_t Ptot = 0, Ttot = 0, meta = 0, words = 0;
-    bool has[4] = {false, false, false, false};
-    bool wg_fit[4] = {false, false, false, false};
     std::vector<glc::ArenaLayout> lay(num_columns);
     b->meta_off.resize(num_columns);
     b->words_off.resize(num_columns);
@@ -201,7 +199,6 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
         if (ni < 0 || ni > 0x7FFFFFFFLL)
             return bail(fail(GLC_ERR_INVALID_ARG, "column " + std::to_string(i) + ": n must be in [0, 2^31)"));
         if (ni > 0 && !b->values[i]) return bail(fail(GLC_ERR_INVALID_ARG, "null values for column " + std::to_string(i)));
-        has[dt] = has[dt] || ni > 0;
         const int64_t P = (ni + partition_size - 1) / partition_size;
         const int64_t n_index = (ni + glc::kIndexTile - 1) / glc::kIndexTile + 1;
         const int64_t T = n_index - 1;
@@ -221,7 +218,6 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
         c.tile_base = Ttot;
         c.dtype = dt;
         c.fit_bs = glc::fit_block_size(std::min<int64_t>(partition_size, ni));
-        if (P > 0 && c.fit_bs != 256) wg_fit[dt] = true;
         c.words_reserved = b->words_res[i];
         part_col.insert(part_col.end(), static_cast<size_t>(P), i);
         tile_col.insert(tile_col.end(), static_cast<size_t>(T), i);
@@ -284,10 +280,6 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
     p.Ttot = Ttot;
     p.C = num_columns;
     p.S = partition_size;
-    for (int d = 0; d < 4; ++d) {
-        p.has_dtype[d] = has[d];
-        p.has_wg_fit[d] = wg_fit[d];
-    }
     if (hipHostMalloc(reinterpret_cast<void**>(&b->h_outs), sizeof(void*) * std::max(num_columns, 1)) != hipSuccess)
         return bail(fail(GLC_ERR_OOM, "pinned allocation of the output table failed"));
     if (hipEventCreateWithFlags(&b->ev_outs, hipEventDisableTiming) != hipSuccess ||

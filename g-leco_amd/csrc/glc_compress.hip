@@ -1,6 +1,6 @@
 // glc_compress.hip -- compress-side gfx950 kernels of libglc.
 //
-//   k_fit         per-partition overflow check + FP64 linear fit + max |delta|
+//   k_fit_*       per-partition overflow check + FP64 linear fit + max |delta|
 //                 -> bit width (compression/CompressionKernels.cuh:46-218)
 //   k_scan        exclusive scan of len*bits -> bit offsets
 //                 (replaces the O(P^2) setBitOffsetsKernel, :222-238)
@@ -20,20 +20,17 @@
 namespace glc {
 namespace {
 
-constexpr int kFitThreads = 256;
 
 // ---------------------------------------------------------------------------
-// Fit.  One workgroup per partition (grid-stride over partitions).
-// The four sums are accumulated by the first `bs` threads over i = t, t+bs, ...
-// and reduced by the shared-memory tree s = bs/2, bs/4, ..., 1 exactly as the
-// reference does (:113-137), so theta0/theta1 are bit-identical for the same
-// contraction form (fma in sum_xx, sum_xy, det, numerator and theta0).
+// Fit.  The reference's block of `bs` threads (a multiple of 32, at most 256)
+// sums over i = t, t + bs, ... in increasing i and reduces by the tree s = bs/2,
+// bs/4, ..., 1 (:113-137); theta0/theta1 are bit-identical for the same
+// contraction form when every value meets the same additions.  Three forms keep
+// that order: a wave with the partition in registers (fit_wave_reg), a workgroup
+// with it in registers (fit_block_reg), both reading it once, and a workgroup
+// reading it twice (fit_block).  A fourth takes the other block sizes
+// (fit_wave_any).
 // ---------------------------------------------------------------------------
-struct FitSmem {
-    double sum[4][kFitThreads];
-    double theta[2];
-    int64_t mx[kFitThreads / 64];
-};
 
 // Contraction form of the fit's FP64 expressions (:113-158 write a*b + c; the
 // reference build lets nvcc fuse them, which the source does not show):
@@ -45,6 +42,17 @@ struct FitSmem {
 template <int FORM> __device__ __forceinline__ double acc_prod(double a, double b, double s) {
     if constexpr (FORM == 0) return __builtin_fma(a, b, s);
     else return s + a * b;
+}
+
+// Sx = sum of i and Sxx = sum of i^2 over i < n without adding them up: where
+// the tree takes in every thread (bs a power of two), each partial sum is an
+// integer, below 2^53 for n <= kExactN, so every addition and product is exact
+// in either form and in any order.
+constexpr int32_t kExactN = 1 << 17;
+__device__ __forceinline__ void exact_x_sums(int32_t n, double& Sx, double& Sxx) {
+    const int64_t m = n;
+    Sx = static_cast<double>(m * (m - 1) / 2);
+    Sxx = static_cast<double>((m - 1) * m * (2 * m - 1) / 6);  // < 2^53 before the division
 }
 
 // theta from the four sums (:140-160): determinant test, then slope and
@@ -69,104 +77,574 @@ template <class T> __device__ __forceinline__ int64_t abs_delta(T val, double t0
     return dl < 0 ? static_cast<int64_t>(0ULL - static_cast<uint64_t>(dl)) : dl;
 }
 
+template <class T, int TIER> __device__ __forceinline__ int64_t abs_delta_fast(T val, double t0, double t1, int32_t i) {
+    const int64_t dl = enc_delta_fast<T, TIER>(val, t0, t1, i);
+    return dl < 0 ? static_cast<int64_t>(0ULL - static_cast<uint64_t>(dl)) : dl;
+}
+
+// enc_tier of a partition's n predictions
+template <class T> __device__ __forceinline__ int fit_tier(int32_t n, double t0, double t1) {
+    return enc_tier<T>(__builtin_fma(t1, 0.0, t0), __builtin_fma(t1, static_cast<double>(n - 1), t0));
+}
+
 __device__ __forceinline__ int32_t bits_for(int64_t m) {
     if (m <= 0) return 0;
     const int32_t bb = 64 - __builtin_clzll(static_cast<unsigned long long>(m)) + 1;
     return bb > 64 ? 64 : bb;
 }
 
-// Partition p of n values at x (n > 0).  Called by the whole workgroup.
-template <class T, int FORM>
-__device__ __forceinline__ void fit_one(const T* __restrict__ x, int32_t n, int bs, int64_t p, int32_t* __restrict__ type,
-                                        double* __restrict__ params, int32_t* __restrict__ bits,
-                                        int64_t* __restrict__ err, FitSmem& sm) {
-    const int tid = threadIdx.x;
-    double a = 0.0, b = 0.0, c = 0.0, d = 0.0;
-    int ovf = 0;
-    if (tid < bs) {
-        for (int32_t i = tid; i < n; i += bs) {
-            const T val = x[i];
-            ovf |= might_overflow_double<T>(val) ? 1 : 0;
-            const double xi = static_cast<double>(i);
-            const double yi = static_cast<double>(val);
-            a = a + xi;
-            b = b + yi;
-            c = acc_prod<FORM>(xi, xi, c);
-            d = acc_prod<FORM>(xi, yi, d);
-        }
-    }
-    if (__syncthreads_or(ovf)) {  // :95-106 DIRECT_COPY
-        if (tid == 0) {
-            type[p] = MODEL_DIRECT_COPY;
-            params[4 * p] = 0.0; params[4 * p + 1] = 0.0; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-            err[p] = 0;
-            bits[p] = static_cast<int32_t>(sizeof(T) * 8);
-        }
-        __syncthreads();
-        return;
-    }
-    sm.sum[0][tid] = a; sm.sum[1][tid] = b; sm.sum[2][tid] = c; sm.sum[3][tid] = d;
-    __syncthreads();
-    for (int h = bs >> 1; h > 0; h >>= 1) {
-        if (tid < h) {
-            sm.sum[0][tid] = sm.sum[0][tid] + sm.sum[0][tid + h];
-            sm.sum[1][tid] = sm.sum[1][tid] + sm.sum[1][tid + h];
-            sm.sum[2][tid] = sm.sum[2][tid] + sm.sum[2][tid + h];
-            sm.sum[3][tid] = sm.sum[3][tid] + sm.sum[3][tid + h];
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        double t0, t1;
-        fit_theta<FORM>(n, sm.sum[0][0], sm.sum[1][0], sm.sum[2][0], sm.sum[3][0], t0, t1);
-        sm.theta[0] = t0; sm.theta[1] = t1;
-        type[p] = MODEL_LINEAR;
-        params[4 * p] = t0; params[4 * p + 1] = t1; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-    }
-    __syncthreads();
-    const double t0 = sm.theta[0], t1 = sm.theta[1];
-    int64_t mx = 0;
-    for (int32_t i = tid; i < n; i += kFitThreads) {
-        const int64_t ab = abs_delta<T>(x[i], t0, t1, i);
-        mx = ab > mx ? ab : mx;
-    }
+// The fit's outputs, one entry per partition.
+struct FitOut {
+    int32_t* __restrict__ type;
+    double* __restrict__ params;
+    int32_t* __restrict__ bits;
+    int64_t* __restrict__ err;
+};
+// one thread
+__device__ __forceinline__ void fit_store(const FitOut& o, int64_t p, double t0, double t1, int64_t mx) {
+    o.type[p] = MODEL_LINEAR;
+    o.params[4 * p] = t0; o.params[4 * p + 1] = t1; o.params[4 * p + 2] = 0.0; o.params[4 * p + 3] = 0.0;
+    o.err[p] = mx;
+    o.bits[p] = bits_for(mx);
+}
+template <class T> __device__ __forceinline__ void fit_store_direct(const FitOut& o, int64_t p) {  // :95-106 DIRECT_COPY
+    o.type[p] = MODEL_DIRECT_COPY;
+    o.params[4 * p] = 0.0; o.params[4 * p + 1] = 0.0; o.params[4 * p + 2] = 0.0; o.params[4 * p + 3] = 0.0;
+    o.err[p] = 0;
+    o.bits[p] = static_cast<int32_t>(sizeof(T) * 8);
+}
+
+__device__ __forceinline__ int64_t wave_max_i64(int64_t mx) {
     for (int o = 32; o > 0; o >>= 1) {
         const int64_t y = __shfl_xor(mx, o, 64);
         mx = y > mx ? y : mx;
     }
-    if ((tid & 63) == 0) sm.mx[tid >> 6] = mx;
-    __syncthreads();
-    if (tid == 0) {
-        int64_t m = sm.mx[0];
-        for (int w = 1; w < kFitThreads / 64; ++w) m = sm.mx[w] > m ? sm.mx[w] : m;
-        err[p] = m;
-        bits[p] = bits_for(m);
-    }
-    __syncthreads();
+    return mx;
 }
 
-// One wave per partition, for the block size 256 (every partition of 256 or
-// more values at the reference's launch, G:519-520).  Lane l plays the
-// reference's threads l, l+64, l+128 and l+192 (sets j = 0..3), each with its
-// own partial sums over i = tid, tid+256, ... in increasing i.  The tree
-// s = 128, 64, 32, ..., 1 then adds the same operands in the same order: the
-// steps 128 and 64 add sets inside a lane (sum[t] += sum[t + s] with t + s in
-// set j + s/64 of the same lane), the steps 32..1 are shuffles.  No LDS and no
-// barrier: a workgroup's waves work on different partitions.
+// A zero the compiler cannot see through.  Index values that depend only on
+// the lane (i, (double)i, i*i) are loop invariants of a loop over
+// partitions; hoisted out of it they would stay live in registers for the
+// whole loop, and the max-error pass would keep the sums pass's (double)i
+// of every value.
+__device__ __forceinline__ int32_t opaque_zero() {
+    int32_t z;
+    asm volatile("v_mov_b32 %0, 0" : "=v"(z));
+    return z;
+}
+
+// Block size 256, partition p of 0 < n <= 512 * NSTEP values, by one wave that
+// holds it in registers: lane l plays the reference's threads l, l+64, l+128 and
+// l+192 (sets j = 0..3), value i = 64 j + l in set j & 3, increasing i within a
+// set.  The tree's steps 128 and 64 add sets inside a lane (sum[t] += sum[t + s]
+// with t + s in set j + s/64 of the same lane), 32..1 are shuffles; the max-error
+// pass reads the same registers.  No LDS, no barrier.
 constexpr int kFitWaves = 4;
 constexpr int kFitWaveBs = 256;
 
-// Partition p of n > 0 values at x, fitted by one wave.
-template <class T, int FORM>
-__device__ __forceinline__ void fit_wave(const T* __restrict__ x, int32_t n, int64_t p, int32_t* __restrict__ type,
-                                         double* __restrict__ params, int32_t* __restrict__ bits,
-                                         int64_t* __restrict__ err, int lane) {
-    double a[4] = {0.0, 0.0, 0.0, 0.0}, b[4] = {0.0, 0.0, 0.0, 0.0};
-    double c[4] = {0.0, 0.0, 0.0, 0.0}, d[4] = {0.0, 0.0, 0.0, 0.0};
+// Both register forms work in FP64 throughout.  64-bit values are kept as the
+// doubles that the sums need anyway (32-bit ones as they are): with |y| <= 2^52
+// and predictions of tier 1, |y - round(pr)| is the difference of two integers
+// below 2^53 in magnitude, exact, and equals |calc_delta|.  FULL: every lane
+// has a value in every row; else a lane past n sums 0 (x + 0 = x, and no sum is
+// ever -0) and adds no residual.  16 instead of 45 vector instructions a value for
+// int64: instructions were 2/3 of the time.  Values above 2^52, tier 2 and
+// predictions that may saturate read the partition again (fit_again).
+constexpr double kFitExact = 4503599627370496.0;  // 2^52
+template <class T> using FitKeep = typename std::conditional<sizeof(T) == 8, double, T>::type;
+
+// Largest residual of values i = i0, i0 + step, ... < n, read from memory, in
+// integers; -1: a uint64 above 2^53 (DIRECT_COPY).  One lane's share.
+template <class T>
+__device__ __forceinline__ int64_t fit_again(const T* __restrict__ x, int32_t i0, int32_t n, int32_t step, double t0,
+                                             double t1) {
+    const int tier = fit_tier<T>(n, t0, t1);
+    int64_t mx = 0;
     int ovf = 0;
-    // 512 values per step: element base + 64k + lane belongs to set k & 3,
-    // and within a set the steps visit i in increasing order.  Loads are
-    // branch-free (index clamped to n - 1) so all eight are in flight at once.
+    for (int32_t base = i0; base < n; base += 8 * step) {
+        T y[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const int32_t i = base + k * step;
+            y[k] = x[i < n ? i : n - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {  // the clamped index repeats element n - 1: same value
+            const int32_t i = base + k * step, j = i < n ? i : n - 1;
+            ovf |= might_overflow_double<T>(y[k]) ? 1 : 0;
+            int64_t ab;
+            if (tier == 1) ab = abs_delta_fast<T, 1>(y[k], t0, t1, j);
+            else if (std::is_same<T, int64_t>::value && tier == 2) ab = abs_delta_fast<T, 2>(y[k], t0, t1, j);
+            else ab = abs_delta<T>(y[k], t0, t1, j);
+            mx = ab > mx ? ab : mx;
+        }
+    }
+    return ovf ? -1 : mx;
+}
+
+// |y - round(pr)| of value i
+template <class K> __device__ __forceinline__ double fit_resid(K y, double xi, double t0, double t1) {
+    return __builtin_fabs(static_cast<double>(y) - round_away(__builtin_fma(t1, xi, t0)));
+}
+
+template <class T, int FORM, int NSTEP, bool FULL>
+__device__ __forceinline__ void fit_wave_form(const T* __restrict__ x, int32_t n, int64_t p, const FitOut& o,
+                                              int lane_) {
+    constexpr int J = 8 * NSTEP;
+    const int lane = lane_ + opaque_zero();
+    T raw[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) {  // branch-free: every load in flight at once
+        const int32_t i = 64 * j + lane;
+        raw[j] = x[FULL || i < n ? i : n - 1];
+    }
+    FitKeep<T> y[J];
+    double b[4] = {0.0, 0.0, 0.0, 0.0}, d[4] = {0.0, 0.0, 0.0, 0.0}, top = 0.0;
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+        const int32_t i = 64 * j + lane;
+        y[j] = FULL || i < n ? static_cast<FitKeep<T>>(raw[j]) : FitKeep<T>(0);
+        const double yi = static_cast<double>(y[j]);
+        b[j & 3] = b[j & 3] + yi;
+        d[j & 3] = acc_prod<FORM>(static_cast<double>(i), yi, d[j & 3]);
+        if constexpr (sizeof(T) == 8) top = __builtin_fmax(top, __builtin_fabs(yi));
+    }
+    double Sy = (b[0] + b[2]) + (b[1] + b[3]);
+    double Sxy = (d[0] + d[2]) + (d[1] + d[3]);
+    for (int h = 32; h > 0; h >>= 1) {
+        Sy = Sy + __shfl_down(Sy, h, 64);
+        Sxy = Sxy + __shfl_down(Sxy, h, 64);
+    }
+    // lane 0 holds the sums; every lane computes the same theta from them
+    Sy = __shfl(Sy, 0, 64);
+    Sxy = __shfl(Sxy, 0, 64);
+    double Sx, Sxx, t0, t1;
+    exact_x_sums(n, Sx, Sxx);
+    fit_theta<FORM>(n, Sx, Sy, Sxx, Sxy, t0, t1);
+    const int lane2 = lane_ + opaque_zero();  // (double)i afresh: not kept live from the sums pass
+    const bool exact = sizeof(T) == 4 || !__any(!(top <= kFitExact));
+    int64_t mx;
+    if (exact && fit_tier<T>(n, t0, t1) == 1) {
+        double md = 0.0;
+#pragma unroll
+        for (int j = 0; j < J; ++j) {
+            const int32_t i = 64 * j + lane2;
+            const double r = fit_resid(y[j], static_cast<double>(i), t0, t1);
+            md = __builtin_fmax(md, FULL || i < n ? r : 0.0);
+        }
+        mx = static_cast<int64_t>(md);
+    } else {
+        mx = fit_again<T>(x, lane2, n, 64, t0, t1);
+        if (__any(mx < 0 && !std::is_signed<T>::value)) {
+            if (lane == 0) fit_store_direct<T>(o, p);
+            return;
+        }
+    }
+    mx = wave_max_i64(mx);
+    if (lane == 0) fit_store(o, p, t0, t1, mx);
+}
+
+template <class T, int FORM, int NSTEP>
+__device__ __forceinline__ void fit_wave_reg(const T* __restrict__ x, int32_t n, int64_t p, const FitOut& o, int lane) {
+    if (n == 512 * NSTEP) fit_wave_form<T, FORM, NSTEP, true>(x, n, p, o, lane);
+    else fit_wave_form<T, FORM, NSTEP, false>(x, n, p, o, lane);
+}
+
+// Any block size, any n, by one wave: lane l plays threads l + 64 j < bs, the
+// tree runs through s_t (bs doubles), truncated as the reference's is for block
+// sizes that are no power of two.  The block size is 256 except where the
+// column's first partition has at most 224 values, which for fixed sizes means
+// that all are as short: two values a thread at most.
+template <class T, int FORM>
+__device__ __forceinline__ void fit_wave_any(const T* __restrict__ x, int32_t n, int bs, int64_t p, const FitOut& o,
+                                             int lane, double* __restrict__ s_t) {
+    double s[4][4] = {};  // sums x, y, xx, xy of sets j = 0..3
+    int ovf = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int t = lane + 64 * j;
+        if (t < bs) {
+            for (int32_t i = t; i < n; i += bs) {
+                const T val = x[i];
+                ovf |= might_overflow_double<T>(val) ? 1 : 0;
+                const double xi = static_cast<double>(i), yi = static_cast<double>(val);
+                s[0][j] = s[0][j] + xi;
+                s[1][j] = s[1][j] + yi;
+                s[2][j] = acc_prod<FORM>(xi, xi, s[2][j]);
+                s[3][j] = acc_prod<FORM>(xi, yi, s[3][j]);
+            }
+        }
+    }
+    if (__any(ovf)) {
+        if (lane == 0) fit_store_direct<T>(o, p);
+        return;
+    }
+    double tot[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (lane + 64 * j < bs) s_t[lane + 64 * j] = s[q][j];
+        wave_lds_fence();
+        for (int h = bs >> 1; h > 0; h >>= 1) {  // reads [h, 2h), writes [0, h)
+            for (int t = lane; t < h; t += 64) s_t[t] = s_t[t] + s_t[t + h];
+            wave_lds_fence();
+        }
+        tot[q] = s_t[0];
+        wave_lds_fence();  // s_t is the next sum's
+    }
+    double t0, t1;
+    fit_theta<FORM>(n, tot[0], tot[1], tot[2], tot[3], t0, t1);
+    int64_t mx = 0;
+    for (int32_t i = lane; i < n; i += 64) {
+        const int64_t ab = abs_delta<T>(x[i], t0, t1, i);
+        mx = ab > mx ? ab : mx;
+    }
+    mx = wave_max_i64(mx);
+    if (lane == 0) fit_store(o, p, t0, t1, mx);
+}
+
+// Any block size, any n > 0, by a 256-thread workgroup: threads t < bs sum
+// with eight loads in flight, the tree runs through s_t, all threads take the
+// maximum.  Uniform arguments.
+template <class T, int FORM>
+__device__ __forceinline__ void fit_block_any(const T* __restrict__ x, int32_t n, int bs, int64_t p, const FitOut& o,
+                                              double* __restrict__ s_t, int64_t* __restrict__ s_mx) {
+    constexpr int K = 8;
+    const int tid = threadIdx.x;
+    double s[4] = {};  // sums x, y, xx, xy
+    int ovf = 0;
+    if (tid < bs) {
+        for (int32_t base = tid; base < n; base += bs * K) {
+            T y[K];
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int32_t i = base + bs * k;
+                y[k] = x[i < n ? i : n - 1];
+            }
+#pragma unroll
+            for (int k = 0; k < K; ++k) {
+                const int32_t i = base + bs * k;
+                if (i < n) {
+                    ovf |= might_overflow_double<T>(y[k]) ? 1 : 0;
+                    const double xi = static_cast<double>(i), yi = static_cast<double>(y[k]);
+                    s[0] = s[0] + xi;
+                    s[1] = s[1] + yi;
+                    s[2] = acc_prod<FORM>(xi, xi, s[2]);
+                    s[3] = acc_prod<FORM>(xi, yi, s[3]);
+                }
+            }
+        }
+    }
+    if (__syncthreads_or(ovf)) {
+        if (tid == 0) fit_store_direct<T>(o, p);
+        return;
+    }
+    double tot[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        if (tid < bs) s_t[tid] = s[q];
+        __syncthreads();
+        for (int h = bs >> 1; h > 0; h >>= 1) {
+            if (tid < h) s_t[tid] = s_t[tid] + s_t[tid + h];
+            __syncthreads();
+        }
+        tot[q] = s_t[0];
+        __syncthreads();
+    }
+    double t0, t1;
+    fit_theta<FORM>(n, tot[0], tot[1], tot[2], tot[3], t0, t1);
+    int64_t mx = 0;
+    const bool fast = fit_tier<T>(n, t0, t1) == 1;
+    for (int32_t base = tid; base < n; base += 256 * K) {
+        T y[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int32_t i = base + 256 * k;
+            y[k] = x[i < n ? i : n - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {  // the clamped index repeats element n - 1: same value
+            const int32_t i = base + 256 * k, j = i < n ? i : n - 1;
+            const int64_t ab = fast ? abs_delta_fast<T, 1>(y[k], t0, t1, j) : abs_delta<T>(y[k], t0, t1, j);
+            mx = ab > mx ? ab : mx;
+        }
+    }
+    mx = wave_max_i64(mx);
+    if ((tid & 63) == 0) s_mx[tid >> 6] = mx;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < 4; ++w) mx = s_mx[w] > mx ? s_mx[w] : mx;
+        fit_store(o, p, t0, t1, mx);
+    }
+    __syncthreads();  // s_t and s_mx are the next partition's
+}
+
+// The reference's block itself (256 threads): the tree of NS sums per thread,
+// s = 128 and 64 through LDS, 32..1 by shuffles in wave 0; theta to every thread.
+struct FitLds {
+    double sum[4][128];
+    double th[2];
+    int64_t mx[4];
+};
+
+template <int NS> __device__ __forceinline__ void block_tree(double (&s)[NS], FitLds& L) {  // result in thread 0
+    const int tid = threadIdx.x;
+    if (tid >= 128)
+#pragma unroll
+        for (int q = 0; q < NS; ++q) L.sum[q][tid - 128] = s[q];
+    __syncthreads();
+    if (tid < 128)
+#pragma unroll
+        for (int q = 0; q < NS; ++q) s[q] = s[q] + L.sum[q][tid];
+    __syncthreads();
+    if (tid >= 64 && tid < 128)
+#pragma unroll
+        for (int q = 0; q < NS; ++q) L.sum[q][tid - 64] = s[q];
+    __syncthreads();
+    if (tid < 64) {
+#pragma unroll
+        for (int q = 0; q < NS; ++q) s[q] = s[q] + L.sum[q][tid];
+        for (int h = 32; h > 0; h >>= 1)
+#pragma unroll
+            for (int q = 0; q < NS; ++q) s[q] = s[q] + __shfl_down(s[q], h, 64);
+    }
+}
+
+__device__ __forceinline__ void block_store(const FitOut& o, int64_t p, double t0, double t1, int64_t mx, FitLds& L) {
+    mx = wave_max_i64(mx);
+    if ((threadIdx.x & 63) == 0) L.mx[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t m = L.mx[0];
+        for (int w = 1; w < 4; ++w) m = L.mx[w] > m ? L.mx[w] : m;
+        fit_store(o, p, t0, t1, m);
+    }
+    __syncthreads();  // L is the workgroup's next partition's
+}
+
+// Block size 256, 0 < n <= 256 K values, by a workgroup: thread t holds its
+// values i = t, t+256, ... in registers for both passes.  Uniform arguments.
+template <class T, int FORM, int K, bool FULL>
+__device__ __forceinline__ void fit_block_form(const T* __restrict__ x, int32_t n, int64_t p, const FitOut& o,
+                                               FitLds& L) {
+    const int tid = static_cast<int>(threadIdx.x) + opaque_zero();
+    T raw[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {  // branch-free: every load in flight at once
+        const int32_t i = tid + 256 * k;
+        raw[k] = x[FULL || i < n ? i : n - 1];
+    }
+    FitKeep<T> y[K];
+    double s[2] = {0.0, 0.0}, top = 0.0;  // sums y, xy
+#pragma unroll
+    for (int k = 0; k < K; ++k) {  // CompressionKernels.cuh:113-120, thread t's own order
+        const int32_t i = tid + 256 * k;
+        y[k] = FULL || i < n ? static_cast<FitKeep<T>>(raw[k]) : FitKeep<T>(0);
+        const double yi = static_cast<double>(y[k]);
+        s[0] = s[0] + yi;
+        s[1] = acc_prod<FORM>(static_cast<double>(i), yi, s[1]);
+        if constexpr (sizeof(T) == 8) top = __builtin_fmax(top, __builtin_fabs(yi));
+    }
+    const bool exact = sizeof(T) == 4 || !__syncthreads_or(!(top <= kFitExact));
+    block_tree<2>(s, L);
+    if (tid == 0) {
+        double Sx, Sxx;
+        exact_x_sums(n, Sx, Sxx);
+        fit_theta<FORM>(n, Sx, s[0], Sxx, s[1], L.th[0], L.th[1]);
+    }
+    __syncthreads();
+    const double t0 = L.th[0], t1 = L.th[1];
+    const int tid2 = static_cast<int>(threadIdx.x) + opaque_zero();  // (double)i afresh, as in fit_wave_reg
+    int64_t mx;
+    if (exact && fit_tier<T>(n, t0, t1) == 1) {
+        double md = 0.0;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int32_t i = 256 * k + tid2;
+            const double r = fit_resid(y[k], static_cast<double>(i), t0, t1);
+            md = __builtin_fmax(md, FULL || i < n ? r : 0.0);
+        }
+        mx = static_cast<int64_t>(md);
+    } else {
+        mx = fit_again<T>(x, tid2, n, 256, t0, t1);
+        if (!std::is_signed<T>::value && __syncthreads_or(mx < 0)) {
+            if (tid == 0) fit_store_direct<T>(o, p);
+            return;
+        }
+    }
+    block_store(o, p, t0, t1, mx, L);
+}
+
+template <class T, int FORM, int K>
+__device__ __forceinline__ void fit_block_reg(const T* __restrict__ x, int32_t n, int64_t p, const FitOut& o,
+                                              FitLds& L) {
+    if (n == 256 * K) fit_block_form<T, FORM, K, true>(x, n, p, o, L);
+    else fit_block_form<T, FORM, K, false>(x, n, p, o, L);
+}
+
+// Block size 256, any n > 0, by a workgroup that reads the partition twice:
+// eight loads a thread in flight; the max-error pass goes from the end back (the
+// part read last is the one most likely still cached; a maximum has no order).
+template <class T, int FORM>
+__device__ __forceinline__ void fit_block(const T* __restrict__ x, int32_t n, int64_t p, const FitOut& o, FitLds& L) {
+    constexpr int K = 8, kStep = 256 * K;
+    const int tid = threadIdx.x;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};  // sums y, xy, x, xx
+    int ovf = 0;
+    const bool xs = n > kExactN;
+    for (int32_t base = 0; base < n; base += kStep) {
+        T y[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int32_t i = base + tid + 256 * k;
+            y[k] = x[i < n ? i : n - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int32_t i = base + tid + 256 * k;
+            if (i < n) {
+                ovf |= might_overflow_double<T>(y[k]) ? 1 : 0;
+                const double xi = static_cast<double>(i), yi = static_cast<double>(y[k]);
+                s[0] = s[0] + yi;
+                s[1] = acc_prod<FORM>(xi, yi, s[1]);
+                if (xs) {
+                    s[2] = s[2] + xi;
+                    s[3] = acc_prod<FORM>(xi, xi, s[3]);
+                }
+            }
+        }
+    }
+    if (__syncthreads_or(ovf)) {
+        if (tid == 0) fit_store_direct<T>(o, p);
+        return;
+    }
+    block_tree<4>(s, L);
+    if (tid == 0) {
+        double Sx = s[2], Sxx = s[3];
+        if (!xs) exact_x_sums(n, Sx, Sxx);
+        fit_theta<FORM>(n, Sx, s[0], Sxx, s[1], L.th[0], L.th[1]);
+    }
+    __syncthreads();
+    const double t0 = L.th[0], t1 = L.th[1];
+    int64_t mx = 0;
+    const bool fast = fit_tier<T>(n, t0, t1) == 1;
+    for (int32_t base = (n - 1) / kStep * kStep; base >= 0; base -= kStep) {
+        T y[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int32_t i = base + tid + 256 * k;
+            y[k] = x[i < n ? i : n - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {  // the clamped index repeats element n - 1: same value
+            const int32_t i = base + tid + 256 * k, j = i < n ? i : n - 1;
+            const int64_t ab = fast ? abs_delta_fast<T, 1>(y[k], t0, t1, j) : abs_delta<T>(y[k], t0, t1, j);
+            mx = ab > mx ? ab : mx;
+        }
+    }
+    block_store(o, p, t0, t1, mx, L);
+}
+
+// Sizes of the forms (block size 256).  A wave holds up to 2048 values, a
+// workgroup 8192; above, two reads.
+constexpr int32_t kFitWaveMax = 2048;
+constexpr int32_t kFitRegMax = 8192;
+
+// Fixed partitions of at most S values, S <= 512 * NSTEP: a wave each.
+template <class T, int FORM, int NSTEP>
+__global__ __launch_bounds__(64 * kFitWaves) void k_fit_waves(const T* __restrict__ v, const int32_t* __restrict__ st,
+                                                              const int32_t* __restrict__ en, FitOut o, int64_t P) {
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * kFitWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (p >= P) return;
+    const int32_t s0 = st[p];
+    const int32_t n = en[p] - s0;
+    if (n > 0) fit_wave_reg<T, FORM, NSTEP>(v + s0, n, p, o, threadIdx.x & 63);
+}
+
+// Fixed partitions of at most S values, S <= 256 K (K = 0: any): a workgroup each.
+template <class T, int FORM, int K>
+__global__ __launch_bounds__(256) void k_fit_block(const T* __restrict__ v, const int32_t* __restrict__ st,
+                                                   const int32_t* __restrict__ en, FitOut o, int64_t P) {
+    __shared__ FitLds L;
+    const int64_t p = blockIdx.x;
+    const int32_t s0 = st[p];
+    const int32_t n = en[p] - s0;
+    if (n <= 0) return;
+    if constexpr (K > 0) fit_block_reg<T, FORM, K>(v + s0, n, p, o, L);
+    else fit_block<T, FORM>(v + s0, n, p, o, L);
+}
+
+// Mixed sizes (V6, split/merge, explicit partitions), block size 256: workgroup
+// g takes partitions g * chunk .. + chunk.  Its waves first fit the partitions of
+// at most kFitWaveMax values, one each, round robin; then the whole workgroup
+// fits the longer ones, one after the other.  Results do not depend on who fits a
+// partition.  chunk: 16 for long lists (2^28 uint64 V6, 122880 partitions: chunks of
+// 4 / 16 / 64 took 492 / 484 / 497 us), down to 1 where workgroups would be too few
+// (3500 partitions of 20000 values, split/merge 2^26: 618 -> 186 us).
+template <class T, int FORM>
+__global__ __launch_bounds__(256, 4) void k_fit_chunk(const T* __restrict__ v, const int32_t* __restrict__ st,
+                                                   const int32_t* __restrict__ en, FitOut o, int64_t P, int chunk) {
+    __shared__ FitLds L;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * chunk;
+    const int64_t p1 = (p0 + chunk < P) ? p0 + chunk : P;
+    for (int64_t p = p0 + wave; p < p1; p += 4) {
+        const int32_t s0 = st[p];
+        const int32_t n = en[p] - s0;
+        if (n <= 0) continue;  // :62, entry keeps its initial values
+        if (n <= 1024) fit_wave_reg<T, FORM, 2>(v + s0, n, p, o, lane);
+        else if (n <= kFitWaveMax) fit_wave_reg<T, FORM, 4>(v + s0, n, p, o, lane);
+    }
+    for (int64_t p = p0; p < p1; ++p) {  // uniform over the workgroup
+        const int32_t s0 = st[p];
+        const int32_t n = en[p] - s0;
+        if (n <= kFitWaveMax) continue;
+        if (n <= kFitRegMax / 2) fit_block_reg<T, FORM, 16>(v + s0, n, p, o, L);
+        else if (n <= kFitRegMax) fit_block_reg<T, FORM, 32>(v + s0, n, p, o, L);
+        else fit_block<T, FORM>(v + s0, n, p, o, L);
+    }
+}
+
+// Other block sizes, in chunks as k_fit_chunk: partitions of up to 1024 values
+// a wave each, longer ones (mixed sizes whose first partition is short) the
+// workgroup.  2e7 int64 values in partitions of 64: 263 us where a workgroup per
+// partition took 602.
+constexpr int kFitAnyMax = 224;  // the largest block size below 256
+template <class T, int FORM>
+__global__ __launch_bounds__(64 * kFitWaves) void k_fit_any(const T* __restrict__ v, const int32_t* __restrict__ st,
+                                                            const int32_t* __restrict__ en, FitOut o, int64_t P,
+                                                            int bs, int chunk) {
+    __shared__ double s_t[kFitWaves][kFitAnyMax];
+    __shared__ int64_t s_mx[kFitWaves];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * chunk;
+    const int64_t p1 = (p0 + chunk < P) ? p0 + chunk : P;
+    int longer = 0;
+    for (int64_t p = p0 + wave; p < p1; p += kFitWaves) {
+        const int32_t s0 = st[p];
+        const int32_t n = en[p] - s0;
+        if (n > 1024) longer = 1;
+        else if (n > 0) fit_wave_any<T, FORM>(v + s0, n, bs, p, o, threadIdx.x & 63, s_t[wave]);
+    }
+    if (!__syncthreads_or(longer)) return;
+    for (int64_t p = p0; p < p1; ++p) {
+        const int32_t s0 = st[p];
+        const int32_t n = en[p] - s0;
+        if (n > 1024) fit_block_any<T, FORM>(v + s0, n, bs, p, o, s_t[0], s_mx);
+    }
+}
+
+// Block size 256, any n > 0, by one wave reading the partition twice (batches
+// with partitions above kFitWaveMax): fit_wave_reg's order, 512 values a step,
+// eight loads in flight.
+template <class T, int FORM>
+__device__ __forceinline__ void fit_wave_long(const T* __restrict__ x, int32_t n, int64_t p, const FitOut& o,
+                                              int lane) {
+    double a[4] = {}, b[4] = {}, c[4] = {}, d[4] = {};
+    int ovf = 0;
+    const bool xs = n > kExactN;
     for (int32_t base = 0; base < n; base += 2 * kFitWaveBs) {
         T y[8];
 #pragma unroll
@@ -179,47 +657,32 @@ __device__ __forceinline__ void fit_wave(const T* __restrict__ x, int32_t n, int
             const int32_t i = base + 64 * k + lane;
             if (i < n) {
                 ovf |= might_overflow_double<T>(y[k]) ? 1 : 0;
-                const double xi = static_cast<double>(i);
-                const double yi = static_cast<double>(y[k]);
-                a[k & 3] = a[k & 3] + xi;
+                const double xi = static_cast<double>(i), yi = static_cast<double>(y[k]);
                 b[k & 3] = b[k & 3] + yi;
-                c[k & 3] = acc_prod<FORM>(xi, xi, c[k & 3]);
                 d[k & 3] = acc_prod<FORM>(xi, yi, d[k & 3]);
+                if (xs) {
+                    a[k & 3] = a[k & 3] + xi;
+                    c[k & 3] = acc_prod<FORM>(xi, xi, c[k & 3]);
+                }
             }
         }
     }
-    if (__any(ovf)) {  // :95-106 DIRECT_COPY
-        if (lane == 0) {
-            type[p] = MODEL_DIRECT_COPY;
-            params[4 * p] = 0.0; params[4 * p + 1] = 0.0; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-            err[p] = 0;
-            bits[p] = static_cast<int32_t>(sizeof(T) * 8);
-        }
+    if (__any(ovf)) {
+        if (lane == 0) fit_store_direct<T>(o, p);
         return;
     }
-    // s = 128: t < 128 adds t + 128 (set j + 2); s = 64: t < 64 adds t + 64 (set 1)
-    double Sx = (a[0] + a[2]) + (a[1] + a[3]);
-    double Sy = (b[0] + b[2]) + (b[1] + b[3]);
-    double Sxx = (c[0] + c[2]) + (c[1] + c[3]);
-    double Sxy = (d[0] + d[2]) + (d[1] + d[3]);
-    for (int h = 32; h > 0; h >>= 1) {
-        Sx = Sx + __shfl_down(Sx, h, 64);
-        Sy = Sy + __shfl_down(Sy, h, 64);
-        Sxx = Sxx + __shfl_down(Sxx, h, 64);
-        Sxy = Sxy + __shfl_down(Sxy, h, 64);
+    double s[4] = {(b[0] + b[2]) + (b[1] + b[3]), (d[0] + d[2]) + (d[1] + d[3]), (a[0] + a[2]) + (a[1] + a[3]),
+                   (c[0] + c[2]) + (c[1] + c[3])};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        for (int h = 32; h > 0; h >>= 1) s[q] = s[q] + __shfl_down(s[q], h, 64);
+        s[q] = __shfl(s[q], 0, 64);
     }
-    // lane 0 holds the sums; every lane computes the same theta from them
-    Sx = __shfl(Sx, 0, 64);
-    Sy = __shfl(Sy, 0, 64);
-    Sxx = __shfl(Sxx, 0, 64);
-    Sxy = __shfl(Sxy, 0, 64);
+    if (!xs) exact_x_sums(n, s[2], s[3]);
     double t0, t1;
-    fit_theta<FORM>(n, Sx, Sy, Sxx, Sxy, t0, t1);
+    fit_theta<FORM>(n, s[2], s[0], s[3], s[1], t0, t1);
     int64_t mx = 0;
-    const bool fast = enc_fast_range<T>(__builtin_fma(t1, 0.0, t0), __builtin_fma(t1, static_cast<double>(n - 1), t0));
-    // last step first: the end of the partition was read last by the sums
-    // pass and is the part most likely still in cache (the maximum does not
-    // depend on the order)
+    const bool fast = fit_tier<T>(n, t0, t1) == 1;
     for (int32_t base = (n - 1) / (2 * kFitWaveBs) * (2 * kFitWaveBs); base >= 0; base -= 2 * kFitWaveBs) {
         T y[8];
 #pragma unroll
@@ -227,373 +690,50 @@ __device__ __forceinline__ void fit_wave(const T* __restrict__ x, int32_t n, int
             const int32_t i = base + 64 * k + lane;
             y[k] = x[i < n ? i : n - 1];
         }
-        // the clamped index repeats element n - 1: same value
-        if (fast) {
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int32_t i = base + 64 * k + lane;
-                const int64_t dl = enc_delta_fast<T>(y[k], t0, t1, i < n ? i : n - 1);
-                const int64_t ab = dl < 0 ? static_cast<int64_t>(0ULL - static_cast<uint64_t>(dl)) : dl;
-                mx = ab > mx ? ab : mx;
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const int32_t i = base + 64 * k + lane;
-                const int64_t ab = abs_delta<T>(y[k], t0, t1, i < n ? i : n - 1);
-                mx = ab > mx ? ab : mx;
-            }
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        const int64_t y = __shfl_xor(mx, o, 64);
-        mx = y > mx ? y : mx;
-    }
-    if (lane == 0) {
-        type[p] = MODEL_LINEAR;
-        params[4 * p] = t0; params[4 * p + 1] = t1; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-        err[p] = mx;
-        bits[p] = bits_for(mx);
-    }
-}
-
-// Partition p of 0 < n <= 512 * NSTEP values, fitted by one wave that holds
-// the partition in registers: lane l keeps values i = 64 j + l (j < 8 NSTEP),
-// which are exactly fit_wave's loads, summed in fit_wave's order (set j & 3,
-// increasing i within a set); the max-error pass reads the same registers,
-// so the partition crosses HBM once.
-// A zero the compiler cannot see through.  Index values that depend only on
-// the lane (i, (double)i, i*i) are loop invariants of a loop over
-// partitions; hoisted out of it they would stay live in registers for the
-// whole loop, and the max-error pass would keep the sums pass's (double)i
-// of every value (256 VGPRs, occupancy 1 for 64-bit values; 160 and 3 with
-// the lane taken afresh from this zero in the loop and again in each pass).
-__device__ __forceinline__ int32_t opaque_zero() {
-    int32_t z;
-    asm volatile("v_mov_b32 %0, 0" : "=v"(z));
-    return z;
-}
-
-template <class T, int FORM, int NSTEP>
-__device__ __forceinline__ void fit_wave_reg(const T* __restrict__ x, int32_t n, int64_t p,
-                                             int32_t* __restrict__ type, double* __restrict__ params,
-                                             int32_t* __restrict__ bits, int64_t* __restrict__ err, int lane_) {
-    constexpr int J = 8 * NSTEP;
-    const int lane = lane_ + opaque_zero();
-    T y[J];
-#pragma unroll
-    for (int j = 0; j < J; ++j) {  // branch-free: every load in flight at once
-        const int32_t i = 64 * j + lane;
-        y[j] = x[i < n ? i : n - 1];
-    }
-    double a[4] = {0.0, 0.0, 0.0, 0.0}, b[4] = {0.0, 0.0, 0.0, 0.0};
-    double c[4] = {0.0, 0.0, 0.0, 0.0}, d[4] = {0.0, 0.0, 0.0, 0.0};
-    int ovf = 0;
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-        const int32_t i = 64 * j + lane;
-        if (i < n) {
-            ovf |= might_overflow_double<T>(y[j]) ? 1 : 0;
-            const double xi = static_cast<double>(i);
-            const double yi = static_cast<double>(y[j]);
-            a[j & 3] = a[j & 3] + xi;
-            b[j & 3] = b[j & 3] + yi;
-            c[j & 3] = acc_prod<FORM>(xi, xi, c[j & 3]);
-            d[j & 3] = acc_prod<FORM>(xi, yi, d[j & 3]);
-        }
-    }
-    if (__any(ovf)) {  // :95-106 DIRECT_COPY
-        if (lane == 0) {
-            type[p] = MODEL_DIRECT_COPY;
-            params[4 * p] = 0.0; params[4 * p + 1] = 0.0; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-            err[p] = 0;
-            bits[p] = static_cast<int32_t>(sizeof(T) * 8);
-        }
-        return;
-    }
-    double Sx = (a[0] + a[2]) + (a[1] + a[3]);
-    double Sy = (b[0] + b[2]) + (b[1] + b[3]);
-    double Sxx = (c[0] + c[2]) + (c[1] + c[3]);
-    double Sxy = (d[0] + d[2]) + (d[1] + d[3]);
-    for (int h = 32; h > 0; h >>= 1) {
-        Sx = Sx + __shfl_down(Sx, h, 64);
-        Sy = Sy + __shfl_down(Sy, h, 64);
-        Sxx = Sxx + __shfl_down(Sxx, h, 64);
-        Sxy = Sxy + __shfl_down(Sxy, h, 64);
-    }
-    Sx = __shfl(Sx, 0, 64);
-    Sy = __shfl(Sy, 0, 64);
-    Sxx = __shfl(Sxx, 0, 64);
-    Sxy = __shfl(Sxy, 0, 64);
-    double t0, t1;
-    fit_theta<FORM>(n, Sx, Sy, Sxx, Sxy, t0, t1);
-    int64_t mx = 0;
-    const int lane2 = lane_ + opaque_zero();  // (double)i afresh: not kept live from the sums pass
-    // the clamped index repeats element n - 1: same value
-    if (enc_fast_range<T>(__builtin_fma(t1, 0.0, t0), __builtin_fma(t1, static_cast<double>(n - 1), t0))) {
-#pragma unroll
-        for (int j = 0; j < J; ++j) {
-            const int32_t i = 64 * j + lane2;
-            const int64_t dl = enc_delta_fast<T>(y[j], t0, t1, i < n ? i : n - 1);
-            const int64_t ab = dl < 0 ? static_cast<int64_t>(0ULL - static_cast<uint64_t>(dl)) : dl;
-            mx = ab > mx ? ab : mx;
-        }
-    } else {  // predictions outside the fast range (rare): read the partition again, in a short loop
-        for (int32_t i = lane2; i < n; i += 64) {
-            const int64_t ab = abs_delta<T>(x[i], t0, t1, i);
+        for (int k = 0; k < 8; ++k) {  // the clamped index repeats element n - 1: same value
+            const int32_t i = base + 64 * k + lane, j = i < n ? i : n - 1;
+            const int64_t ab = fast ? abs_delta_fast<T, 1>(y[k], t0, t1, j) : abs_delta<T>(y[k], t0, t1, j);
             mx = ab > mx ? ab : mx;
         }
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        const int64_t q = __shfl_xor(mx, o, 64);
-        mx = q > mx ? q : mx;
-    }
-    if (lane == 0) {
-        type[p] = MODEL_LINEAR;
-        params[4 * p] = t0; params[4 * p + 1] = t1; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-        err[p] = mx;
-        bits[p] = bits_for(mx);
-    }
+    mx = wave_max_i64(mx);
+    if (lane == 0) fit_store(o, p, t0, t1, mx);
 }
 
-// Partitions of kFitRegMin..kFitRegMax values (block size 256): one
-// 256-thread workgroup per partition, i.e. the reference's block itself.
-// Thread t loads its values i = t, t+256, ... (at most K of them) into
-// registers once, sums them in increasing i, and the tree s = 128, 64 runs
-// through LDS, s = 32..1 by shuffles in wave 0; the max-error pass then reads
-// the same registers, so the partition crosses HBM once.  Measured on int64
-// 2^29 with 4096-value partitions: 0.76 ms against 1.10 ms for the wave form.
-// Smaller partitions stay with the wave forms (a workgroup per 1024 values
-// spends more on its barriers than the second read costs).
-constexpr int kFitRegK = 16;
-constexpr int32_t kFitRegMin = 2048;
-constexpr int32_t kFitRegMax = 256 * kFitRegK;
-constexpr int32_t kFitRegMax32 = 256 * 32;  // the k_fit_chunk form's largest partition
-constexpr int32_t kFitWaveRegMax = 2048;    // fit_wave_reg<.., 4>'s largest partition
-
-struct FitRegLds {
-    double sum[4][128];
-    double th[2];
-    int64_t mx[4];
-};
-
-// Called by the whole 256-thread workgroup (uniform n, 0 < n <= 256 K).
-template <class T, int FORM, int K>
-__device__ __forceinline__ void fit_block_reg(const T* __restrict__ x, int32_t n, int64_t p,
-                                              int32_t* __restrict__ type, double* __restrict__ params,
-                                              int32_t* __restrict__ bits, int64_t* __restrict__ err, FitRegLds& L) {
-    const int tid = static_cast<int>(threadIdx.x) + opaque_zero();
-    const int lane = tid & 63, wave = tid >> 6;
-    T y[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k) {  // branch-free: every load in flight at once
-        const int32_t i = tid + 256 * k;
-        y[k] = x[i < n ? i : n - 1];
-    }
-    double a = 0.0, b = 0.0, c = 0.0, d = 0.0;
-    int ovf = 0;
-#pragma unroll
-    for (int k = 0; k < K; ++k) {  // CompressionKernels.cuh:113-120, thread t's own order
-        const int32_t i = tid + 256 * k;
-        if (i < n) {
-            ovf |= might_overflow_double<T>(y[k]) ? 1 : 0;
-            const double xi = static_cast<double>(i);
-            const double yi = static_cast<double>(y[k]);
-            a = a + xi;
-            b = b + yi;
-            c = acc_prod<FORM>(xi, xi, c);
-            d = acc_prod<FORM>(xi, yi, d);
-        }
-    }
-    if (__syncthreads_or(ovf)) {  // :95-106 DIRECT_COPY
-        if (tid == 0) {
-            type[p] = MODEL_DIRECT_COPY;
-            params[4 * p] = 0.0; params[4 * p + 1] = 0.0; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-            err[p] = 0;
-            bits[p] = static_cast<int32_t>(sizeof(T) * 8);
-        }
-        return;
-    }
-    // tree (:129-137): s = 128 (t < 128 adds t + 128), s = 64, then 32..1 in wave 0
-    if (tid >= 128) {
-        L.sum[0][tid - 128] = a; L.sum[1][tid - 128] = b; L.sum[2][tid - 128] = c; L.sum[3][tid - 128] = d;
-    }
-    __syncthreads();
-    if (tid < 128) {
-        a = a + L.sum[0][tid]; b = b + L.sum[1][tid]; c = c + L.sum[2][tid]; d = d + L.sum[3][tid];
-    }
-    __syncthreads();
-    if (tid >= 64 && tid < 128) {
-        L.sum[0][tid - 64] = a; L.sum[1][tid - 64] = b; L.sum[2][tid - 64] = c; L.sum[3][tid - 64] = d;
-    }
-    __syncthreads();
-    if (wave == 0) {
-        a = a + L.sum[0][tid]; b = b + L.sum[1][tid]; c = c + L.sum[2][tid]; d = d + L.sum[3][tid];
-        for (int h = 32; h > 0; h >>= 1) {
-            a = a + __shfl_down(a, h, 64);
-            b = b + __shfl_down(b, h, 64);
-            c = c + __shfl_down(c, h, 64);
-            d = d + __shfl_down(d, h, 64);
-        }
-        if (lane == 0) {
-            double t0, t1;
-            fit_theta<FORM>(n, a, b, c, d, t0, t1);
-            L.th[0] = t0;
-            L.th[1] = t1;
-        }
-    }
-    __syncthreads();
-    const double t0 = L.th[0], t1 = L.th[1];
-    int64_t mx = 0;
-    const int tid2 = static_cast<int>(threadIdx.x) + opaque_zero();  // (double)i afresh, as in fit_wave_reg
-    // the clamped index repeats element n - 1: same value
-    if (enc_fast_range<T>(__builtin_fma(t1, 0.0, t0), __builtin_fma(t1, static_cast<double>(n - 1), t0))) {
-#pragma unroll
-        for (int k = 0; k < K; ++k) {
-            const int32_t i = tid2 + 256 * k;
-            const int64_t dl = enc_delta_fast<T>(y[k], t0, t1, i < n ? i : n - 1);
-            const int64_t ab = dl < 0 ? static_cast<int64_t>(0ULL - static_cast<uint64_t>(dl)) : dl;
-            mx = ab > mx ? ab : mx;
-        }
-    } else {  // predictions outside the fast range (rare): read the partition again, in a short loop
-        for (int32_t i = tid2; i < n; i += 256) {
-            const int64_t ab = abs_delta<T>(x[i], t0, t1, i);
-            mx = ab > mx ? ab : mx;
-        }
-    }
-    for (int o = 32; o > 0; o >>= 1) {
-        const int64_t q = __shfl_xor(mx, o, 64);
-        mx = q > mx ? q : mx;
-    }
-    if (lane == 0) L.mx[wave] = mx;
-    __syncthreads();
-    if (tid == 0) {
-        int64_t m = L.mx[0];
-        for (int w = 1; w < 4; ++w) m = L.mx[w] > m ? L.mx[w] : m;
-        type[p] = MODEL_LINEAR;
-        params[4 * p] = t0; params[4 * p + 1] = t1; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
-        err[p] = m;
-        bits[p] = bits_for(m);
-    }
-    __syncthreads();  // L is reused by the workgroup's next partition
+// Batched fit, a wave per partition, every element type in one launch (the
+// type comes from the column).  NMAX: the longest partition of the batch, 1024
+// (64 VGPRs instead of 126, twice the waves), 2048, or 0 for longer ones, which
+// take two reads in the wave.
+template <class T, int NMAX>
+__device__ __forceinline__ void fit_batch_one(const BatchCol& c, int64_t p, int32_t s0, int32_t n, int lane,
+                                              double* s_t) {
+    const FitOut o{c.type, c.params, c.bits, c.err};
+    const T* x = static_cast<const T*>(c.values) + s0;
+    if (c.fit_bs != kFitWaveBs) fit_wave_any<T, 0>(x, n, c.fit_bs, p, o, lane, s_t);
+    else if (NMAX == 1024 || n <= 1024) fit_wave_reg<T, 0, 2>(x, n, p, o, lane);
+    else if (NMAX == 2048 || n <= kFitWaveMax) fit_wave_reg<T, 0, NMAX == 1024 ? 2 : 4>(x, n, p, o, lane);
+    else if constexpr (NMAX == 0) fit_wave_long<T, 0>(x, n, p, o, lane);
 }
 
-template <class T, int FORM>
-__global__ __launch_bounds__(256) void k_fit_reg(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                 const int32_t* __restrict__ en, int32_t* __restrict__ type,
-                                                 double* __restrict__ params, int32_t* __restrict__ bits,
-                                                 int64_t* __restrict__ err, int64_t P) {
-    __shared__ FitRegLds L;
-    const int64_t p = blockIdx.x;
-    if (p >= P) return;
-    const int32_t s0 = st[p];
-    const int32_t n = en[p] - s0;
-    if (n < kFitRegMin || n > kFitRegMax) return;  // the wave form's partitions (uniform per workgroup)
-    fit_block_reg<T, FORM, kFitRegK>(v + s0, n, p, type, params, bits, err, L);
-}
-
-template <class T, int FORM>
-__global__ __launch_bounds__(64 * kFitWaves) void k_fit_wave(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                            const int32_t* __restrict__ en, int32_t* __restrict__ type,
-                                                            double* __restrict__ params, int32_t* __restrict__ bits,
-                                                            int64_t* __restrict__ err, int64_t P, bool skip_reg) {
-    const int lane = threadIdx.x & 63;
-    const int64_t p = static_cast<int64_t>(blockIdx.x) * kFitWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (p >= P) return;
-    const int32_t s0 = st[p];
-    const int32_t n = en[p] - s0;
-    if (n <= 0) return;  // :62, entry keeps its initial values
-    if (skip_reg && n >= kFitRegMin && n <= kFitRegMax) return;  // k_fit_reg's partitions
-    fit_wave<T, FORM>(v + s0, n, p, type, params, bits, err, lane);
-}
-
-// Mixed partition sizes (V6, split/merge, other fixed sizes), block size
-// 256, every partition read from HBM once when it has at most kFitRegMax32
-// values: workgroup g takes partitions g*kFitChunk .. + kFitChunk.  Its waves
-// first fit the partitions of at most kFitWaveRegMax values from registers
-// (one wave each, round robin) and those above kFitRegMax32 with the
-// two-pass wave form; then the whole workgroup fits the ones in between, one
-// after the other, from registers (fit_block_reg).  Results do not depend on
-// who fits a partition: each one follows the reference's order on its own.
-constexpr int kFitChunk = 16;
-
-template <class T, int FORM>
-__global__ __launch_bounds__(256) void k_fit_chunk(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                   const int32_t* __restrict__ en, int32_t* __restrict__ type,
-                                                   double* __restrict__ params, int32_t* __restrict__ bits,
-                                                   int64_t* __restrict__ err, int64_t P) {
-    __shared__ FitRegLds L;
+template <int NMAX>
+__global__ __launch_bounds__(64 * kFitWaves, NMAX == 1024 ? 7 : 4) void k_fit_wave_batch(
+    const BatchCol* __restrict__ cols, const int32_t* __restrict__ part_col, int64_t Ptot, int32_t S) {
+    __shared__ double s_t[kFitWaves][kFitAnyMax];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t p0 = static_cast<int64_t>(blockIdx.x) * kFitChunk;
-    const int64_t p1 = (p0 + kFitChunk < P) ? p0 + kFitChunk : P;
-    for (int64_t p = p0 + wave; p < p1; p += 4) {
-        const int32_t s0 = st[p];
-        const int32_t n = en[p] - s0;
-        if (n <= 0) continue;  // :62, entry keeps its initial values
-        if (n <= 1024) fit_wave_reg<T, FORM, 2>(v + s0, n, p, type, params, bits, err, lane);
-        else if (n <= kFitWaveRegMax) fit_wave_reg<T, FORM, 4>(v + s0, n, p, type, params, bits, err, lane);
-        else if (n > kFitRegMax32) fit_wave<T, FORM>(v + s0, n, p, type, params, bits, err, lane);
-    }
-    for (int64_t p = p0; p < p1; ++p) {  // uniform over the workgroup
-        const int32_t s0 = st[p];
-        const int32_t n = en[p] - s0;
-        if (n <= kFitWaveRegMax || n > kFitRegMax32) continue;
-        if (n <= kFitRegMax) fit_block_reg<T, FORM, kFitRegK>(v + s0, n, p, type, params, bits, err, L);
-        else fit_block_reg<T, FORM, 32>(v + s0, n, p, type, params, bits, err, L);
-    }
-}
-
-template <class T, int FORM>
-__global__ __launch_bounds__(kFitThreads) void k_fit(const T* __restrict__ v, const int32_t* __restrict__ st,
-                                                     const int32_t* __restrict__ en, int32_t* __restrict__ type,
-                                                     double* __restrict__ params, int32_t* __restrict__ bits,
-                                                     int64_t* __restrict__ err, int64_t P, int bs) {
-    __shared__ FitSmem sm;
-    for (int64_t p = blockIdx.x; p < P; p += gridDim.x) {
-        const int32_t s0 = st[p];
-        const int32_t n = en[p] - s0;
-        if (n <= 0) continue;  // :62, entry keeps its initial values
-        fit_one<T, FORM>(v + s0, n, bs, p, type, params, bits, err, sm);
-    }
-}
-
-// Batched fit: global partition g belongs to column part_col[g]; only the
-// columns of element type T are visited (one launch per type present).
-template <class T>
-__global__ __launch_bounds__(kFitThreads) void k_fit_batch(const BatchCol* __restrict__ cols,
-                                                           const int32_t* __restrict__ part_col, int64_t Ptot,
-                                                           int dtype) {
-    __shared__ FitSmem sm;
-    for (int64_t g = blockIdx.x; g < Ptot; g += gridDim.x) {
-        const BatchCol& c = cols[part_col[g]];
-        if (c.dtype != dtype || c.fit_bs == kFitWaveBs) continue;  // block size 256: k_fit_wave_batch
-        const int64_t p = g - c.part_base;
-        const int32_t s0 = c.start[p];
-        const int32_t n = c.end[p] - s0;
-        if (n <= 0) continue;
-        fit_one<T, 0>(static_cast<const T*>(c.values) + s0, n, c.fit_bs, p, c.type, c.params, c.bits, c.err, sm);
-    }
-}
-
-// Batched fit, one wave per partition of the columns whose block size is
-// 256, every element type in one launch (the type comes from the column).
-__global__ __launch_bounds__(64 * kFitWaves) void k_fit_wave_batch(const BatchCol* __restrict__ cols,
-                                                                  const int32_t* __restrict__ part_col, int64_t Ptot) {
-    const int lane = threadIdx.x & 63;
-    const int64_t g = static_cast<int64_t>(blockIdx.x) * kFitWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t g = static_cast<int64_t>(blockIdx.x) * kFitWaves + wave;
     if (g >= Ptot) return;
     const BatchCol& c = cols[part_col[g]];
-    if (c.fit_bs != kFitWaveBs) return;
     const int64_t p = g - c.part_base;
-    const int32_t s0 = c.start[p];
-    const int32_t n = c.end[p] - s0;
+    const int32_t s0 = static_cast<int32_t>(p * S);  // as k_fixed_parts_batch writes them; no load to wait for
+    const int32_t n = static_cast<int32_t>(c.n - s0 < S ? c.n - s0 : S);
     if (n <= 0) return;
     switch (c.dtype) {
-        case GLC_I32: fit_wave<int32_t, 0>(static_cast<const int32_t*>(c.values) + s0, n, p, c.type, c.params, c.bits, c.err, lane); break;
-        case GLC_U32: fit_wave<uint32_t, 0>(static_cast<const uint32_t*>(c.values) + s0, n, p, c.type, c.params, c.bits, c.err, lane); break;
-        case GLC_I64: fit_wave<int64_t, 0>(static_cast<const int64_t*>(c.values) + s0, n, p, c.type, c.params, c.bits, c.err, lane); break;
-        default: fit_wave<uint64_t, 0>(static_cast<const uint64_t*>(c.values) + s0, n, p, c.type, c.params, c.bits, c.err, lane); break;
+        case GLC_I32: fit_batch_one<int32_t, NMAX>(c, p, s0, n, lane, s_t[wave]); break;
+        case GLC_U32: fit_batch_one<uint32_t, NMAX>(c, p, s0, n, lane, s_t[wave]); break;
+        case GLC_I64: fit_batch_one<int64_t, NMAX>(c, p, s0, n, lane, s_t[wave]); break;
+        default: fit_batch_one<uint64_t, NMAX>(c, p, s0, n, lane, s_t[wave]); break;
     }
 }
 
@@ -927,12 +1067,21 @@ __device__ __forceinline__ void pack_wave(const T* __restrict__ v, const Desc* _
     }
     // Tiles whose predictions need no saturation (the common case) take the
     // branch-free residual; the codes are the same either way.
-    if (!direct && enc_fast_range<T>(__builtin_fma(x.t1, static_cast<double>(lbase), x.t0),
-                                     __builtin_fma(x.t1, static_cast<double>(lbase + cnt - 1), x.t0))) {
+    const int tier = direct ? 0
+                            : enc_tier<T>(__builtin_fma(x.t1, static_cast<double>(lbase), x.t0),
+                                          __builtin_fma(x.t1, static_cast<double>(lbase + cnt - 1), x.t0));
+    if (tier == 1) {
 #pragma unroll
         for (int r = 0; r < kIndexTile / 64; ++r) {
             const int32_t k = r * 64 + lane;
-            const uint64_t code = static_cast<uint64_t>(enc_delta_fast<T>(val[r], x.t0, x.t1, lbase + k));
+            const uint64_t code = static_cast<uint64_t>(enc_delta_fast<T, 1>(val[r], x.t0, x.t1, lbase + k));
+            s_code[k] = (k < cnt) ? (code & mask) : 0;
+        }
+    } else if (std::is_same<T, int64_t>::value && tier == 2) {
+#pragma unroll
+        for (int r = 0; r < kIndexTile / 64; ++r) {
+            const int32_t k = r * 64 + lane;
+            const uint64_t code = static_cast<uint64_t>(enc_delta_fast<T, 2>(val[r], x.t0, x.t1, lbase + k));
             s_code[k] = (k < cnt) ? (code & mask) : 0;
         }
     } else {
@@ -1074,7 +1223,7 @@ struct alignas(16) SpanDesc {
     int32_t sx;
     uint32_t len;
     uint32_t off;
-    int32_t info;  // bits | DIRECT_COPY << 8 | enc_fast_range << 9
+    int32_t info;  // bits | DIRECT_COPY << 8 | tier 1 of enc_tier << 9
 };
 struct SpanMap {
     SpanDesc d[kManyParts];
@@ -1085,10 +1234,7 @@ template <class T> __device__ __forceinline__ SpanDesc span_desc(const Desc& d, 
     const int b = desc_bits(d.packed);
     const int32_t sx = static_cast<int32_t>(d.start - e0);  // > -2^31: starts are int32 >= 0
     const bool direct = desc_type(d.packed) == MODEL_DIRECT_COPY;
-    const bool fast =
-        !direct && d.len > 0 &&
-        enc_fast_range<T>(__builtin_fma(d.theta1, 0.0, d.theta0),
-                          __builtin_fma(d.theta1, static_cast<double>(d.len - 1), d.theta0));
+    const bool fast = !direct && d.len > 0 && fit_tier<T>(d.len, d.theta0, d.theta1) == 1;
     return SpanDesc{d.theta0, d.theta1, sx, static_cast<uint32_t>(d.len),
                     static_cast<uint32_t>(desc_off(d.packed) - (W0 & ~31LL)) -
                         static_cast<uint32_t>(sx) * static_cast<uint32_t>(b),
@@ -1556,33 +1702,35 @@ inline unsigned grid_for(int64_t work, int64_t per_block, int64_t cap = 1LL << 3
 
 template <class T, int FORM>
 int launch_fit_t(const void* d_values, glc_column* c, int32_t bs, int32_t fixed_size, hipStream_t s) {
-    if (bs == kFitWaveBs) {
-        // fixed partitions of kFitRegMin..kFitRegMax values: the register
-        // form (and k_fit_wave's launch covers only the last, shorter one);
-        // every other layout: k_fit_chunk (one launch; a second launch that
-        // skips the first one's partitions costs more than it saves: 602 us
-        // against 555 us on the uint64 2^28 V6 column)
-        if (fixed_size >= kFitRegMin && fixed_size <= kFitRegMax) {
-            hipLaunchKernelGGL((k_fit_reg<T, FORM>), dim3(static_cast<unsigned>(c->P)), dim3(256), 0, s,
-                               static_cast<const T*>(d_values), c->d_start, c->d_end, c->d_type, c->d_params,
-                               c->d_bits, c->d_err, c->P);
-            GLC_HIP(hipGetLastError());
-            const unsigned g = static_cast<unsigned>((c->P + kFitWaves - 1) / kFitWaves);
-            hipLaunchKernelGGL((k_fit_wave<T, FORM>), dim3(g), dim3(64 * kFitWaves), 0, s,
-                               static_cast<const T*>(d_values), c->d_start, c->d_end, c->d_type, c->d_params,
-                               c->d_bits, c->d_err, c->P, true);
-            GLC_HIP(hipGetLastError());
-            return GLC_OK;
-        }
-        const unsigned g = static_cast<unsigned>((c->P + kFitChunk - 1) / kFitChunk);
-        hipLaunchKernelGGL((k_fit_chunk<T, FORM>), dim3(g), dim3(256), 0, s, static_cast<const T*>(d_values),
-                           c->d_start, c->d_end, c->d_type, c->d_params, c->d_bits, c->d_err, c->P);
-        GLC_HIP(hipGetLastError());
-        return GLC_OK;
+    const T* v = static_cast<const T*>(d_values);
+    const FitOut o{c->d_type, c->d_params, c->d_bits, c->d_err};
+    const dim3 per_wave(static_cast<unsigned>((c->P + kFitWaves - 1) / kFitWaves));
+    const dim3 per_block(static_cast<unsigned>(c->P));
+    const int32_t S = fixed_size;
+    if (bs != kFitWaveBs) {
+        // mixed sizes: a partition a workgroup, as the long ones need; fixed: a wave each
+        const int chunk = S > 0 ? kFitWaves : 1;
+        hipLaunchKernelGGL((k_fit_any<T, FORM>), dim3(static_cast<unsigned>((c->P + chunk - 1) / chunk)),
+                           dim3(64 * kFitWaves), 0, s, v, c->d_start, c->d_end, o, c->P, bs, chunk);
+    } else if (S <= 0) {
+        // about 8192 workgroups, a chunk of 16 at most (k_fit_chunk's note)
+        const int64_t per = (c->P + 8191) / 8192;
+        const int chunk = static_cast<int>(per < 1 ? 1 : per > 16 ? 16 : per);
+        hipLaunchKernelGGL((k_fit_chunk<T, FORM>), dim3(static_cast<unsigned>((c->P + chunk - 1) / chunk)), dim3(256), 0,
+                           s, v, c->d_start, c->d_end, o, c->P, chunk);
+    } else if (S <= 1024) {
+        hipLaunchKernelGGL((k_fit_waves<T, FORM, 2>), per_wave, dim3(64 * kFitWaves), 0, s, v, c->d_start, c->d_end, o,
+                           c->P);
+    } else if (S < kFitWaveMax) {
+        hipLaunchKernelGGL((k_fit_waves<T, FORM, 4>), per_wave, dim3(64 * kFitWaves), 0, s, v, c->d_start, c->d_end, o,
+                           c->P);
+    } else if (S <= kFitRegMax / 2) {
+        hipLaunchKernelGGL((k_fit_block<T, FORM, 16>), per_block, dim3(256), 0, s, v, c->d_start, c->d_end, o, c->P);
+    } else if (S <= kFitRegMax) {
+        hipLaunchKernelGGL((k_fit_block<T, FORM, 32>), per_block, dim3(256), 0, s, v, c->d_start, c->d_end, o, c->P);
+    } else {
+        hipLaunchKernelGGL((k_fit_block<T, FORM, 0>), per_block, dim3(256), 0, s, v, c->d_start, c->d_end, o, c->P);
     }
-    const unsigned g = static_cast<unsigned>(c->P < (1LL << 30) ? c->P : (1LL << 30));
-    hipLaunchKernelGGL((k_fit<T, FORM>), dim3(g), dim3(kFitThreads), 0, s, static_cast<const T*>(d_values), c->d_start,
-                       c->d_end, c->d_type, c->d_params, c->d_bits, c->d_err, c->P, bs);
     GLC_HIP(hipGetLastError());
     return GLC_OK;
 }
@@ -1590,7 +1738,7 @@ int launch_fit_t(const void* d_values, glc_column* c, int32_t bs, int32_t fixed_
 int launch_fit(int dtype, const void* d_values, glc_column* c, int32_t bs, int fit_form, int32_t fixed_size,
                hipStream_t s) {
     if (c->P == 0) return GLC_OK;
-    if (bs < 32 || bs > kFitThreads) return fail(GLC_ERR_INVALID_ARG, "fit block size out of range");
+    if (bs < 32 || bs > kFitWaveBs) return fail(GLC_ERR_INVALID_ARG, "fit block size out of range");
     if (fit_form != 0 && fit_form != 1) return fail(GLC_ERR_INVALID_ARG, "fit_form must be 0 or 1");
     return dispatch_dtype(dtype, [&](auto t) {
         using T = decltype(t);
@@ -1765,22 +1913,14 @@ int launch_batch_compress(const BatchPlan& b, hipStream_t s) {
     hipLaunchKernelGGL(k_fixed_parts_batch, dim3(grid_for(b.Ptot, 256)), dim3(256), 0, s, b.cols, b.part_col, b.Ptot,
                        b.S);
     GLC_HIP(hipGetLastError());
-    const unsigned gf = static_cast<unsigned>(b.Ptot < (1LL << 20) ? b.Ptot : (1LL << 20));
-    hipLaunchKernelGGL(k_fit_wave_batch, dim3(static_cast<unsigned>((b.Ptot + kFitWaves - 1) / kFitWaves)),
-                       dim3(64 * kFitWaves), 0, s, b.cols, b.part_col, b.Ptot);
+    const dim3 gf(static_cast<unsigned>((b.Ptot + kFitWaves - 1) / kFitWaves));
+    if (b.S <= 1024)
+        hipLaunchKernelGGL(k_fit_wave_batch<1024>, gf, dim3(64 * kFitWaves), 0, s, b.cols, b.part_col, b.Ptot, b.S);
+    else if (b.S <= kFitWaveMax)
+        hipLaunchKernelGGL(k_fit_wave_batch<2048>, gf, dim3(64 * kFitWaves), 0, s, b.cols, b.part_col, b.Ptot, b.S);
+    else
+        hipLaunchKernelGGL(k_fit_wave_batch<0>, gf, dim3(64 * kFitWaves), 0, s, b.cols, b.part_col, b.Ptot, b.S);
     GLC_HIP(hipGetLastError());
-    for (int dt = GLC_I32; dt <= GLC_U64; ++dt) {
-        if (!b.has_dtype[dt]) continue;
-        int rc = dispatch_dtype(dt, [&](auto t) {
-            using T = decltype(t);
-            if (b.has_wg_fit[dt]) {
-                hipLaunchKernelGGL(k_fit_batch<T>, dim3(gf), dim3(kFitThreads), 0, s, b.cols, b.part_col, b.Ptot, dt);
-                GLC_HIP(hipGetLastError());
-            }
-            return GLC_OK;
-        });
-        if (rc) return rc;
-    }
     hipLaunchKernelGGL(k_scan_batch, dim3(static_cast<unsigned>(b.C)), dim3(kScanThreads), 0, s, b.cols, b.col_bits);
     GLC_HIP(hipGetLastError());
     hipLaunchKernelGGL(k_build_index_batch, dim3(grid_for(b.Ptot, 256)), dim3(256), 0, s, b.cols, b.part_col, b.Ptot);

@@ -70,22 +70,31 @@ template <class T> __device__ __forceinline__ int64_t calc_delta(T actual, T pre
 }
 
 // Encoder residual without saturation branches, for predictions known to lie
-// in enc_fast_range.  The prediction fma(theta1, i, theta0) is monotonic in
+// in the range of a tier.  The prediction fma(theta1, i, theta0) is monotonic in
 // i (the exact value is, and rounding preserves order), and so are round()
 // and the conversion, so checking the two end indices of a run of indices
 // covers every index between them.  Inside the range:
-//   64-bit T: round(x) is an integer of magnitude <= 2^50, converted exactly
-//             by the 1.5 * 2^52 constant (sat_cast's own fast path);
-//   32-bit T: round(x) lies inside T, converted exactly by one cvt;
-//   uint64:   p <= 2^50, so a - p wraps only when a >= 2^63, and then
+//   tier 1, 64-bit T: round(x) is an integer of magnitude below 2^51,
+//             converted exactly by the 1.5 * 2^52 constant (sat_cast's own fast
+//             path; microsecond timestamps, 1.7e15, are inside);
+//   tier 1, 32-bit T: round(x) lies inside T, converted exactly by one cvt;
+//   tier 2, int64: round(x) lies inside [-2^63, 2^63 - 1024] (the largest
+//             double below the limit), converted exactly by the plain
+//             conversion, and calc_delta is the wrapping difference (nanosecond
+//             timestamps).  uint64 has none: its calc_delta saturates there;
+//   uint64:   p < 2^51, so a - p wraps only when a >= 2^63, and then
 //             calc_delta saturates to INT64_MAX (its a >= p branch).
-// Results equal calc_delta<T>(a, enc_pred<T>(t0, t1, i)) bit for bit.
-template <class T> __device__ __forceinline__ bool enc_fast_range(double x_lo, double x_hi) {
+// Results equal calc_delta<T>(a, enc_pred<T>(t0, t1, i)) bit for bit.  enc_tier
+// gives the tier for a run's end predictions, 0 outside (NaN included).
+template <class T> __device__ __forceinline__ int enc_tier(double x_lo, double x_hi) {
     const double lo = __builtin_fmin(x_lo, x_hi), hi = __builtin_fmax(x_lo, x_hi);
-    if constexpr (std::is_same<T, int32_t>::value) return lo >= -2147483647.0 && hi <= 2147483646.0;
-    else if constexpr (std::is_same<T, uint32_t>::value) return lo >= 0.0 && hi <= 4294967294.0;
-    else if constexpr (std::is_same<T, int64_t>::value) return lo >= -1125899906842624.0 && hi <= 1125899906842624.0;
-    else return lo >= 0.0 && hi <= 1125899906842624.0;
+    constexpr double k51 = 2251799813685247.0;  // 2^51 - 1
+    if (!(x_lo == x_lo && x_hi == x_hi)) return 0;
+    if constexpr (std::is_same<T, int32_t>::value) return lo >= -2147483647.0 && hi <= 2147483646.0 ? 1 : 0;
+    else if constexpr (std::is_same<T, uint32_t>::value) return lo >= 0.0 && hi <= 4294967294.0 ? 1 : 0;
+    else if constexpr (std::is_same<T, int64_t>::value)
+        return lo >= -k51 && hi <= k51 ? 1 : lo >= -9223372036854775808.0 && hi <= 9223372036854774784.0 ? 2 : 0;
+    else return lo >= 0.0 && hi <= k51 ? 1 : 0;
 }
 
 // round(p), half away from zero, for every double p: the sum reaches the next
@@ -96,9 +105,12 @@ __device__ __forceinline__ double round_away(double p) {
     return __builtin_trunc(p + __builtin_copysign(0.49999999999999994, p));
 }
 
-template <class T> __device__ __forceinline__ int64_t enc_delta_fast(T a, double t0, double t1, int32_t i) {
+template <class T, int TIER = 1>
+__device__ __forceinline__ int64_t enc_delta_fast(T a, double t0, double t1, int32_t i) {
     const double r = round_away(__builtin_fma(t1, static_cast<double>(i), t0));
-    if constexpr (sizeof(T) == 4) {
+    if constexpr (TIER == 2) {
+        return static_cast<int64_t>(static_cast<uint64_t>(a) - static_cast<uint64_t>(static_cast<int64_t>(r)));
+    } else if constexpr (sizeof(T) == 4) {
         return static_cast<int64_t>(a) - static_cast<int64_t>(static_cast<T>(r));
     } else {
         const uint64_t p = static_cast<uint64_t>(__double_as_longlong(r + 6755399441055744.0) - 0x4338000000000000LL);
