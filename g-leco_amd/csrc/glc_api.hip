@@ -169,10 +169,11 @@ void* block_get(int device, int64_t bytes, int64_t* got) {
     return p;
 }
 
-void block_put(int device, void* p, int64_t bytes) {
+// synced: the caller has waited for the device since the last use of p
+void block_put(int device, void* p, int64_t bytes, bool synced = false) {
     if (!p) return;
     BlockCache& bc = block_cache(device);
-    if (bytes > 0 && bytes <= block_cache_cap() && hipDeviceSynchronize() == hipSuccess) {
+    if (bytes > 0 && bytes <= block_cache_cap() && (synced || hipDeviceSynchronize() == hipSuccess)) {
         std::lock_guard<std::mutex> g(bc.mu);
         // drop the largest blocks until this one fits under the cap
         while (bc.held + bytes > block_cache_cap() && !bc.blocks.empty()) {
@@ -189,14 +190,16 @@ void block_put(int device, void* p, int64_t bytes) {
     (void)hipFree(p);
 }
 
-int alloc_column(glc_column* c, int64_t P, hipStream_t s) {
+// zero = false: launch_column_setup follows (compress); every array entry is
+// written before it is read.
+int alloc_column(glc_column* c, int64_t P, hipStream_t s, bool zero = true) {
     c->P = P;
     c->n_index = (c->n + kIndexTile - 1) / kIndexTile + 1;
     ArenaLayout L = layout_for(P, c->n_index);
     void* arena = block_get(c->device, L.total, &c->meta_block);
     if (!arena) return fail(GLC_ERR_OOM, "device allocation of column metadata failed (" + std::to_string(L.total) + " B)");
     bind_arena(c, static_cast<char*>(arena), L);
-    GLC_HIP(hipMemsetAsync(arena, 0, L.total, s));
+    if (zero) GLC_HIP(hipMemsetAsync(arena, 0, L.total, s));
     return GLC_OK;
 }
 
@@ -214,55 +217,42 @@ int alloc_payload(glc_column* c, int64_t payload_words, hipStream_t s, bool zero
     return GLC_OK;
 }
 
-void release_words(glc_column* c) {
-    block_put(c->device, c->d_words, c->words_block);
+void release_words(glc_column* c, bool synced = false) {
+    block_put(c->device, c->d_words, c->words_block, synced);
     c->d_words = nullptr;
     c->words_block = 0;
 }
 
 void destroy(glc_column* c) {
     if (!c || c->view) return;
-    if (c->meta_arena) block_put(c->device, c->meta_arena, c->meta_block);
-    if (c->d_words) release_words(c);
+    // one wait for both blocks (block_put waits itself when this one failed)
+    const bool synced = (c->meta_arena || c->d_words) && hipDeviceSynchronize() == hipSuccess;
+    if (c->meta_arena) block_put(c->device, c->meta_arena, c->meta_block, synced);
+    if (c->d_words) release_words(c, synced);
     if (c->d_plain) (void)hipFree(c->d_plain);
     delete c;
 }
 
-// Build the decode index and read the summary back (one D2H).
-int finish_index(glc_column* c, hipStream_t s, IndexSummary* out) {
-    IndexSummary* d_sum = summary_ptr(c);
-    GLC_HIP(hipMemsetAsync(d_sum, 0, sizeof(IndexSummary), s));
-    int rc = launch_build_index(c, d_sum, s);
+// Build the decode index; the summary arrives in pinned memory with the
+// stream's synchronisation.  scan: the bit offsets come from the widths
+// (compress), else they are in the arena.  The summary is clear beforehand.
+int finish_index(glc_column* c, bool scan, const HostWords& h, hipStream_t s, IndexSummary* out) {
+    static_assert(sizeof(IndexSummary) <= HostWords::kWords * 8, "the summary fits the pinned words");
+    bool small = false;
+    *out = IndexSummary{};
+    IndexSummary* h_sum = reinterpret_cast<IndexSummary*>(h.p);
+    int rc = launch_index(c, scan, summary_ptr(c), h_sum, &small, s);
     if (rc) return rc;
-    GLC_HIP(hipMemcpyAsync(out, d_sum, sizeof(IndexSummary), hipMemcpyDeviceToHost, s));
     GLC_HIP(hipStreamSynchronize(s));
     if (c->P > 0) {
+        *out = *h_sum;
         if (out->malformed) return fail(GLC_ERR_FORMAT, "partitions are not sorted, non-overlapping and inside [0, N)");
         if (out->bad_bits) return fail(GLC_ERR_FORMAT, "delta_bits outside [0, 64]");
     }
     c->max_bits = out->max_bits;
     c->has_poly = out->has_poly;
     c->spans = out->unaligned != 0;
-    return launch_build_tinfo(c, s);
-}
-
-
-__global__ void k_fixed_parts(int32_t* st, int32_t* en, int64_t P, int64_t n, int32_t S) {
-    const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (p >= P) return;
-    const int64_t s = p * S;
-    st[p] = static_cast<int32_t>(s);
-    en[p] = static_cast<int32_t>(std::min<int64_t>(s + S, n));
-}
-
-__global__ void k_init_types(int32_t* type, int64_t P) {
-    const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (p < P) type[p] = MODEL_LINEAR;  // host PartitionInfo init, G:409-414
-}
-
-unsigned blocks_for(int64_t work, int threads) {
-    int64_t g = (work + threads - 1) / threads;
-    return static_cast<unsigned>(std::max<int64_t>(g, 1));
+    return small ? GLC_OK : launch_build_tinfo(c, s);
 }
 
 int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, int32_t S, int32_t base,
@@ -283,6 +273,21 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
     c->n = n;
     int rc = GLC_OK;
     int64_t len0 = 0;
+    HostWords host;
+    if (!host.p) return bail(fail(GLC_ERR_OOM, "pinned host allocation failed"));
+    // scratch locks of the partitioners: held until finish_index has waited
+    // for the kernels that read the scratch (declared after c's owner: a return
+    // waits first, below)
+    std::unique_lock<std::mutex> v6_lock;
+    SplitMergeResult sm;
+    struct Drain {  // an error return leaves no kernel on the scratch before the locks go
+        std::unique_lock<std::mutex>& a;
+        std::unique_lock<std::mutex>& b;
+        hipStream_t s;
+        ~Drain() {
+            if (a.owns_lock() || b.owns_lock()) (void)hipStreamSynchronize(s);
+        }
+    } drain{v6_lock, sm.lock, s};
     if (n == 0) {  // G:355-371: an empty column
         if ((rc = alloc_column(c, 0, s))) return bail(rc);
         if ((rc = alloc_payload(c, 0, s))) return bail(rc);
@@ -294,10 +299,8 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
         case GLC_PART_FIXED: {
             if (S <= 0) return bail(fail(GLC_ERR_INVALID_ARG, "partition_size must be > 0"));
             const int64_t P = (n + S - 1) / S;
-            if ((rc = alloc_column(c, P, s))) return bail(rc);
-            hipLaunchKernelGGL(k_fixed_parts, dim3(blocks_for(P, 256)), dim3(256), 0, s, c->d_start, c->d_end, P, n,
-                               S);
-            GLC_HIP_BAIL(hipGetLastError());
+            if ((rc = alloc_column(c, P, s, false))) return bail(rc);
+            if ((rc = launch_column_setup(c, S, nullptr, nullptr, false, s))) return bail(rc);
             len0 = std::min<int64_t>(S, n);
             break;
         }
@@ -308,12 +311,9 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
             const int64_t bytes = align_up(cap * 4, 256) * 2 + align_up((nvb + 1) * 8, 256) +
                                   align_up(nvb * 4, 256) + 256;
             V6Scratch& sc = v6_scratch(c->device);
-            std::lock_guard<std::mutex> scratch_lock(sc.mu);
+            v6_lock = std::unique_lock<std::mutex>(sc.mu);
             if (sc.bytes < bytes) {
-                if (sc.p) {
-                    GLC_HIP_BAIL(hipStreamSynchronize(s));
-                    (void)hipFree(sc.p);
-                }
+                if (sc.p) (void)hipFree(sc.p);  // the previous call ended with its work on it waited for
                 sc.p = nullptr;
                 sc.bytes = 0;
                 const int64_t want = align_up(bytes + bytes / 4, 1 << 20);
@@ -330,30 +330,20 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
             int64_t* tc = reinterpret_cast<int64_t*>(t + 2 * align_up(cap * 4, 256));
             float* tv = reinterpret_cast<float*>(t + 2 * align_up(cap * 4, 256) + align_up((nvb + 1) * 8, 256));
             float* tt = reinterpret_cast<float*>(reinterpret_cast<char*>(tv) + align_up(nvb * 4, 256));
-            rc = launch_v6(dtype, d_values, n, base, ts, te, cap, tc, tc + 1, tv, tt, s);
-            int64_t P = 0;
-            int32_t first[2] = {0, 0};
-            if (!rc && hipMemcpyAsync(&P, tc, 8, hipMemcpyDeviceToHost, s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (!rc && hipMemcpyAsync(&first[0], ts, 4, hipMemcpyDeviceToHost, s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (!rc && hipMemcpyAsync(&first[1], te, 4, hipMemcpyDeviceToHost, s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (!rc && (P < 1 || P > cap)) rc = fail(GLC_ERR_STATE, "V6 produced an invalid partition count");
-            if (!rc) rc = alloc_column(c, P, s);
-            if (!rc && hipMemcpyAsync(c->d_start, ts, P * 4, hipMemcpyDeviceToDevice, s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (!rc && hipMemcpyAsync(c->d_end, te, P * 4, hipMemcpyDeviceToDevice, s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (!rc && hipStreamSynchronize(s) != hipSuccess) rc = GLC_ERR_HIP;
-            if (rc) return bail(rc == GLC_ERR_HIP ? fail(GLC_ERR_HIP, "V6 partitioning failed") : rc);
-            len0 = static_cast<int64_t>(first[1]) - first[0];
+            if ((rc = launch_v6(dtype, d_values, n, base, ts, te, cap, tc, tc + 1, tv, tt, host.p, s))) return bail(rc);
+            GLC_HIP_BAIL(hipStreamSynchronize(s));
+            const int64_t P = host.p[0];
+            if (P < 1 || P > cap) return bail(fail(GLC_ERR_STATE, "V6 produced an invalid partition count"));
+            len0 = host.p[1];
+            if ((rc = alloc_column(c, P, s, false))) return bail(rc);
+            if ((rc = launch_column_setup(c, 0, ts, te, false, s))) return bail(rc);
             break;
         }
         case GLC_PART_GPU_SPLITMERGE: {
-            std::vector<int32_t> st, en;
-            if ((rc = gpu_split_merge(dtype, d_values, n, min_size, st, en, s))) return bail(rc);
-            if ((rc = alloc_column(c, static_cast<int64_t>(st.size()), s))) return bail(rc);
-            GLC_HIP_BAIL(hipMemcpyAsync(c->d_start, st.data(), st.size() * 4, hipMemcpyHostToDevice, s));
-            GLC_HIP_BAIL(hipMemcpyAsync(c->d_end, en.data(), en.size() * 4, hipMemcpyHostToDevice, s));
-            GLC_HIP_BAIL(hipStreamSynchronize(s));
-            len0 = en[0] - st[0];
+            if ((rc = gpu_split_merge(dtype, d_values, n, min_size, &sm, s))) return bail(rc);
+            len0 = sm.first_len;
+            if ((rc = alloc_column(c, sm.P, s, false))) return bail(rc);
+            if ((rc = launch_column_setup(c, 0, sm.d_st, sm.d_en, false, s))) return bail(rc);
             break;
         }
         case GLC_PART_CPU_SPLITMERGE: {
@@ -362,11 +352,12 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
             GLC_HIP_BAIL(hipStreamSynchronize(s));
             std::vector<int32_t> st, en;
             if ((rc = cpu_split_merge(dtype, h.data(), n, min_size, st, en))) return bail(rc);
-            if ((rc = alloc_column(c, static_cast<int64_t>(st.size()), s))) return bail(rc);
+            if ((rc = alloc_column(c, static_cast<int64_t>(st.size()), s, false))) return bail(rc);
             GLC_HIP_BAIL(hipMemcpyAsync(c->d_start, st.data(), st.size() * 4, hipMemcpyHostToDevice, s));
             GLC_HIP_BAIL(hipMemcpyAsync(c->d_end, en.data(), en.size() * 4, hipMemcpyHostToDevice, s));
             GLC_HIP_BAIL(hipStreamSynchronize(s));
             len0 = en[0] - st[0];
+            if ((rc = launch_column_setup(c, 0, nullptr, nullptr, false, s))) return bail(rc);
             break;
         }
         case GLC_PART_EXPLICIT: {
@@ -378,25 +369,24 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
                     (p + 1 < P_explicit && (h_end[p] > h_start[p + 1] || h_start[p + 1] < h_start[p])))
                     return bail(fail(GLC_ERR_FORMAT, "partitions must be sorted, non-overlapping and inside [0, N)"));
             }
-            if ((rc = alloc_column(c, P_explicit, s))) return bail(rc);
+            if ((rc = alloc_column(c, P_explicit, s, false))) return bail(rc);
             GLC_HIP_BAIL(hipMemcpyAsync(c->d_start, h_start, P_explicit * 4, hipMemcpyHostToDevice, s));
             GLC_HIP_BAIL(hipMemcpyAsync(c->d_end, h_end, P_explicit * 4, hipMemcpyHostToDevice, s));
             GLC_HIP_BAIL(hipStreamSynchronize(s));
             len0 = static_cast<int64_t>(h_end[0]) - h_start[0];
+            if ((rc = launch_column_setup(c, 0, nullptr, nullptr, true, s))) return bail(rc);
             break;
         }
         default: return bail(fail(GLC_ERR_INVALID_ARG, "bad partitioner"));
     }
-    hipLaunchKernelGGL(k_init_types, dim3(blocks_for(c->P, 256)), dim3(256), 0, s, c->d_type, c->P);
-    GLC_HIP_BAIL(hipGetLastError());
     c->fit_block = fit_block_size(len0);
     c->fit_form = fit_form;
     if ((rc = launch_fit(dtype, d_values, c, c->fit_block, fit_form, partitioner == GLC_PART_FIXED ? S : 0, s)))
         return bail(rc);
-    int64_t* d_total = reinterpret_cast<int64_t*>(summary_ptr(c)) + 8;  // scratch slot after the summary
-    if ((rc = launch_scan_offsets(c, d_total, s))) return bail(rc);
     IndexSummary sum;
-    if ((rc = finish_index(c, s, &sum))) return bail(rc);
+    if ((rc = finish_index(c, true, host, s, &sum))) return bail(rc);
+    if (v6_lock.owns_lock()) v6_lock.unlock();  // the stream was waited for
+    split_merge_release(sm);
     c->total_bits = sum.total_bits;
     c->fixed_size = sum.not_fixed ? 0 : static_cast<int32_t>(len0);
     if ((rc = alloc_payload(c, (c->total_bits + 31) / 32, s, false))) return bail(rc);
@@ -477,6 +467,40 @@ int check_header(const uint8_t* blob, size_t size, int dtype, bool verify_checks
 }
 
 }  // namespace
+
+namespace {
+struct HostPool {
+    std::mutex mu;
+    std::vector<int64_t*> idle;
+};
+HostPool& host_pool() {
+    static HostPool* pool = new HostPool();  // used until exit
+    return *pool;
+}
+}  // namespace
+HostWords::HostWords() {
+    {
+        HostPool& pool = host_pool();
+        std::lock_guard<std::mutex> g(pool.mu);
+        if (!pool.idle.empty()) {
+            p = pool.idle.back();
+            pool.idle.pop_back();
+            return;
+        }
+    }
+    void* q = nullptr;
+    if (hipHostMalloc(&q, kWords * 8, hipHostMallocPortable) != hipSuccess) {
+        (void)hipGetLastError();
+        return;
+    }
+    p = static_cast<int64_t*>(q);
+}
+HostWords::~HostWords() {
+    if (!p) return;
+    HostPool& pool = host_pool();
+    std::lock_guard<std::mutex> g(pool.mu);
+    pool.idle.push_back(p);
+}
 
 void set_error(const std::string& msg) { g_last_error = msg; }
 int fail(int code, const std::string& msg) {
@@ -673,7 +697,7 @@ int glc_partition_v6_noalloc(int dtype, const void* d_values, int64_t n, int32_t
     if ((rc = noalloc_scratch(&sc))) return rc;
     return launch_v6(dtype, d_values, n, base, d_start, d_end, cap, d_num_partitions,
                      reinterpret_cast<int64_t*>(sc + kNoAllocBaseOff), reinterpret_cast<float*>(sc + kNoAllocVarOff),
-                     reinterpret_cast<float*>(sc + kNoAllocThrOff), s);
+                     reinterpret_cast<float*>(sc + kNoAllocThrOff), nullptr, s);
 }
 
 static bool fixed_compatible(const glc_column* c, int32_t S) {
@@ -900,7 +924,9 @@ int glc_deserialize(const uint8_t* blob, size_t size, int dtype, int preunpack, 
     if ((rc = alloc_payload(c, static_cast<int64_t>((h.delta_bytes + 3) / 4), s))) return bail(rc);
     if (h.delta_bytes) GLC_HIP_BAIL(hipMemcpyAsync(c->d_words, blob + h.delta_off, h.delta_bytes, hipMemcpyHostToDevice, s));
     IndexSummary sum;
-    if ((rc = finish_index(c, s, &sum))) return bail(rc);
+    HostWords host;
+    if (!host.p) return bail(fail(GLC_ERR_OOM, "pinned host allocation failed"));
+    if ((rc = finish_index(c, false, host, s, &sum))) return bail(rc);
     if (static_cast<uint64_t>(sum.total_bits) > h.delta_bytes * 8)
         return bail(fail(GLC_ERR_FORMAT, "partition bit ranges exceed the payload"));
     c->total_bits = sum.total_bits;

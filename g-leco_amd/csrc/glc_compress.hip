@@ -871,81 +871,164 @@ template <class V> __device__ __forceinline__ V wave_max_all(V x) {
 // same-address device atomics serialize, and one set per wave cost ~50 us on
 // 1.2e5 partitions.
 constexpr int kIndexThreads = 1024;
-__global__ __launch_bounds__(kIndexThreads) void k_build_index(const int32_t* __restrict__ st, const int32_t* __restrict__ en,
-                              const int32_t* __restrict__ type, const double* __restrict__ params,
-                              const int32_t* __restrict__ bits, const int64_t* __restrict__ off, int64_t P,
-                              int64_t n, Desc* __restrict__ desc, int32_t* __restrict__ tile_part, int64_t n_index,
-                              IndexSummary* __restrict__ sum) {
-    const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    const bool live = p < P;  // every lane stays for the wave reductions
-    int bad = 0, bad_bits = 0, poly = 0, not_fixed = 0, unaligned = 0;
-    int32_t b = 0;
-    int64_t endbit = 0;
-    int32_t s = 0, s_next = 0x7FFFFFFF;
-    if (live) {
-        const int32_t e = en[p], ty = type[p];
-        s = st[p];
-        b = bits[p];
-        const int32_t len = e > s ? e - s : 0;
-        Desc d;
-        d.theta0 = params[4 * p];
-        d.theta1 = params[4 * p + 1];
-        d.packed = desc_pack(off[p], b, ty);
-        d.start = s;
-        d.len = len;
-        desc[p] = d;
-        // validation (sorted, non-overlapping, inside [0, n))
-        bad = (s < 0 || e < s || static_cast<int64_t>(e) > n) ? 1 : 0;
-        if (p + 1 < P) s_next = st[p + 1];
-        if (p + 1 < P && e > s_next) bad = 1;
-        if (p + 1 < P && s_next < s) bad = 1;
-        bad_bits = (b < 0 || b > 64) ? 1 : 0;
-        poly = ty == MODEL_POLY2 ? 1 : 0;
-        unaligned = (len > 0 && (s % kIndexTile != 0 || (e % kIndexTile != 0 && e != n))) ? 1 : 0;
-        endbit = off[p] + static_cast<int64_t>(len) * b;
-        // fixed-size detection against S = len of partition 0
-        const int64_t S = static_cast<int64_t>(en[0]) - st[0];
-        const int64_t fs = S * p;
-        const int64_t fe = (fs + S < n) ? fs + S : n;
-        not_fixed = (S <= 0 || s != fs || e != fe || (p == P - 1 && e != n)) ? 1 : 0;
-    }
+struct IndexIn {
+    const int32_t* __restrict__ st;
+    const int32_t* __restrict__ en;
+    const int32_t* __restrict__ type;
+    const double* __restrict__ params;
+    const int32_t* __restrict__ bits;
+    int64_t P, n, n_index;
+    Desc* __restrict__ desc;
+    int32_t* __restrict__ tile_part;
+};
+enum { IX_BAD = 1, IX_BITS = 2, IX_POLY = 4, IX_NOT_FIXED = 8, IX_UNALIGNED = 16 };
+struct IndexAcc {
+    int flags = 0;
+    int32_t max_bits = INT32_MIN;
+    uint64_t end = 0;
+};
+
+// Entry p: its descriptor, the tiles whose last partition it is, and its part
+// of the summary.
+__device__ __forceinline__ void index_entry(const IndexIn& a, int64_t p, int64_t off, IndexAcc& acc) {
+    const int32_t s = a.st[p], e = a.en[p], ty = a.type[p], b = a.bits[p];
+    const int32_t len = e > s ? e - s : 0;
+    Desc d;
+    d.theta0 = a.params[4 * p];
+    d.theta1 = a.params[4 * p + 1];
+    d.packed = desc_pack(off, b, ty);
+    d.start = s;
+    d.len = len;
+    a.desc[p] = d;
+    // validation (sorted, non-overlapping, inside [0, n))
+    const bool more = p + 1 < a.P;
+    const int32_t s_next = more ? a.st[p + 1] : 0x7FFFFFFF;
+    const bool bad = s < 0 || e < s || static_cast<int64_t>(e) > a.n || (more && (e > s_next || s_next < s));
+    // fixed-size detection against S = len of partition 0
+    const int64_t S = static_cast<int64_t>(a.en[0]) - a.st[0];
+    const int64_t fs = S * p;
+    const int64_t fe = (fs + S < a.n) ? fs + S : a.n;
+    acc.flags |= (bad ? IX_BAD : 0) | ((b < 0 || b > 64) ? IX_BITS : 0) | (ty == MODEL_POLY2 ? IX_POLY : 0) |
+                 ((S <= 0 || s != fs || e != fe || (!more && e != a.n)) ? IX_NOT_FIXED : 0) |
+                 ((len > 0 && (s % kIndexTile != 0 || (e % kIndexTile != 0 && e != a.n))) ? IX_UNALIGNED : 0);
+    acc.max_bits = b > acc.max_bits ? b : acc.max_bits;
+    const uint64_t end = static_cast<uint64_t>(off + static_cast<int64_t>(len) * b);  // unsigned, as the atomic
+    acc.end = end > acc.end ? end : acc.end;
+    // tile_part[t] = last partition with start <= t*1024, for t in [ceil(s/1024), ceil(s_next/1024))
+    if (bad) return;
+    const int64_t t0 = (p == 0) ? 0 : (static_cast<int64_t>(s) + kIndexTile - 1) >> kIndexShift;
+    int64_t t1 = more ? (static_cast<int64_t>(s_next) + kIndexTile - 1) >> kIndexShift : a.n_index;
+    if (t1 > a.n_index) t1 = a.n_index;
+    for (int64_t t = t0; t < t1; ++t) a.tile_part[t] = static_cast<int32_t>(p);
+}
+
+// The workgroup's summary, valid in thread 0 (all threads call it).
+__device__ __forceinline__ IndexAcc index_reduce(IndexAcc acc) {
     __shared__ int32_t s_flags[kIndexThreads / 64], s_bits[kIndexThreads / 64];
     __shared__ uint64_t s_end[kIndexThreads / 64];
-    const int flags = (__any(bad) ? 1 : 0) | (__any(bad_bits) ? 2 : 0) | (__any(poly) ? 4 : 0) |
-                      (__any(not_fixed) ? 8 : 0) | (__any(live) ? 16 : 0) | (__any(unaligned) ? 32 : 0);
-    const int32_t wmax_bits = wave_max_all(live ? b : INT32_MIN);
-    const uint64_t wend = wave_max_all(live ? static_cast<uint64_t>(endbit) : 0ULL);  // unsigned, as the atomic
+    int flags = 0;
+#pragma unroll
+    for (int f = 1; f <= IX_UNALIGNED; f <<= 1) flags |= __any(acc.flags & f) ? f : 0;
+    const int32_t wb = wave_max_all(acc.max_bits);
+    const uint64_t we = wave_max_all(acc.end);
     if ((threadIdx.x & 63) == 0) {
         s_flags[threadIdx.x >> 6] = flags;
-        s_bits[threadIdx.x >> 6] = wmax_bits;
-        s_end[threadIdx.x >> 6] = wend;
+        s_bits[threadIdx.x >> 6] = wb;
+        s_end[threadIdx.x >> 6] = we;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int f = 0;
-        int32_t mb = INT32_MIN;
-        uint64_t me = 0;
-        for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) {
-            f |= s_flags[w];
-            mb = s_bits[w] > mb ? s_bits[w] : mb;
-            me = s_end[w] > me ? s_end[w] : me;
+    IndexAcc r;
+    if (threadIdx.x == 0)
+        for (int w = 0; w < kIndexThreads / 64; ++w) {
+            r.flags |= s_flags[w];
+            r.max_bits = s_bits[w] > r.max_bits ? s_bits[w] : r.max_bits;
+            r.end = s_end[w] > r.end ? s_end[w] : r.end;
         }
-        if (f & 16) {  // the workgroup holds at least one partition
-            if (f & 1) atomicOr(&sum->malformed, 1);
-            if (f & 2) atomicOr(&sum->bad_bits, 1);
-            if (f & 4) atomicOr(&sum->has_poly, 1);
-            if (f & 8) atomicOr(&sum->not_fixed, 1);
-            if (f & 32) atomicOr(&sum->unaligned, 1);
-            atomicMax(&sum->max_bits, mb);
-            atomicMax(reinterpret_cast<unsigned long long*>(&sum->total_bits), static_cast<unsigned long long>(me));
+    return r;
+}
+
+// sum is zeroed beforehand.  host: pinned memory that receives the summary
+// when the last workgroup is done (no copy to wait for).
+__global__ __launch_bounds__(kIndexThreads) void k_build_index(IndexIn a, const int64_t* __restrict__ off,
+                                                               IndexSummary* __restrict__ sum,
+                                                               IndexSummary* __restrict__ host) {
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * kIndexThreads + threadIdx.x;
+    IndexAcc acc;
+    if (p < a.P) index_entry(a, p, off[p], acc);  // every lane stays for the reductions
+    const IndexAcc r = index_reduce(acc);
+    if (threadIdx.x != 0) return;
+    if (r.flags & IX_BAD) atomicOr(&sum->malformed, 1);
+    if (r.flags & IX_BITS) atomicOr(&sum->bad_bits, 1);
+    if (r.flags & IX_POLY) atomicOr(&sum->has_poly, 1);
+    if (r.flags & IX_NOT_FIXED) atomicOr(&sum->not_fixed, 1);
+    if (r.flags & IX_UNALIGNED) atomicOr(&sum->unaligned, 1);
+    atomicMax(&sum->max_bits, r.max_bits);
+    atomicMax(reinterpret_cast<unsigned long long*>(&sum->total_bits), static_cast<unsigned long long>(r.end));
+    __threadfence();
+    if (atomicAdd(&sum->done, 1) != static_cast<int32_t>(gridDim.x) - 1) return;
+    IndexSummary x{};  // the last workgroup: every other one's atomics are done
+    x.malformed = atomicOr(&sum->malformed, 0);
+    x.bad_bits = atomicOr(&sum->bad_bits, 0);
+    x.has_poly = atomicOr(&sum->has_poly, 0);
+    x.not_fixed = atomicOr(&sum->not_fixed, 0);
+    x.unaligned = atomicOr(&sum->unaligned, 0);
+    x.max_bits = atomicMax(&sum->max_bits, INT32_MIN);
+    x.total_bits = static_cast<int64_t>(atomicMax(reinterpret_cast<unsigned long long*>(&sum->total_bits), 0ULL));
+    *host = x;
+}
+
+// The whole index of a small column in one workgroup and one launch: offsets
+// (SCAN: from the widths; else given), descriptors, tile_part, summary and tile
+// records.  A launch costs 4-5 us with its gap; the six it replaces (three for
+// the scan, index, summary clear, tile records) were a quarter of a 2^16-value
+// compress.  Limits: beyond kIndexSmall partitions or tiles one workgroup takes
+// longer than the launches.
+constexpr int64_t kIndexSmall = 4096;
+template <bool SCAN>
+__global__ __launch_bounds__(kIndexThreads) void k_index_small(IndexIn a, int64_t* __restrict__ off,
+                                                               TileInfo* __restrict__ ti,
+                                                               IndexSummary* __restrict__ sum,
+                                                               IndexSummary* __restrict__ host) {
+    __shared__ int64_t s_w[kScanThreads / 64 + 1];
+    __shared__ int s_bad;
+    static_assert(kIndexThreads == kScanThreads, "one workgroup scans and indexes");
+    IndexAcc acc;
+    int64_t carry = 0;
+    for (int64_t p0 = 0; p0 < a.P; p0 += kIndexThreads) {
+        const int64_t p = p0 + threadIdx.x;
+        int64_t o = 0;
+        if constexpr (SCAN) {
+            int64_t tot;
+            o = carry + block_excl_scan(p < a.P ? static_cast<int64_t>(a.en[p] - a.st[p]) * a.bits[p] : 0, s_w, &tot);
+            carry += tot;
+            if (p < a.P) off[p] = o;
+        } else if (p < a.P) {
+            o = off[p];
         }
+        if (p < a.P) index_entry(a, p, o, acc);
     }
-    // tile_part[t] = last partition with start <= t*1024, for t in [ceil(s/1024), ceil(s_next/1024))
-    if (!live || bad) return;
-    int64_t t0 = (p == 0) ? 0 : (static_cast<int64_t>(s) + kIndexTile - 1) >> kIndexShift;
-    int64_t t1 = (p + 1 < P) ? (static_cast<int64_t>(s_next) + kIndexTile - 1) >> kIndexShift : n_index;
-    if (t1 > n_index) t1 = n_index;
-    for (int64_t t = t0; t < t1; ++t) tile_part[t] = static_cast<int32_t>(p);
+    const IndexAcc r = index_reduce(acc);
+    if (threadIdx.x == 0) {
+        s_bad = r.flags & IX_BAD;
+        IndexSummary x{};
+        x.malformed = (r.flags & IX_BAD) ? 1 : 0;
+        x.bad_bits = (r.flags & IX_BITS) ? 1 : 0;
+        x.has_poly = (r.flags & IX_POLY) ? 1 : 0;
+        x.not_fixed = (r.flags & IX_NOT_FIXED) ? 1 : 0;
+        x.unaligned = (r.flags & IX_UNALIGNED) ? 1 : 0;
+        x.max_bits = r.max_bits > 0 ? r.max_bits : 0;
+        x.total_bits = static_cast<int64_t>(r.end);
+        *sum = x;
+        *host = x;
+    }
+    __threadfence_block();
+    __syncthreads();  // descriptors and tile_part of every thread
+    if (s_bad) return;  // tile_part is incomplete
+    for (int64_t t = threadIdx.x; t < a.n_index - 1; t += kIndexThreads) {
+        const int64_t e0 = t * kIndexTile;
+        const int64_t e1 = (e0 + kIndexTile < a.n) ? e0 + kIndexTile : a.n;
+        ti[t] = make_tile_info(a.desc[a.tile_part[t]], e0, e1);
+    }
 }
 
 // TileInfo per 1024-element tile (after the descriptors and tile_part exist).
@@ -1566,20 +1649,36 @@ __device__ __forceinline__ float key_float(uint32_t k) {
 // nvb <= 1024 * kSelKeys.
 constexpr int kSelKeys = 16;
 
-__device__ __forceinline__ void sel_count(uint32_t k, int pass, uint32_t hmask, int shift, const uint32_t* pre,
-                                          uint32_t (*hist)[256]) {
+// Lanes of a wave that count in the same bin add once: the leading digits of
+// the statistics are nearly all alike, and 16384 LDS atomics on a few addresses
+// were most of the selection's 34 us.  Two rounds take the common digits; what is
+// left counts lane by lane.
+__device__ __forceinline__ void hist_add(uint32_t* hist, uint32_t d, bool on) {
+#pragma unroll
+    for (int round = 0; round < 2; ++round) {
+        const uint64_t m = __ballot(on);
+        if (m == 0) return;
+        const uint32_t lead = __shfl(d, __builtin_ctzll(m), 64);
+        const uint64_t same = __ballot(on && d == lead);
+        if ((threadIdx.x & 63) == __builtin_ctzll(m)) atomicAdd(&hist[lead], static_cast<uint32_t>(__popcll(same)));
+        on = on && d != lead;
+    }
+    if (on) atomicAdd(&hist[d], 1u);
+}
+
+// All lanes call it; live: the lane holds a key.
+__device__ __forceinline__ void sel_count(uint32_t k, bool live, int pass, uint32_t hmask, int shift,
+                                          const uint32_t* pre, uint32_t (*hist)[256]) {
     const uint32_t d = (k >> shift) & 0xFFu;
     if (pass == 0) {
-        atomicAdd(&hist[0][d], 1u);
+        hist_add(hist[0], d, live);
         return;
     }
 #pragma unroll
-    for (int q = 0; q < 3; ++q)
-        if ((k & hmask) == pre[q]) atomicAdd(&hist[q][d], 1u);
+    for (int q = 0; q < 3; ++q) hist_add(hist[q], d, live && (k & hmask) == pre[q]);
 }
 
-__global__ __launch_bounds__(1024) void k_v6_select(const float* __restrict__ var, int64_t nvb,
-                                                    float* __restrict__ thr) {
+__device__ __forceinline__ void v6_select(const float* __restrict__ var, int64_t nvb, float* __restrict__ thr) {
     __shared__ uint32_t hist[3][256];
     __shared__ uint32_t s_prefix[3];
     __shared__ int64_t s_rank[3];
@@ -1607,10 +1706,15 @@ __global__ __launch_bounds__(1024) void k_v6_select(const float* __restrict__ va
         const uint32_t pre[3] = {s_prefix[0], s_prefix[1], s_prefix[2]};
         if (in_regs) {
 #pragma unroll
-            for (int k = 0; k < kSelKeys; ++k)
-                if (tid + 1024LL * k < nvb) sel_count(keys[k], pass, hmask, shift, pre, hist);
+            for (int k = 0; k < kSelKeys; ++k) {
+                if (1024LL * k >= nvb) break;  // uniform
+                sel_count(keys[k], tid + 1024LL * k < nvb, pass, hmask, shift, pre, hist);
+            }
         } else {
-            for (int64_t i = tid; i < nvb; i += 1024) sel_count(float_key(var[i]), pass, hmask, shift, pre, hist);
+            for (int64_t i0 = 0; i0 < nvb; i0 += 1024) {
+                const int64_t i = i0 + tid;
+                sel_count(float_key(var[i < nvb ? i : nvb - 1]), i < nvb, pass, hmask, shift, pre, hist);
+            }
         }
         __syncthreads();
         if (wave < 3) {
@@ -1643,6 +1747,10 @@ __global__ __launch_bounds__(1024) void k_v6_select(const float* __restrict__ va
     }
     if (tid < 3) thr[tid] = key_float(s_prefix[tid]);
 }
+__global__ __launch_bounds__(1024) void k_v6_select(const float* __restrict__ var, int64_t nvb,
+                                                    float* __restrict__ thr) {
+    v6_select(var, nvb, thr);
+}
 
 struct V6Count {
     const float* var;
@@ -1661,17 +1769,55 @@ struct V6Count {
     }
 };
 
-__global__ void k_v6_emit(V6Count f, int64_t nvb, const int64_t* __restrict__ base_idx, int32_t* __restrict__ st,
-                          int32_t* __restrict__ en) {
-    const int64_t b = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (b >= nvb) return;
+// Block b's partitions from entry k on.
+__device__ __forceinline__ void v6_emit(const V6Count& f, int64_t b, int64_t k, int32_t* __restrict__ st,
+                                        int32_t* __restrict__ en) {
     const int64_t s = b * f.vbs;
     const int64_t e = (s + f.vbs < f.n) ? s + f.vbs : f.n;
     const int64_t sz = f.size_of(b);
-    int64_t k = base_idx[b];
     for (int64_t j = s; j < e; j += sz, ++k) {  // PartitioningKernels.cuh:734-741
         st[k] = static_cast<int32_t>(j);
         en[k] = static_cast<int32_t>((j + sz < f.n) ? j + sz : f.n);
+    }
+}
+
+// host (pinned, or null): the number of partitions and the first one's length
+__device__ __forceinline__ void v6_report(const V6Count& f, int64_t total, int64_t* __restrict__ host) {
+    const int64_t sz = f.size_of(0);
+    host[0] = total;
+    host[1] = sz < f.n ? sz : f.n;
+}
+
+__global__ void k_v6_emit(V6Count f, int64_t nvb, const int64_t* __restrict__ base_idx, int32_t* __restrict__ st,
+                          int32_t* __restrict__ en, const int64_t* __restrict__ total, int64_t* __restrict__ host) {
+    const int64_t b = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (b == 0 && host) v6_report(f, *total, host);
+    if (b < nvb) v6_emit(f, b, base_idx[b], st, en);
+}
+
+// Thresholds, counts and partitions of a short list of blocks in one
+// workgroup: one launch instead of five.  Up to kV6Small blocks (2^25 values at
+// the default base); beyond, writing 16 partitions a block from one workgroup
+// takes longer than the launches.
+constexpr int64_t kV6Small = 2048;
+__global__ __launch_bounds__(1024) void k_v6_small(V6Count f, int64_t nvb, float* __restrict__ thr,
+                                                   int32_t* __restrict__ st, int32_t* __restrict__ en,
+                                                   int64_t* __restrict__ total, int64_t* __restrict__ host) {
+    __shared__ int64_t s_w[kScanThreads / 64 + 1];
+    v6_select(f.var, nvb, thr);
+    __threadfence_block();
+    __syncthreads();  // thr
+    int64_t carry = 0;
+    for (int64_t b0 = 0; b0 < nvb; b0 += 1024) {
+        const int64_t b = b0 + threadIdx.x;
+        int64_t tot;
+        const int64_t k = carry + block_excl_scan(b < nvb ? f(b) : 0, s_w, &tot);
+        carry += tot;
+        if (b < nvb) v6_emit(f, b, k, st, en);
+    }
+    if (threadIdx.x == 0) {
+        *total = carry;
+        if (host) v6_report(f, carry, host);
     }
 }
 
@@ -1747,19 +1893,71 @@ int launch_fit(int dtype, const void* d_values, glc_column* c, int32_t bs, int f
     });
 }
 
-int launch_scan_offsets(glc_column* c, int64_t* d_total, hipStream_t s) {
-    LenBits f{c->d_start, c->d_end, c->d_bits};
-    int rc = launch_scan(f, c->P, c->d_off, d_total, s);
-    if (rc) return rc;
+// Offsets (scan: from the widths, else those in the arena), decode index and
+// summary; *small: the tile records are built too (launch_build_tinfo otherwise,
+// once the summary has been checked).
+int launch_index(glc_column* c, bool scan, IndexSummary* d_sum, IndexSummary* h_sum, bool* small, hipStream_t s) {
+    *small = false;
+    if (c->P == 0) return GLC_OK;
+    const IndexIn a{c->d_start, c->d_end, c->d_type, c->d_params, c->d_bits, c->P,
+                    c->n,       c->n_index, c->d_desc, c->d_tile_part};
+    if (c->P <= kIndexSmall && c->n_index - 1 <= kIndexSmall) {
+        *small = true;
+        if (scan)
+            hipLaunchKernelGGL(k_index_small<true>, dim3(1), dim3(kIndexThreads), 0, s, a, c->d_off, c->d_tinfo, d_sum,
+                               h_sum);
+        else
+            hipLaunchKernelGGL(k_index_small<false>, dim3(1), dim3(kIndexThreads), 0, s, a, c->d_off, c->d_tinfo, d_sum,
+                               h_sum);
+        GLC_HIP(hipGetLastError());
+        return GLC_OK;
+    }
+    if (scan) {
+        int64_t* d_total = reinterpret_cast<int64_t*>(d_sum) + 8;  // scratch slot after the summary
+        const int rc = launch_scan(LenBits{c->d_start, c->d_end, c->d_bits}, c->P, c->d_off, d_total, s);
+        if (rc) return rc;
+    }
+    hipLaunchKernelGGL(k_build_index, dim3(grid_for(c->P, kIndexThreads)), dim3(kIndexThreads), 0, s, a, c->d_off, d_sum,
+                       h_sum);
     GLC_HIP(hipGetLastError());
     return GLC_OK;
 }
 
-int launch_build_index(glc_column* c, IndexSummary* d_sum, hipStream_t s) {
-    if (c->P == 0) return GLC_OK;
-    hipLaunchKernelGGL(k_build_index, dim3(grid_for(c->P, kIndexThreads)), dim3(kIndexThreads), 0, s, c->d_start,
-                       c->d_end, c->d_type,
-                       c->d_params, c->d_bits, c->d_off, c->P, c->n, c->d_desc, c->d_tile_part, c->n_index, d_sum);
+// Before a column's kernels, instead of clearing the whole arena: the
+// partitions (fixed: [pS, min((p+1)S, n)); else copied from src_st / src_en, or
+// already there when those are null), the initial model type (host PartitionInfo
+// init, G:409-414), for lists that may hold empty partitions (which the fit
+// skips) zero outputs, and the summary and work-stealing counters.
+__global__ void k_column_setup(int32_t* __restrict__ st, int32_t* __restrict__ en, int32_t* __restrict__ type,
+                               double* __restrict__ params, int32_t* __restrict__ bits, int64_t* __restrict__ err,
+                               int64_t P, int64_t n, int32_t S, const int32_t* __restrict__ src_st,
+                               const int32_t* __restrict__ src_en, bool empties, int32_t* __restrict__ counters,
+                               IndexSummary* __restrict__ sum) {
+    const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (p < 2) counters[p] = 0;
+    if (p == 2) *sum = IndexSummary{};
+    if (p >= P) return;
+    if (S > 0) {
+        const int64_t s0 = p * S;
+        st[p] = static_cast<int32_t>(s0);
+        en[p] = static_cast<int32_t>(s0 + S < n ? s0 + S : n);
+    } else if (src_st) {
+        st[p] = src_st[p];
+        en[p] = src_en[p];
+    }
+    type[p] = MODEL_LINEAR;
+    if (empties) {
+        params[4 * p] = 0.0; params[4 * p + 1] = 0.0; params[4 * p + 2] = 0.0; params[4 * p + 3] = 0.0;
+        bits[p] = 0;
+        err[p] = 0;
+    }
+}
+
+int launch_column_setup(glc_column* c, int32_t S, const int32_t* src_st, const int32_t* src_en, bool empties,
+                        hipStream_t s) {
+    hipLaunchKernelGGL(k_column_setup, dim3(grid_for(c->P > 3 ? c->P : 3, 256)), dim3(256), 0, s, c->d_start, c->d_end,
+                       c->d_type, c->d_params, c->d_bits, c->d_err, c->P, c->n, S, src_st, src_en, empties,
+                       c->d_tile_part + c->n_index, summary_ptr(c));
     GLC_HIP(hipGetLastError());
     return GLC_OK;
 }
@@ -1834,7 +2032,7 @@ int v6_capacity(int64_t n, int32_t base, int64_t* cap, int64_t* nvb) {
 }
 
 int launch_v6(int dtype, const void* d_values, int64_t n, int32_t base, int32_t* d_start, int32_t* d_end,
-              int64_t cap, int64_t* d_total, int64_t* d_base, float* d_var, float* d_thr, hipStream_t s) {
+              int64_t cap, int64_t* d_total, int64_t* d_base, float* d_var, float* d_thr, int64_t* h_out, hipStream_t s) {
     int64_t need = 0, nvb = 0;
     int rc = v6_capacity(n, base, &need, &nvb);
     if (rc) return rc;
@@ -1849,13 +2047,18 @@ int launch_v6(int dtype, const void* d_values, int64_t n, int32_t base, int32_t*
         return GLC_OK;
     });
     if (rc) return rc;
+    const V6Count f{d_var, d_thr, vbs, n, base};
+    if (nvb <= kV6Small) {
+        hipLaunchKernelGGL(k_v6_small, dim3(1), dim3(1024), 0, s, f, nvb, d_thr, d_start, d_end, d_total, h_out);
+        GLC_HIP(hipGetLastError());
+        return GLC_OK;
+    }
     hipLaunchKernelGGL(k_v6_select, dim3(1), dim3(1024), 0, s, d_var, nvb, d_thr);
     GLC_HIP(hipGetLastError());
-    V6Count f{d_var, d_thr, vbs, n, base};
     rc = launch_scan(f, nvb, d_base, d_total, s);  // per-block partition bases, P
     if (rc) return rc;
-    GLC_HIP(hipGetLastError());
-    hipLaunchKernelGGL(k_v6_emit, dim3(grid_for(nvb, 256)), dim3(256), 0, s, f, nvb, d_base, d_start, d_end);
+    hipLaunchKernelGGL(k_v6_emit, dim3(grid_for(nvb, 256)), dim3(256), 0, s, f, nvb, d_base, d_start, d_end, d_total,
+                       h_out);
     GLC_HIP(hipGetLastError());
     return GLC_OK;
 }

@@ -16,6 +16,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <mutex>
 #include <string>
 #include <type_traits>
 #include <vector>
@@ -97,6 +98,7 @@ struct alignas(64) IndexSummary {  // one 64-byte fill clears it (a fill of 40 b
     int32_t bad_bits;       // delta_bits outside [0, 64]
     int64_t total_bits;     // max end bit over partitions
     int32_t unaligned;      // a partition starts, or ends before N, inside a 1024-value tile
+    int32_t done;           // workgroups that have added their part
 };
 static_assert(sizeof(IndexSummary) == 64, "the scratch slot after the summary is at byte 64");
 
@@ -269,18 +271,20 @@ template <class T> __host__ __device__ inline T x86_cast(double r) {
 // fixed_size: S when the partitions are [iS, min((i+1)S, N)), else 0
 int launch_fit(int dtype, const void* d_values, glc_column* c, int32_t bs, int fit_form, int32_t fixed_size,
                hipStream_t s);
-int launch_scan_offsets(glc_column* c, int64_t* d_total, hipStream_t s);
 int launch_pack(int dtype, const void* d_values, glc_column* c, hipStream_t s);
 // zero the payload words a compress leaves partly written by atomics (each
 // 1024-value tile's first word and last three words), after the index
 int launch_zero_edges(glc_column* c, hipStream_t s);
-int launch_build_index(glc_column* c, IndexSummary* d_sum, hipStream_t s);
+int launch_index(glc_column* c, bool scan, IndexSummary* d_sum, IndexSummary* h_sum, bool* small, hipStream_t s);
+int launch_column_setup(glc_column* c, int32_t S, const int32_t* src_st, const int32_t* src_en, bool empties,
+                        hipStream_t s);
 int launch_build_tinfo(glc_column* c, hipStream_t s);  // after a valid index
 // V6 boundaries into d_start/d_end[cap]; *d_total receives P, d_base[nvb]
 // the per-block partition bases; d_var[nvb], d_thr[3] are scratch.  Kernel
 // launches only (no memset, no copy, no host wait).
 int launch_v6(int dtype, const void* d_values, int64_t n, int32_t base, int32_t* d_start, int32_t* d_end,
-              int64_t cap, int64_t* d_total, int64_t* d_base, float* d_var, float* d_thr, hipStream_t s);
+              int64_t cap, int64_t* d_total, int64_t* d_base, float* d_var, float* d_thr, int64_t* h_out,
+              hipStream_t s);
 int v6_capacity(int64_t n, int32_t base, int64_t* cap, int64_t* nvb);
 int launch_fill_u32(uint32_t* p, int64_t n, uint32_t v, hipStream_t s);
 // decode side (glc_decode.hip)
@@ -304,9 +308,32 @@ struct BlobView {            // device pointers into a serialized blob
 };
 int launch_direct_access(int dtype, const BlobView& v, const int32_t* d_pos, int64_t q, void* d_out, hipStream_t s);
 
-// GPU split/merge partitioner (glc_splitmerge.hip); boundaries returned on the host
-int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t min_size, std::vector<int32_t>& st,
-                    std::vector<int32_t>& en, hipStream_t s);
+// A few words of pinned host memory that kernels report to; from a pool that
+// grows to the number of calls in flight and is kept until the process ends
+// (glc_api.hip).  p is null when the allocation failed.
+struct HostWords {
+    static constexpr int kWords = 16;
+    int64_t* p = nullptr;
+    HostWords();
+    ~HostWords();
+    HostWords(const HostWords&) = delete;
+    HostWords& operator=(const HostWords&) = delete;
+};
+
+// GPU split/merge partitioner (glc_splitmerge.hip).  The boundaries stay in the
+// device's scratch: d_st, d_en [P], valid while `lock` is held and the work that
+// reads them is waited for before it is released; first_len is partition 0's length.
+struct SplitMergeResult {
+    const int32_t* d_st = nullptr;
+    const int32_t* d_en = nullptr;
+    int64_t P = 0;
+    int64_t first_len = 0;
+    int device = 0;
+    std::unique_lock<std::mutex> lock;
+};
+// once the stream has been waited for
+void split_merge_release(SplitMergeResult& r);
+int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t min_size, SplitMergeResult* out, hipStream_t s);
 // host-side CPU partitioner (glc_host.cpp)
 int cpu_split_merge(int dtype, const void* h_values, int64_t n, int32_t min_size, std::vector<int32_t>& st,
                     std::vector<int32_t>& en);

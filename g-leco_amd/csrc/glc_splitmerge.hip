@@ -1038,15 +1038,96 @@ __global__ void k_sm_scan_add(int32_t* __restrict__ pos, int64_t N, const int32_
     if (i < N) pos[i] += tile_off[i / kScanTile];
 }
 
-__global__ void k_sm_emit(const int32_t* __restrict__ mark, const int32_t* __restrict__ pos,
-                          const int32_t* __restrict__ best_end, const double* __restrict__ best_cost, int64_t J,
-                          int32_t m, int32_t* __restrict__ st, int32_t* __restrict__ en, double* __restrict__ cost) {
-    const int64_t j = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (j >= J || !mark[j]) return;
-    const int32_t p = pos[j];
-    st[p] = static_cast<int32_t>(j * m);
-    en[p] = best_end[j];
-    cost[p] = best_cost[j];
+// Marked entry i becomes entry p of the next list; entry 0's length is
+// reported to pinned memory (host[1]).
+struct EmitSplit {
+    const int32_t* best_end;
+    const double* best_cost;
+    int32_t m;
+    int32_t *st, *en;
+    double* cost;
+    int64_t* host;
+    __device__ void operator()(int64_t i, int64_t p) const {
+        const int32_t s = static_cast<int32_t>(i * m), e = best_end[i];
+        st[p] = s;
+        en[p] = e;
+        cost[p] = best_cost[i];
+        if (p == 0) host[1] = e - s;
+    }
+};
+struct EmitGroups {
+    const int32_t* gend;
+    const double* gcost;
+    const int32_t *st, *en;
+    int32_t *ost, *oen;
+    double* ocost;
+    int64_t* host;
+    __device__ void operator()(int64_t i, int64_t p) const {
+        const int32_t s = st[i], e = en[gend[i] - 1];
+        ost[p] = s;
+        oen[p] = e;
+        ocost[p] = gcost[i];
+        if (p == 0) host[1] = e - s;
+    }
+};
+template <class E>
+__global__ void k_sm_emit(const int32_t* __restrict__ mark, const int32_t* __restrict__ pos, int64_t N, E emit) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < N && mark[i]) emit(i, pos[i]);
+}
+
+// Chain, scan and emission of a list of at most kChain entries by one
+// workgroup: one launch instead of seven (4-5 us each with its gap), which were
+// half of a 2^16-value call.
+template <class F, class E>
+__global__ __launch_bounds__(kChainThreads) void k_sm_chain_small(F next, E emit, int32_t N, int64_t* __restrict__ host) {
+    __shared__ int32_t s_j[kChain];
+    __shared__ uint8_t s_m[kChain];
+    __shared__ int32_t s_w[kChainThreads / 64 + 1];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    bool inside = false;
+    for (int32_t i = tid; i < N; i += kChainThreads) {
+        s_j[i] = static_cast<int32_t>(next(i));
+        s_m[i] = i == 0;
+        inside = inside || s_j[i] < N;
+    }
+    bool any = __syncthreads_or(inside);
+    while (any) {
+        for (int32_t i = tid; i < N; i += kChainThreads)
+            if (s_m[i] && s_j[i] < N) s_m[s_j[i]] = 1;
+        __syncthreads();
+        any = chain_double(s_j, N);
+    }
+    // positions: thread tid counts entries tid * kChainPer ...
+    int32_t sum = 0;
+#pragma unroll
+    for (int q = 0; q < kChainPer; ++q) {
+        const int32_t i = tid * kChainPer + q;
+        sum += i < N ? s_m[i] : 0;
+    }
+    int32_t incl = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+    }
+    if (lane == 63) s_w[w] = incl;
+    __syncthreads();
+    if (tid == 0) {
+        int32_t acc = 0;
+        for (int k = 0; k < kChainThreads / 64; ++k) {
+            const int32_t t = s_w[k];
+            s_w[k] = acc;
+            acc += t;
+        }
+        host[0] = acc;
+    }
+    __syncthreads();
+    int32_t at = s_w[w] + incl - sum;
+#pragma unroll
+    for (int q = 0; q < kChainPer; ++q) {
+        const int32_t i = tid * kChainPer + q;
+        if (i < N && s_m[i]) emit(i, at++);
+    }
 }
 
 // ---- merge -------------------------------------------------------------------
@@ -1145,19 +1226,6 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_grow(const T* __restrict__ v,
     }
 }
 
-// compaction of the group starts: out lists of the pass
-__global__ void k_sm_emit_groups(const int32_t* __restrict__ spec, const int32_t* __restrict__ pos,
-                                 const int32_t* __restrict__ gend, const double* __restrict__ gcost,
-                                 const int32_t* __restrict__ st, const int32_t* __restrict__ en, int64_t P,
-                                 int32_t* __restrict__ ost, int32_t* __restrict__ oen, double* __restrict__ ocost) {
-    const int64_t a = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (a >= P || !spec[a]) return;
-    const int32_t p = pos[a];
-    ost[p] = st[a];
-    oen[p] = en[gend[a] - 1];
-    ocost[p] = gcost[a];
-}
-
 template <class F> int dispatch_dtype(int dtype, F&& f) {
     switch (dtype) {
         case GLC_I32: return f(int32_t());
@@ -1173,10 +1241,9 @@ unsigned blocks(int64_t n, int b) { return static_cast<unsigned>((n + b - 1) / b
 // Scratch of one split/merge call, kept per device between calls and grown
 // when a larger column needs more (a per-call hipMalloc/hipFree pair costs
 // hundreds of microseconds and the free synchronises the device).  Held
-// until the process ends while it is at most kSmKeep bytes (a column of about
-// 2^28 values at minimum size 128; larger ones give it back, their call is 100
-// times longer than the allocation); the lock covers a whole call, which ends
-// with its stream synchronised.
+// until the process ends; one above kSmKeep bytes (a column of about 2^28 values
+// at minimum size 128) is given back by split_merge_release.  The lock covers a call and its caller's copy of the boundaries, after
+// which the stream has been waited for.
 constexpr int64_t kSmKeep = int64_t(1) << 30;
 struct SmScratch {
     std::mutex mu;
@@ -1194,13 +1261,9 @@ SmScratch& sm_scratch(int device) {
 
 }  // namespace
 
-// Partition d_values[0, n) on the device; the boundaries end up in host
-// vectors (the caller uploads them into the column arena).
-int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::vector<int32_t>& st,
-                    std::vector<int32_t>& en, hipStream_t s) {
-    st.clear();
-    en.clear();
-    if (n <= 0) return GLC_OK;
+// Partition d_values[0, n), n > 0, on the device; the boundaries stay in the
+// scratch, whose lock goes to the caller.
+int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, SplitMergeResult* out, hipStream_t s) {
     if (m <= 0 || m > (1 << 20)) return fail(GLC_ERR_INVALID_ARG, "split/merge minimum size must be in [1, 2^20]");
     const int64_t J = (n + m - 1) / m;
     // blocks: B = m up to kHullMaxB; above, the largest divisor of m from 32
@@ -1232,8 +1295,10 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
     const int64_t bytes = 9 * i4 + 4 * d8 + 256 + 2 * q16 + 2 * c16 + 3 * t4 + (hulls ? hy + hx + hn : 0);
     int dev = 0;
     GLC_HIP(hipGetDevice(&dev));
+    HostWords host;
+    if (!host.p) return fail(GLC_ERR_OOM, "pinned host allocation failed");
     SmScratch& sc = sm_scratch(dev);
-    std::lock_guard<std::mutex> scratch_lock(sc.mu);
+    std::unique_lock<std::mutex> scratch_lock(sc.mu);
     if (sc.bytes < bytes) {
         if (sc.p) (void)hipFree(sc.p);  // the previous call ended synchronised
         sc.p = nullptr;
@@ -1252,7 +1317,6 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
     int32_t *best_end = I(0), *exits = I(1), *mark = I(2), *pos = I(3);
     int32_t *st0 = I(4), *st1 = I(5), *en0 = I(6), *en1 = I(7), *gend = I(8);
     double *best_cost = D(0), *cost0 = D(1), *cost1 = D(2), *gcost = D(3);
-    int64_t* result = reinterpret_cast<int64_t*>(p + 9 * i4 + 4 * d8);
     char* pq = p + 9 * i4 + 4 * d8 + 256;
     i128 *pf1 = reinterpret_cast<i128*>(pq), *pf2 = reinterpret_cast<i128*>(pq + q16);
     i128 *cf1 = reinterpret_cast<i128*>(pq + 2 * q16), *cf2 = reinterpret_cast<i128*>(pq + 2 * q16 + c16);
@@ -1270,16 +1334,25 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
         const int64_t nt = (N + kScanTile - 1) / kScanTile;
         hipLaunchKernelGGL(k_sm_scan_local, dim3(static_cast<unsigned>(nt)), dim3(kSmThreads), 0, s, mark, N, pos,
                            tile_tot);
-        hipLaunchKernelGGL(k_sm_scan, dim3(1), dim3(kScan), 0, s, tile_tot, nt, tile_off, result);
+        hipLaunchKernelGGL(k_sm_scan, dim3(1), dim3(kScan), 0, s, tile_tot, nt, tile_off, host.p);
         hipLaunchKernelGGL(k_sm_scan_add, dim3(blocks(N, 256)), dim3(256), 0, s, pos, N, tile_off);
     };
-    // mark[i] = the walk from entry 0 over next() reaches entry i
-    auto chain = [&](auto next, int64_t N) {
+    // the entries that the walk from entry 0 over next() reaches, in order, to
+    // emit(entry, position); their number to host.p[0]
+    auto chain = [&](auto next, auto emit, int64_t N) {
         using F = decltype(next);
+        using E = decltype(emit);
+        if (N <= kChain) {
+            hipLaunchKernelGGL((k_sm_chain_small<F, E>), dim3(1), dim3(kChainThreads), 0, s, next, emit,
+                               static_cast<int32_t>(N), host.p);
+            return;
+        }
         const unsigned nc = blocks(N, kChain);
         hipLaunchKernelGGL(k_sm_chain_exit<F>, dim3(nc), dim3(kChainThreads), 0, s, next, N, exits);
         hipLaunchKernelGGL(k_sm_chain_walk, dim3(1), dim3(64), 0, s, exits, N, static_cast<int64_t>(nc), entry);
         hipLaunchKernelGGL(k_sm_chain_mark<F>, dim3(nc), dim3(kChainThreads), 0, s, next, N, entry, mark);
+        scan_marks(N);
+        hipLaunchKernelGGL(k_sm_emit<E>, dim3(blocks(N, 256)), dim3(256), 0, s, mark, pos, N, emit);
     };
     int rc = dispatch_dtype(dtype, [&](auto t) -> int {
         using T = decltype(t);
@@ -1303,28 +1376,20 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
                                best_end, best_cost);
         }
         GLC_HIP(hipGetLastError());
-        chain(ChainSplit{best_end, J, m}, J);
-        scan_marks(J);
-        hipLaunchKernelGGL(k_sm_emit, dim3(blocks(J, 256)), dim3(256), 0, s, mark, pos, best_end, best_cost, J, m,
-                           st0, en0, cost0);
+        chain(ChainSplit{best_end, J, m}, EmitSplit{best_end, best_cost, m, st0, en0, cost0, host.p}, J);
         GLC_HIP(hipGetLastError());
-        int64_t P = 0;
-        GLC_HIP(hipMemcpyAsync(&P, result, 8, hipMemcpyDeviceToHost, s));
         GLC_HIP(hipStreamSynchronize(s));
+        int64_t P = host.p[0];
         if (P < 1 || P > J) return fail(GLC_ERR_STATE, "split phase produced an invalid partition count");
         int32_t *sa = st0, *sb = st1, *ea = en0, *eb = en1;
         double *ca = cost0, *cb = cost1;
         for (int iter = 0; iter < 10 && P > 1; ++iter) {  // CpuPartitioner.cuh:198-242
             hipLaunchKernelGGL(k_sm_grow<T>, dim3(blocks(P, kSmThreads / 64)), dim3(kSmThreads), 0, s, v, sa, ea, ca,
                                P, pf, h, gend, gcost);
-            chain(ChainMerge{gend}, P);
-            scan_marks(P);
-            hipLaunchKernelGGL(k_sm_emit_groups, dim3(blocks(P, 256)), dim3(256), 0, s, mark, pos, gend, gcost, sa, ea,
-                               P, sb, eb, cb);
+            chain(ChainMerge{gend}, EmitGroups{gend, gcost, sa, ea, sb, eb, cb, host.p}, P);
             GLC_HIP(hipGetLastError());
-            int64_t Pn = 0;
-            GLC_HIP(hipMemcpyAsync(&Pn, result, 8, hipMemcpyDeviceToHost, s));
             GLC_HIP(hipStreamSynchronize(s));
+            const int64_t Pn = host.p[0];
             if (Pn < 1 || Pn > P) return fail(GLC_ERR_STATE, "merge pass produced an invalid partition count");
             const bool changed = Pn < P;  // every merge removes one entry
             P = Pn;
@@ -1333,20 +1398,30 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, std::
             std::swap(ca, cb);
             if (!changed) break;
         }
-        st.resize(static_cast<size_t>(P));
-        en.resize(static_cast<size_t>(P));
-        GLC_HIP(hipMemcpyAsync(st.data(), sa, P * 4, hipMemcpyDeviceToHost, s));
-        GLC_HIP(hipMemcpyAsync(en.data(), ea, P * 4, hipMemcpyDeviceToHost, s));
-        GLC_HIP(hipStreamSynchronize(s));
+        out->d_st = sa;
+        out->d_en = ea;
+        out->P = P;
+        out->first_len = host.p[1];
         return GLC_OK;
     });
-    if (rc) (void)hipStreamSynchronize(s);  // no kernel of this call may outlive the lock on the scratch
+    if (rc) {
+        (void)hipStreamSynchronize(s);  // no kernel of this call may outlive the lock on the scratch
+        return rc;
+    }
+    out->device = dev;
+    out->lock = std::move(scratch_lock);
+    return GLC_OK;
+}
+
+void split_merge_release(SplitMergeResult& r) {
+    if (!r.lock.owns_lock()) return;
+    SmScratch& sc = sm_scratch(r.device);
     if (sc.bytes > kSmKeep) {
         (void)hipFree(sc.p);
         sc.p = nullptr;
         sc.bytes = 0;
     }
-    return rc;
+    r.lock.unlock();
 }
 
 }  // namespace glc
