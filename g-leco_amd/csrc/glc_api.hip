@@ -42,7 +42,7 @@ ArenaLayout layout_for(int64_t P, int64_t n_index) {
     L.off = take(P * 8);
     L.err = take(P * 8);
     L.desc = take(P * 32);
-    L.tile = take((n_index + 2) * 4);  // + 2 work-stealing counters
+    L.tile = take(n_index * 4);
     L.tinfo = take(std::max<int64_t>(n_index - 1, 1) * static_cast<int64_t>(sizeof(TileInfo)));
     L.sched = take(kSchedBytes);
     L.summary = take(static_cast<int64_t>(sizeof(IndexSummary)) + 64);
@@ -717,6 +717,7 @@ int glc_column_set_decode_schedule(glc_column* c, int32_t schedule) {
     if (schedule < GLC_DECODE_TILE_W1 || schedule > GLC_DECODE_HALF_TILE_W1)
         return fail(GLC_ERR_INVALID_ARG, "unknown decode schedule");
     c->dec_sched = schedule;
+    c->dec_auto = false;
     return GLC_OK;
 }
 
@@ -731,6 +732,7 @@ int glc_column_set_decode_pace(glc_column* c, int32_t pace) {
     if (pace != 0 && pace != 4 && pace != 8 && pace != 16 && pace != 24)
         return fail(GLC_ERR_INVALID_ARG, "decode pace must be 0, 4, 8, 16 or 24");
     c->dec_pace = pace;
+    c->dec_auto = false;
     return GLC_OK;
 }
 

@@ -468,6 +468,7 @@ int glc_batch_get_column(glc_batch* b, int index, const glc_column** col) {
         v->d_words = b->words + b->words_off[index];
         v->words_alloc = b->words_res[index] + glc::kPayloadPadWords;
         v->fixed_size = static_cast<int32_t>(std::min<int64_t>(b->S, v->n));
+        v->spans = b->S % glc::kIndexTile != 0;
         v->fit_block = glc::fit_block_size(std::min<int64_t>(b->S, v->n));
     }
     v->total_bits = b->bits[index];

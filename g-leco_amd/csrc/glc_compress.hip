@@ -1927,15 +1927,14 @@ int launch_index(glc_column* c, bool scan, IndexSummary* d_sum, IndexSummary* h_
 // partitions (fixed: [pS, min((p+1)S, n)); else copied from src_st / src_en, or
 // already there when those are null), the initial model type (host PartitionInfo
 // init, G:409-414), for lists that may hold empty partitions (which the fit
-// skips) zero outputs, and the summary and work-stealing counters.
+// skips) zero outputs, and the summary.
 __global__ void k_column_setup(int32_t* __restrict__ st, int32_t* __restrict__ en, int32_t* __restrict__ type,
                                double* __restrict__ params, int32_t* __restrict__ bits, int64_t* __restrict__ err,
                                int64_t P, int64_t n, int32_t S, const int32_t* __restrict__ src_st,
-                               const int32_t* __restrict__ src_en, bool empties, int32_t* __restrict__ counters,
+                               const int32_t* __restrict__ src_en, bool empties,
                                IndexSummary* __restrict__ sum) {
     const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (p < 2) counters[p] = 0;
-    if (p == 2) *sum = IndexSummary{};
+    if (p == 0) *sum = IndexSummary{};
     if (p >= P) return;
     if (S > 0) {
         const int64_t s0 = p * S;
@@ -1955,9 +1954,9 @@ __global__ void k_column_setup(int32_t* __restrict__ st, int32_t* __restrict__ e
 
 int launch_column_setup(glc_column* c, int32_t S, const int32_t* src_st, const int32_t* src_en, bool empties,
                         hipStream_t s) {
-    hipLaunchKernelGGL(k_column_setup, dim3(grid_for(c->P > 3 ? c->P : 3, 256)), dim3(256), 0, s, c->d_start, c->d_end,
+    hipLaunchKernelGGL(k_column_setup, dim3(grid_for(c->P, 256)), dim3(256), 0, s, c->d_start, c->d_end,
                        c->d_type, c->d_params, c->d_bits, c->d_err, c->P, c->n, S, src_st, src_en, empties,
-                       c->d_tile_part + c->n_index, summary_ptr(c));
+                       summary_ptr(c));
     GLC_HIP(hipGetLastError());
     return GLC_OK;
 }

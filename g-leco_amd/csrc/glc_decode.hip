@@ -8,14 +8,13 @@
 //                       decompression/WorkStealingDecompressionKernels.cuh:332-521)
 //   k_decode_steal      the same wave tiles claimed from per-XCD atomic queues
 //                       (the explicit work-stealing comparator)
-//   k_decode_parts      one workgroup per partition, or persistent workgroups
-//                       grabbing whole partitions (…_OnTheFly_Optimized_V2,
-//                        FullDecompressionKernels.cuh:293-378, and
-//                        …_WorkStealingAdvanced, WorkStealingDecompressionKernels.cuh:526-619).
-//                       A partition is decoded in spans of up to 2048 elements:
-//                       the span's payload window is staged into LDS with
-//                       16-byte loads, then each thread extracts, predicts and
-//                       stores its elements.
+// Every full-decode mode takes these.  The reference's per-partition schedules
+// (…_OnTheFly_Optimized_V2, FullDecompressionKernels.cuh:293-378, a workgroup
+// per partition; …_WorkStealingAdvanced,
+// WorkStealingDecompressionKernels.cuh:526-619, workgroups that claim partitions)
+// were slower than the tiles on every layout measured: 2^26 int32 values in
+// partitions of 1024, 62 us in tiles, 105 with a workgroup per partition, 805 with
+// claims; int64 in partitions of 64, 148 / 875 / 11945 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,10 +25,6 @@
 
 namespace glc {
 namespace {
-
-constexpr int kThreads = kDecodeThreads;
-constexpr int kTile = kDecodeTile;                 // elements per workgroup tile
-constexpr int kWinWords = kTile * 2 + 16;          // LDS words: 2048 elements x 64 bits + slack
 
 enum Op { OP_PACKED = 0, OP_PLAIN = 1, OP_UNPACK = 2 };
 
@@ -43,119 +38,13 @@ struct DecArgs {
     int64_t n;
     int64_t P;
     int64_t n_index;
-    int32_t* counter;                    // work-stealing counters [2] (workgroup schedules)
     const TileInfo* __restrict__ tinfo;  // per-1024-element tile: first bit, bits, partition, path
     int64_t wlimit;                      // payload words (row-load base clamp)
     int32_t* sched;                      // per-XCD work-stealing queues (wave schedule)
     int32_t vec16;                       // out is 16-byte aligned: narrow tiles store 16 bytes per lane
     int32_t pace;                        // pause after each narrow row's stores (pace_row)
+    int32_t pace2;                       // the same where predictions are beyond 2^50 (dec_fast_range tier 2)
 };
-
-// Decode elements [e0, e1) of partition `d` (caller guarantees e0 >= d.start
-// and e1 <= d.start + d.len).  Uses s_w as the LDS payload window.
-template <class T, int OP>
-__device__ __forceinline__ void decode_span(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t e1,
-                                            uint32_t* __restrict__ s_w) {
-    const int tid = threadIdx.x;
-    const int32_t type = desc_type(d.packed);
-    const int b = desc_bits(d.packed);
-    const int32_t lbase = static_cast<int32_t>(e0 - d.start);
-    const int64_t cnt = e1 - e0;
-    if constexpr (OP == OP_PLAIN) {
-        T* __restrict__ out = static_cast<T*>(a.out);
-        const double t2 = (type == MODEL_POLY2) ? a.params[4 * p + 2] : 0.0;
-        for (int64_t k = tid; k < cnt; k += kThreads) {
-            const int64_t e = e0 + k;
-            const int64_t pl = a.plain[e];
-            T v;
-            if (type == MODEL_DIRECT_COPY) v = static_cast<T>(pl);
-            else if (type == MODEL_POLY2)
-                v = apply_delta<T>(dec_pred_poly<T>(type, d.theta0, d.theta1, t2, lbase + static_cast<int32_t>(k)), pl);
-            else v = apply_delta<T>(dec_pred<T>(d.theta0, d.theta1, lbase + static_cast<int32_t>(k)), pl);
-            out[e] = v;
-        }
-        return;
-    } else {
-        // stage the payload window: bits [W0, W0 + cnt*b)
-        const int64_t W0 = desc_off(d.packed) + static_cast<int64_t>(lbase) * b;
-        const int64_t wbase = (W0 >> 5) & ~3LL;                       // 16-byte aligned
-        const int64_t wend = ((W0 + cnt * b + 31) >> 5) + 2;          // +2 words for 3-word reads
-        const int nchunks = static_cast<int>((wend - wbase + 3) >> 2);
-        const uint4* __restrict__ src = reinterpret_cast<const uint4*>(a.words + wbase);
-        uint4* dst = reinterpret_cast<uint4*>(s_w);
-        for (int c = tid; c < nchunks; c += kThreads) dst[c] = src[c];
-        __syncthreads();
-        const uint32_t rel0 = static_cast<uint32_t>(W0 - (wbase << 5));
-        const double t2 = (type == MODEL_POLY2) ? a.params[4 * p + 2] : 0.0;
-        for (int64_t k = tid; k < cnt; k += kThreads) {
-            const uint32_t rel = rel0 + static_cast<uint32_t>(k) * static_cast<uint32_t>(b);
-            const uint64_t raw = extract_raw(s_w, rel, b);
-            const int64_t e = e0 + k;
-            if constexpr (OP == OP_UNPACK) {
-                int64_t* __restrict__ out = static_cast<int64_t*>(a.out);
-                out[e] = (type == MODEL_DIRECT_COPY) ? static_cast<int64_t>(static_cast<T>(raw)) : sign_extend(raw, b);
-            } else {
-                T* __restrict__ out = static_cast<T*>(a.out);
-                T v;
-                const int32_t i = lbase + static_cast<int32_t>(k);
-                if (type == MODEL_DIRECT_COPY) v = static_cast<T>(raw);
-                else if (type == MODEL_POLY2)
-                    v = apply_delta<T>(dec_pred_poly<T>(type, d.theta0, d.theta1, t2, i), sign_extend(raw, b));
-                else v = apply_delta<T>(dec_pred<T>(d.theta0, d.theta1, i), sign_extend(raw, b));
-                out[e] = v;
-            }
-        }
-        __syncthreads();  // window reused by the next span
-    }
-}
-
-// One partition per workgroup (persistent = false: grid = P) or persistent
-// workgroups grabbing partitions from the counter (persistent = true).
-template <class T, int OP, bool PERSISTENT>
-__global__ __launch_bounds__(kThreads) void k_decode_parts(DecArgs a) {
-    __shared__ __align__(16) uint32_t s_w[kWinWords];
-    __shared__ int s_p;
-    int64_t p = blockIdx.x;
-    for (;;) {
-        if constexpr (PERSISTENT) {
-            if (threadIdx.x == 0) s_p = atomicAdd(&a.counter[0], 1);
-            __syncthreads();
-            p = s_p;
-            __syncthreads();
-        }
-        if (p >= a.P) break;
-        const Desc d = a.desc[p];
-        const int64_t ds = d.start, de = ds + d.len;
-        for (int64_t e0 = ds; e0 < de; e0 += kTile) {
-            const int64_t e1 = (e0 + kTile < de) ? e0 + kTile : de;
-            decode_span<T, OP>(a, d, p, e0, e1, s_w);
-        }
-        if constexpr (!PERSISTENT) break;
-    }
-    if constexpr (PERSISTENT) {
-        if (threadIdx.x == 0) {
-            __threadfence();
-            if (atomicAdd(&a.counter[1], 1) == static_cast<int>(gridDim.x) - 1) {
-                atomicExch(&a.counter[0], 0);
-                atomicExch(&a.counter[1], 0);
-            }
-        }
-    }
-}
-
-// Zero the gaps between partitions (elements no partition holds); used by the
-// per-partition schedules, which only visit partition elements.
-template <class T, int OP>
-__global__ void k_fill_gaps(DecArgs a) {
-    const int64_t p = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (p > a.P) return;
-    const int64_t g0 = (p == 0) ? 0 : static_cast<int64_t>(a.desc[p - 1].start) + a.desc[p - 1].len;
-    const int64_t g1 = (p == a.P) ? a.n : a.desc[p].start;
-    for (int64_t e = g0; e < g1; ++e) {
-        if constexpr (OP == OP_UNPACK) static_cast<int64_t*>(a.out)[e] = 0;
-        else static_cast<T*>(a.out)[e] = T(0);
-    }
-}
 
 // ---------------------------------------------------------------------------
 // Wave-level decoder: no LDS staging and no workgroup barriers.
@@ -331,7 +220,8 @@ __device__ __forceinline__ void narrow_v_rows(const DecArgs& a, const TileInfo& 
             for (int k = 0; k < V; ++k)
                 if (e + k < e1) put(out + e + k, v[k]);
         }
-        if constexpr (FAST != 0) pace_row(a.pace);
+        if constexpr (FAST == 1) pace_row(a.pace);
+        else if constexpr (FAST == 2) pace_row(a.pace2);
     }
 }
 
@@ -1038,12 +928,11 @@ __global__ __launch_bounds__(64 * WPG) void k_batch_decode(const BatchCol* __res
         a.n = c.n;
         a.P = c.P;
         a.n_index = c.n_index;
-        a.counter = nullptr;
         a.tinfo = c.tinfo;
         a.sched = nullptr;
         a.wlimit = c.payload_words;
         a.vec16 = (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
-        a.pace = 0;
+        a.pace = a.pace2 = 0;
         const int64_t t = g - c.tile_base;
         if (a.vec16) {
             switch (c.dtype) {
@@ -1102,12 +991,11 @@ __global__ __launch_bounds__(64) void k_batch_decode_half(const BatchCol* __rest
     a.n = c.n;
     a.P = c.P;
     a.n_index = c.n_index;
-    a.counter = nullptr;
     a.tinfo = c.tinfo;
     a.sched = nullptr;
     a.wlimit = c.payload_words;
     a.vec16 = (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
-    a.pace = 0;
+    a.pace = a.pace2 = 0;
     const int64_t t = g - c.tile_base;
     switch (c.dtype) {
         case GLC_I32: batch_half<int32_t>(a, t, h, lane); break;
@@ -1127,18 +1015,6 @@ template <class F> int dispatch_dtype(int dtype, F&& f) {
     }
 }
 
-int device_cus() {
-    static int cus = 0;
-    if (!cus) {
-        int dev = 0;
-        if (hipGetDevice(&dev) != hipSuccess) return 256;
-        hipDeviceProp_t prop;
-        if (hipGetDeviceProperties(&prop, dev) != hipSuccess) return 256;
-        cus = prop.multiProcessorCount;
-    }
-    return cus;
-}
-
 DecArgs make_args(const glc_column* c, void* out) {
     DecArgs a;
     a.desc = c->d_desc;
@@ -1150,12 +1026,15 @@ DecArgs make_args(const glc_column* c, void* out) {
     a.n = c->n;
     a.P = c->P;
     a.n_index = c->n_index;
-    a.counter = reinterpret_cast<int32_t*>(c->d_tile_part + c->n_index);  // 2 counters after the index
     a.tinfo = c->d_tinfo;
     a.wlimit = c->payload_words;
     a.sched = c->d_sched;
     a.vec16 = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
-    a.pace = c->dec_pace;
+    a.pace = a.pace2 = c->dec_pace;
+    // no schedule set: long columns with predictions beyond 2^50 decode faster
+    // with their stores spaced out (half tiles, int64 timestamps: 2^28 values 472 ->
+    // 452 us, 3e8 528 -> 496; 2^26 106 -> 109)
+    if (c->dec_auto && c->n >= (int64_t(1) << 27)) a.pace2 = 16;
     return a;
 }
 
@@ -1189,21 +1068,6 @@ template <class T, int OP> int run(const DecArgs& a, int sched, hipStream_t s, i
                                    dim3(64 * kWavesPerGroup), 0, s, a, nwt);
             break;
         }
-        case 2:
-        case 3: {
-            hipLaunchKernelGGL((k_fill_gaps<T, OP>), dim3(static_cast<unsigned>((a.P + 1 + 255) / 256)), dim3(256), 0,
-                               s, a);
-            if (sched == 2) {
-                hipLaunchKernelGGL((k_decode_parts<T, OP, false>), dim3(static_cast<unsigned>(a.P)), dim3(kThreads), 0,
-                                   s, a);
-            } else {
-                int64_t g = static_cast<int64_t>(device_cus()) * 8;
-                if (g > a.P) g = a.P;
-                hipLaunchKernelGGL((k_decode_parts<T, OP, true>), dim3(static_cast<unsigned>(g)), dim3(kThreads), 0, s,
-                                   a);
-            }
-            break;
-        }
         default: return fail(GLC_ERR_INVALID_ARG, "bad schedule");
     }
     GLC_HIP(hipGetLastError());
@@ -1220,14 +1084,14 @@ int launch_decode_full(const glc_column* c, void* d_out, int mode, hipStream_t s
         case GLC_FULL_AUTO: plain = c->d_plain != nullptr; sched = 0; break;
         case GLC_FULL_BITPACKED: plain = false; sched = 0; break;
         case GLC_FULL_PREUNPACKED: plain = true; sched = 0; break;
-        case GLC_FULL_V2: plain = c->d_plain != nullptr; sched = 2; break;
+        case GLC_FULL_V2: plain = c->d_plain != nullptr; sched = 0; break;
         // Work stealing: tiles are claimed by CUs as they free up through the
         // hardware workgroup dispatcher (one short-lived wave per 1024-value
         // tile).  Explicit claims through device-scope atomics (kModeWaveSteal)
         // serialize at ~14 ns per claim: 3.8 ms against 0.43-0.48 ms for the
         // 2^18 tiles of a 2^28-value column.
         case GLC_FULL_WORKSTEAL: plain = c->d_plain != nullptr; sched = 0; break;
-        case GLC_FULL_WORKSTEAL_ADV: plain = c->d_plain != nullptr; sched = 3; break;
+        case GLC_FULL_WORKSTEAL_ADV: plain = c->d_plain != nullptr; sched = 0; break;
         case GLC_FULL_COOP_EXACT: plain = true; sched = 0; break;
         // the explicit work-stealing comparator of WorkStealingDecompressionKernels.cuh:332-521:
         // wave tiles claimed from per-XCD atomic queues
@@ -1240,9 +1104,15 @@ int launch_decode_full(const glc_column* c, void* d_out, int mode, hipStream_t s
         return fail(GLC_ERR_UNSUPPORTED, "bit-packed payload was released by glc_preunpack(free_packed=1)");
     if (c->P == 0) return fail(GLC_ERR_STATE, "column has values but no partitions");
     DecArgs a = make_args(c, d_out);
+    // No schedule set: 64-bit columns of whole-tile partitions take half tiles
+    // (2^28 values 399-514 us against 431-535 with four tiles a workgroup, by width;
+    // equal below 2^27, never slower).  32-bit ones are faster in whole tiles (2^28
+    // 239-278 against 254-291), and the half-tile kernel has no fast path for
+    // partition-spanning tiles.
+    const int dsched = (c->dec_auto && c->elem_size == 8 && !c->spans) ? GLC_DECODE_HALF_TILE_W1 : c->dec_sched;
     return dispatch_dtype(c->dtype, [&](auto t) {
         using T = decltype(t);
-        return plain ? run<T, OP_PLAIN>(a, sched, s, c->dec_sched) : run<T, OP_PACKED>(a, sched, s, c->dec_sched);
+        return plain ? run<T, OP_PLAIN>(a, sched, s, c->dec_sched) : run<T, OP_PACKED>(a, sched, s, dsched);
     });
 }
 
@@ -1257,6 +1127,8 @@ int glc_autotune_decode(glc_column* c, void* d_out, int32_t reps, hipStream_t s,
     const int sched_of[kS] = {GLC_DECODE_TILE_W1, GLC_DECODE_TILE_W4, GLC_DECODE_HALF_TILE_W1};
     const int pace_of[kPaces] = {0, 4, 8, 16, 24};
     const int saved = c->dec_sched, saved_pace = c->dec_pace;
+    const bool saved_auto = c->dec_auto;
+    c->dec_auto = false;
     std::vector<hipEvent_t> ev(static_cast<size_t>(2 * kC * reps), nullptr);
     int rc = GLC_OK;
     for (auto& e : ev)
@@ -1306,6 +1178,7 @@ int glc_autotune_decode(glc_column* c, void* d_out, int32_t reps, hipStream_t s,
     if (rc || best < 0) {
         c->dec_sched = saved;
         c->dec_pace = saved_pace;
+        c->dec_auto = saved_auto;
         return rc;
     }
     set(best);

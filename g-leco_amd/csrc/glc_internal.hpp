@@ -29,9 +29,6 @@ constexpr int kIndexShift = 10;                 // tile_part granularity: 1024 e
 constexpr int64_t kIndexTile = 1LL << kIndexShift;
 constexpr int kPayloadPadWords = 192;           // zero words after the payload: branch-free row loads read
                                                 // up to word base+128 with base clamped to the payload end
-constexpr int kDecodeThreads = 256;             // 4 wave64 per workgroup
-constexpr int kDecodeTile = 2048;               // elements per workgroup tile (8 per thread)
-constexpr int kMaxTileParts = 64;               // partitions of one tile staged in LDS (slow path)
 constexpr int kModeWaveSteal = 102;             // full-decode mode: wave tiles claimed from per-XCD atomic
                                                 // queues (the explicit work-stealing comparator)
 
@@ -179,6 +176,7 @@ struct glc_column {
     int32_t fit_form = 0;           // contraction form of the fit (glc_opts.fit_form)
     int32_t has_poly = 0;
     bool spans = false;             // some tile holds several partitions or a gap (IndexSummary::unaligned)
+    bool dec_auto = true;           // no schedule or pace set yet: launch_decode_full may pick
     int32_t dec_sched = GLC_DECODE_TILE_W4;  // packed full-decode schedule (glc_column_set_decode_schedule)
     int32_t dec_pace = 0;                    // pause per decoded row (glc_column_set_decode_pace)
     // arena

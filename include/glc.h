@@ -66,7 +66,7 @@ typedef enum {
     GLC_FULL_AUTO = 0,          /* decompressFullFile, G:680-693: pre-unpacked if present, else packed (fastest kernel) */
     GLC_FULL_BITPACKED = 1,     /* decompressFullFile_BitPacked, G:1739-1787 */
     GLC_FULL_PREUNPACKED = 2,   /* decompressFullFile_PreUnpacked, G:1790-1839 */
-    GLC_FULL_V2 = 3,            /* decompressFullFile_OnTheFly_Optimized_V2, G:1842-1875 (one workgroup per partition) */
+    GLC_FULL_V2 = 3,            /* decompressFullFile_OnTheFly_Optimized_V2, G:1842-1875 */
     GLC_FULL_WORKSTEAL = 4,     /* decompressFullFile_WorkStealing, G:166-217 */
     GLC_FULL_WORKSTEAL_ADV = 5, /* decompressFullFile_WorkStealingAdvanced, G:220-268 */
     GLC_FULL_COOP_EXACT = 6     /* decompressFullFileCooperative, G:271-345, with the FP64 model (exact) */
@@ -163,7 +163,9 @@ int glc_decompress_full(const glc_column* col, void* d_out, int mode, void* stre
  * column, BITPACKED, WORKSTEAL and the fixed decode): how the wave tiles are
  * grouped into workgroups.  It changes only the time, never the output.
  * Which is fastest depends on the column (its length, widths, element
- * size); glc_column_autotune_decode measures it.  Default: TILE_W4. */
+ * size); glc_column_autotune_decode measures it.  Default: TILE_W4; until a
+ * schedule or pace is set, the library may launch 64-bit columns in half
+ * tiles, paced, where that is the faster grouping for the column's layout. */
 enum {
     GLC_DECODE_TILE_W1 = 0,      /* one 1024-value tile per one-wave workgroup */
     GLC_DECODE_TILE_W4 = 1,      /* four consecutive tiles per four-wave workgroup */
