@@ -27,15 +27,18 @@
 // width of max |v_i - round(pr_i)|, pr_i = t0 + t1 * i in FP64.  Over a block the
 // real-valued residual of any line is largest at a hull vertex, so with D the
 // largest |v - pr| and H the largest |v - round(pr)| over the vertices,
-//     H <= max <= D + 0.5 + 3 eps,  eps = 2^-52 (|t0| + |t1| n)
-// (eps bounds one prediction's FP64 error; values and predictions within 2^52,
-// where every difference of two integers is exact).  Both ends have the same bit
-// width except when a power of two lies between them; then, and for blocks or
-// candidates outside the exact range, the values themselves are read.  That makes
-// one evaluation about 10 times cheaper than a pass over the values: 2^26 uint64
-// piecewise-linear values, m = 128: split 8.1 -> 1.33 ms, and growing every
-// partition's group takes 0.32 ms a pass where the sequential walk (one
-// workgroup regrowing groups across segments) took 23.4 ms.
+//     max(H, D - f) <= max <= D + f,  f = 0.5 + 4 eps + 2^-50 D,
+//     eps = 2^-52 (|t0| + |t1| n)
+// (one prediction's FP64 error is at most eps; D's own, each vertex as one fused
+// y - t1 x less the block's t0 + t1 x0, at most eps + 2^-52 D; values and
+// predictions within 2^52, where every difference of two integers is exact).  D
+// alone first; H, at more than twice the instructions a vertex, only where a power
+// of two lies between its bounds.  Both ends then have the same bit width except
+// where one lies between these too; there, and for blocks or candidates outside
+// the exact range, the values themselves are read.  That makes one evaluation about 10 times cheaper than a pass over the values: 2^26 uint64
+// piecewise-linear values, m = 128: split 8.1 -> 0.73 ms (1.13 with D and H at
+// once), and growing every partition's group takes 0.28 ms a pass where the
+// sequential walk (one workgroup regrowing groups across segments) took 23.4 ms.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -190,6 +193,11 @@ __device__ __forceinline__ i128 pfx_at(const i128* p, const i128* c, int64_t i) 
     return p[i] + c[i / kPfxChunk];
 }
 
+// the block that starts at position s (s < 2^31: 32-bit division)
+__device__ __forceinline__ int64_t block_of(const SmPrefix& pf, int64_t s) {
+    return static_cast<uint32_t>(s) / static_cast<uint32_t>(pf.B);
+}
+
 // Hull vertices of the blocks: vertex k of block b at
 // ((b / 64) * slots + k) * 64 + b % 64, so that lanes on consecutive blocks read
 // consecutive memory; y its value, x its index in the block.  nv[b]: the number of
@@ -214,7 +222,7 @@ __device__ __forceinline__ int64_t hull_at(int32_t slots, int64_t b, int k) {
 template <class T>
 __device__ __forceinline__ void range_line(const SmPrefix& pf, int64_t s, int64_t e, double& t0, double& t1,
                                            bool& fast) {
-    const int64_t ib = s / pf.B, ie = (e == pf.n) ? pf.JB : e / pf.B;
+    const int64_t ib = block_of(pf, s), ie = (e == pf.n) ? pf.JB : block_of(pf, e);
     const i128 sy = pfx_at(pf.p1, pf.c1, ie) - pfx_at(pf.p1, pf.c1, ib);
     const i128 sxy = pfx_at(pf.p2, pf.c2, ie) - pfx_at(pf.p2, pf.c2, ib) - static_cast<i128>(s) * sy;
     sm_theta(sy, sxy, e - s, t0, t1);
@@ -252,26 +260,40 @@ __device__ __forceinline__ int64_t scan_err(const T* __restrict__ v, int64_t x0,
     return mdi > mx ? mdi : mx;
 }
 
-// D and H (see the top of the file) over the vertices of one block whose
-// first value has index x0 in the range.  y, x: the block's vertices, `stride`
-// apart.
-__device__ __forceinline__ void hull_err(const double* __restrict__ y, const uint8_t* __restrict__ x, int stride,
-                                         int nv, int64_t x0, double t0, double t1, double& D, double& H) {
+// D (see the top of the file) over the vertices of one block whose first value
+// has index x0 in the range.  y, x: the block's vertices, `stride` apart.
+__device__ __forceinline__ double hull_far(const double* __restrict__ y, const uint8_t* __restrict__ x, int stride,
+                                           int nv, int32_t x0, double t0, double t1) {
+    double hi = -DBL_MAX, lo = DBL_MAX;
 #pragma unroll 4
     for (int k = 0; k < nv; ++k) {
-        const double yv = y[k * stride];
-        const double pr = t0 + t1 * static_cast<double>(x0 + x[k * stride]);  // no contraction (-ffp-contract=off)
-        D = __builtin_fmax(D, __builtin_fabs(yv - pr));
-        H = __builtin_fmax(H, __builtin_fabs(yv - round_away(pr)));
+        const double r = __builtin_fma(-t1, static_cast<double>(x[k * stride]), y[k * stride]);
+        hi = __builtin_fmax(hi, r);
+        lo = __builtin_fmin(lo, r);
     }
+    const double base = __builtin_fma(t1, static_cast<double>(x0), t0);
+    return __builtin_fmax(hi - base, base - lo);
+}
+
+// H over the same.
+__device__ __forceinline__ double hull_low(const double* __restrict__ y, const uint8_t* __restrict__ x, int stride,
+                                           int nv, int32_t x0, double t0, double t1) {
+    double H = 0.0;
+    for (int k = 0; k < nv; ++k) {
+        const double pr = t0 + t1 * static_cast<double>(x0 + x[k * stride]);  // no contraction (-ffp-contract=off)
+        H = __builtin_fmax(H, __builtin_fabs(y[k * stride] - round_away(pr)));
+    }
+    return H;
 }
 
 // The bit width that D and H (both <= 2^53 + 1) settle for a range of n
-// values, -1 if a power of two lies between the two bounds.
+// values, -1 if a power of two lies between the two bounds.  H = 0: from D
+// alone.
 __device__ __forceinline__ int32_t hull_bits(double D, double H, double t0, double t1, int64_t n) {
-    const double eps = (__builtin_fabs(t0) + __builtin_fabs(t1) * static_cast<double>(n)) * 2.220446049250313e-16;
-    const int32_t lo = bits_of(static_cast<int64_t>(H));
-    const int32_t hi = bits_of(static_cast<int64_t>(D * (1.0 + 4.44e-16) + 0.5 + 3.0 * eps));  // D is rounded itself
+    const double eps = (__builtin_fabs(t0) + __builtin_fabs(t1) * static_cast<double>(n)) * 0x1p-52;
+    const double far = D * 0x1p-50 + 0.5 + 4.0 * eps;
+    const int32_t lo = bits_of(static_cast<int64_t>(__builtin_ceil(__builtin_fmax(H, D - far))));
+    const int32_t hi = bits_of(static_cast<int64_t>(D + far));
     return lo == hi ? lo : -1;
 }
 
@@ -445,68 +467,197 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split(const T* __restrict__ v
 // Block sums, prefixes and hulls.  One workgroup per chunk of kPfxChunk = 64
 // blocks, staged in LDS (rows of B | 1 values: 64 lanes reading the same index
 // of 64 blocks hit different banks).
-//   filter  a value is no vertex of the upper (lower) hull if the mean of its
-//           neighbours at some equal distance is not below (above) it; the
-//           survivors of distances 1, 2, 4, ..., 32 are one ballot per 64 values;
-//   hull    wave 0 walks the survivors of the upper hulls, wave 1 those of the
-//           lower ones, a block per lane: Andrew's monotone chain with the kept
-//           vertices as a 128-bit mask, cross products exact in int64
-//           (differences <= 2^53, index distances < 2^7);
-//   sums    wave 2, a block per lane, and the scan over the 64 blocks.
+//   filter  a block per wave, twice 64 values: hull_filter;
+//   hull    wave 0 walks the upper hulls, wave 1 the lower ones, a block per
+//           lane: hull_chain;
+//   sums    waves 2 to 5, four lanes a block; the last wave scans the 64 blocks'.
 // p1, p2 receive the exclusive prefix inside the chunk, c1, c2 the chunk's
 // totals (k_sm_chunk_scan turns those into chunk offsets).  A block per lane
 // with values straight from memory (one cache line per lane and step) read the
-// column at 0.55 TB/s.
-struct HullMask {
-    uint64_t lo, hi;
-    __device__ __forceinline__ int top() const {  // highest set bit, -1 if none
-        return hi ? 127 - __builtin_clzll(hi) : lo ? 63 - __builtin_clzll(lo) : -1;
-    }
-    __device__ __forceinline__ int next() const {  // lowest set bit (there is one)
-        return lo ? __builtin_ctzll(lo) : 64 + __builtin_ctzll(hi);
-    }
-    __device__ __forceinline__ void flip(int i) {
-        if (i < 64) lo ^= 1ULL << i;
-        else hi ^= 1ULL << (i - 64);
-    }
-};
+// column at 0.55 TB/s.  Bound by latency: the rows of 64 blocks take half of the
+// LDS, so only two workgroups share a CU, and the walk keeps one wave of each hull
+// busy.  Hence few candidates and few dependent reads a turn for the walk, rows as
+// FP64 (nothing converted in a loop), and 16 waves for the other phases: 2^26
+// uint64 values 1002 -> 394 us, one workgroup alone 42 -> 26 us (with 4 waves, six
+// distances as the filter and a walk in int64 before).
+constexpr int kBlkThreads = 1024;
+constexpr int kSumWaves = 4;
+constexpr int kHullCand = 56;  // candidates of one hull; more: the block is read
 
-// One block's upper (UP) or lower hull among the points of `in`.
+// l <= r (UP) or l >= r for certain, for two products of a difference of values
+// (whole, <= 2^53) and one of indices (< 2^7).  Below 2^50 both are exact and so
+// is the test; above, their error and the test's is less than the margin.
 template <bool UP>
-__device__ __forceinline__ HullMask hull_chain(const int64_t* __restrict__ row, HullMask in) {
-    HullMask out{0, 0};
-    int n = 0, xa = 0, xb = 0, xi = -1;
-    int64_t ya = 0, yb = 0, yi = 0;
-    for (;;) {
-        if (xi < 0) {  // the next point
-            if ((in.lo | in.hi) == 0) break;
-            xi = in.next();
-            in.flip(xi);
-            yi = row[xi];
-        }
-        const int64_t l = (ya - yb) * (xi - xa), r = (yi - ya) * (xa - xb);
-        if (n >= 2 && (UP ? l <= r : l >= r)) {  // the last vertex is not outside the chord past it
-            out.flip(xa);
-            --n;
-            xa = xb;
-            ya = yb;
-            if (n >= 2) {
-                HullMask m = out;
-                m.flip(xa);
-                xb = m.top();
-                yb = row[xb];
-            }
-        } else {
-            out.flip(xi);
-            xb = xa;
-            yb = ya;
-            xa = xi;
-            ya = yi;
-            ++n;
-            xi = -1;
-        }
+__device__ __forceinline__ bool surely_inside(double l, double r) {
+    const double margin = (__builtin_fabs(l) + __builtin_fabs(r)) * 0x1p-51;
+    return UP ? l < (r + 0.5) - margin : l > (r - 0.5) + margin;
+}
+
+template <bool UP>
+__device__ __forceinline__ float row16_best(float x) {  // over the 16 lanes of a row
+#define GLC_ROW_STEP(ror)                                                                                  \
+    {                                                                                                      \
+        const float o = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), ror, 0xF, 0xF, true)); \
+        x = UP ? __builtin_fmaxf(x, o) : __builtin_fminf(x, o);                                            \
     }
-    return out;
+    GLC_ROW_STEP(0x128) GLC_ROW_STEP(0x124) GLC_ROW_STEP(0x122) GLC_ROW_STEP(0x121)
+#undef GLC_ROW_STEP
+    return x;
+}
+
+struct Anchor {
+    double x, y;
+};
+constexpr int kAnchors = kHullMaxB / 16 + 2;  // of one hull: a block's ends and one of every 16 indices
+
+// One block's candidates for the upper and lower hull: their indices in order to
+// lu and ld, 64 apart, and their numbers; index i in lane i % 64.  A point above
+// the line through the block's ends can only be a vertex of the upper hull, one
+// below only of the lower, one on it of neither; and none on or inside a chord of
+// two others is.  Chords: between the neighbours, and between anchors, which are
+// the ends and, of every 16 indices, the point furthest outside the line through
+// them (as float: a poor choice keeps more, nothing else).  One test a point, for
+// its side.  Of 128 values with noise 10 to 12 are left for each hull; neighbours
+// at distances 1, 2, 4, ... 32 without anchors left 25 to 35, tested for both.
+// Where the block has a kink, a line through the ends says little (25 to 50
+// left, up to 67): then once more, with the point furthest outside the chord of
+// the first anchors.
+// a: the wave's, [2][kAnchors].
+constexpr int kFewCand = 24;
+__device__ __forceinline__ void hull_filter(const double* __restrict__ row, int len, int lane, Anchor* a, uint8_t* lu,
+                                            uint8_t* ld, uint8_t* nu, uint8_t* nd) {
+    const double y0 = row[0], yl = row[len - 1], dy = yl - y0, n1 = static_cast<double>(len - 1);
+    const int halves = len > 64 ? 2 : 1, last = 1 + (len + 15) / 16;
+    constexpr uint64_t kRow1 = 0x0001000100010001ULL;  // the first lane of each row
+    wave_lds_fence();
+    if (lane < 2) {
+        a[lane * kAnchors] = Anchor{0.0, y0};
+        a[lane * kAnchors + last] = Anchor{n1, yl};
+    }
+    double y[2];
+    float ku[2], kd[2];  // how far outside above (> 0), below (< 0); infinite: no longer asked
+    bool up[2], dn[2];
+    uint64_t mu[2] = {0, 0}, md[2] = {0, 0};
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (half == halves) break;
+        const int i = half * 64 + lane;
+        const bool in = i < len;
+        y[half] = row[i];  // past the block: anything
+        const double l = (y[half] - y0) * n1, r = dy * static_cast<double>(i);
+        up[half] = in & !surely_inside<true>(l, r);
+        dn[half] = in & !surely_inside<false>(l, r);
+        const float key = static_cast<float>(l - r);
+        ku[half] = in ? key : -__builtin_inff();
+        kd[half] = in ? key : __builtin_inff();
+    }
+    for (int pass = 0;; ++pass) {
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (half == halves) break;
+            const double x = static_cast<double>(half * 64 + lane);
+            const float bu = row16_best<true>(ku[half]), bd = row16_best<false>(kd[half]);
+            const uint64_t eu = __ballot((ku[half] > -__builtin_inff()) & (bu == ku[half]));
+            const uint64_t ed = __ballot((kd[half] < __builtin_inff()) & (bd == kd[half]));
+            // the first of each row; a row without any keeps its anchor
+            const uint64_t zu = eu | kRow1 << 15, zd = ed | kRow1 << 15;
+            const uint64_t fu = zu & ~(zu - kRow1) & eu, fd = zd & ~(zd - kRow1) & ed;
+            const int e = 1 + half * 4 + (lane >> 4);
+            if ((fu >> lane) & 1) a[e] = Anchor{x, y[half]};
+            if ((fd >> lane) & 1) a[kAnchors + e] = Anchor{x, y[half]};
+        }
+        wave_lds_fence();
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (half == halves) break;
+            const int i = half * 64 + lane;
+            const double x = static_cast<double>(i);
+            const Anchor* t = a + (up[half] ? 0 : kAnchors) + half * 4 + (lane >> 4);
+            const Anchor c = t[1], b = t[0], d = t[2];
+            const bool before = x <= c.x, after = x >= c.x;
+            const double px = before ? b.x : c.x, py = before ? b.y : c.y;
+            const double qx = after ? d.x : c.x, qy = after ? d.y : c.y;
+            const double l = (y[half] - py) * (qx - px), r = (qy - py) * (x - px);
+            const double l1 = 2.0 * y[half], r1 = row[i - 1] + row[i + 1];
+            const bool iu = surely_inside<true>(l, r) | (l1 <= r1), id = surely_inside<false>(l, r) | (l1 >= r1);
+            // on an uncertain side of the line: in both lists, without a test for the lower
+            const bool end = (i == 0) | (i == len - 1);
+            const bool u = up[half] & (end | !iu), w = dn[half] & (end | up[half] | !id);
+            const float key = static_cast<float>(l - r) * __builtin_amdgcn_rcpf(static_cast<float>(qx - px));
+            ku[half] = u ? key : -__builtin_inff();
+            kd[half] = w ? key : __builtin_inff();
+            mu[half] = __ballot(u | end);
+            md[half] = __ballot(w | end);
+            up[half] = u;
+            dn[half] = w;
+        }
+        const int cu = __popcll(mu[0]) + __popcll(mu[1]), cd = __popcll(md[0]) + __popcll(md[1]);
+        if (pass == 1 || (cu <= kFewCand && cd <= kFewCand)) {
+            if (lane == 0) *nu = static_cast<uint8_t>(cu), *nd = static_cast<uint8_t>(cd);
+            break;
+        }
+        wave_lds_fence();
+    }
+    auto put = [&](const uint64_t (&m)[2], uint8_t* list) {
+        int before = 0;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (half == halves) break;
+            const int k = before + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                                       m[half] >> 32, __builtin_amdgcn_mbcnt_lo(m[half], 0)));
+            if (((m[half] >> lane) & 1) && k < kHullCand) list[k * 64] = static_cast<uint8_t>(half * 64 + lane);
+            before += __popcll(m[half]);
+        }
+    };
+    put(mu, lu);
+    put(md, ld);
+}
+
+// One block's upper (UP) or lower hull among the `left` points whose indices are
+// list[0], list[64], ..., into the front of the same list; returns their number.
+// A vertex is dropped only where it is inside for certain: one kept in vain costs
+// time, never the result.
+// Lanes walk blocks of their own, so every turn is one straight run, the same for
+// a vertex dropped and a point taken (as two branches the compiler nests them, and
+// all lanes wait for the one with the most drops at every point).  The last three
+// vertices a, b, c, the index of the fourth and the next two points i, j stay in
+// registers, and what a turn reads is first used after the next one's test.
+template <bool UP>
+__device__ __forceinline__ int hull_chain(const double* __restrict__ row, int32_t B, int left, uint8_t* list) {
+    auto at = [&](int k) {  // entries past the points hold anything
+        const int x = list[(k < kHullCand ? k : kHullCand - 1) * 64];
+        return x < B ? x : B - 1;
+    };
+    if (left == 0) return 0;
+    int n = 0, k = 2, xa = 0, xb = 0, xc = 0, xd = 0, xi = at(0), xj = at(1), xn = at(2);
+    double ya = 0.0, yb = 0.0, yc = 0.0, yi = row[xi], yj = row[xj], val = yj;
+    bool dropped = false;  // val belongs to c, not to j
+    do {
+        const bool drop = n >= 2 && surely_inside<UP>((ya - yb) * static_cast<double>(xi - xa),
+                                                      (yi - ya) * static_cast<double>(xa - xb));
+        yc = dropped ? val : yc;
+        yj = dropped ? yj : val;
+        list[n * 64] = static_cast<uint8_t>(xi);  // of no account if dropped
+        val = row[drop ? xd : xn];
+        dropped = drop;
+        const double ta = ya, tb = yb;
+        const int za = xa, zb = xb;
+        ya = drop ? yb : yi;
+        xa = drop ? xb : xi;
+        yb = drop ? yc : ta;
+        xb = drop ? xc : za;
+        yc = tb;  // a drop's is on its way
+        xc = drop ? xd : zb;
+        yi = drop ? yi : yj;
+        xi = drop ? xi : xj;
+        xj = drop ? xj : xn;
+        n += drop ? -1 : 1;
+        k += drop ? 0 : 1;
+        left -= drop ? 0 : 1;
+        xd = at(n < 4 ? 0 : n - 4);
+        xn = at(k);
+    } while (left > 0);
+    return n;
 }
 
 __device__ __forceinline__ i128 shfl_up_i128(i128 v, int o) {
@@ -517,14 +668,20 @@ __device__ __forceinline__ i128 shfl_up_i128(i128 v, int o) {
 }
 
 inline __host__ __device__ int hull_stride(int32_t B) { return B | 1; }
-inline size_t hull_lds(int32_t B) { return static_cast<size_t>(64) * hull_stride(B) * 8; }
+// The filter reads up to index 128 and -1 of a row, whatever its length.
+constexpr int kHullPad0 = 2, kHullPad1 = 66;
+inline size_t hull_lds(int32_t B) { return static_cast<size_t>(64 * hull_stride(B) + kHullPad0 + kHullPad1) * 8; }
 
 template <class T>
-__global__ __launch_bounds__(kSmThreads) void k_sm_blocks(const T* __restrict__ v, int64_t n, int32_t B, int64_t JB,
+__global__ __launch_bounds__(kBlkThreads) void k_sm_blocks(const T* __restrict__ v, int64_t n, int32_t B, int64_t JB,
                                                           i128* __restrict__ p1, i128* __restrict__ p2,
                                                           i128* __restrict__ c1, i128* __restrict__ c2, SmHull h) {
-    extern __shared__ int64_t s_v[];  // 64 rows
-    __shared__ HullMask s_mask[2][64];
+    extern __shared__ double s_rows[];  // 64 rows between pads
+    double* s_v = s_rows + kHullPad0;
+    __shared__ uint8_t s_list[2][kHullCand * 64];  // candidate, then vertex k of block b at k * 64 + b
+    __shared__ uint8_t s_n[2][64];
+    __shared__ i128 s_sum[2][64];
+    __shared__ Anchor s_anchor[kBlkThreads / 64][2 * kAnchors];
     __shared__ int32_t s_big[64];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -534,83 +691,80 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_blocks(const T* __restrict__ 
     const int64_t q0 = b0 * B;
     int32_t cnt = 64 * B;  // values of these 64 blocks
     if (q0 + cnt > n) cnt = n > q0 ? static_cast<int32_t>(n - q0) : 0;
-    if (tid < 64) s_big[tid] = 0;
+    if (tid < 64) s_big[tid] = 0, s_n[0][tid] = s_n[1][tid] = 0;
     __syncthreads();
-    for (int32_t i0 = tid; i0 < cnt; i0 += 8 * kSmThreads) {
+    for (int32_t i0 = tid; i0 < cnt; i0 += 8 * kBlkThreads) {
         T y[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {  // eight loads in flight (index clamped)
-            const int32_t i = i0 + k * kSmThreads;
+            const int32_t i = i0 + k * kBlkThreads;
             y[k] = v[q0 + (i < cnt ? i : cnt - 1)];
         }
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
-            const int32_t i = i0 + k * kSmThreads;
+            const int32_t i = i0 + k * kBlkThreads;
             if (i >= cnt) break;
             const int32_t blk = B == 1 ? i : static_cast<int32_t>(__umulhi(static_cast<uint32_t>(i), rcp));
-            s_v[blk * stride + (i - blk * B)] = static_cast<int64_t>(y[k]);
+            s_v[blk * stride + (i - blk * B)] = static_cast<double>(y[k]);
             if (!small_value<T>(y[k])) s_big[blk] = 1;
         }
     }
     __syncthreads();
-    for (int b = w; b < 64; b += kSmThreads / 64) {  // filter: a block per wave
+    for (int b = w; b < 64; b += kBlkThreads / 64) {  // filter: a block per wave
         const int len = cnt - b * B < B ? cnt - b * B : B;
-        const int64_t* row = s_v + b * stride;
-        HullMask up{0, 0}, dn{0, 0};
-        for (int half = 0; half < 2; ++half) {
-            const int i = half * 64 + lane;
-            bool u = i < len, d = u;
-            if (u) {
-                const int64_t y2 = 2 * row[i];
-#pragma unroll
-                for (int o = 1; o <= 32; o *= 2) {
-                    if (i >= o && i + o < len) {
-                        const int64_t s = row[i - o] + row[i + o];
-                        u = u && y2 > s;
-                        d = d && y2 < s;
-                    }
-                }
-            }
-            const uint64_t bu = __ballot(u), bd = __ballot(d);
-            if (half) up.hi = bu, dn.hi = bd;
-            else up.lo = bu, dn.lo = bd;
-            if (len <= 64) break;
-        }
-        if (lane == 0) s_mask[0][b] = up, s_mask[1][b] = dn;
+        if (len > 0)
+            hull_filter(s_v + b * stride, len, lane, s_anchor[w], s_list[0] + b, s_list[1] + b, &s_n[0][b], &s_n[1][b]);
     }
     __syncthreads();
-    const int64_t* row = s_v + lane * stride;
+    const double* row = s_v + lane * stride;
     if (w == 0) {
-        s_mask[0][lane] = hull_chain<true>(row, s_mask[0][lane]);
+        if (s_n[0][lane] <= kHullCand)
+            s_n[0][lane] = static_cast<uint8_t>(hull_chain<true>(row, B, s_n[0][lane], s_list[0] + lane));
     } else if (w == 1) {
-        s_mask[1][lane] = hull_chain<false>(row, s_mask[1][lane]);
-    } else if (w == 2) {
-        const int len = cnt - lane * B < B ? cnt - lane * B : B;
+        if (s_n[1][lane] <= kHullCand)
+            s_n[1][lane] = static_cast<uint8_t>(hull_chain<false>(row, B, s_n[1][lane], s_list[1] + lane));
+    } else if (w < 2 + kSumWaves) {  // 64 / kSumWaves blocks a wave, kSumWaves lanes a block
+        const int blk = (w - 2) * (64 / kSumWaves) + lane / kSumWaves, sub = lane % kSumWaves;
+        const int len = cnt - blk * B < B ? cnt - blk * B : B;
+        const double* r = s_v + blk * stride;
         i128 a1 = 0, a2 = 0;  // sum of y, of i * y
-        if (s_big[lane]) {
-            for (int i = 0; i < len; ++i) {
-                const i128 y = wide<T>(static_cast<T>(row[i]));
+        if (s_big[blk]) {
+            for (int i = sub; i < len; i += kSumWaves) {
+                const i128 y = wide<T>(v[q0 + static_cast<int64_t>(blk) * B + i]);
                 a1 += y;
                 a2 += y * static_cast<i128>(i);
             }
         } else {  // |y| <= 2^52: a block's sum fits 64 bits, eight products too
             int64_t s1 = 0;
-            for (int i = 0; i < len; i += 8) {
-                int64_t s2 = 0;
+            for (int i = sub; i < len; i += 8 * kSumWaves) {
+                int64_t y[8], s2 = 0;
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+                    y[k] = static_cast<int64_t>(r[i + k * kSumWaves < len ? i + k * kSumWaves : i]);
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
-                    const int64_t y = row[i + k < len ? i + k : i];
-                    if (i + k < len) {
-                        s1 += y;
-                        s2 += y * (i + k);
-                    }
+                    if (i + k * kSumWaves >= len) y[k] = 0;
+                    s1 += y[k];
+                    s2 += y[k] * (i + k * kSumWaves);
                 }
                 a2 += s2;
             }
             a1 = s1;
         }
-        a2 += a1 * static_cast<i128>(q0 + static_cast<int64_t>(lane) * B);  // q = first + i
-        i128 s1 = a1, s2 = a2;  // inclusive scan over the 64 blocks
+        for (int o = 1; o < kSumWaves; o <<= 1) {
+            a1 += shfl_xor_i128(a1, o);
+            a2 += shfl_xor_i128(a2, o);
+        }
+        if (sub == 0) {
+            s_sum[0][blk] = a1;
+            s_sum[1][blk] = a2;
+        }
+    }
+    __syncthreads();
+    if (w == kBlkThreads / 64 - 1) {  // scan over the 64 blocks
+        const i128 a1 = s_sum[0][lane];
+        const i128 a2 = s_sum[1][lane] + a1 * static_cast<i128>(q0 + static_cast<int64_t>(lane) * B);  // q = first + i
+        i128 s1 = a1, s2 = a2;  // inclusive
         for (int o = 1; o < 64; o <<= 1) {
             const i128 x1 = shfl_up_i128(s1, o), x2 = shfl_up_i128(s2, o);
             if (lane >= o) {
@@ -627,25 +781,21 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_blocks(const T* __restrict__ 
             c2[blockIdx.x] = s2;
         }
     }
-    __syncthreads();
-    // vertices: lane = block, wave w the mask bits [32 w, 32 w + 32)
+    // vertices: lane = block, the waves take one in turn; the upper hull's, then
+    // the lower one's without the two ends they share
     const int64_t b = b0 + lane;
-    const uint64_t lo = s_mask[0][lane].lo | s_mask[1][lane].lo, hi = s_mask[0][lane].hi | s_mask[1][lane].hi;
-    const int total = __popcll(lo) + __popcll(hi);
     if (b >= JB) return;
-    if (total > h.slots || s_big[lane]) {
+    const int nu = s_n[0][lane], nl = s_n[1][lane];
+    const int total = nu + (nl > 2 ? nl - 2 : 0);
+    if (nu > kHullCand || nl > kHullCand || total > h.slots || s_big[lane]) {
         if (w == 0) h.nv[b] = kHullScan;
         return;
     }
     if (w == 0) h.nv[b] = static_cast<uint8_t>(total);
-    uint32_t bits = static_cast<uint32_t>((w < 2 ? lo : hi) >> ((w & 1) * 32));
-    int k = (w >= 2 ? __popcll(lo) : 0) + ((w & 1) ? __popc(static_cast<uint32_t>(w < 2 ? lo : hi)) : 0);
-    while (bits) {
-        const int i = w * 32 + __builtin_ctz(bits);
-        bits &= bits - 1;
-        h.y[hull_at(h.slots, b, k)] = static_cast<double>(row[i]);
+    for (int k = w; k < total; k += kBlkThreads / 64) {
+        const int i = k < nu ? s_list[0][k * 64 + lane] : s_list[1][(k - nu + 1) * 64 + lane];
+        h.y[hull_at(h.slots, b, k)] = row[i];
         h.x[hull_at(h.slots, b, k)] = static_cast<uint8_t>(i);
-        ++k;
     }
 }
 
@@ -744,9 +894,11 @@ __global__ __launch_bounds__(kChunkScanThreads) void k_sm_chunk_scan(i128* __res
 // The same evaluation from prefix sums and hulls, S consecutive starts per
 // workgroup (m = U * B, S = 8 / U): their candidates lie in a window of
 // (S - 1 + 29) U blocks, whose vertices are staged in LDS.  Each thread takes
-// (start, candidate, block) triples and raises the candidate's D and H; a
-// candidate that the bounds do not settle is read value by value.
+// (start, candidate, block) triples and raises the candidate's D.  A candidate
+// that D does not settle gets its H from a wave, and one that this does not
+// settle is read value by value.
 constexpr int kSplitMaxU = 8;
+constexpr int kCandUnitSum = 162;
 inline __host__ __device__ int split_starts(int U) { return U >= kSplitMaxU ? 1 : 8 / U; }
 inline __host__ __device__ int split_window(int U) { return (split_starts(U) - 1 + 29) * U; }
 inline size_t split_lds(int U, int32_t slots) { return static_cast<size_t>(split_window(U)) * (slots * 9 + 1); }
@@ -759,9 +911,10 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split_hull(const T* __restric
     constexpr int kS = 8, kTasks = kS * kMaxCand;
     extern __shared__ double s_y[];  // [slots][W], then x [slots][W], nv [W]
     __shared__ double s_t[kTasks][2];
-    __shared__ unsigned long long s_D[kTasks], s_H[kTasks];  // bits of non-negative doubles: ordered as integers
+    __shared__ unsigned long long s_D[kTasks];  // bits of non-negative doubles: ordered as integers
     __shared__ int32_t s_bits[kTasks], s_scan[kTasks], s_fast[kTasks];
-    __shared__ int s_list[kTasks], s_cnt;
+    __shared__ int s_list[2][kTasks], s_cnt[2];
+    __shared__ uint16_t s_unit[kCandUnitSum];  // of one start's candidates' units: candidate, unit of it << 4
     __shared__ int64_t s_mx[kSmThreads / 64];
     __shared__ FitLds L;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -776,13 +929,19 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split_hull(const T* __restric
         s_nv[i] = static_cast<uint8_t>(c);
         most = c != kHullScan && c > most ? c : most;
     }
-    if (tid == 0) s_cnt = 0;
+    if (tid < 2) s_cnt[tid] = 0;
+    if (tid < kCandUnitSum) {
+        int k = 0;
+#pragma unroll
+        for (int c = 1; c < kMaxCand; ++c) k += tid >= kCandCum[c];
+        s_unit[tid] = static_cast<uint16_t>(k | (tid - kCandCum[k]) << 4);
+    }
     // task q * 14 + k: candidate k of start j0 + q
     const int tq = tid / kMaxCand, tk = tid % kMaxCand;
     const int64_t cur = (j0 + tq) * m, size = static_cast<int64_t>(kCandUnits[tk]) * m;
     const bool live = tid < S * kMaxCand && cur + size <= n;
     if (tid < kTasks) {
-        s_D[tid] = s_H[tid] = 0;
+        s_D[tid] = 0;
         s_bits[tid] = live ? 0 : -1;
         s_scan[tid] = 0;
         if (live) {
@@ -793,46 +952,60 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split_hull(const T* __restric
         }
     }
     const int rows = __syncthreads_or(most > 16) ? h.slots : h.slots < 16 ? h.slots : 16;
+    const uint32_t rcp_w = 0xFFFFFFFFu / static_cast<uint32_t>(W) + 1u;  // exact for i * W < 2^32
     for (int i = tid; i < rows * W; i += kSmThreads) {
-        const int k = i / W, b = i - k * W;
+        const int k = static_cast<int>(__umulhi(static_cast<uint32_t>(i), rcp_w)), b = i - k * W;
         if (bw + b < pf.JB) {  // slots past a block's vertices hold whatever was there and are not read below
             s_y[i] = h.y[hull_at(h.slots, bw + b, k)];
             s_x[i] = h.x[hull_at(h.slots, bw + b, k)];
         }
     }
     __syncthreads();
-    const int per = kCandCum[kMaxCand] * U;  // blocks of one start's candidates
+    const int per = kCandUnitSum * U;  // blocks of one start's candidates
+    const uint32_t rcp = 0xFFFFFFFFu / static_cast<uint32_t>(per) + 1u;
     for (int t = tid; t < S * per; t += kSmThreads) {
-        const int q = t / per, r = t - q * per;
-        int k = 0;
-#pragma unroll
-        for (int step = 8; step; step >>= 1)
-            if (k + step < kMaxCand && r >= kCandCum[k + step] * U) k += step;
-        const int task = q * kMaxCand + k;
+        const int q = static_cast<int>(__umulhi(static_cast<uint32_t>(t), rcp)), r = t - q * per;
+        const int x = s_unit[U == 1 ? r : r / U];
+        const int u = (x >> 4) * U + (U == 1 ? 0 : r % U), b = q * U + u;
+        const int task = q * kMaxCand + (x & 15);
         if (s_bits[task] < 0 || s_scan[task]) continue;
-        const int u = r - kCandCum[k] * U, b = q * U + u;
         const int nv = s_nv[b];
         if (nv == kHullScan) {
             s_scan[task] = 1;
             continue;
         }
-        double D = 0.0, H = 0.0;
-        hull_err(s_y + b, s_x + b, W, nv, static_cast<int64_t>(u) * pf.B, s_t[task][0], s_t[task][1], D, H);
+        const double D = hull_far(s_y + b, s_x + b, W, nv, u * pf.B, s_t[task][0], s_t[task][1]);
         atomicMax(&s_D[task], static_cast<unsigned long long>(__double_as_longlong(D)));
-        atomicMax(&s_H[task], static_cast<unsigned long long>(__double_as_longlong(H)));
     }
     __syncthreads();
     if (live) {
-        int32_t b = -1;
-        if (!s_scan[tid])
-            b = hull_bits(__longlong_as_double(static_cast<long long>(s_D[tid])),
-                          __longlong_as_double(static_cast<long long>(s_H[tid])), s_t[tid][0], s_t[tid][1], size);
-        if (b < 0) s_list[atomicAdd(&s_cnt, 1)] = tid;
+        const int32_t b = s_scan[tid] ? -1
+                                      : hull_bits(__longlong_as_double(static_cast<long long>(s_D[tid])), 0.0,
+                                                  s_t[tid][0], s_t[tid][1], size);
+        if (b < 0) s_list[s_scan[tid]][atomicAdd(&s_cnt[s_scan[tid]], 1)] = tid;
         else s_bits[tid] = b;
     }
     __syncthreads();
-    for (int i = 0; i < s_cnt; ++i) {  // read by the whole workgroup
-        const int task = s_list[i];
+    const int open = s_cnt[0];
+    for (int i = w; i < open; i += kSmThreads / 64) {  // a wave each: H
+        const int task = s_list[0][i], k = task % kMaxCand, q = task / kMaxCand;
+        const double t0 = s_t[task][0], t1 = s_t[task][1];
+        double H = 0.0;
+        for (int u = lane; u < kCandUnits[k] * U; u += 64) {
+            const int b = q * U + u;
+            H = __builtin_fmax(H, hull_low(s_y + b, s_x + b, W, s_nv[b], u * pf.B, t0, t1));
+        }
+        for (int o = 32; o > 0; o >>= 1) H = __builtin_fmax(H, __shfl_xor(H, o, 64));
+        const int32_t b = hull_bits(__longlong_as_double(static_cast<long long>(s_D[task])), H, t0, t1,
+                                    static_cast<int64_t>(kCandUnits[k]) * m);
+        if (lane == 0) {
+            if (b < 0) s_list[1][atomicAdd(&s_cnt[1], 1)] = task;
+            else s_bits[task] = b;
+        }
+    }
+    __syncthreads();
+    for (int i = 0; i < s_cnt[1]; ++i) {  // read by the whole workgroup
+        const int task = s_list[1][i];
         const int64_t c = (j0 + task / kMaxCand) * m, z = static_cast<int64_t>(kCandUnits[task % kMaxCand]) * m;
         const int64_t mx = wave_max(
             scan_err<T>(v + c, tid, z, kSmThreads, s_t[task][0], s_t[task][1], s_fast[task] != 0));
@@ -845,22 +1018,18 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_split_hull(const T* __restric
         }
         __syncthreads();
     }
+    if (live) {
+        const double c = cost_of(size, s_bits[tid]);
+        s_t[tid][0] = c / static_cast<double>(size);
+        s_t[tid][1] = c;
+    }
+    __syncthreads();
     if (tid < S && j0 + tid < J && s_bits[tid * kMaxCand] >= 0) {  // smallest cost per value, the first on ties
-        const int64_t c0 = (j0 + tid) * m;
-        double best = DBL_MAX, bc = 0.0;
-        int64_t be = (c0 + m < n) ? c0 + m : n;
-        for (int k = 0; k < kMaxCand && s_bits[tid * kMaxCand + k] >= 0; ++k) {
-            const int64_t z = static_cast<int64_t>(kCandUnits[k]) * m;
-            const double c = cost_of(z, s_bits[tid * kMaxCand + k]);
-            const double cpe = c / static_cast<double>(z);
-            if (cpe < best) {
-                best = cpe;
-                be = c0 + z;
-                bc = c;
-            }
-        }
-        best_end[j0 + tid] = static_cast<int32_t>(be);
-        best_cost[j0 + tid] = bc;
+        int at = 0;
+        for (int k = 1; k < kMaxCand && s_bits[tid * kMaxCand + k] >= 0; ++k)
+            if (s_t[tid * kMaxCand + k][0] < s_t[tid * kMaxCand + at][0]) at = k;
+        best_end[j0 + tid] = static_cast<int32_t>((j0 + tid) * m + static_cast<int64_t>(kCandUnits[at]) * m);
+        best_cost[j0 + tid] = s_t[tid * kMaxCand + at][1];
     }
     // the column's last start may have fewer than m values: one partition [cur, n)
     const int64_t last = (J - 1) * m;
@@ -1150,10 +1319,10 @@ __device__ __forceinline__ int32_t range_bits(const T* __restrict__ v, int64_t g
     const int64_t len = ge - gs;
     int32_t bits = -1;
     if (fast && h.slots > 0) {
-        const int64_t ib = gs / pf.B, ie = (ge == pf.n) ? pf.JB : ge / pf.B;
-        double D = 0.0, H = 0.0;
+        const int64_t ib = block_of(pf, gs), ie = (ge == pf.n) ? pf.JB : block_of(pf, ge);
+        double D = 0.0;
         int64_t mx = 0;  // of blocks read value by value
-        bool settled = true;
+        bool settled = true, read = false;
         for (int64_t b0 = ib; b0 < ie; b0 += 64) {
             const int64_t b = b0 + lane;
             int nv = b < ie ? h.nv[b] : 0;
@@ -1164,8 +1333,9 @@ __device__ __forceinline__ int32_t range_bits(const T* __restrict__ v, int64_t g
             }
             if (nv == kHullScan) nv = 0;
             const int64_t at = hull_at(h.slots, b < ie ? b : ib, 0);
-            hull_err(h.y + at, h.x + at, 64, nv, (b - ib) * pf.B, t0, t1, D, H);
+            D = __builtin_fmax(D, hull_far(h.y + at, h.x + at, 64, nv, static_cast<int32_t>(b - ib) * pf.B, t0, t1));
             while (odd) {  // wave-uniform
+                read = true;
                 const int64_t q = (b0 + __builtin_ctzll(odd)) * pf.B;
                 odd &= odd - 1;
                 const int64_t hi = q + pf.B < ge ? q + pf.B : ge;
@@ -1173,13 +1343,23 @@ __device__ __forceinline__ int32_t range_bits(const T* __restrict__ v, int64_t g
                 mx = a > mx ? a : mx;
             }
         }
-        for (int o = 32; o > 0; o >>= 1) {
-            D = __builtin_fmax(D, __shfl_xor(D, o, 64));
-            H = __builtin_fmax(H, __shfl_xor(H, o, 64));
+        for (int o = 32; o > 0; o >>= 1) D = __builtin_fmax(D, __shfl_xor(D, o, 64));
+        bits = settled ? hull_bits(D, 0.0, t0, t1, len) : -1;
+        if (settled && bits < 0) {
+            double H = 0.0;
+            for (int64_t b = ib + lane; b < ie; b += 64) {
+                const int64_t at = hull_at(h.slots, b, 0);
+                const int nv = h.nv[b];
+                H = __builtin_fmax(H, hull_low(h.y + at, h.x + at, 64, nv == kHullScan ? 0 : nv,
+                                               static_cast<int32_t>(b - ib) * pf.B, t0, t1));
+            }
+            for (int o = 32; o > 0; o >>= 1) H = __builtin_fmax(H, __shfl_xor(H, o, 64));
+            bits = hull_bits(D, H, t0, t1, len);
         }
-        mx = wave_max(mx);
-        bits = settled ? hull_bits(D, H, t0, t1, len) : -1;
-        if (bits >= 0) bits = bits_of(mx) > bits ? bits_of(mx) : bits;
+        if (bits >= 0 && read) {
+            mx = wave_max(mx);
+            bits = bits_of(mx) > bits ? bits_of(mx) : bits;
+        }
     }
     return bits >= 0 ? bits : bits_of(wave_max(scan_err<T>(v + gs, lane, len, 64, t0, t1, fast)));
 }
@@ -1358,7 +1538,7 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, Split
         using T = decltype(t);
         const T* v = static_cast<const T*>(d_values);
         if (hulls) {
-            hipLaunchKernelGGL(k_sm_blocks<T>, dim3(static_cast<unsigned>(C)), dim3(kSmThreads), hull_lds(B), s, v, n,
+            hipLaunchKernelGGL(k_sm_blocks<T>, dim3(static_cast<unsigned>(C)), dim3(kBlkThreads), hull_lds(B), s, v, n,
                                B, JB, pf1, pf2, cf1, cf2, h);
         } else {
             hipLaunchKernelGGL(k_sm_sums<T>, dim3(static_cast<unsigned>(JB)), dim3(kSmThreads), 0, s, v, n, B, pf1,
