@@ -301,14 +301,18 @@ __device__ __forceinline__ void wave_narrow_v(const DecArgs& a, const TileInfo& 
 
 // Wide fast path: one partition, 33..64-bit fields or DIRECT_COPY; two row
 // registers per row (words l and 64 + l) and three bpermute pairs per element.
-template <class T, int OP>
-__device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane) {
+// NP, h: part h of NP of the tile's rows.
+template <class T, int OP, int NP = 1>
+__device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane,
+                                          int h = 0) {
+    constexpr int kRows = kWaveRows / NP;
+    static_assert(kRows % 4 == 0, "whole groups of rows");
     const int b = tile_bits(x.info);
     const uint32_t* __restrict__ w = a.words;
     const int32_t type = tile_type(x.info);
     const int32_t lbase = x.lbase;
     const uint32_t rel_lane = static_cast<uint32_t>(lane) * static_cast<uint32_t>(b);
-    for (int r0 = 0; r0 < kWaveRows; r0 += 4) {
+    for (int r0 = h * kRows; r0 < (h + 1) * kRows; r0 += 4) {
         uint32_t x0[4], x1[4], xs[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {  // branch-free, clamped as in wave_narrow
@@ -838,12 +842,17 @@ __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
     const int h = static_cast<int>(blockIdx.x & 1);
     if (t >= ntiles) return;
     const TileInfo x = a.tinfo[t];
-    if (tile_path(x.info) != TILE_NARROW || !VEC) {
-        if (h == 0) wave_tile<T, OP_PACKED, VEC>(a, t, lane);
-        return;
-    }
+    const int path = tile_path(x.info);
     const int64_t e0 = t * kWaveTile;
     const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
+    if (path == TILE_WIDE) {
+        wave_wide<T, OP_PACKED, 2>(a, x, e0, e1, lane, h);
+        return;
+    }
+    if (path != TILE_NARROW || !VEC) {  // whole, on every XCD (workgroup g runs on XCD g % 8)
+        if (h == static_cast<int>(t >> 2 & 1)) wave_tile<T, OP_PACKED, VEC>(a, t, lane);
+        return;
+    }
     if constexpr (sizeof(T) == 8) wave_narrow_v<T, OP_PACKED, 2, 2>(a, x, e0, e1, lane, h);
     else if (tile_bits(x.info) <= 16) wave_narrow_v<T, OP_PACKED, 4, 2>(a, x, e0, e1, lane, h);
     else wave_narrow_v<T, OP_PACKED, 2, 2>(a, x, e0, e1, lane, h);
