@@ -522,20 +522,28 @@ __device__ __forceinline__ void put_values(O* p, const O (&v)[V], int32_t lo, in
 // time, so that the model and the bit width are wave-uniform and neighbouring
 // lanes read neighbouring words.  Lanes take V adjacent values aligned to V in
 // the tile (one 16-byte store where all of them are the partition's), V fields
-// of V * bits <= 64 from three words loaded together.  The next partition's
-// descriptor is loaded before the current one is decoded.  5e7 uint32 values in
-// partitions of 1000: 67 us, where a search per value (wave_slow) took 225 us and
-// wave_many takes 90; from about 300 values a partition down wave_many is the
-// faster one (300: 81 against 134 us).
+// of V * bits <= 64 from three words loaded together, or two wider ones from five.
+// The next partition's descriptor is loaded before the current one is decoded.
+// 5e7 uint32 values in partitions of 1000: 57 us, where a search per value
+// (wave_slow) took 225 us and wave_many takes 90; from about 300 values a partition
+// down wave_many is the faster one (300: 81 against 134 us).  Bound by the work per
+// row: rows past the partition are left out (64 us with them), and one of two
+// wide fields a lane costs 4/5 of two rows of one (7e7 uint64, 36 bits, S = 1000:
+// 208 -> 160 us).
 constexpr int kSegParts = 3;
 
 // Values [s, t) of partition p (descriptor d; s, t in elements) of the tile at
-// e0.  FAST as in narrow_v_rows; 0 also takes DIRECT_COPY and POLY2.
-template <class T, int OP, int V, int FAST>
+// e0.  FAST as in narrow_v_rows; 0 also takes DIRECT_COPY and POLY2.  WIDE: two
+// fields of up to 64 bits from five words.
+template <class T, int OP, int V, int FAST, bool WIDE = false>
 __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t s, int64_t t,
                                          int lane) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
-    constexpr int kSegRows = V == 4 ? 2 : 4;  // in flight; more only cost registers (V = 1: 128 against 117 us)
+    // in flight; more only cost registers (V = 1 with 8: 128 against 117 us; V = 2
+    // and 4 with as many as a tile has: 2 to 60 % slower)
+    constexpr int kSegRows = V == 4 ? 2 : 4;
+    constexpr int kWords = WIDE ? 5 : 3;
+    static_assert(!WIDE || V == 2, "two wide fields");
     O* __restrict__ out = static_cast<O*>(a.out);
     const int b = desc_bits(d.packed);
     const int32_t type = desc_type(d.packed);
@@ -543,26 +551,29 @@ __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_
     const double t2 = (FAST == 0 && OP != OP_UNPACK && type == MODEL_POLY2) ? a.params[4 * p + 2] : 0.0;
     const int32_t lo = static_cast<int32_t>(s - e0), hi = static_cast<int32_t>(t - e0);  // in the tile
     const int32_t kb = static_cast<int32_t>(e0 - d.start);  // tile position x is value kb + x of the partition
-    for (int32_t x0 = lo / V * V + lane * V; x0 - lane * V < hi; x0 += kSegRows * 64 * V) {
-        uint32_t w[kSegRows][3];
+    constexpr int32_t kLine = 128 / sizeof(O);  // rows on whole lines (partitions of 1000: 1-4 %)
+    for (int32_t row = lo / kLine * kLine; row < hi; row += kSegRows * 64 * V) {
+        const int32_t x0 = row + lane * V;
+        uint32_t w[kSegRows][kWords];
         int64_t pl[kSegRows][V];
 #pragma unroll
         for (int r = 0; r < kSegRows; ++r) {
             const int32_t x = x0 + r * 64 * V;
+            if (r > 0 && row + r * 64 * V >= hi) continue;
             if constexpr (OP == OP_PLAIN) {
 #pragma unroll
                 for (int j = 0; j < V; ++j) pl[r][j] = a.plain[e0 + (x + j < lo ? lo : x + j < hi ? x + j : hi - 1)];
-            } else {  // the three words from the lane's first field of the partition on
+            } else {  // the words from the lane's first field of the partition on
                 const int32_t xf = x < lo ? lo : x < hi ? x : hi - 1;
                 const int64_t wi = (off + static_cast<int64_t>(kb + xf) * b) >> 5;
-                w[r][0] = a.words[wi];
-                w[r][1] = a.words[wi + 1];
-                w[r][2] = a.words[wi + 2];
+#pragma unroll
+                for (int q = 0; q < kWords; ++q) w[r][q] = a.words[wi + q];
             }
         }
 #pragma unroll
         for (int r = 0; r < kSegRows; ++r) {
             const int32_t x = x0 + r * 64 * V;
+            if (r > 0 && row + r * 64 * V >= hi) continue;
             const int32_t xf = x < lo ? lo : x < hi ? x : hi - 1;
             const uint32_t sh = static_cast<uint32_t>(off + static_cast<int64_t>(kb + xf) * b) & 31;
             O v[V];
@@ -576,6 +587,16 @@ __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_
                 } else if constexpr (V == 1) {
                     raw = static_cast<uint64_t>(__builtin_amdgcn_alignbit(w[r][2], w[r][1], sh)) << 32 |
                           __builtin_amdgcn_alignbit(w[r][1], w[r][0], sh);
+                    delta = sign_extend(raw, b);
+                    raw = b >= 64 ? raw : raw & ((1ULL << b) - 1ULL);
+                } else if constexpr (WIDE) {
+                    const uint32_t sk = sh + (x + j > xf ? static_cast<uint32_t>(b) : 0u);  // second field: 33 .. 95
+                    const uint32_t idx = sk >> 5;
+                    const uint32_t l = idx == 0 ? w[r][0] : idx == 1 ? w[r][1] : w[r][2];
+                    const uint32_t m = idx == 0 ? w[r][1] : idx == 1 ? w[r][2] : w[r][3];
+                    const uint32_t h = idx == 0 ? w[r][2] : idx == 1 ? w[r][3] : w[r][4];
+                    raw = static_cast<uint64_t>(__builtin_amdgcn_alignbit(h, m, sk & 31)) << 32 |
+                          __builtin_amdgcn_alignbit(m, l, sk & 31);
                     delta = sign_extend(raw, b);
                     raw = b >= 64 ? raw : raw & ((1ULL << b) - 1ULL);
                 } else {
@@ -624,12 +645,16 @@ __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int6
             else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
         } else if (sizeof(T) == 4 && b <= 32 && u == 1) {
             seg_rows<T, OP, 2, 1>(a, d, p, e0, s, t, lane);
+        } else if constexpr (sizeof(T) == 8) {
+            if (u == 1) seg_rows<T, OP, 2, 1, true>(a, d, p, e0, s, t, lane);
+            else if (u == 2) seg_rows<T, OP, 2, 2, true>(a, d, p, e0, s, t, lane);
+            else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
         } else {
             seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
         }
     } else if constexpr (OP == OP_UNPACK) {
         if (b <= 32) seg_rows<T, OP, 2, 0>(a, d, p, e0, s, t, lane);
-        else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+        else seg_rows<T, OP, 2, 0, true>(a, d, p, e0, s, t, lane);
     } else {
         seg_rows<T, OP, 2, 0>(a, d, p, e0, s, t, lane);
     }
@@ -750,10 +775,9 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
 
 // A tile of the partition-spanning path.  out must be 16-byte aligned (VEC).
 template <class T, int OP>
-__device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int lane,
-                                          ManyLds* L) {
+__device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int64_t phi,
+                                          int lane, ManyLds* L) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
-    const int64_t phi = a.tile_part[(e1 + kIndexTile - 1) >> kIndexShift];
     if (phi - plo >= kSegParts) {
         const int64_t np = phi - plo + 1;
         if (np > kManyParts || !wave_many<T, OP>(a, e0, e1, plo, static_cast<int>(np), lane, *L))
@@ -789,13 +813,19 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
     const int64_t e0 = t * kWaveTile;
     const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
     const TileInfo x = a.tinfo[t];
+    // loaded with the tile's line: spanning tiles need both before anything else
+    int64_t plo = 0, phi = 0;
+    if constexpr (VEC && SEGS) {
+        plo = a.tile_part[t];
+        phi = a.tile_part[(e1 + kIndexTile - 1) >> kIndexShift];
+    }
     const int path = tile_path(x.info);
     if constexpr (OP == OP_PLAIN) {
         if (path != TILE_SLOW) {
             if constexpr (VEC) wave_plain_v<T>(a, x, e0, e1, lane);
             else wave_plain<T>(a, x, e0, e1, lane);
         }
-        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, a.tile_part[t], lane, L);
+        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, plo, phi, lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     } else {
         if (path == TILE_NARROW) {
@@ -805,7 +835,7 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
             else wave_narrow_v<T, OP, 2>(a, x, e0, e1, lane);
         }
         else if (path == TILE_WIDE) wave_wide<T, OP>(a, x, e0, e1, lane);
-        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, a.tile_part[t], lane, L);
+        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, plo, phi, lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     }
 }
@@ -831,10 +861,12 @@ __global__ __launch_bounds__(64 * WPG) void k_decode_wave(DecArgs a) {
     }
 }
 
-// Half tiles (packed decode): one-wave workgroup g decodes half g & 1 of
-// narrow tile g >> 1; a tile of any other path is decoded whole by its
-// first half's wave.  (Quarter tiles, one wave per two 128-value rows, ran
-// 20-55 % slower on every column measured.)
+// Half tiles (packed decode): one-wave workgroup g decodes half g & 1 of narrow
+// or wide tile g >> 1; a tile of any other path is decoded whole by one half's
+// wave, the first's and the second's in turn so that every XCD has such waves
+// (all on the first's: 264 instead of 166 us, 7e7 uint64 of 36 bits).  (Quarter
+// tiles, one wave per two 128-value rows, ran 20-55 % slower on every column
+// measured.)
 template <class T, bool VEC>
 __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
     const int lane = threadIdx.x & 63;
@@ -849,7 +881,7 @@ __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
         wave_wide<T, OP_PACKED, 2>(a, x, e0, e1, lane, h);
         return;
     }
-    if (path != TILE_NARROW || !VEC) {  // whole, on every XCD (workgroup g runs on XCD g % 8)
+    if (path != TILE_NARROW || !VEC) {  // whole (workgroup g runs on XCD g % 8)
         if (h == static_cast<int>(t >> 2 & 1)) wave_tile<T, OP_PACKED, VEC>(a, t, lane);
         return;
     }
@@ -962,20 +994,24 @@ __global__ __launch_bounds__(64 * WPG) void k_batch_decode(const BatchCol* __res
 }
 
 // Batched half tiles: one-wave workgroup g decodes half g & 1 of global tile
-// g >> 1 (tiles of any path but narrow with an aligned output are decoded
-// whole by the first half's wave).
+// g >> 1, the other paths as in k_decode_half.
 template <class T>
 __device__ __forceinline__ void batch_half(const DecArgs& a, int64_t t, int h, int lane) {
     const TileInfo x = a.tinfo[t];
-    if (tile_path(x.info) != TILE_NARROW || !a.vec16) {
-        if (h == 0) {
+    const int path = tile_path(x.info);
+    const int64_t e0 = t * kWaveTile;
+    const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
+    if (path == TILE_WIDE) {
+        wave_wide<T, OP_PACKED, 2>(a, x, e0, e1, lane, h);
+        return;
+    }
+    if (path != TILE_NARROW || !a.vec16) {
+        if (h == static_cast<int>(t >> 2 & 1)) {
             if (a.vec16) wave_tile<T, OP_PACKED, true>(a, t, lane);
             else batch_tile_unaligned<T>(a, t, lane);
         }
         return;
     }
-    const int64_t e0 = t * kWaveTile;
-    const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
     if constexpr (sizeof(T) == 8) wave_narrow_v<T, OP_PACKED, 2, 2>(a, x, e0, e1, lane, h);
     else if (tile_bits(x.info) <= 16) wave_narrow_v<T, OP_PACKED, 4, 2>(a, x, e0, e1, lane, h);
     else wave_narrow_v<T, OP_PACKED, 2, 2>(a, x, e0, e1, lane, h);
@@ -1114,8 +1150,8 @@ int launch_decode_full(const glc_column* c, void* d_out, int mode, hipStream_t s
     if (c->P == 0) return fail(GLC_ERR_STATE, "column has values but no partitions");
     DecArgs a = make_args(c, d_out);
     // No schedule set: 64-bit columns of whole-tile partitions take half tiles
-    // (2^28 values 399-514 us against 431-535 with four tiles a workgroup, by width;
-    // equal below 2^27, never slower).  32-bit ones are faster in whole tiles (2^28
+    // (2^28 values 399-560 us against 431-631 with four tiles a workgroup, by width;
+    // within 3 % below 2^27).  32-bit ones are faster in whole tiles (2^28
     // 239-278 against 254-291), and the half-tile kernel has no fast path for
     // partition-spanning tiles.
     const int dsched = (c->dec_auto && c->elem_size == 8 && !c->spans) ? GLC_DECODE_HALF_TILE_W1 : c->dec_sched;
