@@ -187,7 +187,7 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
 
     std::vector<BatchCol> cols(num_columns);
     std::vector<int32_t> part_col, tile_col;
-    int64_t Ptot = 0, Ttot = 0, meta = 0, words = 0;
+    int64_t Ptot = 0, Ttot = 0, Pmax = 0, Tmax = 0, meta = 0, words = 0;
     std::vector<glc::ArenaLayout> lay(num_columns);
     b->meta_off.resize(num_columns);
     b->words_off.resize(num_columns);
@@ -222,6 +222,8 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
         part_col.insert(part_col.end(), static_cast<size_t>(P), i);
         tile_col.insert(tile_col.end(), static_cast<size_t>(T), i);
         Ptot += P;
+        Pmax = std::max(Pmax, P);
+        Tmax = std::max(Tmax, T);
         Ttot += T;
     }
     b->meta_bytes = meta;
@@ -277,6 +279,8 @@ int glc_batch_create(int num_columns, const int32_t* dtypes, const void* const* 
     p.part_col = reinterpret_cast<const int32_t*>(tb + o_pc);
     p.tile_col = reinterpret_cast<const int32_t*>(tb + o_tc);
     p.Ptot = Ptot;
+    p.Pmax = Pmax;
+    p.Tmax = Tmax;
     p.Ttot = Ttot;
     p.C = num_columns;
     p.S = partition_size;

@@ -135,6 +135,8 @@ struct BatchPlan {
     void* const* outs;        // per-column decompress destinations
     int64_t Ptot;
     int64_t Ttot;
+    int64_t Pmax;             // partitions and tiles of the largest column
+    int64_t Tmax;
     int32_t C;
     int32_t S;
 };
