@@ -15,6 +15,8 @@
 // Positions outside [0, N) or in a gap decode to 0 (RandomAccessKernels.cuh:100-103).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "glc_device.hpp"
 #include "glc_internal.hpp"
 
@@ -111,19 +113,19 @@ __device__ __forceinline__ T ra_lookup(const Desc* __restrict__ desc, const int3
 // tiles of the partition-spanning path take ra_lookup.
 constexpr int kRaBatch = 4;
 
-// Fixed-size partitions: the partition's 32-byte Desc by division, then its
-// payload words (or pre-unpacked delta), four lookups in flight per thread.
-// Elements outside [0, N) return 0; POLY2 partitions (decode-only blobs) go
-// through ra_lookup.
-template <class T, bool PLAIN>
-__device__ __forceinline__ void fixed_batch(const RaArgs& a, int64_t j0, const int64_t (&e)[kRaBatch]) {
+// The elements' partitions known (part(k), asked for elements inside [0, N)):
+// their 32-byte Descs, then the payload words (or pre-unpacked deltas), four
+// lookups in flight per thread.  Elements outside [0, N) and in gaps return 0;
+// POLY2 partitions (decode-only blobs) go through ra_lookup.
+template <class T, bool PLAIN, class F>
+__device__ __forceinline__ void part_batch(const RaArgs& a, int64_t j0, const int64_t (&e)[kRaBatch], F&& part) {
     T* __restrict__ out = static_cast<T*>(a.out);
     bool in[kRaBatch];
     Desc d[kRaBatch];
 #pragma unroll
     for (int k = 0; k < kRaBatch; ++k) {
-        in[k] = e[k] >= 0 && e[k] < a.n;  // n < 2^31: 32-bit division
-        const int64_t p = in[k] ? static_cast<int64_t>(static_cast<uint32_t>(e[k]) / static_cast<uint32_t>(a.fixed)) : 0;
+        in[k] = e[k] >= 0 && e[k] < a.n;
+        const int64_t p = in[k] ? part(k) : 0;
         d[k] = a.desc[p];
     }
     uint32_t w0[kRaBatch], w1[kRaBatch], w2[kRaBatch];
@@ -173,6 +175,77 @@ __device__ __forceinline__ void fixed_batch(const RaArgs& a, int64_t j0, const i
     }
 }
 
+// Fixed-size partitions: p = pos / S (FixedPartitionKernels.cuh:76-77).
+template <class T, bool PLAIN>
+__device__ __forceinline__ void fixed_batch(const RaArgs& a, int64_t j0, const int64_t (&e)[kRaBatch]) {
+    part_batch<T, PLAIN>(a, j0, e, [&](int k) {  // n < 2^31: 32-bit division
+        return static_cast<int64_t>(static_cast<uint32_t>(e[k]) / static_cast<uint32_t>(a.fixed));
+    });
+}
+
+// Partitions by the tile's first and last one and a search between them, the
+// four lookups' steps in flight together.
+template <class T, bool PLAIN>
+__device__ __forceinline__ void search_batch(const RaArgs& a, int64_t j0, const int64_t (&e)[kRaBatch]) {
+    int32_t lo[kRaBatch], hi[kRaBatch];
+#pragma unroll
+    for (int k = 0; k < kRaBatch; ++k) {
+        const bool in = e[k] >= 0 && e[k] < a.n;
+        const int64_t t = in ? e[k] >> kIndexShift : 0;
+        lo[k] = a.tile_part[t];
+        hi[k] = in ? a.tile_part[t + 1] : lo[k];
+    }
+    for (;;) {
+        int32_t m[kRaBatch], st[kRaBatch];
+        bool more = false;
+#pragma unroll
+        for (int k = 0; k < kRaBatch; ++k) more |= lo[k] < hi[k];
+        if (!more) break;
+#pragma unroll
+        for (int k = 0; k < kRaBatch; ++k) {  // a settled lookup reads its own partition again
+            m[k] = static_cast<int32_t>((static_cast<int64_t>(lo[k]) + hi[k] + 1) >> 1);
+            st[k] = a.desc[m[k]].start;
+        }
+#pragma unroll
+        for (int k = 0; k < kRaBatch; ++k) {
+            if (lo[k] >= hi[k]) continue;
+            if (st[k] <= e[k]) lo[k] = m[k];
+            else hi[k] = m[k] - 1;
+        }
+    }
+    part_batch<T, PLAIN>(a, j0, e, [&](int k) { return static_cast<int64_t>(lo[k]); });
+}
+
+template <bool POS64>
+__device__ __forceinline__ int64_t ra_pos(const RaArgs& a, int64_t j) {
+    if (j >= a.q) return -1;
+    return POS64 ? static_cast<const int64_t*>(a.pos)[j] : static_cast<int64_t>(static_cast<const int32_t*>(a.pos)[j]);
+}
+
+// A kernel of its own: as a branch of k_random_access the search cost that one a
+// wave per SIMD (61 -> 70 and 78 -> 83 VGPRs).
+template <class T, bool POS64, bool PLAIN>
+__global__ __launch_bounds__(kThreads) void k_random_search(RaArgs a) {
+    const int64_t per_block = static_cast<int64_t>(kThreads) * kRaBatch;
+    const int64_t step = static_cast<int64_t>(gridDim.x) * per_block;
+    for (int64_t j0 = static_cast<int64_t>(blockIdx.x) * per_block + threadIdx.x; j0 < a.q; j0 += step) {
+        int64_t e[kRaBatch];
+#pragma unroll
+        for (int k = 0; k < kRaBatch; ++k) e[k] = ra_pos<POS64>(a, j0 + k * kThreads);
+        if (a.n <= 0 || (!PLAIN && a.words == nullptr)) {  // as in k_random_access
+#pragma unroll
+            for (int k = 0; k < kRaBatch; ++k) {
+                const int64_t j = j0 + k * kThreads;
+                if (j < a.q)
+                    static_cast<T*>(a.out)[j] = ra_lookup<T, PLAIN>(a.desc, a.tile_part, a.tinfo, a.words, a.plain,
+                                                                    a.params, a.n, 0, e[k]);
+            }
+            continue;
+        }
+        search_batch<T, PLAIN>(a, j0, e);
+    }
+}
+
 template <class T, bool POS64, bool PLAIN>
 __global__ __launch_bounds__(kThreads) void k_random_access(RaArgs a) {
     T* __restrict__ out = static_cast<T*>(a.out);
@@ -182,10 +255,7 @@ __global__ __launch_bounds__(kThreads) void k_random_access(RaArgs a) {
         int64_t e[kRaBatch];
 #pragma unroll
         for (int k = 0; k < kRaBatch; ++k) {
-            const int64_t j = j0 + k * kThreads;
-            e[k] = (j < a.q) ? (POS64 ? static_cast<const int64_t*>(a.pos)[j]
-                                      : static_cast<int64_t>(static_cast<const int32_t*>(a.pos)[j]))
-                             : -1;
+            e[k] = ra_pos<POS64>(a, j0 + k * kThreads);
         }
         // empty columns and a released payload (all widths 0): one at a
         // time through ra_lookup
@@ -390,11 +460,28 @@ int launch_random_access(const glc_column* c, const void* d_pos, int pos64, int6
     // fewer record bytes at S = 4096: int64 2^29, 2^24 lookups 0.597 ->
     // 0.493 ms).
     a.fixed = fixed_size > 0 ? fixed_size : c->fixed_size;
+    // Tiles of several partitions have no record to read.  Columns with such
+    // tiles search the partition, four lookups at once, from tile_part and Desc
+    // alone (2^23 lookups, 2^27 int64 in partitions of 1000: 355 us one at a time, 278
+    // searched; 2^25, split/merge: 225 -> 189).  Pre-unpacked lookups in large columns
+    // of long partitions, few of whose tiles hold two, are bound by the deltas' lines
+    // and keep the records (2^26 uint64, 17000 a partition: 219 against 226 us; 2^20: 109
+    // against 81).
+    const bool search = a.fixed == 0 && c->spans &&
+                        !(plain && c->n >= (int64_t(1) << 24) && c->n / std::max<int64_t>(c->P, 1) >= 8192);
     if (c->P == 0) a.n = 0;  // every query decodes to 0
     return dispatch_dtype(c->dtype, [&](auto t) {
         using T = decltype(t);
         const dim3 g(ra_grid(q, kRaBatch));
-        if (pos64) {
+        if (search) {
+            if (pos64) {
+                if (plain) hipLaunchKernelGGL((k_random_search<T, true, true>), g, dim3(kThreads), 0, s, a);
+                else hipLaunchKernelGGL((k_random_search<T, true, false>), g, dim3(kThreads), 0, s, a);
+            } else {
+                if (plain) hipLaunchKernelGGL((k_random_search<T, false, true>), g, dim3(kThreads), 0, s, a);
+                else hipLaunchKernelGGL((k_random_search<T, false, false>), g, dim3(kThreads), 0, s, a);
+            }
+        } else if (pos64) {
             if (plain) hipLaunchKernelGGL((k_random_access<T, true, true>), g, dim3(kThreads), 0, s, a);
             else hipLaunchKernelGGL((k_random_access<T, true, false>), g, dim3(kThreads), 0, s, a);
         } else {
