@@ -703,8 +703,9 @@ __device__ __forceinline__ void fit_wave_long(const T* __restrict__ x, int32_t n
 
 // Batched fit, a wave per partition, every element type in one launch (the
 // type comes from the column).  NMAX: the longest partition of the batch, 1024
-// (64 VGPRs instead of 126, twice the waves), 2048, or 0 for longer ones, which
-// take two reads in the wave.
+// (92 VGPRs instead of 124, five waves a SIMD; held to seven waves it spills 84
+// bytes: 1000 columns, 2^26 values 100 against 91 us), 2048, or 0 for longer ones,
+// which take two reads in the wave.
 template <class T, int NMAX>
 __device__ __forceinline__ void fit_batch_one(const BatchCol& c, int64_t p, int32_t s0, int32_t n, int lane,
                                               double* s_t) {
@@ -717,7 +718,7 @@ __device__ __forceinline__ void fit_batch_one(const BatchCol& c, int64_t p, int3
 }
 
 template <int NMAX>
-__global__ __launch_bounds__(64 * kFitWaves, NMAX == 1024 ? 7 : 4) void k_fit_wave_batch(
+__global__ __launch_bounds__(64 * kFitWaves, NMAX == 1024 ? 5 : 4) void k_fit_wave_batch(
     const BatchCol* __restrict__ cols, const int32_t* __restrict__ part_col, int64_t Ptot, int32_t S) {
     __shared__ double s_t[kFitWaves][kFitAnyMax];
     const int lane = threadIdx.x & 63;
