@@ -582,8 +582,13 @@ __global__ __launch_bounds__(256) void k_fit_block(const T* __restrict__ v, cons
 // partition.  chunk: 16 for long lists (2^28 uint64 V6, 122880 partitions: chunks of
 // 4 / 16 / 64 took 492 / 484 / 497 us), down to 1 where workgroups would be too few
 // (3500 partitions of 20000 values, split/merge 2^26: 618 -> 186 us).
-template <class T, int FORM>
-__global__ __launch_bounds__(256, 4) void k_fit_chunk(const T* __restrict__ v, const int32_t* __restrict__ st,
+// MINW: waves a SIMD.  With four the 64-bit forms are short of 2 to 10 registers
+// and spill, which the forms that hold 32 values a lane pay for most (2^28 uint64
+// V6 base 2048: 413 us with four, 389 with three; 2^27 int64 base 4096: 234, 214);
+// short partitions and ones of many passes want the fourth wave (2^27 uint64 base
+// 512: 355, 365; split/merge 2^26: 186, 193).
+template <class T, int FORM, int MINW>
+__global__ __launch_bounds__(256, MINW) void k_fit_chunk(const T* __restrict__ v, const int32_t* __restrict__ st,
                                                    const int32_t* __restrict__ en, FitOut o, int64_t P, int chunk) {
     __shared__ FitLds L;
     const int lane = threadIdx.x & 63;
@@ -1925,8 +1930,12 @@ int launch_fit_t(const void* d_values, glc_column* c, int32_t bs, int32_t fixed_
         // about 8192 workgroups, a chunk of 16 at most (k_fit_chunk's note)
         const int64_t per = (c->P + 8191) / 8192;
         const int chunk = static_cast<int>(per < 1 ? 1 : per > 16 ? 16 : per);
-        hipLaunchKernelGGL((k_fit_chunk<T, FORM>), dim3(static_cast<unsigned>((c->P + chunk - 1) / chunk)), dim3(256), 0,
-                           s, v, c->d_start, c->d_end, o, c->P, chunk);
+        const int64_t avg = c->n / c->P;
+        const dim3 g(static_cast<unsigned>((c->P + chunk - 1) / chunk));
+        if (sizeof(T) == 8 && avg > 1024 && avg <= 8192)
+            hipLaunchKernelGGL((k_fit_chunk<T, FORM, 3>), g, dim3(256), 0, s, v, c->d_start, c->d_end, o, c->P, chunk);
+        else
+            hipLaunchKernelGGL((k_fit_chunk<T, FORM, 4>), g, dim3(256), 0, s, v, c->d_start, c->d_end, o, c->P, chunk);
     } else if (S <= 1024) {
         hipLaunchKernelGGL((k_fit_waves<T, FORM, 2>), per_wave, dim3(64 * kFitWaves), 0, s, v, c->d_start, c->d_end, o,
                            c->P);
