@@ -1064,7 +1064,12 @@ DecArgs make_args(const glc_column* c, void* out) {
     DecArgs a;
     a.desc = c->d_desc;
     a.tile_part = c->d_tile_part;
-    a.words = c->d_words;
+    // The tile paths load words whatever the width.  A released payload of no bits
+    // (glc_preunpack with free_packed; launch_decode_full refuses others): every
+    // load is within 128 + 64 words of its first one, and what it brings is masked
+    // to 0 bits, so any 1 KiB of the column's own arena does.
+    static_assert(kSchedBytes >= kPayloadPadWords * 4, "the queues' part alone covers the loads");
+    a.words = c->d_words ? c->d_words : static_cast<const uint32_t*>(c->meta_arena);
     a.plain = c->d_plain;
     a.params = c->d_params;
     a.out = out;
