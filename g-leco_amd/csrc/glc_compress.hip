@@ -312,20 +312,21 @@ __device__ __forceinline__ void fit_block_any(const T* __restrict__ x, int32_t n
                                               double* __restrict__ s_t, int64_t* __restrict__ s_mx) {
     constexpr int K = 8;
     const int tid = threadIdx.x;
+    const uint32_t un = static_cast<uint32_t>(n);  // indices past n may pass 2^31
     double s[4] = {};  // sums x, y, xx, xy
     int ovf = 0;
     if (tid < bs) {
-        for (int32_t base = tid; base < n; base += bs * K) {
+        for (uint32_t base = tid; base < un; base += bs * K) {
             T y[K];
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                const int32_t i = base + bs * k;
-                y[k] = x[i < n ? i : n - 1];
+                const uint32_t i = base + bs * k;
+                y[k] = x[i < un ? i : un - 1];
             }
 #pragma unroll
             for (int k = 0; k < K; ++k) {
-                const int32_t i = base + bs * k;
-                if (i < n) {
+                const uint32_t i = base + bs * k;
+                if (i < un) {
                     ovf |= might_overflow_double<T>(y[k]) ? 1 : 0;
                     const double xi = static_cast<double>(i), yi = static_cast<double>(y[k]);
                     s[0] = s[0] + xi;
@@ -356,16 +357,17 @@ __device__ __forceinline__ void fit_block_any(const T* __restrict__ x, int32_t n
     fit_theta<FORM>(n, tot[0], tot[1], tot[2], tot[3], t0, t1);
     int64_t mx = 0;
     const bool fast = fit_tier<T>(n, t0, t1) == 1;
-    for (int32_t base = tid; base < n; base += 256 * K) {
+    for (uint32_t base = tid; base < un; base += 256 * K) {
         T y[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-            const int32_t i = base + 256 * k;
-            y[k] = x[i < n ? i : n - 1];
+            const uint32_t i = base + 256 * k;
+            y[k] = x[i < un ? i : un - 1];
         }
 #pragma unroll
         for (int k = 0; k < K; ++k) {  // the clamped index repeats element n - 1: same value
-            const int32_t i = base + 256 * k, j = i < n ? i : n - 1;
+            const uint32_t i = base + 256 * k;
+            const int32_t j = static_cast<int32_t>(i < un ? i : un - 1);
             const int64_t ab = fast ? abs_delta_fast<T, 1>(y[k], t0, t1, j) : abs_delta<T>(y[k], t0, t1, j);
             mx = ab > mx ? ab : mx;
         }
@@ -493,7 +495,8 @@ __device__ __forceinline__ void fit_block(const T* __restrict__ x, int32_t n, in
     double s[4] = {0.0, 0.0, 0.0, 0.0};  // sums y, xy, x, xx
     int ovf = 0;
     const bool xs = n > kExactN;
-    for (int32_t base = 0; base < n; base += kStep) {
+    for (uint32_t step = 0; step < static_cast<uint32_t>(n); step += kStep) {  // passes 2^31 at the largest n
+        const int32_t base = static_cast<int32_t>(step);
         T y[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) {
@@ -650,7 +653,8 @@ __device__ __forceinline__ void fit_wave_long(const T* __restrict__ x, int32_t n
     double a[4] = {}, b[4] = {}, c[4] = {}, d[4] = {};
     int ovf = 0;
     const bool xs = n > kExactN;
-    for (int32_t base = 0; base < n; base += 2 * kFitWaveBs) {
+    for (uint32_t step = 0; step < static_cast<uint32_t>(n); step += 2 * kFitWaveBs) {  // passes 2^31 at the largest n
+        const int32_t base = static_cast<int32_t>(step);
         T y[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
