@@ -21,7 +21,10 @@
 //   merge   up to 10 left-to-right passes.  The group that starts at a
 //           partition does not depend on how the walk got there, so every
 //           partition's group is grown at once, one wave each (k_sm_grow), and
-//           the chain keeps the groups the walk from partition 0 reaches.
+//           the chain keeps the groups the walk from partition 0 reaches.  A
+//           wave grows its group for a bounded number of steps; the groups that
+//           want more are grown on, one after the other, where the walk reaches
+//           them (k_sm_more, k_sm_walk).
 //
 // The maximum residual of a line over a range.  A cost needs only the bit
 // width of max |v_i - round(pr_i)|, pr_i = t0 + t1 * i in FP64.  Over a block the
@@ -1304,12 +1307,24 @@ __global__ __launch_bounds__(kChainThreads) void k_sm_chain_small(F next, E emit
 // in partition j while the refitted whole costs less than the group so far and
 // j apart.  Whether the walk starts a group at e or not, what the group would
 // be depends on e alone, so all are grown at once, a wave each; gend[e] is the
-// first partition after the group, gcost[e] its cost.  A group holds at most
-// about 46341 values (past that the cost model's int32 n * (n - 1) wraps and
-// the fit is useless), which bounds the work per start.  The lines of the next
+// first partition after the group, gcost[e] its cost.  The lines of the next
 // kGrowLook candidates are computed by as many lanes at once; one candidate's
 // residuals take the hulls of its blocks, a block per lane.
+//
+// Total work.  Every candidate of every start takes its whole range again: P starts
+// x candidates of a group x blocks of a group / 64 steps.  A group mostly ends by
+// 46341 values, where the cost model's int32 n * (n - 1) wraps: 12 candidates of 362
+// blocks at m = 128, but 1600 at m = 1 (a split partition has up to 29 m values); and
+// values that are all near 0 fit any line, so their group takes in the whole
+// column.  Hence kGrowSteps, after which a wave stops; of the groups left open only
+// those that the walk reaches count, and they are grown on by the whole GPU.  The
+// bound: P x kGrowSteps steps here, then the walk's own candidates x blocks / 64 steps
+// over up to kMoreCand waves.  A candidate counts as a step for every 64 blocks and one for
+// every 256 values (it may come to be read): m = 32 and above end here (4900 at 32),
+// which are 3 times as fast so (2^21 noisy values, bound 4096 against 8192: m = 32
+// 11.6 and 4.1 ms, m = 1 152 and 236 ms).
 constexpr int kGrowLook = 16;
+constexpr float kGrowSteps = 6144.0f;
 
 // Bit width of the residuals of line t0, t1 over [gs, ge), computed by a
 // wave (gs a block start, ge one or n).
@@ -1364,12 +1379,14 @@ __device__ __forceinline__ int32_t range_bits(const T* __restrict__ v, int64_t g
     return bits >= 0 ? bits : bits_of(wave_max(scan_err<T>(v + gs, lane, len, 64, t0, t1, fast)));
 }
 
+// *more (pinned): set where a group is left open after kGrowSteps steps; its
+// gcost is then negative, and gend the first partition not yet asked.
 template <class T>
 __global__ __launch_bounds__(kSmThreads) void k_sm_grow(const T* __restrict__ v, const int32_t* __restrict__ st,
                                                         const int32_t* __restrict__ en,
                                                         const double* __restrict__ cost, int64_t P, SmPrefix pf,
                                                         SmHull h, int32_t* __restrict__ gend,
-                                                        double* __restrict__ gcost) {
+                                                        double* __restrict__ gcost, int64_t* __restrict__ more) {
     const int lane = threadIdx.x & 63;
     const int64_t e = static_cast<int64_t>(blockIdx.x) * (kSmThreads / 64) +
                       __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1378,7 +1395,9 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_grow(const T* __restrict__ v,
     double gc = cost[e];
     int64_t j = e + 1;
     bool open = true;
-    while (open && j < P) {
+    const float per = 1.0f / 256.0f + 1.0f / (64.0f * static_cast<float>(pf.B));
+    float steps = 0.0f;
+    while (open && j < P && steps < kGrowSteps) {
         double lt0 = 0.0, lt1 = 0.0, lc = 0.0;
         int32_t le = 0;
         bool lf = false;
@@ -1388,11 +1407,12 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_grow(const T* __restrict__ v,
             range_line<T>(pf, gs, le, lt0, lt1, lf);
         }
         const int look = P - j < kGrowLook ? static_cast<int>(P - j) : kGrowLook;
-        for (int c = 0; c < look && open; ++c) {
+        for (int c = 0; c < look && open && steps < kGrowSteps; ++c) {
             const int64_t ge = __shfl(le, c, 64);
             const double merged =
                 cost_of(ge - gs, range_bits<T>(v, gs, ge, __shfl(lt0, c, 64), __shfl(lt1, c, 64),
                                                __shfl(static_cast<int>(lf), c, 64) != 0, pf, h, lane));
+            steps += per * static_cast<float>(static_cast<int32_t>(ge - gs));
             open = merged < gc + __shfl(lc, c, 64);
             if (open) {
                 gc = merged;
@@ -1401,8 +1421,103 @@ __global__ __launch_bounds__(kSmThreads) void k_sm_grow(const T* __restrict__ v,
         }
     }
     if (lane == 0) {
+        const bool left = open && j < P;
         gend[e] = static_cast<int32_t>(j);
-        gcost[e] = gc;
+        gcost[e] = left ? -gc : gc;  // a cost is at least 80
+        if (left) *more = 1;
+    }
+}
+
+// The open group that the walk is at (e = P: none left).
+struct SmOpen {
+    int64_t e, j;  // its start, the first partition not yet asked
+    double gc;
+};
+
+// How many candidates the open group is asked for next: as many as it holds, so
+// that what is asked past its end stays in proportion (2^20 noisy values, m = 8: 81 ms
+// with all of kMoreCand at once, 25 so).
+constexpr int kMoreCand = 4096;
+__device__ __forceinline__ int more_cand(const SmOpen& o, int64_t P) {
+    int64_t n = o.j - o.e;
+    n = n < 64 ? 64 : n > kMoreCand ? kMoreCand : n;
+    return static_cast<int>(n < P - o.j ? n : P - o.j);
+}
+
+// Costs of the open group with each of the next candidates taken in, a wave
+// each, as if all before were.
+template <class T>
+__global__ __launch_bounds__(kSmThreads) void k_sm_more(const T* __restrict__ v, const int32_t* __restrict__ st,
+                                                        const int32_t* __restrict__ en, int64_t P, SmPrefix pf,
+                                                        SmHull h, const SmOpen* __restrict__ open,
+                                                        double* __restrict__ merged) {
+    const int q = static_cast<int>(blockIdx.x) * (kSmThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const SmOpen o = *open;
+    if (o.e >= P || q >= more_cand(o, P)) return;
+    const int64_t gs = st[o.e], ge = en[o.j + q];
+    double t0, t1;
+    bool fast;
+    range_line<T>(pf, gs, ge, t0, t1, fast);
+    const double c = cost_of(ge - gs, range_bits<T>(v, gs, ge, t0, t1, fast, pf, h, threadIdx.x & 63));
+    if ((threadIdx.x & 63) == 0) merged[q] = c;
+}
+
+// Takes in the candidates of k_sm_more up to the first that does not pay; where
+// the group ends there, the walk goes on to the next open one.  first: the walk is
+// at partition 0.  *more (pinned): 0 when it has reached the end.  One workgroup.
+constexpr int kWalkThreads = 1024;
+constexpr int kWalkWin = 4096;
+__global__ __launch_bounds__(kWalkThreads) void k_sm_walk(const double* __restrict__ cost,
+                                                          const double* __restrict__ merged, int64_t P, bool first,
+                                                          int32_t* __restrict__ gend, double* __restrict__ gcost,
+                                                          SmOpen* __restrict__ open, int64_t* __restrict__ more) {
+    __shared__ int32_t s_next[kWalkWin];  // gend, negative where open; of the entries from wb on
+    __shared__ int s_end;
+    const int tid = threadIdx.x;
+    int64_t e = 0;  // the same in every thread, as all below
+    if (!first) {
+        const SmOpen o = *open;
+        e = o.e;
+        if (e >= P) return;
+        const int n = more_cand(o, P);
+        if (tid == 0) s_end = n;
+        __syncthreads();
+        for (int c = tid; c < n; c += kWalkThreads)
+            if (!(merged[c] < (c == 0 ? o.gc : merged[c - 1]) + cost[o.j + c])) atomicMin(&s_end, c);
+        __syncthreads();
+        const int end = s_end;
+        const double gc = end == 0 ? o.gc : merged[end - 1];
+        if (end == n && o.j + n < P) {  // still open
+            if (tid == 0) {
+                open->j = o.j + n;
+                open->gc = gc;
+            }
+            return;
+        }
+        if (tid == 0) {
+            gend[e] = static_cast<int32_t>(o.j + end);
+            gcost[e] = gc;
+        }
+        e = o.j + end;
+    }
+    for (int64_t wb = e - kWalkWin; e < P;) {
+        if (e >= wb + kWalkWin) {
+            __syncthreads();
+            wb = e;
+            for (int q = tid; q < kWalkWin && wb + q < P; q += kWalkThreads)
+                s_next[q] = gcost[wb + q] < 0.0 ? -gend[wb + q] : gend[wb + q];
+            __syncthreads();
+        }
+        const int32_t next = s_next[e - wb];
+        if (next < 0) {
+            if (tid == 0) *open = SmOpen{e, -next, -gcost[e]};
+            return;
+        }
+        e = next;
+    }
+    if (tid == 0) {
+        open->e = P;
+        *more = 0;
     }
 }
 
@@ -1461,7 +1576,7 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, Split
     const int U = m / B;
     const int64_t JB = (n + B - 1) / B;
     // scratch: best_end, exits, mark, pos, st x2, en x2, gend (int32 x J each);
-    // best_cost, cost x2, gcost (double x J each); result (2 x int64); block
+    // best_cost, cost x2, gcost (double x J each); the open group (256 bytes); block
     // prefixes p1, p2 (i128 x (JB + 1)) and chunk offsets c1, c2 (i128 x C); scan
     // tile totals and offsets (int32 x T), chain entries (int32); hull vertices
     // y (double), x (byte) x slots and counts (byte) per block, 64 blocks at a time
@@ -1497,6 +1612,7 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, Split
     int32_t *best_end = I(0), *exits = I(1), *mark = I(2), *pos = I(3);
     int32_t *st0 = I(4), *st1 = I(5), *en0 = I(6), *en1 = I(7), *gend = I(8);
     double *best_cost = D(0), *cost0 = D(1), *cost1 = D(2), *gcost = D(3);
+    SmOpen* open = reinterpret_cast<SmOpen*>(p + 9 * i4 + 4 * d8);
     char* pq = p + 9 * i4 + 4 * d8 + 256;
     i128 *pf1 = reinterpret_cast<i128*>(pq), *pf2 = reinterpret_cast<i128*>(pq + q16);
     i128 *cf1 = reinterpret_cast<i128*>(pq + 2 * q16), *cf2 = reinterpret_cast<i128*>(pq + 2 * q16 + c16);
@@ -1564,11 +1680,30 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, Split
         int32_t *sa = st0, *sb = st1, *ea = en0, *eb = en1;
         double *ca = cost0, *cb = cost1;
         for (int iter = 0; iter < 10 && P > 1; ++iter) {  // CpuPartitioner.cuh:198-242
+            const EmitGroups emit{gend, gcost, sa, ea, sb, eb, cb, host.p};
+            host.p[2] = 0;  // the stream is idle
             hipLaunchKernelGGL(k_sm_grow<T>, dim3(blocks(P, kSmThreads / 64)), dim3(kSmThreads), 0, s, v, sa, ea, ca,
-                               P, pf, h, gend, gcost);
-            chain(ChainMerge{gend}, EmitGroups{gend, gcost, sa, ea, sb, eb, cb, host.p}, P);
+                               P, pf, h, gend, gcost, host.p + 2);
+            chain(ChainMerge{gend}, emit, P);
             GLC_HIP(hipGetLastError());
             GLC_HIP(hipStreamSynchronize(s));
+            if (host.p[2]) {  // a group was left open: that list stands only once the walk's are complete
+                hipLaunchKernelGGL(k_sm_walk, dim3(1), dim3(kWalkThreads), 0, s, ca, cb, P, true, gend, gcost, open,
+                                   host.p + 2);
+                while (host.p[2]) {  // each pair ends a group or takes 64 partitions or more into one
+                    for (int k = 0; k < 8; ++k) {
+                        hipLaunchKernelGGL(k_sm_more<T>, dim3(kMoreCand / (kSmThreads / 64)), dim3(kSmThreads), 0, s, v,
+                                           sa, ea, P, pf, h, open, cb);
+                        hipLaunchKernelGGL(k_sm_walk, dim3(1), dim3(kWalkThreads), 0, s, ca, cb, P, false, gend, gcost,
+                                           open, host.p + 2);
+                    }
+                    GLC_HIP(hipGetLastError());
+                    GLC_HIP(hipStreamSynchronize(s));
+                }
+                chain(ChainMerge{gend}, emit, P);
+                GLC_HIP(hipGetLastError());
+                GLC_HIP(hipStreamSynchronize(s));
+            }
             const int64_t Pn = host.p[0];
             if (Pn < 1 || Pn > P) return fail(GLC_ERR_STATE, "merge pass produced an invalid partition count");
             const bool changed = Pn < P;  // every merge removes one entry
