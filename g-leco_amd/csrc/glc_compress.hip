@@ -1750,7 +1750,8 @@ __device__ __forceinline__ void sel_count(uint32_t k, bool live, int pass, uint3
     for (int q = 0; q < 3; ++q) hist_add(hist[q], d, live && (k & hmask) == pre[q]);
 }
 
-__device__ __forceinline__ void v6_select(const float* __restrict__ var, int64_t nvb, float* __restrict__ thr) {
+// thr (LDS) is complete after the caller's next barrier.
+__device__ __forceinline__ void v6_select(const float* __restrict__ var, int64_t nvb, float (&thr)[3]) {
     __shared__ uint32_t hist[3][256];
     __shared__ uint32_t s_prefix[3];
     __shared__ int64_t s_rank[3];
@@ -1821,7 +1822,9 @@ __device__ __forceinline__ void v6_select(const float* __restrict__ var, int64_t
 }
 __global__ __launch_bounds__(1024) void k_v6_select(const float* __restrict__ var, int64_t nvb,
                                                     float* __restrict__ thr) {
-    v6_select(var, nvb, thr);
+    __shared__ float s_thr[3];
+    v6_select(var, nvb, s_thr);
+    if (threadIdx.x < 3) thr[threadIdx.x] = s_thr[threadIdx.x];  // each its own
 }
 
 struct V6Count {
@@ -1872,13 +1875,14 @@ __global__ void k_v6_emit(V6Count f, int64_t nvb, const int64_t* __restrict__ ba
 // the default base); beyond, writing 16 partitions a block from one workgroup
 // takes longer than the launches.
 constexpr int64_t kV6Small = 2048;
-__global__ __launch_bounds__(1024) void k_v6_small(V6Count f, int64_t nvb, float* __restrict__ thr,
-                                                   int32_t* __restrict__ st, int32_t* __restrict__ en,
-                                                   int64_t* __restrict__ total, int64_t* __restrict__ host) {
+__global__ __launch_bounds__(1024) void k_v6_small(V6Count f, int64_t nvb, int32_t* __restrict__ st,
+                                                   int32_t* __restrict__ en, int64_t* __restrict__ total,
+                                                   int64_t* __restrict__ host) {
     __shared__ int64_t s_w[kScanThreads / 64 + 1];
-    v6_select(f.var, nvb, thr);
-    __threadfence_block();
-    __syncthreads();  // thr
+    __shared__ float s_thr[3];
+    v6_select(f.var, nvb, s_thr);
+    __syncthreads();
+    f.thr = s_thr;
     int64_t carry = 0;
     for (int64_t b0 = 0; b0 < nvb; b0 += 1024) {
         const int64_t b = b0 + threadIdx.x;
@@ -2124,7 +2128,7 @@ int launch_v6(int dtype, const void* d_values, int64_t n, int32_t base, int32_t*
     if (rc) return rc;
     const V6Count f{d_var, d_thr, vbs, n, base};
     if (nvb <= kV6Small) {
-        hipLaunchKernelGGL(k_v6_small, dim3(1), dim3(1024), 0, s, f, nvb, d_thr, d_start, d_end, d_total, h_out);
+        hipLaunchKernelGGL(k_v6_small, dim3(1), dim3(1024), 0, s, f, nvb, d_start, d_end, d_total, h_out);
         GLC_HIP(hipGetLastError());
         return GLC_OK;
     }
