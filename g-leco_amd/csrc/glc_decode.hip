@@ -42,6 +42,7 @@ struct DecArgs {
     int64_t wlimit;                      // payload words (row-load base clamp)
     int32_t* sched;                      // per-XCD work-stealing queues (wave schedule)
     int32_t vec16;                       // out is 16-byte aligned: narrow tiles store 16 bytes per lane
+    bool spans;                          // for the host: some tile holds several partitions (glc_column::spans)
     int32_t pace;                        // pause after each narrow row's stores (pace_row)
     int32_t pace2;                       // the same where predictions are beyond 2^50 (dec_fast_range tier 2)
 };
@@ -803,11 +804,13 @@ __device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t 
 // VEC: narrow tiles take the wide-store path (wave_narrow_v), which needs a
 // 16-byte aligned output; the host picks the instantiation by the output's
 // alignment, so each kernel carries one narrow path only.
-// SEGS: partition-spanning tiles take wave_segs.  Left out where no tile of the
-// launch can span partitions (batches) and of the half-tile kernel: its
-// extra registers (46 -> 72 VGPRs for 64-bit types) leave the whole-tile
-// kernels as fast on columns without such tiles (uint64 2^28 430 against 437
-// us) but cost the half tiles 4 % (420 against 404 us).
+// SEGS: partition-spanning tiles take wave_segs.  Its registers (int64: 46 -> 80
+// VGPRs packed, 30 -> 60 pre-unpack) move packed and pre-unpacked decodes of columns
+// without such tiles by 3 % at most, to either side (without and with, 2^28 int32 215
+// and 214 us, int64 491 and 478; 2^27 int64, pre-unpacked, 385 and 391).  Left out of
+// batches whose tiles cannot span partitions, of pre-unpacking columns without such
+// tiles (2^27 int32: 223 us without, 228 with) and of the half-tile kernel (uint64
+// 2^28: 404 us without, 420 with).
 template <class T, int OP, bool VEC = true, bool SEGS = false>
 __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane, ManyLds* L = nullptr) {
     const int64_t e0 = t * kWaveTile;
@@ -847,17 +850,17 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
 // the uint64 2^28 column: 0.410 ms against 0.422-0.431 ms with four waves
 // (four consecutive tiles) per workgroup; the plain write of 2 GiB in 8-KB
 // per-wave runs takes 0.370 ms against 0.397 ms the same way.
-template <class T, int OP, bool VEC, int WPG>
+template <class T, int OP, bool VEC, bool SEGS, int WPG>
 __global__ __launch_bounds__(64 * WPG) void k_decode_wave(DecArgs a) {
     const int lane = threadIdx.x & 63;
     const int wave = (WPG == 1) ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t t = static_cast<int64_t>(blockIdx.x) * WPG + wave;
     if (t * kWaveTile >= a.n) return;
-    if constexpr (VEC) {
+    if constexpr (VEC && SEGS) {
         __shared__ ManyLds L[WPG];
         wave_tile<T, OP, true, true>(a, t, lane, &L[wave]);
     } else {
-        wave_tile<T, OP, false>(a, t, lane);
+        wave_tile<T, OP, VEC>(a, t, lane);
     }
 }
 
@@ -1080,6 +1083,7 @@ DecArgs make_args(const glc_column* c, void* out) {
     a.wlimit = c->payload_words;
     a.sched = c->d_sched;
     a.vec16 = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    a.spans = c->spans;
     a.pace = a.pace2 = c->dec_pace;
     // no schedule set: long columns with predictions beyond 2^50 decode faster
     // with their stores spaced out (half tiles, int64 timestamps: 2^28 values 472 ->
@@ -1088,23 +1092,29 @@ DecArgs make_args(const glc_column* c, void* out) {
     return a;
 }
 
-template <class T, int OP, bool VEC>
+template <class T, int OP, bool VEC, bool SEGS>
 void launch_static(const DecArgs& a, int dsched, int64_t nwt, hipStream_t s) {
     if (dsched == GLC_DECODE_HALF_TILE_W1 && OP == OP_PACKED)
         hipLaunchKernelGGL((k_decode_half<T, VEC>), dim3(static_cast<unsigned>(2 * nwt)), dim3(64), 0, s, a, nwt);
     else if (dsched != GLC_DECODE_TILE_W4)
-        hipLaunchKernelGGL((k_decode_wave<T, OP, VEC, 1>), dim3(static_cast<unsigned>(nwt)), dim3(64), 0, s, a);
+        hipLaunchKernelGGL((k_decode_wave<T, OP, VEC, SEGS, 1>), dim3(static_cast<unsigned>(nwt)), dim3(64), 0, s, a);
     else
-        hipLaunchKernelGGL((k_decode_wave<T, OP, VEC, 4>), dim3(static_cast<unsigned>((nwt + 3) / 4)), dim3(256), 0, s,
-                           a);
+        hipLaunchKernelGGL((k_decode_wave<T, OP, VEC, SEGS, 4>), dim3(static_cast<unsigned>((nwt + 3) / 4)), dim3(256),
+                           0, s, a);
 }
 
 template <class T, int OP> int run(const DecArgs& a, int sched, hipStream_t s, int dsched = GLC_DECODE_TILE_W4) {
     const int64_t nwt = (a.n + kWaveTile - 1) / kWaveTile;
     switch (sched) {
         case 0:
-            if (a.vec16) launch_static<T, OP, true>(a, dsched, nwt, s);
-            else launch_static<T, OP, false>(a, dsched, nwt, s);
+            if constexpr (OP == OP_UNPACK) {  // wave_tile's note
+                if (a.vec16 && !a.spans) {
+                    launch_static<T, OP, true, false>(a, dsched, nwt, s);
+                    break;
+                }
+            }
+            if (a.vec16) launch_static<T, OP, true, true>(a, dsched, nwt, s);
+            else launch_static<T, OP, false, false>(a, dsched, nwt, s);
             break;
         case 1: {
             hipLaunchKernelGGL(k_zero_queues, dim3(1), dim3(kStealQueues * kQueueStride), 0, s, a.sched);
