@@ -1382,7 +1382,7 @@ struct alignas(16) SpanDesc {
 };
 struct SpanMap {
     SpanDesc d[kManyParts];
-    uint32_t bits[kIndexTile / 32];
+    uint32_t bits[kManyBits];
 };
 
 template <class T> __device__ __forceinline__ SpanDesc span_desc(const Desc& d, int64_t e0, int64_t W0) {

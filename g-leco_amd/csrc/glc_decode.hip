@@ -42,6 +42,7 @@ struct DecArgs {
     int64_t wlimit;                      // payload words (row-load base clamp)
     int32_t* sched;                      // per-XCD work-stealing queues (wave schedule)
     int32_t vec16;                       // out is 16-byte aligned: narrow tiles store 16 bytes per lane
+    int32_t skew;                        // values from a 128-byte line's start to out (and to every tile of it)
     bool spans;                          // for the host: some tile holds several partitions (glc_column::spans)
     int32_t pace;                        // pause after each narrow row's stores (pace_row)
     int32_t pace2;                       // the same where predictions are beyond 2^50 (dec_fast_range tier 2)
@@ -82,48 +83,74 @@ __device__ __forceinline__ void emit(const DecArgs& a, int64_t e, int32_t type, 
     }
 }
 
-// Narrow fast path: the tile lies in one partition with bits <= 32 (linear model).
-template <class T, int OP>
-__device__ __forceinline__ void wave_narrow(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane) {
+// Rows of a tile whose output is not 16-byte aligned: row 0 ends at a line of the
+// output, the others are 64 values from there on, so that only a tile's two ends
+// share a line with another wave's stores (5e7 int64 values in partitions of 64: 134
+// us with rows across lines, 103 so).  SKEW = false: plain rows of 64.
+constexpr int kSkewRows = kWaveRows + 1;
+template <bool SKEW> __device__ __forceinline__ int32_t row_start(int r, int32_t skew) {
+    return SKEW && r > 0 ? r * 64 - skew : r * 64;
+}
+template <bool SKEW> __device__ __forceinline__ int32_t row_end(int r, int32_t skew) {
+    return SKEW ? (r + 1) * 64 - skew : (r + 1) * 64;
+}
+
+// Index in the partition of the tile's value k; past the tile's end (k up to 1087,
+// never stored) it may wrap.
+__device__ __forceinline__ int32_t local_of(const TileInfo& x, int32_t k) {
+    return static_cast<int32_t>(static_cast<uint32_t>(x.lbase) + static_cast<uint32_t>(k));
+}
+
+// Narrow fast path, outputs that are not 16-byte aligned: the tile lies in one
+// partition with bits <= 32 (linear model).  FAST as in narrow_v_rows.
+template <class T, int FAST>
+__device__ __forceinline__ void narrow_rows(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane,
+                                            const uint32_t (&x0)[kSkewRows], const uint32_t (&xs)[kSkewRows]) {
     const int b = tile_bits(x.info);
-    const uint32_t* __restrict__ w = a.words;
-    uint32_t x0[kWaveRows], xs[kWaveRows];
-    // Branch-free loads: lane l reads word wb + l of the row, plus word wb + 64.
-    // wb is clamped to the payload end (rows past the column end are never
-    // stored), and the payload carries kPayloadPadWords zero words, so every
-    // read stays inside the allocation.
-#pragma unroll
-    for (int r = 0; r < kWaveRows; ++r) {
-        const int64_t R = x.W + static_cast<int64_t>(r * 64) * b;
-        const int64_t wb = (R >> 5) < a.wlimit ? (R >> 5) : a.wlimit;
-        x0[r] = w[wb + lane];
-        xs[r] = w[wb + 64];
-    }
-    const int32_t type = tile_type(x.info);
-    const int32_t lbase = x.lbase;
     const uint32_t rel_lane = static_cast<uint32_t>(lane) * static_cast<uint32_t>(b);
+    T* __restrict__ out = static_cast<T*>(a.out);
 #pragma unroll
-    for (int r = 0; r < kWaveRows; ++r) {
-        const int64_t e = e0 + r * 64 + lane;
-        const int64_t R = x.W + static_cast<int64_t>(r * 64) * b;
+    for (int r = 0; r < kSkewRows; ++r) {
+        const int32_t k = row_start<true>(r, a.skew) + lane;
+        const int64_t R = x.W + static_cast<int64_t>(row_start<true>(r, a.skew)) * b;
         const uint32_t rel = static_cast<uint32_t>(R & 31) + rel_lane;
         const uint32_t wi = rel >> 5;
         const uint32_t lo = bperm(x0[r], wi);
         const uint32_t hb = bperm(x0[r], wi + 1);
         const uint32_t hi = (wi + 1 < 64) ? hb : xs[r];
         const uint32_t raw = __builtin_amdgcn_alignbit(hi, lo, rel & 31);
-        uint64_t rawv;
-        int64_t delta;
-        if (b == 32) {
-            rawv = raw;
-            delta = static_cast<int32_t>(raw);
-        } else {
-            rawv = raw & ((1u << b) - 1u);
-            // the builtin returns an unsigned: sign-extend through int32
-            delta = static_cast<int32_t>(__builtin_amdgcn_sbfe(static_cast<int>(raw), 0u, static_cast<unsigned>(b)));
-        }
-        if (e < e1) emit<T, OP>(a, e, type, x.t0, x.t1, lbase + r * 64 + lane, rawv, delta);
+        // the builtin returns an unsigned: sign-extend through int32
+        const int64_t delta = b == 32 ? static_cast<int64_t>(static_cast<int32_t>(raw))
+                                      : static_cast<int64_t>(static_cast<int32_t>(__builtin_amdgcn_sbfe(
+                                            static_cast<int>(raw), 0u, static_cast<unsigned>(b))));
+        T v;
+        const int32_t i = local_of(x, k);
+        if constexpr (FAST != 0) v = apply_delta<T>(dec_pred_fast<T, FAST>(x.t0, x.t1, i), delta);
+        else v = apply_delta<T>(dec_pred<T>(x.t0, x.t1, i), delta);
+        if (k < row_end<true>(r, a.skew) && e0 + k < e1) put(out + e0 + k, v);
     }
+}
+
+template <class T, int TIER = 1> __device__ __forceinline__ bool tile_fast(const TileInfo& x, int32_t i0, int32_t i1);
+
+template <class T>
+__device__ __forceinline__ void wave_narrow(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane) {
+    const int b = tile_bits(x.info);
+    const uint32_t* __restrict__ w = a.words;
+    uint32_t x0[kSkewRows], xs[kSkewRows];
+    // Branch-free loads: lane l reads word wb + l of the row, plus word wb + 64.
+    // wb is clamped to the payload end (rows past the column end are never
+    // stored), and the payload carries kPayloadPadWords zero words, so every
+    // read stays inside the allocation.
+#pragma unroll
+    for (int r = 0; r < kSkewRows; ++r) {
+        const int64_t R = x.W + static_cast<int64_t>(row_start<true>(r, a.skew)) * b;
+        const int64_t wb = (R >> 5) < a.wlimit ? (R >> 5) : a.wlimit;
+        x0[r] = w[wb + lane];
+        xs[r] = w[wb + 64];
+    }
+    if (tile_fast<T, 1>(x, x.lbase, x.lbase + kWaveTile - 1)) narrow_rows<T, 1>(a, x, e0, e1, lane, x0, xs);
+    else narrow_rows<T, 0>(a, x, e0, e1, lane, x0, xs);
 }
 
 // Narrow path with V adjacent values per lane and one 16-byte store per lane
@@ -228,7 +255,7 @@ __device__ __forceinline__ void narrow_v_rows(const DecArgs& a, const TileInfo& 
 
 // True when every prediction of local indices i0 .. i1 of the tile's
 // partition lies in dec_fast_range<T, TIER> (the same on every lane).
-template <class T, int TIER = 1>
+template <class T, int TIER>
 __device__ __forceinline__ bool tile_fast(const TileInfo& x, int32_t i0, int32_t i1) {
     const bool f = dec_fast_range<T, TIER>(__builtin_fma(x.t1, static_cast<double>(i0), x.t0),
                                            __builtin_fma(x.t1, static_cast<double>(i1), x.t0));
@@ -302,22 +329,22 @@ __device__ __forceinline__ void wave_narrow_v(const DecArgs& a, const TileInfo& 
 
 // Wide fast path: one partition, 33..64-bit fields or DIRECT_COPY; two row
 // registers per row (words l and 64 + l) and three bpermute pairs per element.
-// NP, h: part h of NP of the tile's rows.
-template <class T, int OP, int NP = 1>
+// NP, h: part h of NP of the tile's rows.  SKEW: the output is not 16-byte aligned.
+template <class T, int OP, int NP = 1, bool SKEW = false>
 __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane,
                                           int h = 0) {
     constexpr int kRows = kWaveRows / NP;
-    static_assert(kRows % 4 == 0, "whole groups of rows");
+    static_assert(kRows % 4 == 0 && (NP == 1 || !SKEW), "whole groups of rows");
     const int b = tile_bits(x.info);
     const uint32_t* __restrict__ w = a.words;
     const int32_t type = tile_type(x.info);
-    const int32_t lbase = x.lbase;
     const uint32_t rel_lane = static_cast<uint32_t>(lane) * static_cast<uint32_t>(b);
-    for (int r0 = h * kRows; r0 < (h + 1) * kRows; r0 += 4) {
+    for (int r0 = h * kRows; r0 < (h + 1) * kRows + (SKEW ? 1 : 0); r0 += 4) {
         uint32_t x0[4], x1[4], xs[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {  // branch-free, clamped as in wave_narrow
-            const int64_t R = x.W + static_cast<int64_t>((r0 + k) * 64) * b;
+            if (SKEW && k > 0 && r0 == kRows) break;
+            const int64_t R = x.W + static_cast<int64_t>(row_start<SKEW>(r0 + k, a.skew)) * b;
             const int64_t wb = (R >> 5) < a.wlimit ? (R >> 5) : a.wlimit;
             x0[k] = w[wb + lane];
             x1[k] = w[wb + 64 + lane];
@@ -325,8 +352,9 @@ __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, i
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int64_t e = e0 + (r0 + k) * 64 + lane;
-            const int64_t R = x.W + static_cast<int64_t>((r0 + k) * 64) * b;
+            if (SKEW && k > 0 && r0 == kRows) break;
+            const int32_t i = row_start<SKEW>(r0 + k, a.skew) + lane;
+            const int64_t R = x.W + static_cast<int64_t>(row_start<SKEW>(r0 + k, a.skew)) * b;
             const uint32_t rel = static_cast<uint32_t>(R & 31) + rel_lane;
             const uint32_t wi = rel >> 5;
             const uint32_t w1 = wi + 1, w2 = wi + 2;
@@ -342,29 +370,30 @@ __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, i
             const uint64_t rawv = (b >= 64) ? raw : (raw & ((1ULL << b) - 1ULL));
             const int64_t delta =
                 (b >= 64) ? static_cast<int64_t>(raw) : static_cast<int64_t>(raw << (64 - b)) >> (64 - b);
-            if (e < e1) emit<T, OP>(a, e, type, x.t0, x.t1, lbase + (r0 + k) * 64 + lane, rawv, delta);
+            if ((!SKEW || i < row_end<true>(r0 + k, a.skew)) && e0 + i < e1)
+                emit<T, OP>(a, e0 + i, type, x.t0, x.t1, local_of(x, i), rawv, delta);
         }
     }
 }
 
-// Pre-unpacked deltas: one coalesced 8-byte load per element.
+// Pre-unpacked deltas, outputs that are not 16-byte aligned: one coalesced
+// 8-byte load per element.
 template <class T>
 __device__ __forceinline__ void wave_plain(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane) {
-    int64_t pl[kWaveRows];
+    int64_t pl[kSkewRows];
 #pragma unroll
-    for (int r = 0; r < kWaveRows; ++r) {
-        const int64_t e = e0 + r * 64 + lane;
+    for (int r = 0; r < kSkewRows; ++r) {
+        const int64_t e = e0 + row_start<true>(r, a.skew) + lane;
         pl[r] = (e < e1) ? a.plain[e] : 0;
     }
     const int32_t type = tile_type(x.info);
-    const int32_t lbase = x.lbase;
     T* __restrict__ out = static_cast<T*>(a.out);
 #pragma unroll
-    for (int r = 0; r < kWaveRows; ++r) {
-        const int64_t e = e0 + r * 64 + lane;
+    for (int r = 0; r < kSkewRows; ++r) {
+        const int32_t k = row_start<true>(r, a.skew) + lane;
         const T v = (type == MODEL_DIRECT_COPY) ? static_cast<T>(pl[r])
-                                                : apply_delta<T>(dec_pred<T>(x.t0, x.t1, lbase + r * 64 + lane), pl[r]);
-        if (e < e1) put(out + e, v);
+                                                : apply_delta<T>(dec_pred<T>(x.t0, x.t1, local_of(x, k)), pl[r]);
+        if (k < row_end<true>(r, a.skew) && e0 + k < e1) put(out + e0 + k, v);
     }
 }
 
@@ -536,7 +565,7 @@ constexpr int kSegParts = 3;
 // Values [s, t) of partition p (descriptor d; s, t in elements) of the tile at
 // e0.  FAST as in narrow_v_rows; 0 also takes DIRECT_COPY and POLY2.  WIDE: two
 // fields of up to 64 bits from five words.
-template <class T, int OP, int V, int FAST, bool WIDE = false>
+template <class T, int OP, int V, int FAST, bool WIDE = false, bool VEC = true>
 __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t s, int64_t t,
                                          int lane) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
@@ -553,7 +582,8 @@ __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_
     const int32_t lo = static_cast<int32_t>(s - e0), hi = static_cast<int32_t>(t - e0);  // in the tile
     const int32_t kb = static_cast<int32_t>(e0 - d.start);  // tile position x is value kb + x of the partition
     constexpr int32_t kLine = 128 / sizeof(O);  // rows on whole lines (partitions of 1000: 1-4 %)
-    for (int32_t row = lo / kLine * kLine; row < hi; row += kSegRows * 64 * V) {
+    const int32_t skew = VEC ? 0 : a.skew;
+    for (int32_t row = (lo + skew) / kLine * kLine - skew; row < hi; row += kSegRows * 64 * V) {
         const int32_t x0 = row + lane * V;
         uint32_t w[kSegRows][kWords];
         int64_t pl[kSegRows][V];
@@ -628,7 +658,8 @@ __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_
 }
 
 // Values [s, t) of one partition of the tile at e0 (wave-uniform arguments).
-template <class T, int OP>
+// Outputs that are not 16-byte aligned (!VEC): a value a lane.
+template <class T, int OP, bool VEC>
 __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t s,
                                            int64_t t, int lane) {
     constexpr int kWide = (OP == OP_UNPACK || sizeof(T) == 8) ? 2 : 4;  // values of a 16-byte store
@@ -640,7 +671,11 @@ __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int6
         const bool line = type != MODEL_DIRECT_COPY && type != MODEL_POLY2;
         const int tier = !line ? 0 : dec_fast_range<T, 1>(p0, p1) ? 1 : (sizeof(T) == 8 && dec_fast_range<T, 2>(p0, p1)) ? 2 : 0;
         const int u = __builtin_amdgcn_readfirstlane(tier);
-        if (b <= 64 / kWide && b <= 32) {
+        if constexpr (!VEC) {
+            if (u == 1) seg_rows<T, OP, 1, 1, false, false>(a, d, p, e0, s, t, lane);
+            else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, 1, 2, false, false>(a, d, p, e0, s, t, lane);
+            else seg_rows<T, OP, 1, 0, false, false>(a, d, p, e0, s, t, lane);
+        } else if (b <= 64 / kWide && b <= 32) {
             if (u == 1) seg_rows<T, OP, kWide, 1>(a, d, p, e0, s, t, lane);
             else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, kWide, 2>(a, d, p, e0, s, t, lane);
             else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
@@ -679,10 +714,10 @@ struct alignas(8) ManyDesc {
 };
 struct ManyLds {
     ManyDesc d[kManyParts];
-    uint32_t bits[kWaveTile / 32];
+    uint32_t bits[kManyBits];
 };
 
-template <class T, int OP>
+template <class T, int OP, bool SKEW>
 __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int np, int lane,
                                           ManyLds& L) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
@@ -707,14 +742,16 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
     const bool any_wide = __any(wide) != 0;
     const int32_t cnt = static_cast<int32_t>(e1 - e0);
     int base = 0;  // partitions that start in the rows before
-    for (int r0 = 0; r0 < kWaveRows; r0 += 4) {
+    for (int r0 = 0; r0 < kWaveRows + (SKEW ? 1 : 0); r0 += 4) {
         int idx[4];
         uint32_t w0[4], w1[4], w2[4];
         int64_t pl[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            idx[k] = many_index(L.bits, r0 + k, lane, base);
-            const int32_t x = (r0 + k) * 64 + lane;
+            if (SKEW && k > 0 && r0 == kWaveRows) break;
+            const int32_t x = row_start<SKEW>(r0 + k, a.skew) + lane;
+            idx[k] = SKEW ? many_index_at(L.bits, x - lane, row_end<SKEW>(r0 + k, a.skew), lane, base)
+                          : many_index(L.bits, r0 + k, lane, base);
             const ManyDesc& d = L.d[idx[k]];
             const bool in = x < cnt && static_cast<uint32_t>(x - d.sx) < d.len;
             if constexpr (OP == OP_PLAIN) {
@@ -728,7 +765,8 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            const int32_t x = (r0 + k) * 64 + lane;
+            if (SKEW && k > 0 && r0 == kWaveRows) break;
+            const int32_t x = row_start<SKEW>(r0 + k, a.skew) + lane;
             const ManyDesc& d = L.d[idx[k]];
             const int32_t i = x - d.sx;
             const int32_t type = (d.info >> 8) & 15;
@@ -768,20 +806,22 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
                                            delta);
                 }
             }
-            if (x < cnt) put(out + x, v);
+            if (x < cnt && (!SKEW || x < row_end<true>(r0 + k, a.skew))) put(out + x, v);
         }
     }
     return true;
 }
 
-// A tile of the partition-spanning path.  out must be 16-byte aligned (VEC).
-template <class T, int OP>
+// A tile of the partition-spanning path.  VEC: the output is 16-byte aligned.  Where
+// it is not, pre-unpacked tiles take the staged map for few partitions too (5e7 int32
+// values in partitions of 1000: 112 us, a partition at a time 149).
+template <class T, int OP, bool VEC>
 __device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int64_t phi,
                                           int lane, ManyLds* L) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
-    if (phi - plo >= kSegParts) {
+    if ((OP == OP_PLAIN && !VEC) || phi - plo >= kSegParts) {
         const int64_t np = phi - plo + 1;
-        if (np > kManyParts || !wave_many<T, OP>(a, e0, e1, plo, static_cast<int>(np), lane, *L))
+        if (np > kManyParts || !wave_many<T, OP, !VEC>(a, e0, e1, plo, static_cast<int>(np), lane, *L))
             wave_slow<T, OP>(a, e0, e1, plo, lane);
         return;
     }
@@ -795,7 +835,7 @@ __device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t 
         const int64_t s = ds > e0 ? ds : e0, t = de < e1 ? de : e1;
         if (s >= t) continue;
         for (int64_t e = done + lane; e < s; e += 64) out[e] = O(0);  // a gap
-        seg_decode<T, OP>(a, d, p, e0, s, t, lane);
+        seg_decode<T, OP, VEC>(a, d, p, e0, s, t, lane);
         done = t;
     }
     for (int64_t e = done + lane; e < e1; e += 64) out[e] = O(0);
@@ -818,7 +858,7 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
     const TileInfo x = a.tinfo[t];
     // loaded with the tile's line: spanning tiles need both before anything else
     int64_t plo = 0, phi = 0;
-    if constexpr (VEC && SEGS) {
+    if constexpr (SEGS) {
         plo = a.tile_part[t];
         phi = a.tile_part[(e1 + kIndexTile - 1) >> kIndexShift];
     }
@@ -828,17 +868,17 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
             if constexpr (VEC) wave_plain_v<T>(a, x, e0, e1, lane);
             else wave_plain<T>(a, x, e0, e1, lane);
         }
-        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, plo, phi, lane, L);
+        else if constexpr (SEGS) wave_segs<T, OP, VEC>(a, e0, e1, plo, phi, lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     } else {
         if (path == TILE_NARROW) {
-            if constexpr (!VEC) wave_narrow<T, OP>(a, x, e0, e1, lane);
+            if constexpr (!VEC) wave_narrow<T>(a, x, e0, e1, lane);
             else if constexpr (OP == OP_UNPACK || sizeof(T) == 8) wave_narrow_v<T, OP, 2>(a, x, e0, e1, lane);
             else if (tile_bits(x.info) <= 16) wave_narrow_v<T, OP, 4>(a, x, e0, e1, lane);
             else wave_narrow_v<T, OP, 2>(a, x, e0, e1, lane);
         }
-        else if (path == TILE_WIDE) wave_wide<T, OP>(a, x, e0, e1, lane);
-        else if constexpr (VEC && SEGS) wave_segs<T, OP>(a, e0, e1, plo, phi, lane, L);
+        else if (path == TILE_WIDE) wave_wide<T, OP, 1, !VEC>(a, x, e0, e1, lane);
+        else if constexpr (SEGS) wave_segs<T, OP, VEC>(a, e0, e1, plo, phi, lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     }
 }
@@ -856,9 +896,9 @@ __global__ __launch_bounds__(64 * WPG) void k_decode_wave(DecArgs a) {
     const int wave = (WPG == 1) ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t t = static_cast<int64_t>(blockIdx.x) * WPG + wave;
     if (t * kWaveTile >= a.n) return;
-    if constexpr (VEC && SEGS) {
+    if constexpr (SEGS) {
         __shared__ ManyLds L[WPG];
-        wave_tile<T, OP, true, true>(a, t, lane, &L[wave]);
+        wave_tile<T, OP, VEC, true>(a, t, lane, &L[wave]);
     } else {
         wave_tile<T, OP, VEC>(a, t, lane);
     }
@@ -880,7 +920,7 @@ __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
     const int path = tile_path(x.info);
     const int64_t e0 = t * kWaveTile;
     const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
-    if (path == TILE_WIDE) {
+    if (path == TILE_WIDE && VEC) {
         wave_wide<T, OP_PACKED, 2>(a, x, e0, e1, lane, h);
         return;
     }
@@ -976,6 +1016,7 @@ __global__ __launch_bounds__(64 * WPG) void k_batch_decode(const BatchCol* __res
         a.sched = nullptr;
         a.wlimit = c.payload_words;
         a.vec16 = (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+        a.skew = 0;  // outputs that are not aligned take batch_tile_unaligned
         a.pace = a.pace2 = 0;
         const int64_t t = g - c.tile_base;
         if (a.vec16) {
@@ -1043,6 +1084,7 @@ __global__ __launch_bounds__(64) void k_batch_decode_half(const BatchCol* __rest
     a.sched = nullptr;
     a.wlimit = c.payload_words;
     a.vec16 = (reinterpret_cast<uintptr_t>(a.out) & 15) == 0;
+    a.skew = 0;
     a.pace = a.pace2 = 0;
     const int64_t t = g - c.tile_base;
     switch (c.dtype) {
@@ -1083,6 +1125,7 @@ DecArgs make_args(const glc_column* c, void* out) {
     a.wlimit = c->payload_words;
     a.sched = c->d_sched;
     a.vec16 = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    a.skew = static_cast<int32_t>((reinterpret_cast<uintptr_t>(out) & 127) / c->elem_size);
     a.spans = c->spans;
     a.pace = a.pace2 = c->dec_pace;
     // no schedule set: long columns with predictions beyond 2^50 decode faster
@@ -1107,14 +1150,16 @@ template <class T, int OP> int run(const DecArgs& a, int sched, hipStream_t s, i
     const int64_t nwt = (a.n + kWaveTile - 1) / kWaveTile;
     switch (sched) {
         case 0:
-            if constexpr (OP == OP_UNPACK) {  // wave_tile's note
-                if (a.vec16 && !a.spans) {
-                    launch_static<T, OP, true, false>(a, dsched, nwt, s);
-                    break;
-                }
+            if constexpr (OP == OP_UNPACK) {  // into its own block, aligned; wave_tile's note
+                if (a.spans) launch_static<T, OP, true, true>(a, dsched, nwt, s);
+                else launch_static<T, OP, true, false>(a, dsched, nwt, s);
+            } else if (a.vec16) {
+                launch_static<T, OP, true, true>(a, dsched, nwt, s);
+            } else if (a.spans) {
+                launch_static<T, OP, false, true>(a, dsched, nwt, s);
+            } else {
+                launch_static<T, OP, false, false>(a, dsched, nwt, s);
             }
-            if (a.vec16) launch_static<T, OP, true, true>(a, dsched, nwt, s);
-            else launch_static<T, OP, false, false>(a, dsched, nwt, s);
             break;
         case 1: {
             hipLaunchKernelGGL(k_zero_queues, dim3(1), dim3(kStealQueues * kQueueStride), 0, s, a.sched);

@@ -242,6 +242,7 @@ __device__ __forceinline__ T decode_value(int32_t type, double t0, double t1, in
 // before and a masked count in its own, no search.  At most kManyParts partitions
 // (3-4 KB of LDS a wave).
 constexpr int kManyParts = 96;
+constexpr int kManyBits = kIndexTile / 32 + 3;  // many_index_at reads up to three words past the tile
 
 __device__ __forceinline__ void wave_lds_fence() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -256,7 +257,7 @@ __device__ __forceinline__ void wave_lds_fence() {
 // cannot tell them apart.
 template <class F>
 __device__ __forceinline__ bool many_stage(int64_t plo, int np, int lane, uint32_t* bits, F stage) {
-    if (lane < kIndexTile / 32) bits[lane] = 0;
+    if (lane < kManyBits) bits[lane] = 0;
     wave_lds_fence();
     int starts = 0;
     for (int i = lane; i < np; i += 64) {
@@ -283,6 +284,21 @@ __device__ __forceinline__ int many_index(const uint32_t* bits, int r, int lane,
     const uint32_t own = lane < 32 ? (lo >> lane) & 1 : (hi >> (lane - 32)) & 1;
     const int idx = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, own)));
     base += __popc(lo) + __popc(hi);
+    return idx;
+}
+
+// The same for a row of the values s .. end - 1 (end - s <= 64; lanes past it: the
+// last one's or a later partition), rows in order.
+__device__ __forceinline__ int many_index_at(const uint32_t* bits, int s, int end, int lane, int& base) {
+    const int w = s >> 5;
+    const uint32_t b0 = __builtin_amdgcn_readfirstlane(bits[w]), b1 = __builtin_amdgcn_readfirstlane(bits[w + 1]),
+                   b2 = __builtin_amdgcn_readfirstlane(bits[w + 2]);
+    const uint64_t m = (static_cast<uint64_t>(__builtin_amdgcn_alignbit(b2, b1, s & 31)) << 32) |
+                       __builtin_amdgcn_alignbit(b1, b0, s & 31);
+    const uint32_t lo = static_cast<uint32_t>(m), hi = static_cast<uint32_t>(m >> 32);
+    const uint32_t own = lane < 32 ? (lo >> lane) & 1 : (hi >> (lane - 32)) & 1;
+    const int idx = base + static_cast<int>(__builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, own)));
+    base += __popcll(end - s < 64 ? m & ((1ULL << (end - s)) - 1) : m);
     return idx;
 }
 
