@@ -6,15 +6,20 @@
 //                       _PreUnpacked, decompression/FullDecompressionKernels.cuh:48-288,
 //                       and decompressFullFile_WorkStealing,
 //                       decompression/WorkStealingDecompressionKernels.cuh:332-521)
-//   k_decode_steal      the same wave tiles claimed from per-XCD atomic queues
+//   k_decode_plain      pre-unpacked columns of whole-tile partitions, a workgroup per tile
+//   k_decode_half       half tiles (GLC_DECODE_HALF_TILE_W1)
+//   k_decode_steal      wave tiles claimed from per-XCD atomic queues
 //                       (the explicit work-stealing comparator)
 // Every full-decode mode takes these.  The reference's per-partition schedules
 // (…_OnTheFly_Optimized_V2, FullDecompressionKernels.cuh:293-378, a workgroup
 // per partition; …_WorkStealingAdvanced,
-// WorkStealingDecompressionKernels.cuh:526-619, workgroups that claim partitions)
-// were slower than the tiles on every layout measured: 2^26 int32 values in
-// partitions of 1024, 62 us in tiles, 105 with a workgroup per partition, 805 with
-// claims; int64 in partitions of 64, 148 / 875 / 11945 us.
+// WorkStealingDecompressionKernels.cuh:526-619, workgroups that claim partitions) have no
+// kernels of their own: a workgroup per partition was slower than the tiles or within 2 %
+// on the layouts measured (tiles / per partition: 2^26 int32 values in partitions of
+// 1024, 62 / 105 us; 5e7 int64 in partitions of 64, 100 / 634, of 3000, 75 / 103; 2^27
+// int64 pre-unpacked in partitions of 1024, 343 / 358, of 1000, 366 / 372; 5e7 so, into
+// an unaligned output, 154 / 152), and claims were slower everywhere (805 and 8913 us on
+// the first two).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -376,96 +381,104 @@ __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, i
     }
 }
 
-// Pre-unpacked deltas, outputs that are not 16-byte aligned: one coalesced
-// 8-byte load per element.
-template <class T>
-__device__ __forceinline__ void wave_plain(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane) {
-    int64_t pl[kSkewRows];
+// V adjacent values of a lane at p: those with index in [lo, hi) of them, one
+// 16- or 8-byte store when that is all (p is aligned to it).
+template <class O, int V>
+__device__ __forceinline__ void put_values(O* p, const O (&v)[V], int32_t lo, int32_t hi) {
+    if (lo <= 0 && hi >= V) {
+        if constexpr (V * sizeof(O) == 16) {
+            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+            u32x4 q;
+            if constexpr (sizeof(O) == 8) {
+                q.x = static_cast<uint32_t>(static_cast<uint64_t>(v[0]));
+                q.y = static_cast<uint32_t>(static_cast<uint64_t>(v[0]) >> 32);
+                q.z = static_cast<uint32_t>(static_cast<uint64_t>(v[1]));
+                q.w = static_cast<uint32_t>(static_cast<uint64_t>(v[1]) >> 32);
+            } else {
+                q.x = static_cast<uint32_t>(v[0]);
+                q.y = static_cast<uint32_t>(v[1]);
+                q.z = static_cast<uint32_t>(v[2]);
+                q.w = static_cast<uint32_t>(v[3]);
+            }
+            put(reinterpret_cast<u32x4*>(p), q);
+        } else if constexpr (V == 2) {
+            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+            u32x2 q;
+            q.x = static_cast<uint32_t>(v[0]);
+            q.y = static_cast<uint32_t>(v[1]);
+            put(reinterpret_cast<u32x2*>(p), q);
+        } else {
+            put(p, v[0]);
+        }
+    } else {
 #pragma unroll
-    for (int r = 0; r < kSkewRows; ++r) {
-        const int64_t e = e0 + row_start<true>(r, a.skew) + lane;
-        pl[r] = (e < e1) ? a.plain[e] : 0;
-    }
-    const int32_t type = tile_type(x.info);
-    T* __restrict__ out = static_cast<T*>(a.out);
-#pragma unroll
-    for (int r = 0; r < kSkewRows; ++r) {
-        const int32_t k = row_start<true>(r, a.skew) + lane;
-        const T v = (type == MODEL_DIRECT_COPY) ? static_cast<T>(pl[r])
-                                                : apply_delta<T>(dec_pred<T>(x.t0, x.t1, local_of(x, k)), pl[r]);
-        if (k < row_end<true>(r, a.skew) && e0 + k < e1) put(out + e0 + k, v);
+        for (int k = 0; k < V; ++k)
+            if (k >= lo && k < hi) put(p + k, v[k]);
     }
 }
 
 // Pre-unpacked deltas, two per lane: one 16-byte load of two adjacent int64
 // deltas and one 16-byte (8-byte for 32-bit values) store per lane and row
-// of 128 values.  The delta array is a device allocation (16-byte aligned)
-// and e is even, so the vector loads are aligned; the output's alignment is
-// the caller's (VEC instantiation).  PRED: 0 = DIRECT_COPY, 1 = dec_pred,
+// of 128 values.  SKEW: the output is not 16-byte aligned; row r starts at tile
+// value 128 r - skew, on a line of it, so that the stores are aligned all the same and
+// the deltas' loads to 8 bytes (1e8 int64 values: a value a lane in rows of 64 across
+// lines 381 us, 265 so).  PRED: 0 = DIRECT_COPY, 1 = dec_pred,
 // 2 / 3 = dec_pred_fast of tier 1 / 2.
-typedef int64_t i64x2 __attribute__((ext_vector_type(2)));
+typedef int64_t i64x2 __attribute__((ext_vector_type(2), aligned(8)));
 constexpr int kPlainRows = kWaveTile / 128;
 
-template <class T, int PRED>
+template <class T, int PRED, int NR, bool SKEW>
 __device__ __forceinline__ void plain_v_rows(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane,
-                                             const i64x2 (&pl)[kPlainRows]) {
-    const int32_t lbase = x.lbase;
+                                             int rbase, const i64x2 (&pl)[NR]) {
     T* __restrict__ out = static_cast<T*>(a.out);
+    const int32_t cnt = static_cast<int32_t>(e1 - e0);
 #pragma unroll
-    for (int r = 0; r < kPlainRows; ++r) {
-        const int64_t e = e0 + r * 128 + 2 * lane;
-        const int32_t i = lbase + r * 128 + 2 * lane;
+    for (int r = 0; r < NR; ++r) {
+        const int32_t k = (rbase + r) * 128 + 2 * lane - (SKEW ? a.skew : 0);
+        const int32_t i = local_of(x, k);
         T v[2];
         if constexpr (PRED == 0) {
             v[0] = static_cast<T>(pl[r].x);
             v[1] = static_cast<T>(pl[r].y);
         } else if constexpr (PRED == 1) {
             v[0] = apply_delta<T>(dec_pred<T>(x.t0, x.t1, i), pl[r].x);
-            v[1] = apply_delta<T>(dec_pred<T>(x.t0, x.t1, i + 1), pl[r].y);
+            v[1] = apply_delta<T>(dec_pred<T>(x.t0, x.t1, local_of(x, k + 1)), pl[r].y);
         } else {
             v[0] = apply_delta<T>(dec_pred_fast<T, PRED - 1>(x.t0, x.t1, i), pl[r].x);
-            v[1] = apply_delta<T>(dec_pred_fast<T, PRED - 1>(x.t0, x.t1, i + 1), pl[r].y);
+            v[1] = apply_delta<T>(dec_pred_fast<T, PRED - 1>(x.t0, x.t1, local_of(x, k + 1)), pl[r].y);
         }
-        if (e + 2 <= e1) {
-            if constexpr (sizeof(T) == 8) {
-                typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-                u32x4 q;
-                q.x = static_cast<uint32_t>(static_cast<uint64_t>(v[0]));
-                q.y = static_cast<uint32_t>(static_cast<uint64_t>(v[0]) >> 32);
-                q.z = static_cast<uint32_t>(static_cast<uint64_t>(v[1]));
-                q.w = static_cast<uint32_t>(static_cast<uint64_t>(v[1]) >> 32);
-                put(reinterpret_cast<u32x4*>(out + e), q);
-            } else {
-                typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-                u32x2 q;
-                q.x = static_cast<uint32_t>(v[0]);
-                q.y = static_cast<uint32_t>(v[1]);
-                put(reinterpret_cast<u32x2*>(out + e), q);
-            }
-        } else if (e < e1) {
-            put(out + e, v[0]);
-        }
+        put_values<T, 2>(out + e0 + k, v, SKEW ? -k : 0, cnt - k);
     }
 }
 
-template <class T>
-__device__ __forceinline__ void wave_plain_v(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane) {
-    i64x2 pl[kPlainRows];
+// NP, h: part h of NP of the tile's rows (SKEW: the last part's with what row 0
+// leaves over).
+template <class T, int NP = 1, bool SKEW = false>
+__device__ __forceinline__ void wave_plain_v(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane,
+                                             int h = 0) {
+    constexpr int kRows = kPlainRows / NP + (SKEW ? 1 : 0);
+    const int rbase = h * (kPlainRows / NP);
+    // values of this part
+    const int64_t end = SKEW && h < NP - 1 ? e0 + (rbase + kRows - 1) * 128 - a.skew : e1;
+    const int32_t cnt = static_cast<int32_t>((end < e1 ? end : e1) - e0);
+    i64x2 pl[kRows];
 #pragma unroll
-    for (int r = 0; r < kPlainRows; ++r) {
-        const int64_t e = e0 + r * 128 + 2 * lane;
-        if (e + 2 <= e1) {
-            pl[r] = *reinterpret_cast<const i64x2*>(a.plain + e);
+    for (int r = 0; r < kRows; ++r) {
+        const int32_t k = (rbase + r) * 128 + 2 * lane - (SKEW ? a.skew : 0);
+        if (k >= 0 && k + 2 <= cnt) {
+            pl[r] = *reinterpret_cast<const i64x2*>(a.plain + e0 + k);
         } else {
-            pl[r].x = (e < e1) ? a.plain[e] : 0;
-            pl[r].y = 0;
+            pl[r].x = (k >= 0 && k < cnt) ? a.plain[e0 + k] : 0;
+            pl[r].y = (k + 1 >= 0 && k + 1 < cnt) ? a.plain[e0 + k + 1] : 0;
         }
     }
-    if (tile_type(x.info) == MODEL_DIRECT_COPY) plain_v_rows<T, 0>(a, x, e0, e1, lane, pl);
-    else if (tile_fast<T, 1>(x, x.lbase, x.lbase + kWaveTile - 1)) plain_v_rows<T, 2>(a, x, e0, e1, lane, pl);
+    const int64_t stop = e0 + cnt;
+    if (tile_type(x.info) == MODEL_DIRECT_COPY) plain_v_rows<T, 0, kRows, SKEW>(a, x, e0, stop, lane, rbase, pl);
+    else if (tile_fast<T, 1>(x, x.lbase, x.lbase + kWaveTile - 1))
+        plain_v_rows<T, 2, kRows, SKEW>(a, x, e0, stop, lane, rbase, pl);
     else if (sizeof(T) == 8 && tile_fast<T, 2>(x, x.lbase, x.lbase + kWaveTile - 1))
-        plain_v_rows<T, 3>(a, x, e0, e1, lane, pl);
-    else plain_v_rows<T, 1>(a, x, e0, e1, lane, pl);
+        plain_v_rows<T, 3, kRows, SKEW>(a, x, e0, stop, lane, rbase, pl);
+    else plain_v_rows<T, 1, kRows, SKEW>(a, x, e0, stop, lane, rbase, pl);
 }
 
 // Slow path: a tile spanning several partitions, gaps, or a decode-only
@@ -508,42 +521,6 @@ __device__ __forceinline__ void wave_slow(const DecArgs& a, int64_t e0, int64_t 
                 emit<T, OP>(a, e, type, d.theta0, d.theta1, i, raw, delta);
             }
         }
-    }
-}
-
-// V adjacent values of a lane at p: those with index in [lo, hi) of them, one
-// 16- or 8-byte store when that is all (p is aligned to it).
-template <class O, int V>
-__device__ __forceinline__ void put_values(O* p, const O (&v)[V], int32_t lo, int32_t hi) {
-    if (lo <= 0 && hi >= V) {
-        if constexpr (V * sizeof(O) == 16) {
-            typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-            u32x4 q;
-            if constexpr (sizeof(O) == 8) {
-                q.x = static_cast<uint32_t>(static_cast<uint64_t>(v[0]));
-                q.y = static_cast<uint32_t>(static_cast<uint64_t>(v[0]) >> 32);
-                q.z = static_cast<uint32_t>(static_cast<uint64_t>(v[1]));
-                q.w = static_cast<uint32_t>(static_cast<uint64_t>(v[1]) >> 32);
-            } else {
-                q.x = static_cast<uint32_t>(v[0]);
-                q.y = static_cast<uint32_t>(v[1]);
-                q.z = static_cast<uint32_t>(v[2]);
-                q.w = static_cast<uint32_t>(v[3]);
-            }
-            put(reinterpret_cast<u32x4*>(p), q);
-        } else if constexpr (V == 2) {
-            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-            u32x2 q;
-            q.x = static_cast<uint32_t>(v[0]);
-            q.y = static_cast<uint32_t>(v[1]);
-            put(reinterpret_cast<u32x2*>(p), q);
-        } else {
-            put(p, v[0]);
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < V; ++k)
-            if (k >= lo && k < hi) put(p + k, v[k]);
     }
 }
 
@@ -658,7 +635,6 @@ __device__ __forceinline__ void seg_rows(const DecArgs& a, const Desc& d, int64_
 }
 
 // Values [s, t) of one partition of the tile at e0 (wave-uniform arguments).
-// Outputs that are not 16-byte aligned (!VEC): a value a lane.
 template <class T, int OP, bool VEC>
 __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int64_t p, int64_t e0, int64_t s,
                                            int64_t t, int lane) {
@@ -671,28 +647,28 @@ __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int6
         const bool line = type != MODEL_DIRECT_COPY && type != MODEL_POLY2;
         const int tier = !line ? 0 : dec_fast_range<T, 1>(p0, p1) ? 1 : (sizeof(T) == 8 && dec_fast_range<T, 2>(p0, p1)) ? 2 : 0;
         const int u = __builtin_amdgcn_readfirstlane(tier);
-        if constexpr (!VEC) {
-            if (u == 1) seg_rows<T, OP, 1, 1, false, false>(a, d, p, e0, s, t, lane);
-            else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, 1, 2, false, false>(a, d, p, e0, s, t, lane);
-            else seg_rows<T, OP, 1, 0, false, false>(a, d, p, e0, s, t, lane);
+        if constexpr (sizeof(T) == 8 && !VEC) {  // 5e7 values, S = 3000: 81 us, two a lane 94
+            if (u == 1) seg_rows<T, OP, 1, 1, false, VEC>(a, d, p, e0, s, t, lane);
+            else if (u == 2) seg_rows<T, OP, 1, 2, false, VEC>(a, d, p, e0, s, t, lane);
+            else seg_rows<T, OP, 1, 0, false, VEC>(a, d, p, e0, s, t, lane);
         } else if (b <= 64 / kWide && b <= 32) {
-            if (u == 1) seg_rows<T, OP, kWide, 1>(a, d, p, e0, s, t, lane);
-            else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, kWide, 2>(a, d, p, e0, s, t, lane);
-            else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+            if (u == 1) seg_rows<T, OP, kWide, 1, false, VEC>(a, d, p, e0, s, t, lane);
+            else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, kWide, 2, false, VEC>(a, d, p, e0, s, t, lane);
+            else seg_rows<T, OP, 1, 0, false, VEC>(a, d, p, e0, s, t, lane);
         } else if (sizeof(T) == 4 && b <= 32 && u == 1) {
-            seg_rows<T, OP, 2, 1>(a, d, p, e0, s, t, lane);
+            seg_rows<T, OP, 2, 1, false, VEC>(a, d, p, e0, s, t, lane);
         } else if constexpr (sizeof(T) == 8) {
-            if (u == 1) seg_rows<T, OP, 2, 1, true>(a, d, p, e0, s, t, lane);
-            else if (u == 2) seg_rows<T, OP, 2, 2, true>(a, d, p, e0, s, t, lane);
-            else seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+            if (u == 1) seg_rows<T, OP, 2, 1, true, VEC>(a, d, p, e0, s, t, lane);
+            else if (u == 2) seg_rows<T, OP, 2, 2, true, VEC>(a, d, p, e0, s, t, lane);
+            else seg_rows<T, OP, 1, 0, false, VEC>(a, d, p, e0, s, t, lane);
         } else {
-            seg_rows<T, OP, 1, 0>(a, d, p, e0, s, t, lane);
+            seg_rows<T, OP, 1, 0, false, VEC>(a, d, p, e0, s, t, lane);
         }
     } else if constexpr (OP == OP_UNPACK) {
         if (b <= 32) seg_rows<T, OP, 2, 0>(a, d, p, e0, s, t, lane);
         else seg_rows<T, OP, 2, 0, true>(a, d, p, e0, s, t, lane);
     } else {
-        seg_rows<T, OP, 2, 0>(a, d, p, e0, s, t, lane);
+        seg_rows<T, OP, 2, 0, false, VEC>(a, d, p, e0, s, t, lane);
     }
 }
 
@@ -812,14 +788,13 @@ __device__ __forceinline__ bool wave_many(const DecArgs& a, int64_t e0, int64_t 
     return true;
 }
 
-// A tile of the partition-spanning path.  VEC: the output is 16-byte aligned.  Where
-// it is not, pre-unpacked tiles take the staged map for few partitions too (5e7 int32
-// values in partitions of 1000: 112 us, a partition at a time 149).
+// A tile of the partition-spanning path.  VEC: the output is 16-byte aligned; where
+// it is not, seg_rows' rows are shifted to its lines.
 template <class T, int OP, bool VEC>
 __device__ __forceinline__ void wave_segs(const DecArgs& a, int64_t e0, int64_t e1, int64_t plo, int64_t phi,
                                           int lane, ManyLds* L) {
     typedef typename std::conditional<OP == OP_UNPACK, int64_t, T>::type O;
-    if ((OP == OP_PLAIN && !VEC) || phi - plo >= kSegParts) {
+    if (phi - plo >= kSegParts) {
         const int64_t np = phi - plo + 1;
         if (np > kManyParts || !wave_many<T, OP, !VEC>(a, e0, e1, plo, static_cast<int>(np), lane, *L))
             wave_slow<T, OP>(a, e0, e1, plo, lane);
@@ -865,8 +840,9 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
     const int path = tile_path(x.info);
     if constexpr (OP == OP_PLAIN) {
         if (path != TILE_SLOW) {
-            if constexpr (VEC) wave_plain_v<T>(a, x, e0, e1, lane);
-            else wave_plain<T>(a, x, e0, e1, lane);
+            // by halves: with the whole tile in registers the spanning paths run in
+            // fewer waves (int64: 79 VGPRs; 5e7 values in partitions of 300 144 -> 151 us)
+            for (int h = 0; h < 2; ++h) wave_plain_v<T, 2, !VEC>(a, x, e0, e1, lane, h);
         }
         else if constexpr (SEGS) wave_segs<T, OP, VEC>(a, e0, e1, plo, phi, lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
@@ -901,6 +877,25 @@ __global__ __launch_bounds__(64 * WPG) void k_decode_wave(DecArgs a) {
         wave_tile<T, OP, VEC, true>(a, t, lane, &L[wave]);
     } else {
         wave_tile<T, OP, VEC>(a, t, lane);
+    }
+}
+
+// Pre-unpacked columns of whole-tile partitions: a workgroup of NP waves a tile, a
+// part each.  Bound by memory; shorter runs of loads and stores a wave keep both
+// going at once (2^27 values, a tile a wave against 4 or 8 parts: int32 283 and 268
+// us, int64 384 and 341; the other way round 283 and 367).
+template <class T, bool VEC, int NP>
+__global__ __launch_bounds__(64 * NP) void k_decode_plain(DecArgs a) {
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t t = blockIdx.x;
+    const int64_t e0 = t * kWaveTile;
+    const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
+    const TileInfo x = a.tinfo[t];
+    if (tile_path(x.info) == TILE_SLOW) {  // a gap, or a decode-only polynomial model
+        if (wave == static_cast<int>(t % NP)) wave_slow<T, OP_PLAIN>(a, e0, e1, a.tile_part[t], lane);
+    } else {
+        wave_plain_v<T, NP, !VEC>(a, x, e0, e1, lane, wave);
     }
 }
 
@@ -1153,12 +1148,17 @@ template <class T, int OP> int run(const DecArgs& a, int sched, hipStream_t s, i
             if constexpr (OP == OP_UNPACK) {  // into its own block, aligned; wave_tile's note
                 if (a.spans) launch_static<T, OP, true, true>(a, dsched, nwt, s);
                 else launch_static<T, OP, true, false>(a, dsched, nwt, s);
+            } else if (OP == OP_PLAIN && !a.spans) {
+                constexpr int kParts = sizeof(T) == 8 ? 8 : 4;
+                const dim3 g(static_cast<unsigned>(nwt));
+                if (a.vec16) hipLaunchKernelGGL((k_decode_plain<T, true, kParts>), g, dim3(64 * kParts), 0, s, a);
+                else hipLaunchKernelGGL((k_decode_plain<T, false, kParts>), g, dim3(64 * kParts), 0, s, a);
             } else if (a.vec16) {
                 launch_static<T, OP, true, true>(a, dsched, nwt, s);
-            } else if (a.spans) {
+            } else if (OP == OP_PLAIN || a.spans) {
                 launch_static<T, OP, false, true>(a, dsched, nwt, s);
             } else {
-                launch_static<T, OP, false, false>(a, dsched, nwt, s);
+                launch_static<T, OP, false, OP == OP_PLAIN>(a, dsched, nwt, s);
             }
             break;
         case 1: {
