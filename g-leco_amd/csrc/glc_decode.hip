@@ -49,6 +49,7 @@ struct DecArgs {
     int32_t vec16;                       // out is 16-byte aligned: narrow tiles store 16 bytes per lane
     int32_t skew;                        // values from a 128-byte line's start to out (and to every tile of it)
     bool spans;                          // for the host: some tile holds several partitions (glc_column::spans)
+    bool wide;                           // for the host: some field has more than 32 bits
     int32_t pace;                        // pause after each narrow row's stores (pace_row)
     int32_t pace2;                       // the same where predictions are beyond 2^50 (dec_fast_range tier 2)
 };
@@ -334,22 +335,21 @@ __device__ __forceinline__ void wave_narrow_v(const DecArgs& a, const TileInfo& 
 
 // Wide fast path: one partition, 33..64-bit fields or DIRECT_COPY; two row
 // registers per row (words l and 64 + l) and three bpermute pairs per element.
-// NP, h: part h of NP of the tile's rows.  SKEW: the output is not 16-byte aligned.
-template <class T, int OP, int NP = 1, bool SKEW = false>
+// NP, h: part h of NP of the tile's rows.
+template <class T, int OP, int NP = 1>
 __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, int64_t e0, int64_t e1, int lane,
                                           int h = 0) {
     constexpr int kRows = kWaveRows / NP;
-    static_assert(kRows % 4 == 0 && (NP == 1 || !SKEW), "whole groups of rows");
+    static_assert(kRows % 4 == 0, "whole groups of rows");
     const int b = tile_bits(x.info);
     const uint32_t* __restrict__ w = a.words;
     const int32_t type = tile_type(x.info);
     const uint32_t rel_lane = static_cast<uint32_t>(lane) * static_cast<uint32_t>(b);
-    for (int r0 = h * kRows; r0 < (h + 1) * kRows + (SKEW ? 1 : 0); r0 += 4) {
+    for (int r0 = h * kRows; r0 < (h + 1) * kRows; r0 += 4) {
         uint32_t x0[4], x1[4], xs[4];
 #pragma unroll
         for (int k = 0; k < 4; ++k) {  // branch-free, clamped as in wave_narrow
-            if (SKEW && k > 0 && r0 == kRows) break;
-            const int64_t R = x.W + static_cast<int64_t>(row_start<SKEW>(r0 + k, a.skew)) * b;
+            const int64_t R = x.W + static_cast<int64_t>((r0 + k) * 64) * b;
             const int64_t wb = (R >> 5) < a.wlimit ? (R >> 5) : a.wlimit;
             x0[k] = w[wb + lane];
             x1[k] = w[wb + 64 + lane];
@@ -357,9 +357,8 @@ __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, i
         }
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
-            if (SKEW && k > 0 && r0 == kRows) break;
-            const int32_t i = row_start<SKEW>(r0 + k, a.skew) + lane;
-            const int64_t R = x.W + static_cast<int64_t>(row_start<SKEW>(r0 + k, a.skew)) * b;
+            const int64_t e = e0 + (r0 + k) * 64 + lane;
+            const int64_t R = x.W + static_cast<int64_t>((r0 + k) * 64) * b;
             const uint32_t rel = static_cast<uint32_t>(R & 31) + rel_lane;
             const uint32_t wi = rel >> 5;
             const uint32_t w1 = wi + 1, w2 = wi + 2;
@@ -375,8 +374,7 @@ __device__ __forceinline__ void wave_wide(const DecArgs& a, const TileInfo& x, i
             const uint64_t rawv = (b >= 64) ? raw : (raw & ((1ULL << b) - 1ULL));
             const int64_t delta =
                 (b >= 64) ? static_cast<int64_t>(raw) : static_cast<int64_t>(raw << (64 - b)) >> (64 - b);
-            if ((!SKEW || i < row_end<true>(r0 + k, a.skew)) && e0 + i < e1)
-                emit<T, OP>(a, e0 + i, type, x.t0, x.t1, local_of(x, i), rawv, delta);
+            if (e < e1) emit<T, OP>(a, e, type, x.t0, x.t1, x.lbase + (r0 + k) * 64 + lane, rawv, delta);
         }
     }
 }
@@ -647,11 +645,7 @@ __device__ __forceinline__ void seg_decode(const DecArgs& a, const Desc& d, int6
         const bool line = type != MODEL_DIRECT_COPY && type != MODEL_POLY2;
         const int tier = !line ? 0 : dec_fast_range<T, 1>(p0, p1) ? 1 : (sizeof(T) == 8 && dec_fast_range<T, 2>(p0, p1)) ? 2 : 0;
         const int u = __builtin_amdgcn_readfirstlane(tier);
-        if constexpr (sizeof(T) == 8 && !VEC) {  // 5e7 values, S = 3000: 81 us, two a lane 94
-            if (u == 1) seg_rows<T, OP, 1, 1, false, VEC>(a, d, p, e0, s, t, lane);
-            else if (u == 2) seg_rows<T, OP, 1, 2, false, VEC>(a, d, p, e0, s, t, lane);
-            else seg_rows<T, OP, 1, 0, false, VEC>(a, d, p, e0, s, t, lane);
-        } else if (b <= 64 / kWide && b <= 32) {
+        if (b <= 64 / kWide && b <= 32) {
             if (u == 1) seg_rows<T, OP, kWide, 1, false, VEC>(a, d, p, e0, s, t, lane);
             else if (sizeof(T) == 8 && u == 2) seg_rows<T, OP, kWide, 2, false, VEC>(a, d, p, e0, s, t, lane);
             else seg_rows<T, OP, 1, 0, false, VEC>(a, d, p, e0, s, t, lane);
@@ -853,7 +847,12 @@ __device__ __forceinline__ void wave_tile(const DecArgs& a, int64_t t, int lane,
             else if (tile_bits(x.info) <= 16) wave_narrow_v<T, OP, 4>(a, x, e0, e1, lane);
             else wave_narrow_v<T, OP, 2>(a, x, e0, e1, lane);
         }
-        else if (path == TILE_WIDE) wave_wide<T, OP, 1, !VEC>(a, x, e0, e1, lane);
+        else if (path == TILE_WIDE) {
+            // shifted rows: two wide fields a lane (1.3e8 int64 values of 41 bits: 312 us, one
+            // a lane 330; of 51 bits 330, 350)
+            if constexpr (!VEC && SEGS) seg_decode<T, OP, false>(a, a.desc[plo], plo, e0, e0, e1, lane);
+            else wave_wide<T, OP>(a, x, e0, e1, lane);
+        }
         else if constexpr (SEGS) wave_segs<T, OP, VEC>(a, e0, e1, plo, phi, lane, L);
         else wave_slow<T, OP>(a, e0, e1, a.tile_part[t], lane);
     }
@@ -899,13 +898,13 @@ __global__ __launch_bounds__(64 * NP) void k_decode_plain(DecArgs a) {
     }
 }
 
-// Half tiles (packed decode): one-wave workgroup g decodes half g & 1 of narrow
-// or wide tile g >> 1; a tile of any other path is decoded whole by one half's
+// Half tiles (packed decode into 16-byte aligned outputs; others take whole tiles by
+// one wave): one-wave workgroup g decodes half g & 1 of narrow or wide tile g >> 1; a tile of any other path is decoded whole by one half's
 // wave, the first's and the second's in turn so that every XCD has such waves
 // (all on the first's: 264 instead of 166 us, 7e7 uint64 of 36 bits).  (Quarter
 // tiles, one wave per two 128-value rows, ran 20-55 % slower on every column
 // measured.)
-template <class T, bool VEC>
+template <class T>
 __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
     const int lane = threadIdx.x & 63;
     const int64_t t = static_cast<int64_t>(blockIdx.x) >> 1;
@@ -915,12 +914,12 @@ __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
     const int path = tile_path(x.info);
     const int64_t e0 = t * kWaveTile;
     const int64_t e1 = (e0 + kWaveTile < a.n) ? e0 + kWaveTile : a.n;
-    if (path == TILE_WIDE && VEC) {
+    if (path == TILE_WIDE) {
         wave_wide<T, OP_PACKED, 2>(a, x, e0, e1, lane, h);
         return;
     }
-    if (path != TILE_NARROW || !VEC) {  // whole (workgroup g runs on XCD g % 8)
-        if (h == static_cast<int>(t >> 2 & 1)) wave_tile<T, OP_PACKED, VEC>(a, t, lane);
+    if (path != TILE_NARROW) {  // whole (workgroup g runs on XCD g % 8)
+        if (h == static_cast<int>(t >> 2 & 1)) wave_tile<T, OP_PACKED>(a, t, lane);
         return;
     }
     if constexpr (sizeof(T) == 8) wave_narrow_v<T, OP_PACKED, 2, 2>(a, x, e0, e1, lane, h);
@@ -1122,18 +1121,15 @@ DecArgs make_args(const glc_column* c, void* out) {
     a.vec16 = (reinterpret_cast<uintptr_t>(out) & 15) == 0;
     a.skew = static_cast<int32_t>((reinterpret_cast<uintptr_t>(out) & 127) / c->elem_size);
     a.spans = c->spans;
+    a.wide = c->max_bits > 32;
     a.pace = a.pace2 = c->dec_pace;
-    // no schedule set: long columns with predictions beyond 2^50 decode faster
-    // with their stores spaced out (half tiles, int64 timestamps: 2^28 values 472 ->
-    // 452 us, 3e8 528 -> 496; 2^26 106 -> 109)
-    if (c->dec_auto && c->n >= (int64_t(1) << 27)) a.pace2 = 16;
     return a;
 }
 
 template <class T, int OP, bool VEC, bool SEGS>
 void launch_static(const DecArgs& a, int dsched, int64_t nwt, hipStream_t s) {
-    if (dsched == GLC_DECODE_HALF_TILE_W1 && OP == OP_PACKED)
-        hipLaunchKernelGGL((k_decode_half<T, VEC>), dim3(static_cast<unsigned>(2 * nwt)), dim3(64), 0, s, a, nwt);
+    if (dsched == GLC_DECODE_HALF_TILE_W1 && OP == OP_PACKED && VEC)
+        hipLaunchKernelGGL(k_decode_half<T>, dim3(static_cast<unsigned>(2 * nwt)), dim3(64), 0, s, a, nwt);
     else if (dsched != GLC_DECODE_TILE_W4)
         hipLaunchKernelGGL((k_decode_wave<T, OP, VEC, SEGS, 1>), dim3(static_cast<unsigned>(nwt)), dim3(64), 0, s, a);
     else
@@ -1155,7 +1151,7 @@ template <class T, int OP> int run(const DecArgs& a, int sched, hipStream_t s, i
                 else hipLaunchKernelGGL((k_decode_plain<T, false, kParts>), g, dim3(64 * kParts), 0, s, a);
             } else if (a.vec16) {
                 launch_static<T, OP, true, true>(a, dsched, nwt, s);
-            } else if (OP == OP_PLAIN || a.spans) {
+            } else if (OP == OP_PLAIN || a.spans || a.wide) {
                 launch_static<T, OP, false, true>(a, dsched, nwt, s);
             } else {
                 launch_static<T, OP, false, OP == OP_PLAIN>(a, dsched, nwt, s);
@@ -1211,10 +1207,22 @@ int launch_decode_full(const glc_column* c, void* d_out, int mode, hipStream_t s
     DecArgs a = make_args(c, d_out);
     // No schedule set: 64-bit columns of whole-tile partitions take half tiles
     // (2^28 values 399-560 us against 431-631 with four tiles a workgroup, by width;
-    // within 3 % below 2^27).  32-bit ones are faster in whole tiles (2^28
-    // 239-278 against 254-291), and the half-tile kernel has no fast path for
-    // partition-spanning tiles.
-    const int dsched = (c->dec_auto && c->elem_size == 8 && !c->spans) ? GLC_DECODE_HALF_TILE_W1 : c->dec_sched;
+    // within 3 % below 2^27).  Long ones of wide fields whose predictions are beyond
+    // 2^50 (timestamps) also space their stores out: 2^28 values of 17 / 19 / 21 / 24 / 29
+    // bits take 411 / 422 / 463 / 478 / 512 us without, 454 / 452 / 449 / 446 / 497 with;
+    // 2^26 of 20 bits 106 and 109.  32-bit columns are faster in whole tiles (2^28 239-278
+    // against 254-291), and the half-tile kernel has no fast path for
+    // partition-spanning tiles and none for outputs that are not 16-byte aligned.
+    // Those decode in one-wave workgroups (1.3e8 int64 values of 41 bits, S = 1000: 321
+    // us in fours, 316 so; S = 3000: 351, 331, and of 13 bits 244, 236; int32 of 25 bits
+    // 187, 178).
+    int dsched = c->dec_sched;
+    if (c->dec_auto && !a.vec16) {
+        dsched = GLC_DECODE_TILE_W1;
+    } else if (c->dec_auto && c->elem_size == 8 && !c->spans) {
+        dsched = GLC_DECODE_HALF_TILE_W1;
+        if (c->n >= (int64_t(1) << 27) && c->total_bits >= 21 * c->n) a.pace2 = 16;
+    }
     return dispatch_dtype(c->dtype, [&](auto t) {
         using T = decltype(t);
         return plain ? run<T, OP_PLAIN>(a, sched, s, c->dec_sched) : run<T, OP_PACKED>(a, sched, s, dsched);
