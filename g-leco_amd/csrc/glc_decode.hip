@@ -899,11 +899,11 @@ __global__ __launch_bounds__(64 * NP) void k_decode_plain(DecArgs a) {
 }
 
 // Half tiles (packed decode into 16-byte aligned outputs; others take whole tiles by
-// one wave): one-wave workgroup g decodes half g & 1 of narrow or wide tile g >> 1; a tile of any other path is decoded whole by one half's
-// wave, the first's and the second's in turn so that every XCD has such waves
-// (all on the first's: 264 instead of 166 us, 7e7 uint64 of 36 bits).  (Quarter
-// tiles, one wave per two 128-value rows, ran 20-55 % slower on every column
-// measured.)
+// one wave): one-wave workgroup g decodes half g & 1 of narrow or wide tile g >> 1; a
+// tile of any other path is decoded whole by one half's wave, the first's and the
+// second's in turn so that every XCD has such waves (all on the first's: 264 instead
+// of 166 us, 7e7 uint64 of 36 bits).  (Quarter tiles, one wave per two 128-value rows,
+// ran 20-55 % slower on every column measured.)
 template <class T>
 __global__ __launch_bounds__(64) void k_decode_half(DecArgs a, int64_t ntiles) {
     const int lane = threadIdx.x & 63;
@@ -1033,8 +1033,8 @@ __global__ __launch_bounds__(64 * WPG) void k_batch_decode(const BatchCol* __res
 
 // Batched half tiles: one-wave workgroup g decodes half g & 1 of global tile
 // g >> 1, the other paths as in k_decode_half.
-template <class T>
-__device__ __forceinline__ void batch_half(const DecArgs& a, int64_t t, int h, int lane) {
+template <class T, bool SEGS>
+__device__ __forceinline__ void batch_half(const DecArgs& a, int64_t t, int h, int lane, ManyLds* L) {
     const TileInfo x = a.tinfo[t];
     const int path = tile_path(x.info);
     const int64_t e0 = t * kWaveTile;
@@ -1045,7 +1045,7 @@ __device__ __forceinline__ void batch_half(const DecArgs& a, int64_t t, int h, i
     }
     if (path != TILE_NARROW || !a.vec16) {
         if (h == static_cast<int>(t >> 2 & 1)) {
-            if (a.vec16) wave_tile<T, OP_PACKED, true>(a, t, lane);
+            if (a.vec16) wave_tile<T, OP_PACKED, true, SEGS>(a, t, lane, L);
             else batch_tile_unaligned<T>(a, t, lane);
         }
         return;
@@ -1055,10 +1055,16 @@ __device__ __forceinline__ void batch_half(const DecArgs& a, int64_t t, int h, i
     else wave_narrow_v<T, OP_PACKED, 2, 2>(a, x, e0, e1, lane, h);
 }
 
+template <bool SEGS>
 __global__ __launch_bounds__(64) void k_batch_decode_half(const BatchCol* __restrict__ cols,
                                                           const int32_t* __restrict__ tile_col,
                                                           void* const* __restrict__ outs, int64_t Ttot) {
     const int lane = threadIdx.x & 63;
+    ManyLds* L = nullptr;
+    if constexpr (SEGS) {
+        __shared__ ManyLds s_many;
+        L = &s_many;
+    }
     const int64_t g = static_cast<int64_t>(blockIdx.x) >> 1;
     const int h = static_cast<int>(blockIdx.x & 1);
     if (g >= Ttot) return;
@@ -1082,10 +1088,10 @@ __global__ __launch_bounds__(64) void k_batch_decode_half(const BatchCol* __rest
     a.pace = a.pace2 = 0;
     const int64_t t = g - c.tile_base;
     switch (c.dtype) {
-        case GLC_I32: batch_half<int32_t>(a, t, h, lane); break;
-        case GLC_U32: batch_half<uint32_t>(a, t, h, lane); break;
-        case GLC_I64: batch_half<int64_t>(a, t, h, lane); break;
-        default: batch_half<uint64_t>(a, t, h, lane); break;
+        case GLC_I32: batch_half<int32_t, SEGS>(a, t, h, lane, L); break;
+        case GLC_U32: batch_half<uint32_t, SEGS>(a, t, h, lane, L); break;
+        case GLC_I64: batch_half<int64_t, SEGS>(a, t, h, lane, L); break;
+        default: batch_half<uint64_t, SEGS>(a, t, h, lane, L); break;
     }
 }
 
@@ -1306,20 +1312,16 @@ int launch_batch_decode(const BatchPlan& b, int wpg, int tpw, hipStream_t s) {
         return dim3(static_cast<unsigned>((b.Ttot + static_cast<int64_t>(w) * t - 1) / (static_cast<int64_t>(w) * t)));
     };
     // partitions that are no multiple of a tile leave partition-spanning tiles
-    // all over: the instantiation with the segment rows, one or four waves per
-    // workgroup (the other schedules group whole-partition tiles)
-    if (b.S % kIndexTile != 0) {
-        if (wpg == 1) hipLaunchKernelGGL((k_batch_decode<1, 1, true>), grid(1, 1), dim3(64), 0, s, b.cols, b.tile_col,
-                                         b.outs, b.Ttot);
-        else hipLaunchKernelGGL((k_batch_decode<4, 1, true>), grid(4, 1), dim3(256), 0, s, b.cols, b.tile_col, b.outs,
-                                b.Ttot);
-        GLC_HIP(hipGetLastError());
-        return GLC_OK;
-    }
+    // all over: the instantiations with the spanning paths
+    const bool segs = b.S % kIndexTile != 0;
 #define GLC_BATCH_CASE(W, TP)                                                                                     \
     if (wpg == W && tpw == TP) {                                                                                  \
-        hipLaunchKernelGGL((k_batch_decode<W, TP, false>), grid(W, TP), dim3(64 * W), 0, s, b.cols, b.tile_col,    \
-                           b.outs, b.Ttot);                                                               \
+        if (segs)                                                                                                 \
+            hipLaunchKernelGGL((k_batch_decode<W, TP, true>), grid(W, TP), dim3(64 * W), 0, s, b.cols, b.tile_col, \
+                               b.outs, b.Ttot);                                                                   \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_batch_decode<W, TP, false>), grid(W, TP), dim3(64 * W), 0, s, b.cols,           \
+                               b.tile_col, b.outs, b.Ttot);                                                       \
         GLC_HIP(hipGetLastError());                                                                               \
         return GLC_OK;                                                                                            \
     }
@@ -1331,8 +1333,9 @@ int launch_batch_decode(const BatchPlan& b, int wpg, int tpw, hipStream_t s) {
     GLC_BATCH_CASE(2, 4)
 #undef GLC_BATCH_CASE
     if (wpg == 1 && tpw == 0) {
-        hipLaunchKernelGGL(k_batch_decode_half, dim3(static_cast<unsigned>(2 * b.Ttot)), dim3(64), 0, s, b.cols,
-                           b.tile_col, b.outs, b.Ttot);
+        const dim3 g(static_cast<unsigned>(2 * b.Ttot));
+        if (segs) hipLaunchKernelGGL(k_batch_decode_half<true>, g, dim3(64), 0, s, b.cols, b.tile_col, b.outs, b.Ttot);
+        else hipLaunchKernelGGL(k_batch_decode_half<false>, g, dim3(64), 0, s, b.cols, b.tile_col, b.outs, b.Ttot);
         GLC_HIP(hipGetLastError());
         return GLC_OK;
     }
