@@ -85,19 +85,13 @@ thread_local std::string g_last_error;
 // device between calls and grown when a larger column needs more: a
 // per-call hipMalloc/hipFree pair costs hundreds of microseconds and the
 // free synchronises the device.  Held until the process ends; the lock
-// covers the scratch from the first V6 kernel to the last copy out of it.
-struct V6Scratch {
-    std::mutex mu;
-    void* p = nullptr;
-    int64_t bytes = 0;
-};
-
-V6Scratch& v6_scratch(int device) {
+// covers the scratch from the first V6 kernel to the launch of the last that reads it.
+SharedScratch& v6_scratch(int device) {
     static std::mutex table_mu;
-    static std::map<int, V6Scratch*>* table = new std::map<int, V6Scratch*>();
+    static std::map<int, SharedScratch*>* table = new std::map<int, SharedScratch*>();
     std::lock_guard<std::mutex> g(table_mu);
-    V6Scratch*& e = (*table)[device];
-    if (!e) e = new V6Scratch();
+    SharedScratch*& e = (*table)[device];
+    if (!e) e = new SharedScratch();
     return *e;
 }
 
@@ -275,9 +269,9 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
     int64_t len0 = 0;
     HostWords host;
     if (!host.p) return bail(fail(GLC_ERR_OOM, "pinned host allocation failed"));
-    // scratch locks of the partitioners: held until finish_index has waited
-    // for the kernels that read the scratch (declared after c's owner: a return
-    // waits first, below)
+    // scratch locks of the partitioners: held until the last kernel that reads
+    // the scratch has been launched (declared after c's owner: an error return waits
+    // first, below)
     std::unique_lock<std::mutex> v6_lock;
     SplitMergeResult sm;
     struct Drain {  // an error return leaves no kernel on the scratch before the locks go
@@ -310,20 +304,9 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
             // temp: start[cap], end[cap], count[nvb+1] (int64), var[nvb], thr[3]
             const int64_t bytes = align_up(cap * 4, 256) * 2 + align_up((nvb + 1) * 8, 256) +
                                   align_up(nvb * 4, 256) + 256;
-            V6Scratch& sc = v6_scratch(c->device);
+            SharedScratch& sc = v6_scratch(c->device);
             v6_lock = std::unique_lock<std::mutex>(sc.mu);
-            if (sc.bytes < bytes) {
-                if (sc.p) (void)hipFree(sc.p);  // the previous call ended with its work on it waited for
-                sc.p = nullptr;
-                sc.bytes = 0;
-                const int64_t want = align_up(bytes + bytes / 4, 1 << 20);
-                if (hipMalloc(&sc.p, want) != hipSuccess) {
-                    (void)hipGetLastError();
-                    sc.p = nullptr;
-                    return bail(fail(GLC_ERR_OOM, "V6 scratch allocation failed"));
-                }
-                sc.bytes = want;
-            }
+            if ((rc = scratch_acquire(sc, bytes, s))) return bail(rc);
             char* t = static_cast<char*>(sc.p);
             int32_t* ts = reinterpret_cast<int32_t*>(t);
             int32_t* te = reinterpret_cast<int32_t*>(t + align_up(cap * 4, 256));
@@ -337,6 +320,8 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
             len0 = host.p[1];
             if ((rc = alloc_column(c, P, s, false))) return bail(rc);
             if ((rc = launch_column_setup(c, 0, ts, te, false, s))) return bail(rc);
+            if ((rc = scratch_release(sc, INT64_MAX, s))) return bail(rc);
+            v6_lock.unlock();
             break;
         }
         case GLC_PART_GPU_SPLITMERGE: {
@@ -344,6 +329,7 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
             len0 = sm.first_len;
             if ((rc = alloc_column(c, sm.P, s, false))) return bail(rc);
             if ((rc = launch_column_setup(c, 0, sm.d_st, sm.d_en, false, s))) return bail(rc);
+            if ((rc = split_merge_release(sm, s))) return bail(rc);
             break;
         }
         case GLC_PART_CPU_SPLITMERGE: {
@@ -385,8 +371,6 @@ int compress_impl(int dtype, const void* d_values, int64_t n, int partitioner, i
         return bail(rc);
     IndexSummary sum;
     if ((rc = finish_index(c, true, host, s, &sum))) return bail(rc);
-    if (v6_lock.owns_lock()) v6_lock.unlock();  // the stream was waited for
-    split_merge_release(sm);
     c->total_bits = sum.total_bits;
     c->fixed_size = sum.not_fixed ? 0 : static_cast<int32_t>(len0);
     if ((rc = alloc_payload(c, (c->total_bits + 31) / 32, s, false))) return bail(rc);
@@ -500,6 +484,39 @@ HostWords::~HostWords() {
     HostPool& pool = host_pool();
     std::lock_guard<std::mutex> g(pool.mu);
     pool.idle.push_back(p);
+}
+
+int scratch_acquire(SharedScratch& sc, int64_t bytes, hipStream_t s) {
+    if (sc.bytes < bytes) {
+        if (sc.p) {
+            if (sc.last) GLC_HIP(hipEventSynchronize(sc.last));
+            (void)hipFree(sc.p);
+        }
+        sc.p = nullptr;
+        sc.bytes = 0;
+        const int64_t want = align_up(bytes + bytes / 4, 1 << 20);
+        if (hipMalloc(&sc.p, static_cast<size_t>(want)) != hipSuccess) {
+            (void)hipGetLastError();
+            sc.p = nullptr;
+            return fail(GLC_ERR_OOM, "device allocation of partitioning scratch failed");
+        }
+        sc.bytes = want;
+    }
+    if (sc.last) GLC_HIP(hipStreamWaitEvent(s, sc.last, 0));
+    return GLC_OK;
+}
+
+int scratch_release(SharedScratch& sc, int64_t keep, hipStream_t s) {
+    if (sc.bytes > keep) {
+        GLC_HIP(hipStreamSynchronize(s));
+        (void)hipFree(sc.p);
+        sc.p = nullptr;
+        sc.bytes = 0;
+        return GLC_OK;
+    }
+    if (!sc.last) GLC_HIP(hipEventCreateWithFlags(&sc.last, hipEventDisableTiming));
+    GLC_HIP(hipEventRecord(sc.last, s));
+    return GLC_OK;
 }
 
 void set_error(const std::string& msg) { g_last_error = msg; }

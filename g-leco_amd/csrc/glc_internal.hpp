@@ -320,9 +320,24 @@ struct HostWords {
     HostWords& operator=(const HostWords&) = delete;
 };
 
+// Device scratch kept between calls and shared by them.  mu is held while one
+// call's kernels on it are being launched; `last` is recorded after its last one, so
+// that the next call's stream waits on the device, while the first call goes on
+// without the lock.
+struct SharedScratch {
+    std::mutex mu;
+    void* p = nullptr;
+    int64_t bytes = 0;
+    hipEvent_t last = nullptr;
+};
+// with mu held: s waits for the last call's kernels; p has at least `bytes`
+int scratch_acquire(SharedScratch& sc, int64_t bytes, hipStream_t s);
+// with mu held, after the call's last launch on it; above `keep` bytes it is given back
+int scratch_release(SharedScratch& sc, int64_t keep, hipStream_t s);
+
 // GPU split/merge partitioner (glc_splitmerge.hip).  The boundaries stay in the
-// device's scratch: d_st, d_en [P], valid while `lock` is held and the work that
-// reads them is waited for before it is released; first_len is partition 0's length.
+// device's scratch: d_st, d_en [P], valid while `lock` is held and for what is
+// launched meanwhile; first_len is partition 0's length.
 struct SplitMergeResult {
     const int32_t* d_st = nullptr;
     const int32_t* d_en = nullptr;
@@ -331,8 +346,8 @@ struct SplitMergeResult {
     int device = 0;
     std::unique_lock<std::mutex> lock;
 };
-// once the stream has been waited for
-void split_merge_release(SplitMergeResult& r);
+// once what reads the boundaries has been launched on s
+int split_merge_release(SplitMergeResult& r, hipStream_t s);
 int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t min_size, SplitMergeResult* out, hipStream_t s);
 // host-side CPU partitioner (glc_host.cpp)
 int cpu_split_merge(int dtype, const void* h_values, int64_t n, int32_t min_size, std::vector<int32_t>& st,

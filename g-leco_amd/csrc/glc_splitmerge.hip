@@ -1537,20 +1537,15 @@ unsigned blocks(int64_t n, int b) { return static_cast<unsigned>((n + b - 1) / b
 // when a larger column needs more (a per-call hipMalloc/hipFree pair costs
 // hundreds of microseconds and the free synchronises the device).  Held
 // until the process ends; one above kSmKeep bytes (a column of about 2^28 values
-// at minimum size 128) is given back by split_merge_release.  The lock covers a call and its caller's copy of the boundaries, after
-// which the stream has been waited for.
+// at minimum size 128) is given back by split_merge_release.  The lock covers a call
+// and the launch of its caller's copy of the boundaries.
 constexpr int64_t kSmKeep = int64_t(1) << 30;
-struct SmScratch {
-    std::mutex mu;
-    void* p = nullptr;
-    int64_t bytes = 0;
-};
-SmScratch& sm_scratch(int device) {
+SharedScratch& sm_scratch(int device) {
     static std::mutex table_mu;
-    static std::map<int, SmScratch*>* table = new std::map<int, SmScratch*>();  // never freed: used until exit
+    static std::map<int, SharedScratch*>* table = new std::map<int, SharedScratch*>();  // never freed: used until exit
     std::lock_guard<std::mutex> g(table_mu);
-    SmScratch*& e = (*table)[device];
-    if (!e) e = new SmScratch();
+    SharedScratch*& e = (*table)[device];
+    if (!e) e = new SharedScratch();
     return *e;
 }
 
@@ -1592,20 +1587,10 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, Split
     GLC_HIP(hipGetDevice(&dev));
     HostWords host;
     if (!host.p) return fail(GLC_ERR_OOM, "pinned host allocation failed");
-    SmScratch& sc = sm_scratch(dev);
+    SharedScratch& sc = sm_scratch(dev);
     std::unique_lock<std::mutex> scratch_lock(sc.mu);
-    if (sc.bytes < bytes) {
-        if (sc.p) (void)hipFree(sc.p);  // the previous call ended synchronised
-        sc.p = nullptr;
-        sc.bytes = 0;
-        const int64_t want = align_up(bytes + bytes / 4, 1 << 20);
-        if (hipMalloc(&sc.p, static_cast<size_t>(want)) != hipSuccess) {
-            (void)hipGetLastError();
-            sc.p = nullptr;
-            return fail(GLC_ERR_OOM, "split/merge scratch allocation failed");
-        }
-        sc.bytes = want;
-    }
+    const int ac = scratch_acquire(sc, bytes, s);
+    if (ac) return ac;
     char* p = static_cast<char*>(sc.p);
     auto I = [&](int k) { return reinterpret_cast<int32_t*>(p + k * i4); };
     auto D = [&](int k) { return reinterpret_cast<double*>(p + 9 * i4 + k * d8); };
@@ -1728,15 +1713,10 @@ int gpu_split_merge(int dtype, const void* d_values, int64_t n, int32_t m, Split
     return GLC_OK;
 }
 
-void split_merge_release(SplitMergeResult& r) {
-    if (!r.lock.owns_lock()) return;
-    SmScratch& sc = sm_scratch(r.device);
-    if (sc.bytes > kSmKeep) {
-        (void)hipFree(sc.p);
-        sc.p = nullptr;
-        sc.bytes = 0;
-    }
-    r.lock.unlock();
+int split_merge_release(SplitMergeResult& r, hipStream_t s) {
+    const int rc = scratch_release(sm_scratch(r.device), kSmKeep, s);
+    if (!rc) r.lock.unlock();
+    return rc;
 }
 
 }  // namespace glc
