@@ -70,8 +70,8 @@ def decode_traffic(workload: str, sched: int):
 DECODER_KERNEL = {
     "worksteal": "{K} (GLC_FULL_WORKSTEAL: wave tiles handed to CUs by the hardware workgroup dispatcher)",
     "bitpacked": "{K} (GLC_FULL_BITPACKED)",
-    "v2": "k_decode_parts<persistent=false> (GLC_FULL_V2: one workgroup per partition)",
-    "worksteal_adv": "k_decode_parts<persistent=true> (GLC_FULL_WORKSTEAL_ADV: workgroups claim partitions from a counter)",
+    "v2": "{K} (GLC_FULL_V2)",
+    "worksteal_adv": "{K} (GLC_FULL_WORKSTEAL_ADV)",
 }
 
 
@@ -1049,8 +1049,7 @@ def main():
         "compress_ms": round(compress_ms_steady, 2), "compress_ms_first_call": round(compress_ms, 2),
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic, "traffic_source": traffic_src,
-                     "kernel": (SCHEDULE_KERNEL[sched].format(T="uint64") if args.mode in ("worksteal", "bitpacked")
-                                else DECODER_KERNEL[args.mode].split(" (")[0]),
+                     "kernel": SCHEDULE_KERNEL[sched].format(T="uint64"),
                      "algorithmic_bytes": alg_bytes},
         "cpu_baseline": cpu,
     }

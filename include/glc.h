@@ -164,8 +164,12 @@ int glc_decompress_full(const glc_column* col, void* d_out, int mode, void* stre
  * grouped into workgroups.  It changes only the time, never the output.
  * Which is fastest depends on the column (its length, widths, element
  * size); glc_column_autotune_decode measures it.  Default: TILE_W4; until a
- * schedule or pace is set, the library may launch 64-bit columns in half
- * tiles, paced, where that is the faster grouping for the column's layout. */
+ * schedule or pace is set, the library launches another grouping where that is
+ * the faster one for the column's layout and the output's alignment (half tiles,
+ * paced for wide timestamps; TILE_W1 for outputs that are not 16-byte aligned).
+ * get returns what was set or tuned, TILE_W4 before; to set that value ends the
+ * library's choice.  HALF_TILE_W1 is for 16-byte aligned outputs; others take
+ * TILE_W1 under it. */
 enum {
     GLC_DECODE_TILE_W1 = 0,      /* one 1024-value tile per one-wave workgroup */
     GLC_DECODE_TILE_W4 = 1,      /* four consecutive tiles per four-wave workgroup */
